@@ -53,7 +53,7 @@ extern "C" {
 #define MI355X_FP8_VARIANT_TILED   1  /* LDS-tiled persistent MFMA kernel (compute-bound shapes) */
 #define MI355X_FP8_VARIANT_SKINNY  2  /* kernels that own all of K per workgroup and stream B (HBM-bound): M <= 64, \
                                          and M <= 256 where the narrow-tile form below fits */
-#define MI355X_FP8_VARIANT_GENERIC 3  /* byte loads and f32 multiply-adds, no requirement on K, the leading dimensions or \
+#define MI355X_FP8_VARIANT_GENERIC 3  /* unaligned loads and 16-bit MFMA, no requirement on K, the leading dimensions or \
                                          the alignment of a and b: what AUTO runs for operands the two MFMA families   \
                                          cannot take (a few TFLOP/s) */
 

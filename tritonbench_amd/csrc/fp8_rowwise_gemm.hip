@@ -23,7 +23,8 @@
 //   gemm_narrow_kernel       M <= 64 (M <= 256 in row blocks), K in 512-byte steps, at most one tile of
 //                            up to 64 columns per CU: a workgroup owns all of K (no split, no second
 //                            launch); separate waves fetch A and B.
-//   gemm_generic_kernel      any K, leading dimension and alignment: byte loads, f32 multiply-adds.
+//   gemm_any_kernel          any K, leading dimension and alignment (more than 64 rows; up to 64 the skinny
+//                            kernel has a form for them): unaligned loads, binary16 MFMA on the widened codes.
 //   quantize_rows_*_kernel   row-wise e4m3fn quantiser (amax, scale, convert), one row per workgroup.
 //   quantize_blocks_kernel   128 x 128 block-wise e4m3fn quantiser, one block per workgroup.
 //   fused_rowwise_quant_kernel  RMSNorm or SiLU-mul of bf16 rows followed by the same quantiser, one pass.
@@ -1183,66 +1184,208 @@ __global__ __launch_bounds__(256) void splitk_finalize_kernel(GemmParams p) {
 }
 
 // ------------------------------------------------------------------------------------
-// Generic kernel: operands the other families cannot take (K, lda or ldb not a multiple of 16,
-// A or B not 16-byte aligned, leading dimensions beyond a buffer descriptor's range). Byte loads,
-// codes widened to f32 in LDS, f32 multiply-adds (the product of two e4m3fn values is exact in
-// f32), 64x64 tile per workgroup, 4x4 outputs per lane. A few TFLOP/s: a correct answer for
-// odd shapes, not a fast one. Same epilogue arithmetic as the other kernels.
+// Generic kernels: operands the other families cannot take (K, lda or ldb not a multiple of 16,
+// A or B not 16-byte aligned, leading dimensions beyond a buffer descriptor's range). Rows start at
+// any byte, so a lane's 16 bytes are an unaligned load (one instruction on this chip; the pieces of a
+// row lie across two cache lines more often than not), and the last chunk of a row is put
+// together byte by byte: nothing outside a row's K bytes is ever read.
+//
+// The products run on the 16-bit matrix instructions with the codes widened to binary16, which is
+// exact (e4m3fn reaches from 2^-9 to 448), and f32 accumulation that is as accurate as a chain of f32
+// multiply-adds (measured over K = 1024 standard normal codes: 4e-8 of the result's norm for both,
+// 1.5e-5 for the fp8 matrix instructions, which align a group of products before they add). One
+// conversion instruction widens two codes, and the conversions are what bounds the large tiles (a
+// 128x128 tile runs at 0.39 of the 16-bit matrix rate). Against byte loads and f32 multiply-adds on the
+// vector ALU, which this family was before: 517x3000x1041 212 -> 12.7 us.
 // ------------------------------------------------------------------------------------
-__device__ __forceinline__ float e4m3fn_to_f32(uint8_t code) {
-  const uint32_t mag = code & 0x7fu;
-  // the 7 magnitude bits placed at an f32's exponent/mantissa boundary are the value times 2^-120
-  // (subnormal codes become subnormal floats, which the multiply takes as they are)
-  float v = __uint_as_float(mag << 20) * 0x1p120f;
-  if (mag == 0x7fu) v = __uint_as_float(0x7fc00000u);
-  return (code & 0x80u) ? -v : v;
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+
+// bytes [k, k + 16) of a row of K bytes; those at or past K count as zero
+__device__ __forceinline__ v4i load16_any(const uint8_t* row, int k, int K) {
+  if (k + kChunk <= K) return *(const v4i_any*)(row + k);
+  uint64_t lo = 0, hi = 0;
+  if (K >= kChunk) {  // the row's last 16 bytes, moved down to where the chunk wants them
+    if (k < K) {
+      const v4i x = *(const v4i_any*)(row + K - kChunk);
+      lo = (uint32_t)x[0] | ((uint64_t)(uint32_t)x[1] << 32);
+      hi = (uint32_t)x[2] | ((uint64_t)(uint32_t)x[3] << 32);
+      const int n = 8 * (k + kChunk - K);  // 8 .. 120
+      lo = n < 64 ? (lo >> n) | (hi << (64 - n)) : hi >> (n & 63);
+      hi = n < 64 ? hi >> n : 0;
+    }
+  } else {
+    for (int e = 0; e < kChunk; ++e)
+      if (k + e < K) (e < 8 ? lo : hi) |= (uint64_t)row[k + e] << (8 * (e & 7));
+  }
+  return (v4i){(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)};
 }
 
-constexpr int kGenericTile = 64, kGenericStepK = 32;
+// eight e4m3fn codes in two registers -> binary16 (exact; NaN codes become NaN)
+__device__ __forceinline__ v8h e4m3fn_to_f16x8(int lo, int hi) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const v2h a = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, false), b = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 1.0f, true);
+  const v2h c = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, false), d = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 1.0f, true);
+  return (v8h){a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+#else
+  return (v8h){};
+#endif
+}
 
-__global__ __launch_bounds__(256) void gemm_generic_kernel(GemmParams p) {
-  __shared__ float as[kGenericStepK][kGenericTile + 1];
-  __shared__ float bs[kGenericStepK][kGenericTile + 1];
+// Generic form for more than 64 rows: BM x BN tile per workgroup of 2 x 2 waves, K in 128-byte steps.
+// Global memory -> registers (DEPTH steps ahead) -> LDS in the tiled kernel's swizzled layout, two stages,
+// one barrier per step; a fragment's codes are widened as they are read from LDS. The partial step
+// at the end of K is multiplied first, so that the loop over whole steps has no conditional loads (its wait
+// counts are then exact and DEPTH steps stay in flight).
+constexpr size_t any_lds_bytes(int BM, int BN) { return (size_t)2 * (BM + BN) * kStepK; }
+
+template <int BM, int BN, int DEPTH>
+__global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
+  constexpr int WTM = BM / 2, WTN = BN / 2, MT = WTM / 32, NT = WTN / 32;
+  constexpr int STAGE = (BM + BN) * kStepK;  // A's rows, then B's
+  constexpr int LA = BM / 32, LOADS = (BM + BN) / 32;  // chunks of A, and of both, a lane fetches per step
+  fetch_arguments_now(p);
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   const int tid = threadIdx.x;
-  const long m0 = (long)blockIdx.y * kGenericTile, n0 = (long)blockIdx.x * kGenericTile;
-  const int ld_row = tid / 4, ld_k = (tid % 4) * 8;  // the 8 bytes of one tile row a lane widens per step
-  const int ty = tid / 16, tx = tid % 16;
-  float acc[4][4] = {};
-  for (long k0 = 0; k0 < p.K; k0 += kGenericStepK) {
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1, l32 = lane & 31, half = lane >> 5;
+
+  // each XCD takes a contiguous run of the tile list (kGroupM tile rows at a time, column-major inside)
+  const TileWalk walk = make_walk(p.tiles_m * p.tiles_n);
+  if (walk.slot >= walk.chunk_len) return;
+  int tm, tn;
+  tile_coords(walk.chunk_begin + walk.slot, p.tiles_m, p.tiles_n, p.div_group_mul, p.div_group_shift, tm, tn);
+  const long m0 = (long)tm * BM, n0 = (long)tn * BN;
+
+  // lane's chunk ld_c of rows ld_row, ld_row + 32, ... (rows past an edge repeat the last one)
+  const int ld_row = tid >> 3, ld_c = tid & 7;
+  const uint8_t* row[LOADS];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const long k = k0 + ld_k + e;
-      const bool in_k = k < p.K;
-      as[ld_k + e][ld_row] = in_k && m0 + ld_row < p.M ? e4m3fn_to_f32(p.a[(size_t)(m0 + ld_row) * p.lda + k]) : 0.0f;
-      bs[ld_k + e][ld_row] = in_k && n0 + ld_row < p.N ? e4m3fn_to_f32(p.b[(size_t)(n0 + ld_row) * p.ldb + k]) : 0.0f;
-    }
-    __syncthreads();
-#pragma unroll 8
-    for (int kk = 0; kk < kGenericStepK; ++kk) {
-      float av[4], bv[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = as[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bv[j] = bs[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(av[i], bv[j], acc[i][j]);
-    }
-    __syncthreads();
+  for (int i = 0; i < LOADS; ++i) {
+    const int r = ld_row + 32 * (i < LA ? i : i - LA);
+    row[i] = i < LA ? p.a + (size_t)min(m0 + r, (long)p.M - 1) * p.lda : p.b + (size_t)min(n0 + r, (long)p.N - 1) * p.ldb;
   }
+  const int park_pos = ld_row * kStepK + ((ld_c ^ swz128(ld_row)) * kChunk);  // (32 rows on: the same swizzle)
+  auto park = [&](const v4i (&from)[LOADS], int stage) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const long m = m0 + ty * 4 + i;
-    if (m >= p.M) continue;
-    const float sa_m = p.a_scale[m];
+    for (int i = 0; i < LOADS; ++i) *(v4i*)(lds + stage * STAGE + i * 32 * kStepK + park_pos) = from[i];
+  };
+  auto join = [&]() {  // this wave's LDS accesses are done, then everyone's; global loads stay in flight
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+  };
+
+  v16f acc[MT][NT];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const long n = n0 + tx * 4 + j;
-      if (n >= p.N) continue;
-      const float t = acc[i][j] * sa_m;
-      const float r = p.bias ? __builtin_fmaf(t, p.b_scale[n], bf16_to_f32(p.bias[n])) : t * p.b_scale[n];
-      p.c[(size_t)m * p.ldc + n] = (uint16_t)pack_out_x2(r, 0.0f, p.out_f16);
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = (v16f){0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int stage) {
+    const uint8_t* rows_a = lds + stage * STAGE + (wm * WTM + l32) * kStepK;
+    const uint8_t* rows_b = lds + stage * STAGE + (BM + wn * WTN + l32) * kStepK;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {  // lane half h multiplies chunk 2c + h of its row: 8 codes per instruction
+      const int off = ((2 * c + half) ^ swz128(l32)) * kChunk;
+      v8h fa[MT][2], fb[NT][2];
+#pragma unroll
+      for (int i = 0; i < MT; ++i) {
+        const v4i x = *(const v4i*)(rows_a + i * 32 * kStepK + off);
+        fa[i][0] = e4m3fn_to_f16x8(x[0], x[1]);
+        fa[i][1] = e4m3fn_to_f16x8(x[2], x[3]);
+      }
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const v4i x = *(const v4i*)(rows_b + j * 32 * kStepK + off);
+        fb[j][0] = e4m3fn_to_f16x8(x[0], x[1]);
+        fb[j][1] = e4m3fn_to_f16x8(x[2], x[3]);
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[j][u], fa[i][u], acc[i][j], 0, 0, 0);
+    }
+  };
+
+  const int full = p.K / kStepK;
+  v4i land[DEPTH][LOADS];
+  auto fetch = [&](v4i (&to)[LOADS], int s) {  // past the last whole step: that one again, for nobody
+    const int k = min(s, full - 1) * kStepK + ld_c * kChunk;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) to[i] = *(const v4i_any*)(row[i] + k);
+  };
+  if (full > 0)
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) fetch(land[d], d);
+  if (full * kStepK < p.K) {
+    v4i tail[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) tail[i] = load16_any(row[i], full * kStepK + ld_c * kChunk, p.K);
+    park(tail, 1);
+    join();
+    multiply(1);
+  }
+  if (full > 0) {
+    // step s on the stage it was parked in; its registers take step s + DEPTH, the other stage step s + 1
+    auto step = [&](int d, int s) {
+      fetch(land[d], s + DEPTH);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(s & 1);
+      park(land[(d + 1) % DEPTH], (s + 1) & 1);
+      join();
+    };
+    park(land[0], 0);
+    join();
+    int s = 0;
+    for (; s + DEPTH <= full; s += DEPTH)
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) step(d, s + d);
+#pragma unroll
+    for (int d = 0; d < DEPTH - 1; ++d)
+      if (s + d < full) step(d, s + d);
+  }
+
+  // lane (l32, half): row l32 of every 32x32 block, columns 8q + 4*half + 0..3
+  const bool vec = ((p.ldc & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.c) & 7) == 0);
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    float sb[4][4], bias[4][4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const long ne = min(n0 + wn * WTN + j * 32 + 8 * q + 4 * half + e, (long)p.N - 1);
+        sb[q][e] = p.b_scale[ne];
+        bias[q][e] = p.bias ? bf16_to_f32(p.bias[ne]) : 0.0f;
+      }
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const long m = m0 + wm * WTM + i * 32 + l32;
+      if (m >= p.M) continue;
+      const float sa_m = p.a_scale[m];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const long n = n0 + wn * WTN + j * 32 + 8 * q + 4 * half;
+        float r[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float t = acc[i][j][4 * q + e] * sa_m;
+          r[e] = p.bias ? __builtin_fmaf(t, sb[q][e], bias[q][e]) : t * sb[q][e];
+        }
+        const uint32_t lo = pack_out_x2(r[0], r[1], p.out_f16), hi = pack_out_x2(r[2], r[3], p.out_f16);
+        uint16_t* dst = p.c + (size_t)m * p.ldc + n;
+        if (vec && n + 3 < p.N) {
+          *(v2u*)dst = (v2u){lo, hi};
+        } else {
+          if (n < p.N) dst[0] = (uint16_t)lo;
+          if (n + 1 < p.N) dst[1] = (uint16_t)(lo >> 16);
+          if (n + 2 < p.N) dst[2] = (uint16_t)hi;
+          if (n + 3 < p.N) dst[3] = (uint16_t)(hi >> 16);
+        }
+      }
     }
   }
 }
@@ -1261,8 +1404,11 @@ __global__ __launch_bounds__(256) void gemm_generic_kernel(GemmParams p) {
 // operations in order, so the loop needs no barrier. A [16*MT rows] takes the same route.
 // Partial 16x16 results are summed across the waves through LDS at the end.
 // ------------------------------------------------------------------------------------
-template <int MT, int NTW, int DEPTH, int KW>
+// ANY: the generic family's form for up to 64 rows: unaligned loads, 16-bit matrix instructions on the
+// widened codes, any K (see the generic kernels above).
+template <int MT, int NTW, int DEPTH, int KW, bool ANY = false>
 __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
+  using Chunk = std::conditional_t<ANY, v4i_any, v4i>;
   constexpr int TILE = 16 * kStepK;                 // one 16-row operand tile of one step: 2 KB
   constexpr int NTILE = NTW + MT;                   // tiles per step: B tiles then A tiles
   constexpr int BUF = NTILE * TILE;                 // wave-private transpose buffer
@@ -1334,28 +1480,51 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
     for (int t = 0; t < NTILE; ++t)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        // B is read once and never again: stream it past the caches; A is shared by everyone
-        if (t < NTW) dst[t][h] = __builtin_nontemporal_load((const v4i*)(src[t][h] + kb));
-        else dst[t][h] = *(const v4i*)(src[t][h] + kb);
+        // B is read once and never again: stream it past the caches; A is shared by everyone. (ANY: an
+        // unaligned piece shares its lines with the neighbouring steps, which the streaming policy would
+        // fetch again: 1x8192x8191 19.6 -> 14.4 us without it, 16x8192x8191 25.6 -> 19.1.)
+        if (t < NTW && !ANY) dst[t][h] = __builtin_nontemporal_load((const Chunk*)(src[t][h] + kb));
+        else dst[t][h] = *(const Chunk*)(src[t][h] + kb);
       }
+  };
+  // one step's products; ANY: a lane's 32 codes of a row are four 16-bit instructions of 8 codes per lane
+  auto multiply = [&](const v8i (&bf)[NTW], const v8i (&af)[MT]) {
+    if constexpr (ANY) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        v8h hb[NTW], ha[MT];
+#pragma unroll
+        for (int t = 0; t < NTW; ++t) hb[t] = e4m3fn_to_f16x8(bf[t][2 * q], bf[t][2 * q + 1]);
+#pragma unroll
+        for (int u = 0; u < MT; ++u) ha[u] = e4m3fn_to_f16x8(af[u][2 * q], af[u][2 * q + 1]);
+#pragma unroll
+        for (int t = 0; t < NTW; ++t)
+#pragma unroll
+          for (int u = 0; u < MT; ++u) acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hb[t], ha[u], acc[t][u], 0, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < NTW; ++t)
+#pragma unroll
+        for (int u = 0; u < MT; ++u)
+          acc[t][u] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf[t], af[u], acc[t][u], 0, 0, 0, 0, 0, 0);
+    }
   };
   auto consume = [&](const v4i (&got)[NTILE][2]) {
 #pragma unroll
     for (int t = 0; t < NTILE; ++t)
 #pragma unroll
       for (int h = 0; h < 2; ++h) *(v4i*)(buf + t * TILE + wr_off[h]) = got[t][h];
-    v8i f[NTILE];
+    v8i bf[NTW], af[MT];
 #pragma unroll
     for (int t = 0; t < NTILE; ++t) {
       const v4i lo = *(const v4i*)(buf + t * TILE + rd0);
       const v4i hi = *(const v4i*)(buf + t * TILE + rd1);
-      f[t] = (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      const v8i f = (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      if (t < NTW) bf[t] = f;
+      else af[t - NTW] = f;
     }
-#pragma unroll
-    for (int t = 0; t < NTW; ++t)
-#pragma unroll
-      for (int u = 0; u < MT; ++u)
-        acc[t][u] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(f[t], f[NTW + u], acc[t][u], 0, 0, 0, 0, 0, 0);
+    multiply(bf, af);
   };
 
   // The loop is unrolled DEPTH times so every register set has a fixed name; the compiler's
@@ -1399,31 +1568,27 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
     }
   }
   // K tail (K % 128 != 0): one partial step, taken by the wave whose turn it would be; the
-  // lanes fetch their own 16-byte chunks and chunks at or past K count as zero
+  // lanes fetch their own 16-byte chunks and chunks (ANY: bytes) at or past K count as zero
   if (k_tail && (k_full % KW) == wave) {
-    const size_t kb = (size_t)k_full * kStepK;
-    const bool in0 = (2 * g4) * kChunk < k_tail, in1 = (2 * g4 + 1) * kChunk < k_tail;
-    const v4i z = {0, 0, 0, 0};
+    const int kb = k_full * kStepK;
+    auto chunk_of = [&](const uint8_t* row, int c) -> v4i {
+      if constexpr (ANY) return load16_any(row, kb + c * kChunk, p.K);
+      return c * kChunk < k_tail ? *(const v4i*)(row + kb + c * kChunk) : (v4i){0, 0, 0, 0};
+    };
     v8i bf[NTW], af[MT];
 #pragma unroll
     for (int t = 0; t < NTW; ++t) {
-      const uint8_t* row = p.b + (size_t)min(n0 + t * 16 + r16, p.N - 1) * p.ldb + kb;
-      const v4i lo = in0 ? *(const v4i*)(row + 2 * g4 * kChunk) : z;
-      const v4i hi = in1 ? *(const v4i*)(row + (2 * g4 + 1) * kChunk) : z;
+      const uint8_t* row = p.b + (size_t)min(n0 + t * 16 + r16, p.N - 1) * p.ldb;
+      const v4i lo = chunk_of(row, 2 * g4), hi = chunk_of(row, 2 * g4 + 1);
       bf[t] = (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     }
 #pragma unroll
     for (int u = 0; u < MT; ++u) {
-      const uint8_t* row = p.a + (size_t)min(u * 16 + r16, p.M - 1) * p.lda + kb;
-      const v4i lo = in0 ? *(const v4i*)(row + 2 * g4 * kChunk) : z;
-      const v4i hi = in1 ? *(const v4i*)(row + (2 * g4 + 1) * kChunk) : z;
+      const uint8_t* row = p.a + (size_t)min(u * 16 + r16, p.M - 1) * p.lda;
+      const v4i lo = chunk_of(row, 2 * g4), hi = chunk_of(row, 2 * g4 + 1);
       af[u] = (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     }
-#pragma unroll
-    for (int t = 0; t < NTW; ++t)
-#pragma unroll
-      for (int u = 0; u < MT; ++u)
-        acc[t][u] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf[t], af[u], acc[t][u], 0, 0, 0, 0, 0, 0);
+    multiply(bf, af);
   }
 
   // ---- cross-wave reduction through each wave's own (now idle) buffer
@@ -3179,11 +3344,11 @@ MI355X_DEFINE_TILED_PART(6, 128, 128, 2, 2, false, true)  // (never with the str
 
 #if !defined(MI355X_TILED_PART)  // (everything from here on belongs to the main unit)
 namespace {
-template <int MT, int NTW, int DEPTH, int KW>
+template <int MT, int NTW, int DEPTH, int KW, bool ANY = false>
 int launch_skinny(const GemmParams& p, hipStream_t stream) {
   constexpr size_t lds_bytes = (size_t)KW * (NTW + MT) * 16 * kStepK;
   static_assert(lds_bytes <= 160 * 1024, "transpose buffers must fit the 160 KB LDS");
-  constexpr auto kern = gemm_skinny_kernel<MT, NTW, DEPTH, KW>;
+  constexpr auto kern = gemm_skinny_kernel<MT, NTW, DEPTH, KW, ANY>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   if (const int st = ready_device()) return st;
   const unsigned grid = (unsigned)((p.N + 16 * NTW - 1) / (16 * NTW));
@@ -3191,6 +3356,40 @@ int launch_skinny(const GemmParams& p, hipStream_t stream) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "skinny kernel launch: %s", hipGetErrorString(e));
   return MI355X_FP8_OK;
+}
+
+template <int BM, int BN, int DEPTH>
+int launch_any(GemmParams p, hipStream_t stream) {
+  constexpr size_t lds_bytes = any_lds_bytes(BM, BN);
+  constexpr auto kern = gemm_any_kernel<BM, BN, DEPTH>;
+  (void)LdsLimit<kern, lds_bytes>::registered;
+  p.tiles_m = (p.M + BM - 1) / BM;
+  p.tiles_n = (p.N + BN - 1) / BN;
+  const long tiles = (long)p.tiles_m * p.tiles_n;
+  if (tiles > (long)INT32_MAX - kNumXcd || (long)kGroupM * p.tiles_n > (long)INT32_MAX)
+    return fail(MI355X_FP8_ENOTSUP, "more than 2^31-1 tiles");
+  make_fast_div((uint32_t)kGroupM * (uint32_t)p.tiles_n, p.div_group_mul, p.div_group_shift);
+  if (const int st = ready_device()) return st;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((tiles + kNumXcd - 1) / kNumXcd * kNumXcd)), dim3(256), lds_bytes, stream, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "generic kernel launch: %s", hipGetErrorString(e));
+  return MI355X_FP8_OK;
+}
+
+// The generic family: the streaming kernel's unaligned form up to 64 rows (measured cold: 1x8192x8191 14.4 us,
+// 16x8192x8191 19.1, 64x8192x8191 29.7, where 64x64 tiles take 33), tiles beyond. 128x128 tiles from two
+// rounds of the CUs on (4096x8192x8191 563 us = 977 TFLOP/s); below, 64x64 tiles. With at most one of
+// those per CU nothing but its own loads covers a step's latency, and they run two steps ahead
+// (128x8192x8191 61.7 -> 36.7 us, 256x4096x4097 27.9 -> 19.6); with more, the CU's other workgroups do, and
+// the second step's registers would cost one of them (517x3000x1041 13.9 -> 12.7, 1024x2048x1025 13.7 -> 12.5).
+int launch_generic(const GemmParams& p, hipStream_t s) {
+  if (p.M > 65535 * 64) return fail(MI355X_FP8_ENOTSUP, "the generic family takes M <= %d", 65535 * 64);
+  if (p.M <= 16) return launch_skinny<1, 1, 4, 8, true>(p, s);
+  if (p.M <= 32) return launch_skinny<2, 1, 2, 8, true>(p, s);
+  if (p.M <= 64) return launch_skinny<4, 2, 2, 8, true>(p, s);
+  auto tiles = [&](long edge) { return ((p.M + edge - 1) / edge) * ((p.N + edge - 1) / edge); };
+  if (tiles(128) >= 2 * kNumCu) return launch_any<128, 128, 1>(p, s);
+  return tiles(64) <= kNumCu ? launch_any<64, 64, 2>(p, s) : launch_any<64, 64, 1>(p, s);
 }
 
 // ---- built-in scratch of the entry point that allocates nothing
@@ -3538,15 +3737,8 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
       if (M <= 32) return launch_skinny<2, 1, 2, 8>(p, s);
       if (M <= 48) return launch_skinny<3, 1, 2, 8>(p, s);
       return launch_skinny<4, 2, 2, 8>(p, s);  // 32 rows of B per workgroup: A passes L1 half as often
-    case MI355X_FP8_VARIANT_GENERIC: {
-      if (const int gs = ready_device()) return gs;
-      const dim3 grid((unsigned)((N + kGenericTile - 1) / kGenericTile), (unsigned)((M + kGenericTile - 1) / kGenericTile));
-      if (grid.y > 65535) return fail(MI355X_FP8_ENOTSUP, "the generic family takes M <= %d", 65535 * kGenericTile);
-      hipLaunchKernelGGL(gemm_generic_kernel, grid, dim3(256), 0, s, p);
-      const hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "generic kernel launch: %s", hipGetErrorString(e));
-      return MI355X_FP8_OK;
-    }
+    case MI355X_FP8_VARIANT_GENERIC:
+      return launch_generic(p, s);
     default:
       return fail(MI355X_FP8_EINVAL, "unknown variant %d", variant);
   }
