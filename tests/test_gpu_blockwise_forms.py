@@ -1,0 +1,59 @@
+"""The forms of the block-scaled GEMM at the edges of their tiles, K blocks and dispatch, against
+float64. Needs an MI355X."""
+import pytest
+import torch
+
+from tritonbench_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _expand(codes, scales):
+    s = scales.double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+    return codes.double() * s[: codes.shape[0], : codes.shape[1]]
+
+
+def _check(m, n, k, dev, seed=0):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    gk = -(-k // 128)
+    xq = torch.randn((m, k), generator=g, device=dev).to(torch.float8_e4m3fn)
+    wq = torch.randn((n, k), generator=g, device=dev).to(torch.float8_e4m3fn)
+    # factors over eight binades, so that a product added with a neighbour's factor would show; one block of
+    # zeros with a factor of zero
+    xs = torch.exp2(torch.rand((-(-m // 128), gk), generator=g, device=dev) * 8 - 4)
+    ws = torch.exp2(torch.rand((-(-n // 128), gk), generator=g, device=dev) * 8 - 4)
+    if gk > 2:
+        wq[:128, 128:256] = 0
+        ws[0, 1] = 0.0
+    canvas = torch.full((m + 2, n + 8), 7.0, dtype=torch.bfloat16, device=dev)
+    aligned = n % 8 == 0
+    out = canvas[1:-1, :n] if aligned else canvas[1:-1, 3 : n + 3]
+    ops.fp8_gemm_blockwise(xq, wq, xs, ws, out=out)
+    torch.cuda.synchronize()
+    a, b = _expand(xq, xs), _expand(wq, ws)
+    exact = a @ b.t()
+    # One rounding to bf16; f32 sums of k products with two roundings of scale per block of 128; and the fp8 matrix
+    # instruction's own sum of 64 products, which aligns them to the largest before it adds: over 300k such sums it
+    # was off by up to 2^-11.9 of the largest product (two instructions per block; the largest product is at most
+    # the product of the rows' largest elements).
+    ulp = torch.exp2(torch.floor(torch.log2(exact.abs().clamp(min=2.0**-126))) - 7)
+    slack = (a.abs() @ b.abs().t()) * (k + 4 * gk + 8) * 2.0**-24
+    largest = [torch.nn.functional.pad(t.abs(), (0, gk * 128 - k)).view(-1, gk, 128).amax(2) for t in (a, b)]
+    slack += (largest[0] @ largest[1].t()) * 2 * 2.0**-11.5
+    excess = ((out.double() - exact).abs() - ulp - slack).max().item()
+    assert excess <= 0, f"{m}x{n}x{k}: {excess} beyond the bound"
+    rel = ((out.double() - exact).norm() / exact.norm()).item()
+    assert rel < 4e-3, f"{m}x{n}x{k}: relative error {rel} (rounding alone: 1.7e-3)"
+    guard = canvas.clone()
+    guard[1:-1, (slice(0, n) if aligned else slice(3, n + 3))] = 7.0
+    assert (guard == 7.0).all()
+
+
+# 256x256 tiles of two alternating groups of waves: one step, two, three (the depth of the ring of B), a partial last step,
+# ragged rows and columns (also less than a wave's share of a tile), stores element by element, several tiles per
+# workgroup and a last round that reaches few of them
+@pytest.mark.parametrize("m,n,k", [(4096, 4096, 96), (4100, 4090, 144), (4350, 4100, 384), (3000, 5000, 3008), (6000, 3000, 528),
+                                   (4097, 13313, 640), (8200, 4104, 1040)])
+def test_large_tiles_against_float64(gpu_device, m, n, k):
+    print(f"case m={m} n={n} k={k}", flush=True)
+    _check(m, n, k, gpu_device)

@@ -317,6 +317,13 @@ __device__ __forceinline__ void wait_loads_and_barrier() {
   __builtin_amdgcn_s_barrier();
 }
 
+// waits until at most VM of this wave's global loads are outstanding (LDS operations are not waited for)
+template <int VM>
+__device__ __forceinline__ void wait_loads() {
+  constexpr int imm = (VM & 15) | ((VM >> 4) << 14) | (7 << 4) | (15 << 8);
+  __builtin_amdgcn_s_waitcnt(imm);
+}
+
 // Cursor over the (tile, K step) sequence a workgroup walks; one for the A loads, one for
 // the B loads (which run a step further ahead).
 struct StepCursor {
@@ -1130,6 +1137,290 @@ void gemm_tiled_kernel(GemmParams p) {
   }
 }
 
+// ------------------------------------------------------------------------------------
+// Block-scaled kernel for shapes that fill the chip with 256x256 tiles: two groups of four waves take turns.
+//
+// The accumulators are kept in units of the current K block's factor (see the tiled kernel's BLOCKSCALE
+// form): one multiply per accumulator and step on the vector ALU, which reaches accumulators in
+// ordinary registers only. A 256x256 tile therefore needs eight waves (128x64 each: 128 accumulators), two per
+// SIMD. Each wave alternates between a memory phase (all of a step's operand fragments from LDS, the
+// rescaling) and a matrix phase (the step's 16 MFMAs); waves 4..7 run one phase behind waves 0..3, and
+// a SIMD hosts one wave of either group, so one of its waves feeds the matrix pipe while the other one
+// reads and rescales. A barrier ends every phase.
+//
+//   phase 2k      waves 0..3: memory(k)    waves 4..7: matrix(k-1)     everyone loads A(k+1)
+//   phase 2k + 1  waves 0..3: matrix(k)    waves 4..7: memory(k)       everyone loads B(k+2), then waits for
+//                                                                       its own loads of A(k+1) and B(k+1)
+//
+// LDS: two stages of A, three of B (32 KB each), as in the plain 256x256 tile. B(k+2) goes where B(k-1) was,
+// last read in phase 2k-1; A(k+1) where A(k-1) was, last read in the same phase.
+//
+// What bounds it: 8192^3 416 us (2.64 PFLOP/s), with the rescaling taken out 366, which is what the plain 256x256 tile
+// takes; the 128x128 form 542. The eight waves read 192 KB of fragments from LDS per step (four waves of
+// 128x128 would read 128, but have no registers the multiplies can reach), beside the 64 KB that arrive there.
+// Measured on the way: the same waves in step with each other (the tiled kernel's schedule) 464-470 us; this one with
+// the cursors' scalar work in the memory phase 430; all 128 multiplies in the memory phase 426, all behind the
+// MFMAs 447; the loads in front of the fragment reads instead of behind them 427.
+// ------------------------------------------------------------------------------------
+constexpr int kBlockTile = 256, kBlockWaves = 8;
+constexpr size_t kBlockLdsBytes = tiled_lds_bytes(kBlockTile, kBlockTile);
+
+template <bool KTAIL>
+__global__ __launch_bounds__(kBlockWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void gemm_block_kernel(GemmParams p) {
+  constexpr int BT = kBlockTile, NW = kBlockWaves, MT = 4, NT = 2;  // wave tile: 4 x 2 blocks of 32x32
+  constexpr int STAGE = BT * kStepK;
+  constexpr int LDS_B0 = 2 * STAGE;
+  constexpr int GROUPS = BT / 8 / NW;  // 8-row groups of A, and of B, a wave fetches per step
+  fetch_arguments_now(p);
+  fetch_tiled_arguments_now(p);
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool lead = wave < NW / 2;         // waves 0..3
+  const int wm = (wave >> 1) & 1, wn = (wave & 1) * 2 + (wave >> 2);
+  const int l32 = lane & 31, half = lane >> 5;
+
+  const TileWalk walk = make_walk(p.tiles_m * p.tiles_n);
+  if (walk.slot >= walk.chunk_len) return;  // uniform over the workgroup
+  const int k_full = p.K / kStepK, k_tail = p.K - k_full * kStepK;
+  const int k_steps = k_full + (k_tail ? 1 : 0);
+  const int total_steps = ((walk.chunk_len - walk.slot + walk.slots - 1) / walk.slots) * k_steps;
+  auto tile_of = [&](int li, int& m0, int& n0) {
+    int tm, tn;
+    tile_coords(walk.chunk_begin + li, p.tiles_m, p.tiles_n, p.div_group_mul, p.div_group_shift, tm, tn);
+    m0 = tm * BT;
+    n0 = tn * BT;
+  };
+
+  // ---- load side: one cursor per operand. `mem` is the operand a wave loads in its memory phases, `mat` the one
+  // it loads in its matrix phases: A and B for waves 0..3, the other way round for waves 4..7.
+  struct Cursor {
+    bool is_a;
+    int item, kt, issued, stage;
+    const uint8_t* base;
+    uint32_t extent, wave_off, group_stride, lane_off, lane_off_tail;
+  };
+  const int ld_row = lane >> 3, ld_pc = lane & 7;
+  const uint32_t chunk = (uint32_t)((ld_pc ^ swz128(wave * 8 + ld_row)) * kChunk);  // (a wave's groups share their parity)
+  auto enter_item = [&](Cursor& c) {
+    int m0, n0;
+    tile_of(c.item, m0, n0);
+    const int row0 = c.is_a ? m0 : n0, rows = min((c.is_a ? p.M : p.N) - row0, BT);
+    const long ld = c.is_a ? p.lda : p.ldb;
+    const uintptr_t b = reinterpret_cast<uintptr_t>(c.is_a ? p.a : p.b) + (size_t)row0 * ld;
+    c.base = reinterpret_cast<const uint8_t*>(
+        ((uintptr_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32) |
+        (uintptr_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b));
+    c.extent = (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)rows * (uint32_t)ld));
+    c.kt = 0;
+  };
+  auto make_cursor = [&](bool is_a) {
+    Cursor c;
+    c.is_a = is_a;
+    c.item = walk.slot;
+    c.issued = 0;
+    c.stage = 0;
+    const uint32_t ld = (uint32_t)(is_a ? p.lda : p.ldb);
+    c.wave_off = 8u * (uint32_t)wave * ld;
+    c.group_stride = 8u * NW * ld;
+    c.lane_off = __umul24((uint32_t)ld_row, ld) + chunk;
+    c.lane_off_tail = (int)chunk < k_tail ? c.lane_off : 0x80000000u;  // past K: outside every extent, zeros arrive
+    enter_item(c);
+    return c;
+  };
+  auto load_one = [&](const Cursor& c, int i) {
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(c.base), 0, (int)c.extent, 0x00020000);
+    uint8_t* const stage = lds + (c.is_a ? 0 : LDS_B0) + c.stage * STAGE;
+    load_chunk_to_lds<false>(rsrc, stage + (wave + NW * i) * 1024, KTAIL && c.kt >= k_full ? c.lane_off_tail : c.lane_off,
+                             (uint32_t)c.kt * kStepK + c.wave_off + (uint32_t)i * c.group_stride);
+  };
+  // past the last step the last one is fetched again, into a stage nobody reads any more
+  auto advance = [&](Cursor& c) {
+    c.stage = c.stage + 1 == (c.is_a ? 2 : 3) ? 0 : c.stage + 1;
+    if (++c.issued >= total_steps) return;
+    if (++c.kt == k_steps) {
+      c.item += walk.slots;
+      enter_item(c);
+    }
+  };
+  Cursor c_mem = make_cursor(lead), c_mat = make_cursor(!lead);
+  auto load_step = [&](Cursor& c) {
+#pragma unroll
+    for (int i = 0; i < GROUPS; ++i) load_one(c, i);
+    advance(c);
+  };
+
+  // ---- factors: one per wave and step; a factor of zero (a block of zeros) counts as 2^-60
+  typedef const __attribute__((address_space(4))) float* scalar_floats;  // scalar loads
+  scalar_floats sa_row = nullptr, sb_row = nullptr;
+  auto factor = [&](float a, float b) {
+    const float f = a * b;
+    return f == 0.0f ? 0x1p-60f : f;
+  };
+
+  v16f acc[MT][NT];
+  v4i fa[MT][4], fb[NT][4];
+  int rd[4];  // logical chunks 4*half + 0..3 of row l32
+#pragma unroll
+  for (int c = 0; c < 4; ++c) rd[c] = l32 * kStepK + (((4 * half + c) ^ swz128(l32)) * kChunk);
+  const int a_rows = wm * 128 * kStepK, b_rows = LDS_B0 + wn * 64 * kStepK;
+  int sa = 0, sb = 0;  // stages of the step being computed
+  // factor of the step whose products the accumulators are in units of, of the step after it, and their ratio
+  float s_now = 1.0f, s_next = 1.0f, ratio = 1.0f;
+
+  // A wave issues an instruction every four cycles at best, so a phase of 1024 cycles (its 16 MFMAs, or the other
+  // group's) has room for 256 instructions: the memory phase is kept to the loads, the fragment reads and as much
+  // of the rescaling as fits beside them; the last FOLD_LATE blocks are rescaled and everything scalar is done
+  // behind the MFMAs of the matrix phase.
+  constexpr int FOLD_LATE = 3, READS_PER_BLOCK = 8;
+  auto rescale = [&](int t, int v0, int v1) {
+    v16f& block = acc[t / NT][t % NT];
+#pragma unroll
+    for (int v = v0; v < v1; ++v) block[v] *= ratio;
+    asm volatile("" : "+v"(block));  // here: the compiler would sink the multiplies to the MFMAs
+  };
+  auto memory_phase = [&](auto first_tag) {
+    constexpr bool FIRST = decltype(first_tag)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    const uint8_t* rows_a = lds + sa * STAGE + a_rows;
+    const uint8_t* rows_b = lds + sb * STAGE + b_rows;
+#pragma unroll
+    for (int t = 0; t < MT * NT; ++t) {
+#pragma unroll
+      for (int u = READS_PER_BLOCK * t; u < READS_PER_BLOCK * (t + 1); ++u) {
+        const int c = u / (MT + NT), f = u % (MT + NT);
+        if (u >= 4 * (MT + NT)) continue;
+        if (f < NT) fb[f < NT ? f : 0][c] = *(const v4i*)(rows_b + f * 32 * kStepK + rd[c]);
+        else fa[f < NT ? 0 : f - NT][c] = *(const v4i*)(rows_a + (f - NT) * 32 * kStepK + rd[c]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (!FIRST && t < MT * NT - FOLD_LATE) rescale(t, 0, 16);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = 0; i < GROUPS; ++i) load_one(c_mem, i);
+    if (!lead) wait_loads<GROUPS>();
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the fragments are in registers, the stage may be written
+    __builtin_amdgcn_s_barrier();
+  };
+  auto matrix_phase = [&](auto first_tag, int kt) {
+    constexpr bool FIRST = decltype(first_tag)::value;
+    const v16f zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    auto join = [](const v4i& lo, const v4i& hi) { return (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}; };
+    float next_a = 0.f, next_b = 0.f;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < 2 * MT * NT; ++t) {
+      const int h = t / (MT * NT), i = t / NT % MT, j = t % NT;
+      acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(join(fb[j][2 * h], fb[j][2 * h + 1]), join(fa[i][2 * h], fa[i][2 * h + 1]),
+                                                                  FIRST && h == 0 ? zero : acc[i][j], 0, 0, 0, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (t == 0) {
+        const int kn = min(kt + 1, k_steps - 1);
+        next_a = sa_row[kn];
+        next_b = sb_row[kn];
+        sa = sa ^ 1;
+        sb = sb == 2 ? 0 : sb + 1;
+      }
+      if (!FIRST && FOLD_LATE && t < 2 * FOLD_LATE) rescale(MT * NT - FOLD_LATE + t / 2, 8 * (t & 1), 8 * (t & 1) + 8);
+      if (t >= 5 && t < 5 + GROUPS) load_one(c_mat, t - 5);
+      if (t == 5 + GROUPS) advance(c_mat);
+      if (t == 6 + GROUPS) advance(c_mem);
+      if (t == 13) {
+        s_now = FIRST ? s_now : s_next;
+        s_next = factor(next_a, next_b);
+        ratio = s_now / s_next;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (lead) wait_loads<GROUPS>();
+    __builtin_amdgcn_s_barrier();
+  };
+
+  // ---- epilogue: each 32-row block of the wave's tile is turned through LDS as 16-bit values, in the four
+  // 1 KB groups this wave fetches itself of the B stage the tile's last step was read from
+  auto epilogue = [&](int m0, int n0, uint8_t* table, auto vector_tag) {
+    constexpr bool VECTOR = decltype(vector_tag)::value;
+    int lane_e;  // (an opaque copy: see the tiled kernel's epilogue)
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_e));
+    const int row = lane_e & 31, hi = lane_e >> 5, rd_row = lane_e >> 3, rd_c = lane_e & 7;
+    auto at = [&](int r, int c) { return table + (wave + NW * (r >> 3)) * 1024 + (r & 7) * 128 + ((c ^ (r & 7)) * 16); };
+    const int m_wave = m0 + wm * 128, n_wave = n0 + wn * 64;
+    const uint32_t c_row_bytes = (uint32_t)p.ldc * 2u;
+    const int c_rows = __builtin_amdgcn_readfirstlane(min(max(p.M - m_wave, 0), 128));
+    const __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.c + ((size_t)m_wave * p.ldc + n_wave), 0,
+                                                                            (int)((uint32_t)c_rows * c_row_bytes), 0x00020000);
+    const int n = n_wave + rd_c * 8;
+    const uint32_t c_lane = n < p.N ? (uint32_t)rd_row * c_row_bytes + (uint32_t)rd_c * 16u : 0x80000000u;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          *(v2u*)(at(row, j * 4 + q) + hi * 8) = (v2u){pack_bf16x2(acc[i][j][4 * q] * s_now, acc[i][j][4 * q + 1] * s_now),
+                                                       pack_bf16x2(acc[i][j][4 * q + 2] * s_now, acc[i][j][4 * q + 3] * s_now)};
+      __builtin_amdgcn_sched_barrier(0);
+      v4i out[4];
+#pragma unroll
+      for (int it = 0; it < 4; ++it) out[it] = *(const v4i*)at(it * 8 + rd_row, rd_c);
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        if (VECTOR) {
+          store_chunk_streaming(out[it], c_rsrc, c_lane, (uint32_t)(i * 32 + it * 8) * c_row_bytes);
+        } else {
+          const int m = m_wave + i * 32 + it * 8 + rd_row;
+          uint16_t* dst = p.c + (size_t)m * p.ldc + n;
+          if (m < p.M) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              if (n + e < p.N) dst[e] = (uint16_t)((unsigned)out[it][e / 2] >> (16 * (e & 1)));
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  // ---- A(0) B(0) B(1) in flight; step 0 landed at the first barrier
+  if (lead) {
+    load_step(c_mem);
+    load_step(c_mat);
+    load_step(c_mat);
+  } else {
+    load_step(c_mat);
+    load_step(c_mem);
+    load_step(c_mem);
+  }
+  wait_loads<GROUPS>();
+  __builtin_amdgcn_s_barrier();
+  if (!lead) {  // the phase the second group runs behind: it loads its share of A(1) (its matrix phases' operand)
+    load_step(c_mat);
+    __builtin_amdgcn_s_barrier();
+  }
+  const bool vec = ((reinterpret_cast<uintptr_t>(p.c) | (uintptr_t)(p.ldc * 2) | (uintptr_t)(p.N * 2)) & 15) == 0;
+  for (int item = walk.slot; item < walk.chunk_len; item += walk.slots) {
+    int m0, n0;
+    tile_of(item, m0, n0);
+    // the scale block of this wave's tile (clamped for waves that lie past the matrix edge)
+    sa_row = (scalar_floats)(p.a_scale + (size_t)(min(m0 + wm * 128, p.M - 1) / 128) * k_steps);
+    sb_row = (scalar_floats)(p.b_scale + (size_t)(min(n0 + wn * 64, p.N - 1) / 128) * k_steps);
+    s_now = factor(sa_row[0], sb_row[0]);
+    memory_phase(std::true_type{});
+    matrix_phase(std::true_type{}, 0);
+    for (int kt = 1; kt < k_steps; ++kt) {
+      memory_phase(std::false_type{});
+      matrix_phase(std::false_type{}, kt);
+    }
+    uint8_t* table = lds + LDS_B0 + (sb == 0 ? 2 : sb - 1) * STAGE;
+    if (vec) epilogue(m0, n0, table, std::true_type{});
+    else epilogue(m0, n0, table, std::false_type{});
+  }
+  if (lead) __builtin_amdgcn_s_barrier();  // the second group's last phase
+  wait_loads<0>();  // (loads into LDS land before it is released)
+}
+
 // Second pass of a split-K launch: sums the splits' partials in a fixed order (results do not
 // depend on scheduling), applies the scales and the bias and rounds to bf16. One thread per
 // 4 consecutive columns.
@@ -1865,13 +2156,6 @@ constexpr size_t narrow_lds_bytes(int MB, int NB) {
 }
 static_assert(narrow_lds_bytes(2, 1) <= 160 * 1024 && narrow_lds_bytes(1, 2) <= 160 * 1024 && narrow_lds_bytes(2, 2) <= 160 * 1024,
               "stage rings must fit the LDS");
-
-// waits until at most VM of this wave's global loads are outstanding (LDS operations are not waited for)
-template <int VM>
-__device__ __forceinline__ void wait_loads() {
-  constexpr int imm = (VM & 15) | ((VM >> 4) << 14) | (7 << 4) | (15 << 8);
-  __builtin_amdgcn_s_waitcnt(imm);
-}
 
 template <int MB, int NB>
 __global__ __launch_bounds__(512) void gemm_narrow_kernel(GemmParams p) {
@@ -3358,6 +3642,46 @@ int launch_skinny(const GemmParams& p, hipStream_t stream) {
   return MI355X_FP8_OK;
 }
 
+// Estimated times of the block-scaled forms over MFMA-bound shapes, from launches with 4 to 104 steps (us a 128-byte
+// step of a round of tiles, and what a round costs beside its steps). 128x128 tiles, two workgroups per CU: 8192^3
+// 545 us (8 rounds of 64 steps), 4096x10240x8192 350; alone on their CUs 1024x2048x4096 20 (128 tiles of 32
+// steps), 2048x2048x4096 22.6 (256).
+inline float block_small_cost_us(int64_t M, int64_t N, int64_t K) {
+  const long tiles = ((M + 127) / 128) * ((N + 127) / 128), full = tiles / (2 * kNumCu), rest = tiles % (2 * kNumCu);
+  const float steps = (float)k_steps_of(K);
+  float t = (float)full * (steps + 5.0f);
+  if (rest) t += steps * (rest <= kNumCu ? 0.45f + 0.1f * (float)rest / (float)kNumCu : 1.0f) + 5.0f;
+  return t;
+}
+// 256x256 tiles: 8192^3 416-425 us (4 rounds of 64 steps), 2048x8192x2048 33.7 (one of 16), 4096x2304x13312 129 (144
+// tiles of 104 steps), 1024x8192x8192 76.5 (128 of 64), 512x4096x4096 38.6 (64 of 32): a step slows down with the
+// share of the chip at work beyond one half.
+inline float block_large_cost_us(int64_t M, int64_t N, int64_t K) {
+  const long tiles = ((M + kBlockTile - 1) / kBlockTile) * ((N + kBlockTile - 1) / kBlockTile), full = tiles / kNumCu, rest = tiles % kNumCu;
+  const float steps = (float)k_steps_of(K), share = (float)rest / (float)kNumCu;
+  float t = (float)full * (steps * 1.55f + 8.0f);
+  if (rest) t += steps * (share <= 0.5f ? 1.1f : 1.1f + 0.9f * (share - 0.5f)) + 6.0f;
+  return t;
+}
+
+template <bool KTAIL>
+int launch_block_form(GemmParams p, hipStream_t stream) {
+  constexpr auto kern = gemm_block_kernel<KTAIL>;
+  (void)LdsLimit<kern, kBlockLdsBytes>::registered;
+  p.tiles_m = (p.M + kBlockTile - 1) / kBlockTile;
+  p.tiles_n = (p.N + kBlockTile - 1) / kBlockTile;
+  make_fast_div((uint32_t)kGroupM * (uint32_t)p.tiles_n, p.div_group_mul, p.div_group_shift);
+  const long total = (long)p.tiles_m * p.tiles_n;
+  if (total > (long)INT32_MAX) return fail(MI355X_FP8_ENOTSUP, "more than 2^31-1 tiles");
+  const long grid = total < kNumCu ? (total + kNumXcd - 1) / kNumXcd * kNumXcd : kNumCu;
+  if (const int st = ready_device()) return st;
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kBlockWaves * 64), kBlockLdsBytes, stream, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "block-scaled kernel launch: %s", hipGetErrorString(e));
+  return MI355X_FP8_OK;
+}
+int launch_block(const GemmParams& p, hipStream_t s) { return p.K % kStepK ? launch_block_form<true>(p, s) : launch_block_form<false>(p, s); }
+
 template <int BM, int BN, int DEPTH>
 int launch_any(GemmParams p, hipStream_t stream) {
   constexpr size_t lds_bytes = any_lds_bytes(BM, BN);
@@ -3860,8 +4184,7 @@ int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale
   p.m_sizes = nullptr; p.groups = 0; p.out_f16 = 0;
   p.div_tiles_mul = p.div_tiles_shift = p.div_group_mul = p.div_group_shift = 0; p.stamps = nullptr;
   hipStream_t s = (hipStream_t)stream;
-  // 128x128 tiles: with 256x128 tiles (64 more accumulators and 64 more partial products per
-  // lane) the fold no longer fits the 256 registers VALU instructions can address
+  if (block_large_cost_us(M, N, K) < block_small_cost_us(M, N, K)) return launch_block(p, s);
   return (K % kStepK) ? launch_tiled<128, 128, 2, 2, true, kEpiPlain, false, true>(p, s)
                       : launch_tiled<128, 128, 2, 2, false, kEpiPlain, false, true>(p, s);
 }
