@@ -57,3 +57,22 @@ def _check(m, n, k, dev, seed=0):
 def test_large_tiles_against_float64(gpu_device, m, n, k):
     print(f"case m={m} n={n} k={k}", flush=True)
     _check(m, n, k, gpu_device)
+
+
+# the streaming forms: rows around 16, 32, 48 and 64, tiles whose columns straddle two column blocks (20 and 40 columns a
+# tile), column counts that are no multiple of 4, one K block, fewer K blocks than waves, partial last blocks; row
+# blocks (65 .. 256 rows) in every tile size
+@pytest.mark.parametrize("m,n,k", [(1, 2304, 2048), (16, 130, 96), (17, 1000, 144), (33, 515, 1040), (48, 640, 3008), (49, 300, 400),
+                                   (64, 2050, 1168), (16, 5000, 8192), (30, 10007, 2000), (64, 9999, 4112), (65, 515, 1040),
+                                   (128, 2300, 6656), (200, 1030, 2064), (256, 4090, 528)])
+def test_streaming_forms_against_float64(gpu_device, m, n, k):
+    print(f"case m={m} n={n} k={k}", flush=True)
+    _check(m, n, k, gpu_device)
+
+
+# 128x128 tiles whose walk over K starts at a step of its own per tile column and wraps around (one tile row, wide panel): the
+# factors' ratios have to wrap with it; one step, few steps, many steps with a partial last one
+@pytest.mark.parametrize("m,n,k", [(100, 24600, 128), (128, 25000, 400), (77, 26001, 2064)])
+def test_rotated_walk_against_float64(gpu_device, m, n, k):
+    print(f"case m={m} n={n} k={k}", flush=True)
+    _check(m, n, k, gpu_device)

@@ -317,6 +317,9 @@ __device__ __forceinline__ void wait_loads_and_barrier() {
   __builtin_amdgcn_s_barrier();
 }
 
+// what the block-scaled kernels read their factors through: constant memory, wave-uniform addresses, scalar loads
+typedef const __attribute__((address_space(4))) float* scalar_floats;
+
 // waits until at most VM of this wave's global loads are outstanding (LDS operations are not waited for)
 template <int VM>
 __device__ __forceinline__ void wait_loads() {
@@ -352,9 +355,13 @@ constexpr int kEpiPlain = 0, kEpiBias = 1, kEpiPartial = 2;
 constexpr size_t tiled_lds_bytes(int BM, int BN, int dist = kDefaultDist) {
   return (size_t)(dist * BM + (dist + 1) * BN) * kStepK;
 }
-constexpr int tiled_wgs_per_cu(int BM, int BN, bool blockscale = false, int dist = kDefaultDist) {
-  (void)blockscale;
-  return tiled_lds_bytes(BM, BN, dist) <= 80 * 1024 ? 2 : 1;
+constexpr int tiled_wgs_per_cu(int BM, int BN, int dist = kDefaultDist) { return tiled_lds_bytes(BM, BN, dist) <= 80 * 1024 ? 2 : 1; }
+// waves per SIMD the registers are budgeted for. The block-scaled form is always held to 256 registers: with more
+// the compiler puts the accumulators where the vector ALU cannot reach them and copies them back and
+// forth in every step (512x4096x4096, deep ring: 28.5 us that way).
+constexpr int tiled_waves_per_simd(int BM, int BN, int waves, bool blockscale, int dist) {
+  const int n = tiled_wgs_per_cu(BM, BN, dist) * waves / 4;
+  return blockscale && n < 2 ? 2 : n;
 }
 
 //
@@ -374,13 +381,13 @@ constexpr int tiled_wgs_per_cu(int BM, int BN, bool blockscale = false, int dist
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool KTAIL, int EPI, bool GROUPED = false, bool BLOCKSCALE = false,
           int DIST = kDefaultDist, bool STREAM_B = false>
 __global__ __launch_bounds__(WAVES_M* WAVES_N * 64)
-__attribute__((amdgpu_waves_per_eu(tiled_wgs_per_cu(BM, BN, BLOCKSCALE, DIST) * WAVES_M * WAVES_N / 4,
-                                   tiled_wgs_per_cu(BM, BN, BLOCKSCALE, DIST) * WAVES_M * WAVES_N / 4)))
+__attribute__((amdgpu_waves_per_eu(tiled_waves_per_simd(BM, BN, WAVES_M * WAVES_N, BLOCKSCALE, DIST),
+                                   tiled_waves_per_simd(BM, BN, WAVES_M * WAVES_N, BLOCKSCALE, DIST))))
 void gemm_tiled_kernel(GemmParams p) {
   constexpr int kStagesA = DIST, kStagesB = DIST + 1;
   static_assert(DIST >= 2 && tiled_lds_bytes(BM, BN, DIST) <= 160 * 1024, "the stage rings must fit the LDS");
   static_assert(!GROUPED || EPI == kEpiPlain, "the grouped form has neither bias nor split-K");
-  static_assert(!STREAM_B || (!BLOCKSCALE && !GROUPED), "the rotated K order is for the plain form only");
+  static_assert(!STREAM_B || !GROUPED, "the rotated K order is not for the grouped form");
   static_assert(!BLOCKSCALE || (128 % (BM / WAVES_M) == 0 && 128 % (BN / WAVES_N) == 0 && EPI == kEpiPlain && !GROUPED),
                 "a wave's tile must lie inside one 128x128 scale block: one factor per wave and step");
   constexpr bool HAS_BIAS = EPI == kEpiBias;
@@ -505,11 +512,14 @@ void gemm_tiled_kernel(GemmParams p) {
   // share panels of B through the L2 keep the common order: there the sharing needs it. So do
   // plans with more than two splits, whose items are already spread over K (M=128, N=K=8192 with
   // four splits lost 5 % to the rotation; two splits gain 5 %, unsplit plans 11-28 %).
+  auto first_step = [&](const TileLoc& loc, int begin, int count) {
+    return begin + (STREAM_B && p.splits <= 2 ? (loc.n0 / BN) % count : 0);
+  };
   auto start_cursor = [&](StepCursor& c, int li, const TileLoc& loc) {
     c.kt_begin = split_begin(item_split(li));
     c.kt_end = split_end(item_split(li));
     c.left = c.kt_end - c.kt_begin;
-    c.kt = c.kt_begin + (STREAM_B && p.splits <= 2 ? (loc.n0 / BN) % c.left : 0);
+    c.kt = first_step(loc, c.kt_begin, c.left);
   };
   // Source of the loads: one buffer descriptor per operand and tile, base = the tile's first row,
   // extent = its valid rows (the hardware returns zeros for anything past the extent, so rows past
@@ -678,10 +688,11 @@ void gemm_tiled_kernel(GemmParams p) {
     for (int r = 0; r < SC_REGS; ++r) {
       const int kb = min(r * 64 + lane, k_steps - 1);
       sc[r] = factor(kb);
-      rt[r] = kb > 0 ? factor(kb - 1) / sc[r] : 1.0f;
+      rt[r] = factor(kb > 0 ? kb - 1 : k_steps - 1) / sc[r];  // (a rotated walk passes from the last step to the first)
     }
   };
-  auto lane_value = [&](const float (&regs)[SC_REGS], int kt) -> float {
+  auto lane_value = [&](const float (&regs)[SC_REGS], int kt) -> float {  // (kt at most k_steps past the end)
+    if (kt >= k_steps) kt -= k_steps;
     const int r = kt >> 6;
     const float v = r == 0 ? regs[0] : r == 1 ? regs[1] : r == 2 ? regs[2] : regs[3];
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), kt & 63));
@@ -1032,8 +1043,8 @@ void gemm_tiled_kernel(GemmParams p) {
       if (t == B_LAST) advance_b(plain_tag);
       if (t == PREP_T) prepare_a_loads();
       if (BLOCKSCALE && t == PREP_T) {
-        n_pend = lane_value(rt, min(kt_c + 2, k_steps - 1));
-        n_last = lane_value(sc, min(kt_c + 1, k_steps - 1));
+        n_pend = lane_value(rt, k_steps == 1 ? 0 : kt_c + 2);
+        n_last = lane_value(sc, kt_c + 1);
       }
       if (t == PREP_T2) {
         sa = (sa + 1 == kStagesA) ? 0 : sa + 1;
@@ -1073,7 +1084,7 @@ void gemm_tiled_kernel(GemmParams p) {
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (BLOCKSCALE) ++kt_c;
+    if (BLOCKSCALE) kt_c = kt_c + 1 == k_steps ? 0 : kt_c + 1;
   };
   auto read_first_half = [&]() {
 #pragma unroll
@@ -1089,9 +1100,10 @@ void gemm_tiled_kernel(GemmParams p) {
     const int c_split = item_split(c_item);
     const int n_steps = split_end(c_split) - split_begin(c_split);
     if (BLOCKSCALE) {
-      load_block_scales(locate(walk_c, c_item));
-      kt_c = split_begin(c_split);
-      n_pend = lane_value(rt, min(kt_c + 1, k_steps - 1));
+      const TileLoc loc = locate(walk_c, c_item);
+      load_block_scales(loc);
+      kt_c = first_step(loc, 0, k_steps);
+      n_pend = lane_value(rt, kt_c + 1);
       n_last = lane_value(sc, kt_c);
     }
     if (n_steps == 1) {
@@ -1252,7 +1264,6 @@ void gemm_block_kernel(GemmParams p) {
   };
 
   // ---- factors: one per wave and step; a factor of zero (a block of zeros) counts as 2^-60
-  typedef const __attribute__((address_space(4))) float* scalar_floats;  // scalar loads
   scalar_floats sa_row = nullptr, sb_row = nullptr;
   auto factor = [&](float a, float b) {
     const float f = a * b;
@@ -1697,8 +1708,11 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
 // ------------------------------------------------------------------------------------
 // ANY: the generic family's form for up to 64 rows: unaligned loads, 16-bit matrix instructions on the
 // widened codes, any K (see the generic kernels above).
-template <int MT, int NTW, int DEPTH, int KW, bool ANY = false>
+// BLOCK: the block-scaled form (a step is one K block, all rows of A are in one row block and a tile of B in one
+// column block): a step's products are scaled by its factor as they are added up.
+template <int MT, int NTW, int DEPTH, int KW, bool ANY = false, bool BLOCK = false>
 __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
+  static_assert(!ANY || !BLOCK, "one or the other");
   using Chunk = std::conditional_t<ANY, v4i_any, v4i>;
   constexpr int TILE = 16 * kStepK;                 // one 16-row operand tile of one step: 2 KB
   constexpr int NTILE = NTW + MT;                   // tiles per step: B tiles then A tiles
@@ -1753,7 +1767,7 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
   const int fin_m = (fin_tu % MT) * 16 + (lane & 15);
   const int fin_n = n0 + (fin_tu / MT) * 16 + 4 * (lane >> 4);
   float fin_sa = 0.f, fin_sb[4] = {0.f, 0.f, 0.f, 0.f}, fin_bias[4] = {0.f, 0.f, 0.f, 0.f};
-  if (finisher) {
+  if (finisher && !BLOCK) {
     fin_sa = p.a_scale[min(fin_m, p.M - 1)];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -1763,9 +1777,27 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
     }
   }
 
+  // the factors of K block kb: a_scale's and, per 16 rows of B, b_scale's
+  const int k_blocks = k_full + (k_tail ? 1 : 0);
+  scalar_floats block_a = (scalar_floats)p.a_scale, block_b[NTW];
+#pragma unroll
+  for (int t = 0; t < NTW; ++t) block_b[t] = (scalar_floats)(p.b_scale + (size_t)(min(n0 + t * 16, p.N - 1) / 128) * k_blocks);
+  struct Factors {
+    float a, b[NTW];
+  };
+  auto fetch_factors = [&](int kb, Factors& f) {
+    if constexpr (BLOCK) {
+      f.a = block_a[kb];
+#pragma unroll
+      for (int t = 0; t < NTW; ++t) f.b[t] = block_b[t][kb];
+    }
+  };
+
   // DEPTH register sets, one per step in flight
   v4i land[DEPTH][NTILE][2];
-  auto fetch = [&](int i, v4i (&dst)[NTILE][2]) {
+  Factors land_f[DEPTH];
+  auto fetch = [&](int i, v4i (&dst)[NTILE][2], Factors& f) {
+    fetch_factors(wave + KW * i, f);
     const size_t kb = (size_t)(wave + KW * i) * kStepK;
 #pragma unroll
     for (int t = 0; t < NTILE; ++t)
@@ -1779,8 +1811,24 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
       }
   };
   // one step's products; ANY: a lane's 32 codes of a row are four 16-bit instructions of 8 codes per lane
-  auto multiply = [&](const v8i (&bf)[NTW], const v8i (&af)[MT]) {
-    if constexpr (ANY) {
+  auto multiply = [&](const v8i (&bf)[NTW], const v8i (&af)[MT], const Factors& f) {
+    if constexpr (BLOCK) {
+      const v4f zero = {0.f, 0.f, 0.f, 0.f};
+      v4f part[NTW][MT];
+#pragma unroll
+      for (int t = 0; t < NTW; ++t)
+#pragma unroll
+        for (int u = 0; u < MT; ++u)
+          part[t][u] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf[t], af[u], zero, 0, 0, 0, 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < NTW; ++t) {
+        const float s = f.a * f.b[t];
+#pragma unroll
+        for (int u = 0; u < MT; ++u)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[t][u][e] = __builtin_fmaf(part[t][u][e], s, acc[t][u][e]);
+      }
+    } else if constexpr (ANY) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         v8h hb[NTW], ha[MT];
@@ -1801,7 +1849,7 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
           acc[t][u] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf[t], af[u], acc[t][u], 0, 0, 0, 0, 0, 0);
     }
   };
-  auto consume = [&](const v4i (&got)[NTILE][2]) {
+  auto consume = [&](const v4i (&got)[NTILE][2], const Factors& factors) {
 #pragma unroll
     for (int t = 0; t < NTILE; ++t)
 #pragma unroll
@@ -1815,7 +1863,7 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
       if (t < NTW) bf[t] = f;
       else af[t - NTW] = f;
     }
-    multiply(bf, af);
+    multiply(bf, af, factors);
   };
 
   // The loop is unrolled DEPTH times so every register set has a fixed name; the compiler's
@@ -1831,30 +1879,30 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
   int i = 0;
   if (kSteadyLoop && my_steps >= DEPTH) {
 #pragma unroll
-    for (int d = 0; d < DEPTH; ++d) fetch(d, land[d]);
+    for (int d = 0; d < DEPTH; ++d) fetch(d, land[d], land_f[d]);
     for (; i + 2 * DEPTH <= my_steps; i += DEPTH) {
 #pragma unroll
       for (int d = 0; d < DEPTH; ++d) {
-        consume(land[d]);
-        fetch(i + d + DEPTH, land[d]);
+        consume(land[d], land_f[d]);
+        fetch(i + d + DEPTH, land[d], land_f[d]);
       }
     }
     if (i + DEPTH == my_steps) {
 #pragma unroll
-      for (int d = 0; d < DEPTH; ++d) consume(land[d]);
+      for (int d = 0; d < DEPTH; ++d) consume(land[d], land_f[d]);
       i += DEPTH;
     }
   } else {
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d)
-      if (d < my_steps) fetch(d, land[d]);
+      if (d < my_steps) fetch(d, land[d], land_f[d]);
   }
   for (; i < my_steps; i += DEPTH) {
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) {
       if (i + d < my_steps) {
-        consume(land[d]);
-        if (i + d + DEPTH < my_steps) fetch(i + d + DEPTH, land[d]);
+        consume(land[d], land_f[d]);
+        if (i + d + DEPTH < my_steps) fetch(i + d + DEPTH, land[d], land_f[d]);
       }
     }
   }
@@ -1879,7 +1927,9 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
       const v4i lo = chunk_of(row, 2 * g4), hi = chunk_of(row, 2 * g4 + 1);
       af[u] = (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     }
-    multiply(bf, af);
+    Factors f;
+    fetch_factors(k_full, f);
+    multiply(bf, af, f);
   }
 
   // ---- cross-wave reduction through each wave's own (now idle) buffer
@@ -1897,8 +1947,8 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
     float r[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      r[e] = sum[e] * fin_sa * fin_sb[e];
-      if (p.bias) r[e] += fin_bias[e];
+      r[e] = BLOCK ? sum[e] : sum[e] * fin_sa * fin_sb[e];
+      if (!BLOCK && p.bias) r[e] += fin_bias[e];
     }
     const uint32_t lo = pack_out_x2(r[0], r[1], p.out_f16), hi = pack_out_x2(r[2], r[3], p.out_f16);
     uint16_t* dst = p.c + (size_t)fin_m * p.ldc + fin_n;
@@ -2157,7 +2207,10 @@ constexpr size_t narrow_lds_bytes(int MB, int NB) {
 static_assert(narrow_lds_bytes(2, 1) <= 160 * 1024 && narrow_lds_bytes(1, 2) <= 160 * 1024 && narrow_lds_bytes(2, 2) <= 160 * 1024,
               "stage rings must fit the LDS");
 
-template <int MB, int NB>
+// BLOCK: the block-scaled form. A wave's slab of a step is one K block; the slab's products are scaled by that
+// block's factor as they are added up. A tile's columns may straddle two column blocks of B: every group of 4
+// columns takes the factor of its own.
+template <int MB, int NB, bool BLOCK = false>
 __global__ __launch_bounds__(512) void gemm_narrow_kernel(GemmParams p) {
   constexpr int BM = 32 * MB, BN = 32 * NB, KS = kNarrowKS;
   constexpr int DA = narrow_a_dist(MB, NB), DB = narrow_b_dist(MB, NB);
@@ -2220,16 +2273,34 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(GemmParams p) {
     const int l32 = lane & 31, half = lane >> 5;
     const int nq = n0 + 8 * wave + 4 * half;
     float sa[MB], sb[NB][4], bias_f[NB][4];
+    if (!BLOCK) {
 #pragma unroll
-    for (int i = 0; i < MB; ++i) sa[i] = p.a_scale[min(m0 + i * 32 + l32, p.M - 1)];
+      for (int i = 0; i < MB; ++i) sa[i] = p.a_scale[min(m0 + i * 32 + l32, p.M - 1)];
 #pragma unroll
-    for (int jb = 0; jb < NB; ++jb)
+      for (int jb = 0; jb < NB; ++jb)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int ne = min(nq + 32 * jb + e, p.N - 1);
-        sb[jb][e] = p.b_scale[ne];
-        bias_f[jb][e] = p.bias ? bf16_to_f32(p.bias[ne]) : 0.0f;
+        for (int e = 0; e < 4; ++e) {
+          const int ne = min(nq + 32 * jb + e, p.N - 1);
+          sb[jb][e] = p.b_scale[ne];
+          bias_f[jb][e] = p.bias ? bf16_to_f32(p.bias[ne]) : 0.0f;
+        }
+    }
+    // BLOCK: rows of factors of this row block and of the (at most two) column blocks 32 columns lie in
+    const int k_blocks = (p.K + kStepK - 1) / kStepK;
+    scalar_floats block_a = nullptr, block_lo[NB], block_hi[NB];
+    bool in_lo[NB][4];
+    if (BLOCK) {
+      const int last_nb = (p.N - 1) / 128;
+      block_a = (scalar_floats)(p.a_scale + (size_t)(m0 / 128) * k_blocks);
+#pragma unroll
+      for (int jb = 0; jb < NB; ++jb) {
+        const int nb = min((n0 + 32 * jb) / 128, last_nb);
+        block_lo[jb] = (scalar_floats)(p.b_scale + (size_t)nb * k_blocks);
+        block_hi[jb] = (scalar_floats)(p.b_scale + (size_t)min(nb + 1, last_nb) * k_blocks);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) in_lo[jb][q] = n0 + 32 * jb + 8 * q + 4 * half < (nb + 1) * 128;
       }
+    }
 #pragma unroll
     for (int s = 0; s < DA; ++s) issue_a(s);
     if (ksteps > DA) wait_loads<(DA - 1) * LA>(); else wait_loads<0>();
@@ -2264,7 +2335,8 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(GemmParams p) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) fah[i][j] = *(const v4i*)(sa_rows + i * 32 * kStepK + rd[sh][j]);
     };
-    auto mfma_half = [&](const v4i (&fbh)[NB][2], const v4i (&fah)[MB][2]) {
+    v16f part[BLOCK ? MB : 1][BLOCK ? NB : 1];  // BLOCK: the step's products
+    auto mfma_half = [&](const v4i (&fbh)[NB][2], const v4i (&fah)[MB][2], bool first) {
 #pragma unroll
       for (int jb = 0; jb < NB; ++jb) {
         const v8i vb = (v8i){fbh[jb][0][0], fbh[jb][0][1], fbh[jb][0][2], fbh[jb][0][3],
@@ -2273,16 +2345,46 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(GemmParams p) {
         for (int i = 0; i < MB; ++i) {
           const v8i va = (v8i){fah[i][0][0], fah[i][0][1], fah[i][0][2], fah[i][0][3],
                                fah[i][1][0], fah[i][1][1], fah[i][1][2], fah[i][1][3]};
-          acc[i][jb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vb, va, acc[i][jb], 0, 0, 0, 0, 0, 0);
+          if constexpr (BLOCK) {
+            part[i][jb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vb, va, first ? zero : part[i][jb], 0, 0, 0, 0, 0, 0);
+          } else {
+            acc[i][jb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vb, va, acc[i][jb], 0, 0, 0, 0, 0, 0);
+          }
+        }
+      }
+    };
+    // (a slab past K: its products are zero, any factor will do)
+    auto add_scaled = [&](float fa, const float (&flo)[NB], const float (&fhi)[NB]) {
+#pragma unroll
+      for (int jb = 0; jb < NB; ++jb) {
+        const float lo = fa * flo[jb], hi = fa * fhi[jb];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float f = in_lo[jb][q] ? lo : hi;
+#pragma unroll
+          for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              acc[i][jb][4 * q + e] = __builtin_fmaf(part[BLOCK ? i : 0][BLOCK ? jb : 0][4 * q + e], f, acc[i][jb][4 * q + e]);
         }
       }
     };
     v4i fb0[NB][2], fa0[MB][2], fb1[NB][2], fa1[MB][2];
     read_half(0, 0, fb0, fa0);
     for (int s = 0; s < ksteps; ++s) {
+      float f_a = 0.f, f_lo[NB] = {}, f_hi[NB] = {};
+      if (BLOCK) {
+        const int kb = min(step_of(s) * 4 + wave, k_blocks - 1);
+        f_a = block_a[kb];
+#pragma unroll
+        for (int jb = 0; jb < NB; ++jb) {
+          f_lo[jb] = block_lo[jb][kb];
+          f_hi[jb] = block_hi[jb][kb];
+        }
+      }
       read_half(s, 1, fb1, fa1);
       __builtin_amdgcn_sched_barrier(0);
-      mfma_half(fb0, fa0);
+      mfma_half(fb0, fa0, true);
       // every fragment of the step is in registers: this wave's slab of the A stage is free again, and
       // the loads of step s + DA go into it (nobody else reads or writes that slab)
       __builtin_amdgcn_sched_barrier(0);
@@ -2294,7 +2396,8 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(GemmParams p) {
       __builtin_amdgcn_s_barrier();
       if (s + 1 < ksteps) read_half(s + 1, 0, fb0, fa0);
       __builtin_amdgcn_sched_barrier(0);
-      mfma_half(fb1, fa1);
+      mfma_half(fb1, fa1, false);
+      if (BLOCK) add_scaled(f_a, f_lo, f_hi);
       __builtin_amdgcn_sched_barrier(0);
     }
 
@@ -2322,8 +2425,8 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(GemmParams p) {
           float r[4];
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const float t = sum[e] * sa[i];
-            r[e] = p.bias ? __builtin_fmaf(t, sb[jb][e], bias_f[jb][e]) : t * sb[jb][e];
+            const float t = BLOCK ? sum[e] : sum[e] * sa[i];
+            r[e] = BLOCK ? t : p.bias ? __builtin_fmaf(t, sb[jb][e], bias_f[jb][e]) : t * sb[jb][e];
           }
           const uint32_t lo = pack_out_x2(r[0], r[1], p.out_f16), hi = pack_out_x2(r[2], r[3], p.out_f16);
           uint16_t* dst = p.c + (size_t)m * p.ldc + n;
@@ -3553,7 +3656,7 @@ int launch_tiled(GemmParams p, hipStream_t stream) {
   make_fast_div((uint32_t)kGroupM * (uint32_t)p.tiles_n, p.div_group_mul, p.div_group_shift);
   const long total = (long)p.tiles_m * p.tiles_n * p.splits;
   if (total > (long)INT32_MAX) return fail(MI355X_FP8_ENOTSUP, "more than 2^31-1 work items");
-  const long slots = (long)kNumCu * tiled_wgs_per_cu(BM, BN, BLOCKSCALE, DIST);
+  const long slots = (long)kNumCu * tiled_wgs_per_cu(BM, BN, DIST);
   long grid = total < slots ? ((total + kNumXcd - 1) / kNumXcd) * kNumXcd : slots;
   constexpr auto kern = gemm_tiled_kernel<BM, BN, WAVES_M, WAVES_N, KTAIL, EPI, GROUPED, BLOCKSCALE, DIST, STREAM_B>;
   (void)LdsLimit<kern, lds_bytes>::registered;
@@ -3628,11 +3731,11 @@ MI355X_DEFINE_TILED_PART(6, 128, 128, 2, 2, false, true)  // (never with the str
 
 #if !defined(MI355X_TILED_PART)  // (everything from here on belongs to the main unit)
 namespace {
-template <int MT, int NTW, int DEPTH, int KW, bool ANY = false>
+template <int MT, int NTW, int DEPTH, int KW, bool ANY = false, bool BLOCK = false>
 int launch_skinny(const GemmParams& p, hipStream_t stream) {
   constexpr size_t lds_bytes = (size_t)KW * (NTW + MT) * 16 * kStepK;
   static_assert(lds_bytes <= 160 * 1024, "transpose buffers must fit the 160 KB LDS");
-  constexpr auto kern = gemm_skinny_kernel<MT, NTW, DEPTH, KW, ANY>;
+  constexpr auto kern = gemm_skinny_kernel<MT, NTW, DEPTH, KW, ANY, BLOCK>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   if (const int st = ready_device()) return st;
   const unsigned grid = (unsigned)((p.N + 16 * NTW - 1) / (16 * NTW));
@@ -3646,11 +3749,18 @@ int launch_skinny(const GemmParams& p, hipStream_t stream) {
 // step of a round of tiles, and what a round costs beside its steps). 128x128 tiles, two workgroups per CU: 8192^3
 // 545 us (8 rounds of 64 steps), 4096x10240x8192 350; alone on their CUs 1024x2048x4096 20 (128 tiles of 32
 // steps), 2048x2048x4096 22.6 (256).
+// One tile row against a wide panel is bound by the stream of B and fetches it with the streaming policy: K = 8192,
+// N = 57344 78 / 83 / 98 us with 16 / 64 / 128 rows (96 / 109 / 117 without the policy), N = 28672 48 with 64 rows (63);
+// with fewer workgroups it costs: 24x20480x5120 30.9 -> 31.9, 128x2304x6656 28 -> 34.
+inline bool block_streams(int64_t M, int64_t N) { return M <= 128 && N >= 192 * 128; }
 inline float block_small_cost_us(int64_t M, int64_t N, int64_t K) {
-  const long tiles = ((M + 127) / 128) * ((N + 127) / 128), full = tiles / (2 * kNumCu), rest = tiles % (2 * kNumCu);
   const float steps = (float)k_steps_of(K);
+  if (block_streams(M, N)) return fmaxf(5.0f + (float)N * (float)K * (1.0f + (float)M / 400.0f) / 6.4e6f, 6.0f + 0.62f * steps);
+  const long tiles = ((M + 127) / 128) * ((N + 127) / 128), full = tiles / (2 * kNumCu), rest = tiles % (2 * kNumCu);
+  // (one tile row: its steps wait for HBM, 16x8192x8192 40 us, 16x13312x13312 67)
+  const float alone = M <= 128 ? 0.58f : 0.45f + 0.1f * (float)rest / (float)kNumCu;
   float t = (float)full * (steps + 5.0f);
-  if (rest) t += steps * (rest <= kNumCu ? 0.45f + 0.1f * (float)rest / (float)kNumCu : 1.0f) + 5.0f;
+  if (rest) t += steps * (rest <= kNumCu ? alone : 1.0f) + 5.0f;
   return t;
 }
 // 256x256 tiles: 8192^3 416-425 us (4 rounds of 64 steps), 2048x8192x2048 33.7 (one of 16), 4096x2304x13312 129 (144
@@ -3661,7 +3771,28 @@ inline float block_large_cost_us(int64_t M, int64_t N, int64_t K) {
   const float steps = (float)k_steps_of(K), share = (float)rest / (float)kNumCu;
   float t = (float)full * (steps * 1.55f + 8.0f);
   if (rest) t += steps * (share <= 0.5f ? 1.1f : 1.1f + 0.9f * (share - 0.5f)) + 6.0f;
-  return t;
+  // (one tile row against a wide panel: 128x57344x8192 122 us, 200x57344x4096 62)
+  return M <= kBlockTile ? fmaxf(t, 4.0f + (float)N * (float)K / 4.0e6f) : t;
+}
+
+// Up to 64 rows (256 where row blocks of it are one round) the streaming forms of the row-wise product take over, whose waves
+// share out the K blocks of a tile: measured against 128x128 tiles 1x2304x2048 12.1 -> 3.4 us, 16x8192x8192 40.0 -> 13.6,
+// 16x2048x16384 76.8 -> 13.2, 32x8192x28672 142 -> 46, 64x4096x2048 12.2 -> 6.4, 128x8192x8192 42.9 -> 21.9,
+// 256x4096x4096 19.9 -> 12.2. Their times are those of the row-wise forms within 3 %, and so are the estimates.
+enum BlockForm { kBlockOneTile, kBlockNarrow, kBlockSmall, kBlockSmallStream, kBlockLarge };
+inline BlockForm block_form(int64_t M, int64_t N, int64_t K) {
+  BlockForm best = block_streams(M, N) ? kBlockSmallStream : kBlockSmall;
+  float cost = block_small_cost_us(M, N, K);
+  auto weigh = [&](BlockForm form, float us) {
+    if (us < cost) {
+      best = form;
+      cost = us;
+    }
+  };
+  weigh(kBlockLarge, block_large_cost_us(M, N, K));
+  if (M <= kSkinnyMaxM) weigh(kBlockOneTile, one_tile_cost_us(M, N, K));
+  if (narrow_fits(M, N, K)) weigh(kBlockNarrow, narrow_cost_us(M, N, K));
+  return best;
 }
 
 template <bool KTAIL>
@@ -3835,10 +3966,10 @@ int launch_skinny_persistent_steps(const GemmParams& p, hipStream_t s) {
   }
 }
 
-template <int MB, int NB>
+template <int MB, int NB, bool BLOCK>
 int launch_narrow(const GemmParams& p, hipStream_t stream) {
   constexpr size_t lds_bytes = narrow_lds_bytes(MB, NB);
-  constexpr auto kern = gemm_narrow_kernel<MB, NB>;
+  constexpr auto kern = gemm_narrow_kernel<MB, NB, BLOCK>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   if (const int st = ready_device()) return st;
   const unsigned row_blocks = (unsigned)((p.M + 32 * MB - 1) / (32 * MB));
@@ -3855,10 +3986,11 @@ int launch_narrow(const GemmParams& p, hipStream_t stream) {
 }
 
 // the narrow-tile instantiation for a shape
+template <bool BLOCK = false>
 int launch_narrow_for(const GemmParams& p, hipStream_t s) {
   const NarrowForm f = narrow_form(p.M, p.N);
-  if (f.mb == 1) return f.nb == 1 ? launch_narrow<1, 1>(p, s) : launch_narrow<1, 2>(p, s);
-  return f.nb == 1 ? launch_narrow<2, 1>(p, s) : launch_narrow<2, 2>(p, s);
+  if (f.mb == 1) return f.nb == 1 ? launch_narrow<1, 1, BLOCK>(p, s) : launch_narrow<1, 2, BLOCK>(p, s);
+  return f.nb == 1 ? launch_narrow<2, 1, BLOCK>(p, s) : launch_narrow<2, 2, BLOCK>(p, s);
 }
 
 int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_scale, const void* bias, void* c,
@@ -4034,15 +4166,15 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
           return fail(MI355X_FP8_ENOTSUP,
                       "the narrow-tile kernel takes M <= %d, and M <= %d where 64x64 tiles give every CU at most one (got %lldx%lld)",
                       kSkinnyMaxM, kNarrowMaxM, (long long)M, (long long)N);
-        return launch_narrow_for(p, s);
+        return launch_narrow_for<>(p, s);
       }
       if (M > kSkinnyMaxM) {
         if (plan_bits & MI355X_FP8_SKINNY_ONE_TILE)
           return fail(MI355X_FP8_ENOTSUP, "the one-tile-per-workgroup form takes M <= %d (got M=%lld)", kSkinnyMaxM, (long long)M);
-        return launch_narrow_for(p, s);
+        return launch_narrow_for<>(p, s);
       }
       if (!(plan_bits & (MI355X_FP8_SKINNY_ONE_TILE | MI355X_FP8_SKINNY_RESIDENT)) && narrow_preferred(M, N, K))
-        return launch_narrow_for(p, s);
+        return launch_narrow_for<>(p, s);
       if ((plan_bits & MI355X_FP8_SKINNY_RESIDENT) && !pair_skinny_fits(M, N, K) && !persistent_skinny_fits(M, N, K))
         return fail(MI355X_FP8_ENOTSUP, "neither form that keeps A on chip takes %lldx%lldx%lld", (long long)M, (long long)N, (long long)K);
       if ((pair_skinny_fits(M, N, K) || persistent_skinny_fits(M, N, K)) && !(plan_bits & MI355X_FP8_SKINNY_ONE_TILE)) {
@@ -4184,9 +4316,22 @@ int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale
   p.m_sizes = nullptr; p.groups = 0; p.out_f16 = 0;
   p.div_tiles_mul = p.div_tiles_shift = p.div_group_mul = p.div_group_shift = 0; p.stamps = nullptr;
   hipStream_t s = (hipStream_t)stream;
-  if (block_large_cost_us(M, N, K) < block_small_cost_us(M, N, K)) return launch_block(p, s);
-  return (K % kStepK) ? launch_tiled<128, 128, 2, 2, true, kEpiPlain, false, true>(p, s)
-                      : launch_tiled<128, 128, 2, 2, false, kEpiPlain, false, true>(p, s);
+  const bool ktail = K % kStepK;
+  switch (block_form(M, N, K)) {
+    case kBlockNarrow: return launch_narrow_for<true>(p, s);
+    case kBlockOneTile:
+      if (M <= 16) return launch_skinny<1, 1, 4, 8, false, true>(p, s);
+      if (M <= 32) return launch_skinny<2, 1, 2, 8, false, true>(p, s);
+      if (M <= 48) return launch_skinny<3, 1, 2, 8, false, true>(p, s);
+      return launch_skinny<4, 2, 2, 8, false, true>(p, s);
+    case kBlockLarge: return launch_block(p, s);
+    case kBlockSmallStream:
+      return ktail ? launch_tiled<128, 128, 2, 2, true, kEpiPlain, false, true, kDefaultDist, true>(p, s)
+                   : launch_tiled<128, 128, 2, 2, false, kEpiPlain, false, true, kDefaultDist, true>(p, s);
+    default:
+      return ktail ? launch_tiled<128, 128, 2, 2, true, kEpiPlain, false, true>(p, s)
+                   : launch_tiled<128, 128, 2, 2, false, kEpiPlain, false, true>(p, s);
+  }
 }
 
 namespace {
