@@ -377,7 +377,8 @@ constexpr int tiled_waves_per_simd(int BM, int BN, int waves, bool blockscale, i
 // STREAM_B: the rows of B are fetched with the streaming cache policy. For launches with one or
 // two tile rows, where a panel of B is read by one or two workgroups and never again
 // (measured: M=128, N=K=8192 27.6 -> 24.2 us, M=64 22.5 -> 19.6 us; with more tile rows the
-// panels are shared through the L2 and the same policy costs 5-8 %).
+// panels are shared through the L2 and the same policy costs 5-8 %). The grouped form has it for groups of
+// about one tile row (grouped_form).
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool KTAIL, int EPI, bool GROUPED = false, bool BLOCKSCALE = false,
           int DIST = kDefaultDist, bool STREAM_B = false>
 __global__ __launch_bounds__(WAVES_M* WAVES_N * 64)
@@ -387,7 +388,6 @@ void gemm_tiled_kernel(GemmParams p) {
   constexpr int kStagesA = DIST, kStagesB = DIST + 1;
   static_assert(DIST >= 2 && tiled_lds_bytes(BM, BN, DIST) <= 160 * 1024, "the stage rings must fit the LDS");
   static_assert(!GROUPED || EPI == kEpiPlain, "the grouped form has neither bias nor split-K");
-  static_assert(!STREAM_B || !GROUPED, "the rotated K order is not for the grouped form");
   static_assert(!BLOCKSCALE || (128 % (BM / WAVES_M) == 0 && 128 % (BN / WAVES_N) == 0 && EPI == kEpiPlain && !GROUPED),
                 "a wave's tile must lie inside one 128x128 scale block: one factor per wave and step");
   constexpr bool HAS_BIAS = EPI == kEpiBias;
@@ -1692,6 +1692,53 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
   }
 }
 
+// Grouped form: the group that row block `item` belongs to when every group's rows are cut into blocks of BM, and what
+// precedes it. Each lane takes one size of 64, and two scans across the wave give the rows and the blocks in front of
+// every group: one trip to memory however many groups there are (up to 64), where a walk over the sizes makes one each.
+// Sizes are clamped as in the tiled kernel (negative -> 0, the running sum cut at M): additions that saturate at M, which
+// a scan may regroup. group < 0: there is no such block.
+struct RowBlock {
+  int group, row_begin, row_end, blocks, blocks_before;
+};
+template <int BM>
+__device__ __forceinline__ RowBlock find_row_block(const GemmParams& p, int item) {
+  const int lane = threadIdx.x & 63;
+  int rows_before = 0, blocks_before = 0;
+  for (int g0 = 0; g0 < p.groups; g0 += 64) {
+    const int size = g0 + lane < p.groups ? min(max(p.m_sizes[g0 + lane], 0), p.M) : 0;
+    uint32_t row_end = (uint32_t)size + (lane == 0 ? (uint32_t)rows_before : 0u);
+    row_end = min(row_end, (uint32_t)p.M);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t below = __shfl_up(row_end, o);
+      if (lane >= o) row_end = min(row_end + below, (uint32_t)p.M);
+    }
+    const uint32_t prev = __shfl_up(row_end, 1);
+    const int row_begin = lane == 0 ? rows_before : (int)prev;
+    const int blocks = ((int)row_end - row_begin + BM - 1) / BM;
+    int blocks_end = blocks + (lane == 0 ? blocks_before : 0);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int below = __shfl_up(blocks_end, o);
+      if (lane >= o) blocks_end += below;
+    }
+    const uint64_t past = __ballot(item < blocks_end);
+    if (past) {
+      const int at = __builtin_ctzll(past);
+      RowBlock r;
+      r.group = g0 + at;
+      r.row_begin = __builtin_amdgcn_readlane(row_begin, at);
+      r.row_end = __builtin_amdgcn_readlane((int)row_end, at);
+      r.blocks = __builtin_amdgcn_readlane(blocks, at);
+      r.blocks_before = __builtin_amdgcn_readlane(blocks_end, at) - r.blocks;
+      return r;
+    }
+    rows_before = __builtin_amdgcn_readlane((int)row_end, 63);
+    blocks_before = __builtin_amdgcn_readlane(blocks_end, 63);
+  }
+  return RowBlock{-1, 0, 0, 0, 0};
+}
+
 // ------------------------------------------------------------------------------------
 // Skinny kernel (M <= 16*MT, HBM-bound): B is streamed exactly once and nothing is reused, so
 // what matters is whole-line coalesced loads and as many bytes in flight as a plain copy has.
@@ -1710,9 +1757,13 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
 // widened codes, any K (see the generic kernels above).
 // BLOCK: the block-scaled form (a step is one K block, all rows of A are in one row block and a tile of B in one
 // column block): a step's products are scaled by its factor as they are added up.
-template <int MT, int NTW, int DEPTH, int KW, bool ANY = false, bool BLOCK = false>
+// GROUPED: the grouped form for few rows a group. A workgroup is 16*NTW columns of one block of up to 16*MT rows of
+// a group; the row blocks of one group's columns are neighbours on one XCD (workgroup ids go round the XCDs), so that
+// the group's rows of B come from HBM once. The grid covers the most row blocks that any sizes with these M and G can
+// give; the surplus comes last and returns at once.
+template <int MT, int NTW, int DEPTH, int KW, bool ANY = false, bool BLOCK = false, bool GROUPED = false>
 __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
-  static_assert(!ANY || !BLOCK, "one or the other");
+  static_assert((int)ANY + (int)BLOCK + (int)GROUPED <= 1, "at most one of them");
   using Chunk = std::conditional_t<ANY, v4i_any, v4i>;
   constexpr int TILE = 16 * kStepK;                 // one 16-row operand tile of one step: 2 KB
   constexpr int NTILE = NTW + MT;                   // tiles per step: B tiles then A tiles
@@ -1725,7 +1776,24 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint8_t* buf = lds + wave * BUF;
-  const int n0 = blockIdx.x * (16 * NTW);
+  int n0 = blockIdx.x * (16 * NTW), m0 = 0, m_end = p.M;
+  const uint8_t* b_rows = p.b;
+  const float* b_scales = p.b_scale;
+  if constexpr (GROUPED) {
+    const int tiles = (p.tiles_n + kNumXcd - 1) / kNumXcd * kNumXcd;
+    const RowBlock at = find_row_block<16 * MT>(p, (int)blockIdx.x / tiles);
+    if (at.group < 0) return;
+    // t runs over the group's tiles and row blocks: the XCD's place, then the row block, then the round of tiles
+    const int t = (int)blockIdx.x - at.blocks_before * tiles;
+    const int slot = t / kNumXcd;
+    const int tile = slot / at.blocks * kNumXcd + t % kNumXcd;
+    if (tile >= p.tiles_n) return;
+    n0 = tile * (16 * NTW);
+    m0 = at.row_begin + slot % at.blocks * (16 * MT);
+    m_end = at.row_end;
+    b_rows += (size_t)at.group * p.N * p.ldb;
+    b_scales += (size_t)at.group * p.N;
+  }
 
   // global load: lane (ld_row, ld_c) of a wave-wide load fetches chunk ld_c (16 bytes) of row
   // ld_row of an 8-row half tile and parks it in LDS at the swizzled chunk position
@@ -1738,10 +1806,10 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
     wr_off[h] = r * kStepK + ((ld_c ^ swz128(r)) * kChunk);
 #pragma unroll
     for (int t = 0; t < NTW; ++t)
-      src[t][h] = p.b + (size_t)min(n0 + t * 16 + r, p.N - 1) * p.ldb + ld_c * kChunk;
+      src[t][h] = b_rows + (size_t)min(n0 + t * 16 + r, p.N - 1) * p.ldb + ld_c * kChunk;
 #pragma unroll
     for (int t = 0; t < MT; ++t)
-      src[NTW + t][h] = p.a + (size_t)min(t * 16 + r, p.M - 1) * p.lda + ld_c * kChunk;
+      src[NTW + t][h] = p.a + (size_t)min(m0 + t * 16 + r, m_end - 1) * p.lda + ld_c * kChunk;
   }
   // LDS->register: lane (r, g) of the 16x16x128 MFMA takes logical chunks 2g, 2g+1 of row r
   const int r16 = lane & 15, g4 = lane >> 4;
@@ -1764,15 +1832,15 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
   static_assert(NTW * MT * 64 <= KW * 64, "one finishing lane per output quad");
   const bool finisher = threadIdx.x < NTW * MT * 64;
   const int fin_tu = threadIdx.x >> 6;
-  const int fin_m = (fin_tu % MT) * 16 + (lane & 15);
+  const int fin_m = m0 + (fin_tu % MT) * 16 + (lane & 15);
   const int fin_n = n0 + (fin_tu / MT) * 16 + 4 * (lane >> 4);
   float fin_sa = 0.f, fin_sb[4] = {0.f, 0.f, 0.f, 0.f}, fin_bias[4] = {0.f, 0.f, 0.f, 0.f};
   if (finisher && !BLOCK) {
-    fin_sa = p.a_scale[min(fin_m, p.M - 1)];
+    fin_sa = p.a_scale[min(fin_m, m_end - 1)];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int ne = min(fin_n + e, p.N - 1);
-      fin_sb[e] = p.b_scale[ne];
+      fin_sb[e] = b_scales[ne];
       if (p.bias) fin_bias[e] = bf16_to_f32(p.bias[ne]);
     }
   }
@@ -1917,13 +1985,13 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
     v8i bf[NTW], af[MT];
 #pragma unroll
     for (int t = 0; t < NTW; ++t) {
-      const uint8_t* row = p.b + (size_t)min(n0 + t * 16 + r16, p.N - 1) * p.ldb;
+      const uint8_t* row = b_rows + (size_t)min(n0 + t * 16 + r16, p.N - 1) * p.ldb;
       const v4i lo = chunk_of(row, 2 * g4), hi = chunk_of(row, 2 * g4 + 1);
       bf[t] = (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     }
 #pragma unroll
     for (int u = 0; u < MT; ++u) {
-      const uint8_t* row = p.a + (size_t)min(u * 16 + r16, p.M - 1) * p.lda;
+      const uint8_t* row = p.a + (size_t)min(m0 + u * 16 + r16, m_end - 1) * p.lda;
       const v4i lo = chunk_of(row, 2 * g4), hi = chunk_of(row, 2 * g4 + 1);
       af[u] = (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     }
@@ -1940,7 +2008,7 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
     for (int u = 0; u < MT; ++u) mine[(t * MT + u) * 64 + lane] = acc[t][u];
   __syncthreads();
 
-  if (finisher && fin_m < p.M && fin_n < p.N) {
+  if (finisher && fin_m < m_end && fin_n < p.N) {
     v4f sum = ((const v4f*)lds)[fin_tu * 64 + lane];
 #pragma unroll
     for (int w = 1; w < KW; ++w) sum += ((const v4f*)(lds + w * BUF))[fin_tu * 64 + lane];
@@ -3745,6 +3813,52 @@ int launch_skinny(const GemmParams& p, hipStream_t stream) {
   return MI355X_FP8_OK;
 }
 
+// The grouped form for few rows a group. The most row blocks any sizes can give: every group that has rows at all
+// wastes at most all but one row of a block.
+template <int MT, int NTW, int DEPTH, int KW>
+int launch_grouped_skinny(const GemmParams& p, hipStream_t stream) {
+  constexpr int BM = 16 * MT, BN = 16 * NTW;
+  constexpr size_t lds_bytes = (size_t)KW * (NTW + MT) * 16 * kStepK;
+  static_assert(lds_bytes <= 160 * 1024, "transpose buffers must fit the 160 KB LDS");
+  constexpr auto kern = gemm_skinny_kernel<MT, NTW, DEPTH, KW, false, false, true>;
+  (void)LdsLimit<kern, lds_bytes>::registered;
+  GemmParams q = p;
+  q.tiles_n = (p.N + BN - 1) / BN;
+  const long tiles = (q.tiles_n + kNumXcd - 1) / kNumXcd * kNumXcd;
+  const long row_blocks = ((long)p.M + (long)(BM - 1) * (p.groups < p.M ? p.groups : p.M)) / BM;
+  if (tiles * row_blocks > (long)INT32_MAX) return fail(MI355X_FP8_ENOTSUP, "more than 2^31-1 workgroups");
+  if (const int st = ready_device()) return st;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * row_blocks)), dim3(KW * 64), lds_bytes, stream, q);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "grouped skinny kernel launch: %s", hipGetErrorString(e));
+  return MI355X_FP8_OK;
+}
+
+// Which form runs a grouped launch whose groups are up to a tile high on average: such a launch is bound by the
+// stream of B, and the sizes themselves are on the device. Measured over G = 2 ... 64 with rows sent to groups at random
+// and B read from memory, us, 128x128 tiles with B through the caches -> the form:
+// * up to 8 rows a group on average, the 16-row streaming form (a group with more takes several blocks): 16 groups of
+//   4096x4096 67 -> 50, 8 of 2048x7168 37 -> 21, 8 of 14336x4096 99 -> 83, 64 of 1536x1024 46 -> 32. Its tiles are 32
+//   columns wide so that A passes the L1 half as often: 16-column tiles 57, 37 and 97 on the first, third and last but one.
+// * launches of at most 128 tiles leave half of the chip idle; on long rows the streaming forms with 32 and 64 rows are
+//   ahead of them up to 16 and 32 rows a group: 8 groups of 2048x7168 38 -> 25 and 38 -> 31, 2 of 4096x4096 20 -> 13
+//   with 32 rows. (64 rows a group: 39 -> 48.)
+// * else tiles of one tile row with the streaming policy and the rotated walk: 16 groups of 4096x4096 with 16 to 64
+//   rows 68 -> 51-53, 8 of 14336x4096 with 32 101 -> 88. (Fewer than 128 tiles: 18 -> 22. K = 1024: 14.4 -> 15.7.)
+// * groups of 65 to 128 rows often are two tile rows high; 128x256 tiles then make fewer rounds: 16 groups of 4096x4096
+//   with 128 rows 88 -> 73 (128x128 tiles with the streaming policy 99), 8 of 14336x4096 145 -> 109, 16 of 7168x2048
+//   72 -> 63. (Fewer than 128 of them: 8 groups of 2048x7168 42 -> 57.)
+enum GroupedForm { kGroupedTiles, kGroupedRows16, kGroupedRows32, kGroupedRows64, kGroupedStream128, kGroupedStream256 };
+inline GroupedForm grouped_form(int64_t G, int64_t M, int64_t N, int64_t K) {
+  const bool rows_forms = G <= 256;  // (a workgroup's look-up goes over 64 groups at a time, the tiled kernel's once a launch)
+  if (M <= 8 * G && rows_forms) return kGroupedRows16;
+  const int64_t tiles_128 = G * ((N + 127) / 128), tiles_256 = G * ((N + 255) / 256);
+  if (rows_forms && K >= 4096 && tiles_128 <= 128 && M <= 32 * G) return M <= 16 * G ? kGroupedRows32 : kGroupedRows64;
+  if (K < 2048 || M > 128 * G) return kGroupedTiles;
+  if (M > 64 * G) return tiles_256 >= 128 ? kGroupedStream256 : kGroupedTiles;
+  return tiles_128 >= 128 ? kGroupedStream128 : kGroupedTiles;
+}
+
 // Estimated times of the block-scaled forms over MFMA-bound shapes, from launches with 4 to 104 steps (us a 128-byte
 // step of a round of tiles, and what a round costs beside its steps). 128x128 tiles, two workgroups per CU: 8192^3
 // 545 us (8 rounds of 64 steps), 4096x10240x8192 350; alone on their CUs 1024x2048x4096 20 (128 tiles of 32
@@ -4264,6 +4378,19 @@ int mi355x_fp8_rowwise_grouped_gemm(const void* a, const void* b, const float* a
   p.m_sizes = m_sizes; p.groups = (int)G; p.out_f16 = 0;
   p.div_tiles_mul = p.div_tiles_shift = p.div_group_mul = p.div_group_shift = 0; p.stamps = nullptr;
   hipStream_t s = (hipStream_t)stream;
+  const bool ktail = K % kStepK;
+  switch (tile_config < 0 ? grouped_form(G, M, N, K) : kGroupedTiles) {
+    case kGroupedRows16: return launch_grouped_skinny<1, 2, 2, 8>(p, s);
+    case kGroupedRows32: return launch_grouped_skinny<2, 2, 2, 8>(p, s);
+    case kGroupedRows64: return launch_grouped_skinny<4, 2, 2, 8>(p, s);
+    case kGroupedStream128:
+      return ktail ? launch_tiled<128, 128, 2, 2, true, kEpiPlain, true, false, kDefaultDist, true>(p, s)
+                   : launch_tiled<128, 128, 2, 2, false, kEpiPlain, true, false, kDefaultDist, true>(p, s);
+    case kGroupedStream256:
+      return ktail ? launch_tiled<128, 256, 2, 2, true, kEpiPlain, true, false, kDefaultDist, true>(p, s)
+                   : launch_tiled<128, 256, 2, 2, false, kEpiPlain, true, false, kDefaultDist, true>(p, s);
+    default: break;
+  }
   // Large tiles when an average group fills most of one and there are enough of them for every
   // CU, small tiles otherwise (the group sizes themselves are on the device; M / G is what the
   // host knows). Where 256x256 tiles are too few and 256x128 tiles come to about one round of workgroups,
@@ -4275,7 +4402,6 @@ int mi355x_fp8_rowwise_grouped_gemm(const void* a, const void* b, const float* a
     const int64_t tiles_256 = (M / 256) * (N / 256), tiles_128 = (M / 256) * (N / 128);
     tile_config = rows_fill && tiles_256 >= 192 ? 0 : rows_fill && tiles_128 >= 192 && tiles_128 <= 288 && K >= 4096 ? 2 : 1;
   }
-  const bool ktail = K % kStepK;
   if (tile_config == 0)
     return ktail ? launch_tiled<256, 256, 2, 2, true, kEpiPlain, true>(p, s)
                  : launch_tiled<256, 256, 2, 2, false, kEpiPlain, true>(p, s);
