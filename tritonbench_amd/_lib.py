@@ -5,11 +5,13 @@ tritonbench_amd.build). There is no fallback: if the library is missing or does 
 load, every entry point raises.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 from ctypes import c_char_p, c_int, c_int64, c_size_t, c_void_p
 
-from .build import LIB_PATH
+from .build import BINDING_PATH, LIB_PATH
 
 ABI_VERSION = 2
 
@@ -158,6 +160,26 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+_binding = None
+
+
+def binding():
+    """The native module that takes everyday calls from PyTorch tensors to the library (csrc/torch_binding.cpp), loaded once,
+    behind the library it calls."""
+    global _binding
+    if _binding is None:
+        load()
+        with _lock:
+            if _binding is None:
+                if not os.path.exists(BINDING_PATH):
+                    raise LibraryNotBuilt(f"{BINDING_PATH} does not exist; build it with `python -m tritonbench_amd.build`")
+                loader = importlib.machinery.ExtensionFileLoader("mi355x_torch_binding", BINDING_PATH)
+                module = importlib.util.module_from_spec(importlib.util.spec_from_loader(loader.name, loader))
+                loader.exec_module(module)
+                _binding = module
+    return _binding
+
+
 _initialised = set()
 
 
@@ -172,6 +194,7 @@ def init_device(index: int) -> None:
     with torch.cuda.device(index):
         check(load().mi355x_fp8_rowwise_init(), "mi355x_fp8_rowwise_init")
     _initialised.add(index)
+    binding().mark_ready(index)
 
 
 def last_error() -> str:

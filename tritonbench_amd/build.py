@@ -1,16 +1,19 @@
-"""Builds the gfx950 shared library from the HIP sources next to this file.
+"""Builds the gfx950 shared library from the HIP sources next to this file, and the PyTorch binding beside it.
 
 The library has no dependency on PyTorch headers: it is plain HIP behind a C ABI
-(include/mi355x_fp8_rowwise.h), compiled with hipcc for gfx950 only.
+(include/mi355x_fp8_rowwise.h), compiled with hipcc for gfx950 only. The binding is host code (g++).
 """
 import os
 import shutil
 import subprocess
+import sysconfig
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 SOURCES = [os.path.join(_PKG, "csrc", "fp8_rowwise_gemm.hip")]
 LIB_DIR = os.path.join(_PKG, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libmi355x_fp8_rowwise.so")
+BINDING_SOURCE = os.path.join(_PKG, "csrc", "torch_binding.cpp")
+BINDING_PATH = os.path.join(LIB_DIR, "mi355x_torch_binding.so")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -42,6 +45,28 @@ def _run(cmd, verbose):
         raise RuntimeError("hipcc failed:\n" + " ".join(cmd) + "\n" + proc.stdout)
 
 
+def _binding_object(verbose):
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    obj = os.path.join(BUILD_DIR, "torch_binding.o")
+    includes = [sysconfig.get_paths()["include"], *include_paths(), os.path.join(os.path.dirname(find_hipcc()), "..", "include")]
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{d}" for d in includes),
+          "-c", BINDING_SOURCE, "-o", obj], verbose)
+    return obj
+
+
+def _link_binding(obj, verbose):
+    """Links the binding against the library beside it (found through its own directory at run time) and PyTorch's."""
+    import torch
+
+    tmp = BINDING_PATH + ".tmp"
+    _run(["g++", "-shared", "-o", tmp, obj, f"-L{LIB_DIR}", "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN",
+          f"-L{os.path.join(os.path.dirname(torch.__file__), 'lib')}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"], verbose)
+    os.replace(tmp, BINDING_PATH)
+
+
 def build_library(verbose: bool = False, jobs: int = 0) -> str:
     """Compiles the library unconditionally and returns its path.
 
@@ -56,6 +81,8 @@ def build_library(verbose: bool = False, jobs: int = 0) -> str:
     if jobs == 1:
         _run([hipcc, *HIPCC_FLAGS, "-o", tmp, *SOURCES], verbose)
         os.replace(tmp, LIB_PATH)
+        os.makedirs(BUILD_DIR, exist_ok=True)
+        _link_binding(_binding_object(verbose), verbose)
         return LIB_PATH
     from concurrent.futures import ThreadPoolExecutor
 
@@ -66,10 +93,13 @@ def build_library(verbose: bool = False, jobs: int = 0) -> str:
     with ThreadPoolExecutor(max_workers=workers) as pool:
         futures = [pool.submit(_run, [hipcc, *flags, *defs, "-c", SOURCES[0], "-o", obj], verbose)
                    for (name, defs), obj in zip(units, objects)]
+        binding = pool.submit(_binding_object, verbose)
         for f in futures:
             f.result()
+        binding_obj = binding.result()
     _run([hipcc, "--offload-arch=gfx950", "-fPIC", "-shared", "-o", tmp, *objects], verbose)
     os.replace(tmp, LIB_PATH)
+    _link_binding(binding_obj, verbose)
     return LIB_PATH
 
 
