@@ -1503,6 +1503,8 @@ __global__ __launch_bounds__(256) void splitk_finalize_kernel(GemmParams p) {
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t v2u_any __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
 
 // bytes [k, k + 16) of a row of K bytes; those at or past K count as zero
 __device__ __forceinline__ v4i load16_any(const uint8_t* row, int k, int K) {
@@ -2888,7 +2890,11 @@ struct VecTraits<uint16_t> {
 // THREADS lanes per row, ROWS rows per workgroup. Rows short enough for one wave's registers take
 // THREADS = 64 with several rows per workgroup: no LDS, no barrier, and a fraction of the workgroups
 // (short rows are bound by the rate at which workgroups start, about one per 1.2-2 ns).
-template <typename SrcT, int CACHE, int THREADS, int ROWS = 1>
+// ANY: rows that start at any element and end anywhere (K >= one chunk): the same passes on unaligned accesses, which cost
+// a wave-wide load one line more. The last chunk is the row's last 16 bytes, which may repeat part of the chunk before it:
+// harmless for the maximum, and the codes come out and are stored the same twice. Its loads do without the streaming
+// policy (neighbouring waves share the lines at their borders).
+template <typename SrcT, int CACHE, int THREADS, int ROWS = 1, bool ANY = false>
 __global__ __launch_bounds__(THREADS* ROWS) void quantize_rows_vec_kernel(const SrcT* x, uint8_t* xq,
                                                                         float* inv_scale, int K, long ldx,
                                                                         long ldq, long rows) {
@@ -2899,9 +2905,16 @@ __global__ __launch_bounds__(THREADS* ROWS) void quantize_rows_vec_kernel(const 
   __shared__ float wave_max[THREADS / 64];
   const long row = (long)blockIdx.x * ROWS + (ROWS > 1 ? (long)(threadIdx.x >> 6) : 0);
   if (ROWS > 1 && row >= rows) return;  // (whole waves; this form has no barrier)
-  const v4i* xr = (const v4i*)(x + row * ldx);
+  using Chunk = std::conditional_t<ANY, v4i_any, v4i>;
+  using Codes = std::conditional_t<ANY, v4i_any, v4i>;
+  using Codes8 = std::conditional_t<ANY, v2u_any, v2u>;
+  using Codes4 = std::conditional_t<ANY, u32_any, uint32_t>;
+  const SrcT* xr = x + row * ldx;
   uint8_t* qr = xq + row * ldq;
-  const int nchunks = K / EPV;
+  const int nchunks = ANY ? (K + EPV - 1) / EPV : K / EPV;
+  // first element of chunk c
+  auto start = [&](int c) { return ANY ? min(c * EPV, K - EPV) : c * EPV; };
+  auto load = [&](int c) -> v4i { return *(const Chunk*)(xr + start(c)); };
   const int tid = ROWS > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
 
   v4i cache[CACHE];
@@ -2916,11 +2929,13 @@ __global__ __launch_bounds__(THREADS* ROWS) void quantize_rows_vec_kernel(const 
   for (int i = 0; i < CACHE; ++i) {
     // past the row's end a lane re-reads the last chunk: harmless for the maximum, never
     // stored, and it keeps the loads free of branches
-    cache[i] = __builtin_nontemporal_load(xr + min(tid + THREADS * i, nchunks - 1));
+    const int c = min(tid + THREADS * i, nchunks - 1);
+    if constexpr (ANY) cache[i] = load(c);
+    else cache[i] = __builtin_nontemporal_load((const v4i*)xr + c);
   }
 #pragma unroll
   for (int i = 0; i < CACHE; ++i) fold(cache[i]);
-  for (int c = tid + THREADS * CACHE; c < nchunks; c += THREADS) fold(xr[c]);
+  for (int c = tid + THREADS * CACHE; c < nchunks; c += THREADS) fold(load(c));
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) amax = max_keep_nan(amax, __shfl_xor(amax, o));
   if (THREADS > 64) {
@@ -2956,8 +2971,8 @@ __global__ __launch_bounds__(THREADS* ROWS) void quantize_rows_vec_kernel(const 
   auto convert_store = [&](const v4i& src, int c) {
     uint32_t out[EPV / 4];
     convert(src, out);
-    if (EPV == 4) *(uint32_t*)(qr + (size_t)c * 4) = out[0];
-    else *(v2u*)(qr + (size_t)c * 8) = (v2u){out[0], out[EPV / 4 - 1]};
+    if (EPV == 4) *(Codes4*)(qr + start(c)) = out[0];
+    else *(Codes8*)(qr + start(c)) = (v2u){out[0], out[EPV / 4 - 1]};
   };
   // A chunk turns into EPV output bytes per lane (4 or 8): too little per store instruction.
   // BATCH = 16 / EPV consecutive rounds of the cached chunks are therefore gathered through
@@ -2971,7 +2986,7 @@ __global__ __launch_bounds__(THREADS* ROWS) void quantize_rows_vec_kernel(const 
   constexpr int LPR = 64 / BATCH;  // lanes that store one round's bytes of this wave
 #pragma unroll
   for (int i0 = 0; i0 < CACHE; i0 += BATCH) {
-    if (THREADS * (i0 + BATCH) <= nchunks) {  // uniform: every lane of every wave has all BATCH rounds
+    if (THREADS * (i0 + BATCH) <= K / EPV) {  // uniform: every lane of every wave has all BATCH rounds
 #pragma unroll
       for (int b = 0; b < BATCH; ++b) {
         uint32_t out[EPV / 4];
@@ -2982,7 +2997,7 @@ __global__ __launch_bounds__(THREADS* ROWS) void quantize_rows_vec_kernel(const 
       const int b = lane / LPR, piece = lane % LPR;
       const v4i bytes = *(const v4i*)(mine + lane * 16);
       // round i0+b, this wave's 64 chunks start at chunk THREADS*(i0+b) + 64*wave
-      *(v4i*)(qr + ((size_t)THREADS * (i0 + b) + (tid & ~63)) * EPV + piece * 16) = bytes;
+      *(Codes*)(qr + ((size_t)THREADS * (i0 + b) + (tid & ~63)) * EPV + piece * 16) = bytes;
     } else {
 #pragma unroll
       for (int b = 0; b < BATCH; ++b) {
@@ -2991,7 +3006,7 @@ __global__ __launch_bounds__(THREADS* ROWS) void quantize_rows_vec_kernel(const 
       }
     }
   }
-  for (int c = tid + THREADS * CACHE; c < nchunks; c += THREADS) convert_store(xr[c], c);
+  for (int c = tid + THREADS * CACHE; c < nchunks; c += THREADS) convert_store(load(c), c);
 }
 
 
@@ -4315,6 +4330,36 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
 }
 }  // namespace
 
+namespace {
+constexpr int kWaveRows = 4;
+
+// The quantiser on rows that do not start 16-byte aligned or do not hold whole 16-byte chunks: the vector kernel's
+// unaligned forms, by the same lines as the aligned ones (fewer of them: this is the rare case). The element-by-element
+// kernel, which ran them all before, is left for rows shorter than one chunk. Measured, sources rotated through memory, before
+// -> now: f32 4096x8191 72 -> 28 us (2.3 -> 6.0 TB/s), 8192x2047 40 -> 15, 2048x20001 99 -> 36, 512x53247 181 -> 30; bf16
+// 4096x8191 73 -> 22 (4.6 TB/s), 8192x2047 40 -> 15, 1024x28671 107 -> 23.
+template <typename SrcT>
+void launch_quantize_any(const SrcT* x, uint8_t* xq, float* inv_scale, int64_t R, int64_t K, int64_t ldx, int64_t ldq, hipStream_t s) {
+  constexpr int epv = VecTraits<SrcT>::EPV;
+  constexpr int very_long_cache = epv == 4 ? 8 : 4;
+  const int64_t chunks = (K + epv - 1) / epv;
+  auto go = [&](auto kern, int64_t grid, int threads) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3((unsigned)threads), 0, s, x, xq, inv_scale, (int)K, (long)ldx, (long)ldq, (long)R);
+  };
+  if (K < epv) {
+    hipLaunchKernelGGL(quantize_rows_kernel<SrcT>, dim3((unsigned)R), dim3(256), 0, s, x, xq, inv_scale, (int)K, (long)ldx, (long)ldq);
+  } else if (chunks <= 8 * 64 && R > 2048) {
+    go(quantize_rows_vec_kernel<SrcT, 8, 64, kWaveRows, true>, (R + kWaveRows - 1) / kWaveRows, 64 * kWaveRows);
+  } else if (chunks <= 4 * 256) {
+    go(quantize_rows_vec_kernel<SrcT, 4, 256, 1, true>, R, 256);
+  } else if (chunks <= 8 * 512) {
+    go(quantize_rows_vec_kernel<SrcT, 8, 512, 1, true>, R, 512);
+  } else {
+    go(quantize_rows_vec_kernel<SrcT, very_long_cache, 1024, 1, true>, R, 1024);
+  }
+}
+}  // namespace
+
 extern "C" {
 
 int mi355x_fp8_rowwise_gemm_noalloc(const void* a, const void* b, const float* a_scale, const float* b_scale,
@@ -4466,10 +4511,10 @@ namespace {
 // workgroup per row -> wave per row: 16384 x 2048 quantiser 28.7 -> 19.9 us, RMSNorm form 40.8 -> 21.0,
 // SiLU-mul form 49.0 -> 27.9; 65536 x 512 75 -> 27, 132 -> 29, 170 -> 32; eight rows per workgroup
 // instead of four changed nothing.)
-constexpr int kWaveRows = 4;
 inline int row_chunks_per_lane(int64_t chunks) { return chunks <= 64 * 4 ? 4 : chunks <= 64 * 8 ? 8 : 0; }
 // (bf16 rows of up to 1024 elements: two rounds per lane instead of four, of which at least two would be idle)
 inline int bf16_row_chunks_per_lane(int64_t chunks) { return chunks <= 64 * 2 ? 2 : row_chunks_per_lane(chunks); }
+
 }  // namespace
 
 int mi355x_fp8_rowwise_quantize(const void* x, int src_type, void* xq, float* inv_scale, int64_t R,
@@ -4523,11 +4568,9 @@ int mi355x_fp8_rowwise_quantize(const void* x, int src_type, void* xq, float* in
                          (const uint16_t*)x, (uint8_t*)xq, inv_scale, (int)K, (long)ldx, (long)ldq, (long)R);
     }
   } else if (src_type == MI355X_FP8_SRC_F32) {
-    hipLaunchKernelGGL(quantize_rows_kernel<float>, dim3((unsigned)R), dim3(256), 0, s, (const float*)x,
-                       (uint8_t*)xq, inv_scale, (int)K, (long)ldx, (long)ldq);
+    launch_quantize_any<float>((const float*)x, (uint8_t*)xq, inv_scale, R, K, ldx, ldq, s);
   } else if (src_type == MI355X_FP8_SRC_BF16) {
-    hipLaunchKernelGGL(quantize_rows_kernel<uint16_t>, dim3((unsigned)R), dim3(256), 0, s,
-                       (const uint16_t*)x, (uint8_t*)xq, inv_scale, (int)K, (long)ldx, (long)ldq);
+    launch_quantize_any<uint16_t>((const uint16_t*)x, (uint8_t*)xq, inv_scale, R, K, ldx, ldq, s);
   } else {
     return fail(MI355X_FP8_EINVAL, "unknown src_type %d", src_type);
   }
