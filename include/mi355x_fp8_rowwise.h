@@ -245,6 +245,17 @@ int mi355x_fp8_rowwise_grouped_gemm(const void* a, const void* b,
                                     int tile_config, void* stream);
 
 /*
+ * The same, and with a non-zero `clear_rest` the rows of C past the sum of the sizes are set to zero
+ * in the same launch: for a result whose memory has not been written before.
+ */
+int mi355x_fp8_rowwise_grouped_gemm_ex(const void* a, const void* b,
+                                       const float* a_scale, const float* b_scale,
+                                       const int32_t* m_sizes, void* c,
+                                       int64_t G, int64_t M, int64_t N, int64_t K,
+                                       int64_t lda, int64_t ldb, int64_t ldc,
+                                       int tile_config, int clear_rest, void* stream);
+
+/*
  * Block-scaled form: one scale per 128x128 block of A and of B,
  *
  *   C[m, n] = bf16( sum_kb (sum_{k in block kb} A[m,k] * B[n,k]) * a_scale[m/128][kb] * b_scale[n/128][kb] )

@@ -87,3 +87,21 @@ def test_a_captured_launch_follows_new_sizes(gpu_device):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+# (a form of each kernel; N a whole number of 16-byte pieces or not; no rest, a row, nearly everything, everything)
+@pytest.mark.parametrize("g,m,n,k", [(16, 100, 96, 640), (16, 100, 97, 640), (2, 32, 128, 4096), (8, 500, 2048, 2048), (16, 1100, 2048, 2048),
+                                     (3, 900, 520, 256), (3, 900, 513, 256), (4, 4096, 4096, 512), (130, 900, 64, 256)])
+@pytest.mark.parametrize("rest", ["none", "a row", "most", "all"])
+def test_a_result_made_by_the_call_is_zero_past_the_groups(gpu_device, g, m, n, k, rest):
+    x, w, xs, ws = _operands(gpu_device, g, m, n, k)
+    rows = {"none": m, "a row": m - 1, "most": 3, "all": 0}[rest]
+    ms = torch.tensor(_spread(g, rows), dtype=torch.int32, device=gpu_device)
+    want = torch.zeros((m, n), dtype=torch.bfloat16, device=gpu_device)
+    ops.fp8_gemm_rowwise_grouped(x, w, ms, xs, ws, out=want)
+    stale = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)  # what the allocator hands out next
+    del stale
+    for config in (-1, 0, 1, 2):
+        got = ops.fp8_gemm_rowwise_grouped(x, w, ms, xs, ws, tile_config=config)
+        assert torch.equal(got, want), config
+        got.fill_(float("nan"))

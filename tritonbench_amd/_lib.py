@@ -94,6 +94,12 @@ SIGNATURES = {
          c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64,
          c_int, c_void_p],
     ),
+    "mi355x_fp8_rowwise_grouped_gemm_ex": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+         c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64,
+         c_int, c_int, c_void_p],
+    ),
     "mi355x_fp8_blockwise_gemm": (
         c_int,
         [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,

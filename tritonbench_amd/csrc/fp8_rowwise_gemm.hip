@@ -77,6 +77,7 @@ struct GemmParams {
   // (device memory) multiplied with rows [g*N, (g+1)*N) of B and scaled by b_scale[g*N + n]
   const int32_t* m_sizes;
   int groups;
+  int clear_rest;  // rows of C past the last group's are set to zero (else they are left alone)
   int out_f16;  // C holds IEEE binary16 instead of bf16 (same size, same stores)
   // tiled kernel, plain form: reciprocals of the two run-time divisors of the tile walk (the number
   // of tiles, and the tiles of a full group of tile rows), prepared on the host: see fast_div()
@@ -175,6 +176,21 @@ __device__ __forceinline__ void fetch_arguments_now(const GemmParams& p) {
                "s"(p.lda), "s"(p.ldb), "s"(p.ldc), "s"(p.tiles_m), "s"(p.tiles_n), "s"(p.out_f16));
 }
 // the same for what only the tiled kernel and its second pass read
+// Grouped form: zeros into rows first .. M-1 of C, shared out over `of` workgroups of this launch (this one is number `who`).
+// As a fill of all of C in front of the launch it took a launch of its own and a write of everything that the product
+// then writes again (8192 x 4096: 10 us of 115).
+__device__ __forceinline__ void clear_rows(const GemmParams& p, int first, int who, int of) {
+  const int threads = (int)blockDim.x, tid = (int)threadIdx.x;
+  if (p.ldc == p.N && p.N % 8 == 0 && (reinterpret_cast<uintptr_t>(p.c) & 15) == 0) {
+    v4i* c = (v4i*)(p.c + (size_t)first * p.N);
+    const size_t count = (size_t)(p.M - first) * p.N / 8;
+    for (size_t i = (size_t)who * threads + tid; i < count; i += (size_t)of * threads) c[i] = (v4i){0, 0, 0, 0};
+  } else {
+    for (long r = (long)first + who; r < p.M; r += of)
+      for (long n = tid; n < p.N; n += threads) p.c[(size_t)r * p.ldc + n] = 0;
+  }
+}
+
 __device__ __forceinline__ void fetch_tiled_arguments_now(const GemmParams& p) {
   asm volatile("" ::"s"(p.splits), "s"(p.steps_per_split), "s"(p.partial), "s"(p.m_sizes), "s"(p.groups), "s"(p.div_tiles_mul),
                "s"(p.div_tiles_shift), "s"(p.div_group_mul), "s"(p.div_group_shift), "s"(p.stamps));
@@ -445,11 +461,13 @@ void gemm_tiled_kernel(GemmParams p) {
   auto group_rows = [&](int g, int row_begin) { return min(max(p.m_sizes[g], 0), p.M - row_begin); };
   if (GROUPED) {
     total_tiles = 0;
-    for (int g = 0, rows = 0; g < p.groups; ++g) {
+    int rows = 0;
+    for (int g = 0; g < p.groups; ++g) {
       const int mg = group_rows(g, rows);
       total_tiles += ((mg + BM - 1) / BM) * p.tiles_n;
       rows += mg;
     }
+    if (p.clear_rest && rows < p.M) clear_rows(p, rows, (int)blockIdx.x, (int)gridDim.x);
   }
   const TileWalk walk = make_walk(total_tiles * p.splits);
   if (walk.slot >= walk.chunk_len) return;  // uniform over the workgroup
@@ -1698,7 +1716,7 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
 // precedes it. Each lane takes one size of 64, and two scans across the wave give the rows and the blocks in front of
 // every group: one trip to memory however many groups there are (up to 64), where a walk over the sizes makes one each.
 // Sizes are clamped as in the tiled kernel (negative -> 0, the running sum cut at M): additions that saturate at M, which
-// a scan may regroup. group < 0: there is no such block.
+// a scan may regroup. group < 0: there is no such block, and row_end and blocks_before are the totals.
 struct RowBlock {
   int group, row_begin, row_end, blocks, blocks_before;
 };
@@ -1738,7 +1756,7 @@ __device__ __forceinline__ RowBlock find_row_block(const GemmParams& p, int item
     rows_before = __builtin_amdgcn_readlane((int)row_end, 63);
     blocks_before = __builtin_amdgcn_readlane(blocks_end, 63);
   }
-  return RowBlock{-1, 0, 0, 0, 0};
+  return RowBlock{-1, rows_before, rows_before, 0, blocks_before};
 }
 
 // ------------------------------------------------------------------------------------
@@ -1784,7 +1802,13 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
   if constexpr (GROUPED) {
     const int tiles = (p.tiles_n + kNumXcd - 1) / kNumXcd * kNumXcd;
     const RowBlock at = find_row_block<16 * MT>(p, (int)blockIdx.x / tiles);
-    if (at.group < 0) return;
+    if (at.group < 0) {  // surplus
+      if (p.clear_rest && at.row_end < p.M) {
+        const int used = at.blocks_before * tiles;
+        clear_rows(p, at.row_end, (int)blockIdx.x - used, (int)gridDim.x - used);
+      }
+      return;
+    }
     // t runs over the group's tiles and row blocks: the XCD's place, then the row block, then the round of tiles
     const int t = (int)blockIdx.x - at.blocks_before * tiles;
     const int slot = t / kNumXcd;
@@ -3840,7 +3864,8 @@ int launch_grouped_skinny(const GemmParams& p, hipStream_t stream) {
   GemmParams q = p;
   q.tiles_n = (p.N + BN - 1) / BN;
   const long tiles = (q.tiles_n + kNumXcd - 1) / kNumXcd * kNumXcd;
-  const long row_blocks = ((long)p.M + (long)(BM - 1) * (p.groups < p.M ? p.groups : p.M)) / BM;
+  // (one more where rows past the groups' are to be cleared, so that there is a surplus to do it)
+  const long row_blocks = ((long)p.M + (long)(BM - 1) * (p.groups < p.M ? p.groups : p.M)) / BM + (p.clear_rest ? 1 : 0);
   if (tiles * row_blocks > (long)INT32_MAX) return fail(MI355X_FP8_ENOTSUP, "more than 2^31-1 workgroups");
   if (const int st = ready_device()) return st;
   hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * row_blocks)), dim3(KW * 64), lds_bytes, stream, q);
@@ -3853,8 +3878,10 @@ int launch_grouped_skinny(const GemmParams& p, hipStream_t stream) {
 // stream of B, and the sizes themselves are on the device. Measured over G = 2 ... 64 with rows sent to groups at random
 // and B read from memory, us, 128x128 tiles with B through the caches -> the form:
 // * up to 8 rows a group on average, the 16-row streaming form (a group with more takes several blocks): 16 groups of
-//   4096x4096 67 -> 50, 8 of 2048x7168 37 -> 21, 8 of 14336x4096 99 -> 83, 64 of 1536x1024 46 -> 32. Its tiles are 32
-//   columns wide so that A passes the L1 half as often: 16-column tiles 57, 37 and 97 on the first, third and last but one.
+//   4096x4096 67 -> 47, 8 of 2048x7168 37 -> 21, 8 of 14336x4096 99 -> 77, 64 of 1536x1024 46 -> 21. Its tiles are 32
+//   columns wide so that A passes the L1 half as often (16 columns: 57 on the first, 97 on the third). Four waves rather than
+//   eight, so that twice as many workgroups are on a CU at different places of their short lives: eight waves 49, 21, 82
+//   and 31, sixteen 60, 24, 101 and 50.
 // * launches of at most 128 tiles leave half of the chip idle; on long rows the streaming forms with 32 and 64 rows are
 //   ahead of them up to 16 and 32 rows a group: 8 groups of 2048x7168 38 -> 25 and 38 -> 31, 2 of 4096x4096 20 -> 13
 //   with 32 rows. (64 rows a group: 39 -> 48.)
@@ -4248,7 +4275,7 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
   p.lda = lda; p.ldb = ldb; p.ldc = ldc;
   p.tiles_m = p.tiles_n = 0; p.group_m = 1;
   p.splits = 1; p.steps_per_split = k_steps_of(K); p.partial = nullptr;
-  p.m_sizes = nullptr; p.groups = 0; p.out_f16 = out_type == MI355X_FP8_OUT_F16;
+  p.m_sizes = nullptr; p.groups = 0; p.clear_rest = 0; p.out_f16 = out_type == MI355X_FP8_OUT_F16;
   p.div_tiles_mul = p.div_tiles_shift = p.div_group_mul = p.div_group_shift = 0; p.stamps = stamps;
   hipStream_t s = (hipStream_t)stream;
 
@@ -4393,6 +4420,13 @@ int mi355x_fp8_rowwise_grouped_gemm(const void* a, const void* b, const float* a
                                     const int32_t* m_sizes, void* c, int64_t G, int64_t M, int64_t N,
                                     int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int tile_config,
                                     void* stream) {
+  return mi355x_fp8_rowwise_grouped_gemm_ex(a, b, a_scale, b_scale, m_sizes, c, G, M, N, K, lda, ldb, ldc, tile_config, 0, stream);
+}
+
+int mi355x_fp8_rowwise_grouped_gemm_ex(const void* a, const void* b, const float* a_scale, const float* b_scale,
+                                       const int32_t* m_sizes, void* c, int64_t G, int64_t M, int64_t N,
+                                       int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int tile_config,
+                                       int clear_rest, void* stream) {
   int st = check_shape(M, N, K);
   if (st == MI355X_FP8_OK) st = check_fast_shape(K);
   if (st != MI355X_FP8_OK) return st;
@@ -4420,12 +4454,12 @@ int mi355x_fp8_rowwise_grouped_gemm(const void* a, const void* b, const float* a
   p.lda = lda; p.ldb = ldb; p.ldc = ldc;
   p.tiles_m = p.tiles_n = 0; p.group_m = 1;
   p.splits = 1; p.steps_per_split = k_steps_of(K); p.partial = nullptr;
-  p.m_sizes = m_sizes; p.groups = (int)G; p.out_f16 = 0;
+  p.m_sizes = m_sizes; p.groups = (int)G; p.clear_rest = clear_rest != 0; p.out_f16 = 0;
   p.div_tiles_mul = p.div_tiles_shift = p.div_group_mul = p.div_group_shift = 0; p.stamps = nullptr;
   hipStream_t s = (hipStream_t)stream;
   const bool ktail = K % kStepK;
   switch (tile_config < 0 ? grouped_form(G, M, N, K) : kGroupedTiles) {
-    case kGroupedRows16: return launch_grouped_skinny<1, 2, 2, 8>(p, s);
+    case kGroupedRows16: return launch_grouped_skinny<1, 2, 2, 4>(p, s);
     case kGroupedRows32: return launch_grouped_skinny<2, 2, 2, 8>(p, s);
     case kGroupedRows64: return launch_grouped_skinny<4, 2, 2, 8>(p, s);
     case kGroupedStream128:
@@ -4484,7 +4518,7 @@ int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale
   p.lda = lda; p.ldb = ldb; p.ldc = ldc;
   p.tiles_m = p.tiles_n = 0; p.group_m = 1;
   p.splits = 1; p.steps_per_split = k_steps_of(K); p.partial = nullptr;
-  p.m_sizes = nullptr; p.groups = 0; p.out_f16 = 0;
+  p.m_sizes = nullptr; p.groups = 0; p.clear_rest = 0; p.out_f16 = 0;
   p.div_tiles_mul = p.div_tiles_shift = p.div_group_mul = p.div_group_shift = 0; p.stamps = nullptr;
   hipStream_t s = (hipStream_t)stream;
   const bool ktail = K % kStepK;

@@ -10,7 +10,6 @@
 #include <Python.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
-#include <ATen/ops/zeros.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -151,12 +150,12 @@ PyObject* gemm_grouped(PyObject* const* a, Py_ssize_t count) {
     out = operand(a[5]);
     if (!result(out, at::kBFloat16, m, n)) return nullptr;
   } else {
-    made = at::zeros({m, n}, at::TensorOptions().dtype(at::kBFloat16).device(xq->device()));
+    made = fresh({m, n}, at::kBFloat16, *xq);
   }
   void* stream = current_stream();
-  const bool ok = enqueue(mi355x_fp8_rowwise_grouped_gemm, xq->data_ptr(), wq->data_ptr(), f32(*xs), f32(*ws), (const int32_t*)sizes->data_ptr(),
+  const bool ok = enqueue(mi355x_fp8_rowwise_grouped_gemm_ex, xq->data_ptr(), wq->data_ptr(), f32(*xs), f32(*ws), (const int32_t*)sizes->data_ptr(),
                                            out->data_ptr(), groups, m, n, k, xq->stride(0), wq->stride(0), out->stride(0),
-                                           (int)config, stream);
+                                           (int)config, a[5] == Py_None, stream);
   if (!ok) return nullptr;
   if (a[5] == Py_None) return one(made);
   Py_INCREF(a[5]);

@@ -225,15 +225,17 @@ def fp8_gemm_rowwise_grouped(
     if group_a.stride(1) != 1 or group_b.stride(1) != 1:
         raise ValueError("group_a and group_b must be K-contiguous")
     if out is None:
-        out = torch.zeros((m, n), dtype=torch.bfloat16, device=group_a.device)
+        out = torch.empty((m, n), dtype=torch.bfloat16, device=group_a.device)
+        clear_rest = 1
     else:
+        clear_rest = 0
         _require_gpu(out, "out")
         if out.dtype != torch.bfloat16 or tuple(out.shape) != (m, n) or out.stride(1) != 1:
             raise ValueError("out must be bfloat16 [M,N] with unit column stride")
-    st = lib.mi355x_fp8_rowwise_grouped_gemm(
+    st = lib.mi355x_fp8_rowwise_grouped_gemm_ex(
         group_a.data_ptr(), group_b.data_ptr(), a_scale.data_ptr(), b_scale.data_ptr(), m_sizes.data_ptr(),
         out.data_ptr(), g, m, n, k, group_a.stride(0), group_b.stride(0), out.stride(0), tile_config,
-        _stream_ptr(),
+        clear_rest, _stream_ptr(),
     )
     _lib.check(st, "mi355x_fp8_rowwise_grouped_gemm")
     return out
