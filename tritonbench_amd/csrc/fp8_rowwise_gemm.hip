@@ -77,7 +77,6 @@ struct GemmParams {
   // (device memory) multiplied with rows [g*N, (g+1)*N) of B and scaled by b_scale[g*N + n]
   const int32_t* m_sizes;
   int groups;
-  int clear_rest;  // rows of C past the last group's are set to zero (else they are left alone)
   int out_f16;  // C holds IEEE binary16 instead of bf16 (same size, same stores)
   // tiled kernel, plain form: reciprocals of the two run-time divisors of the tile walk (the number
   // of tiles, and the tiles of a full group of tile rows), prepared on the host: see fast_div()
@@ -85,6 +84,10 @@ struct GemmParams {
   // tiled kernel: where every workgroup leaves its start and end readings of the shader clock and of
   // the constant 100 MHz clock (4 values per workgroup), or nullptr
   unsigned long long* stamps;
+  // grouped form: rows of C past the last group's are set to zero (else they are left alone). Last, because the others
+  // lie so that the kernels' argument fetch is a few wide loads: between `groups` and `out_f16` this field took it
+  // apart, with a wait between the pieces (1000x3000x4112, one round of workgroups: 22.67 -> 22.87 us)
+  int clear_rest;
 };
 
 extern thread_local char err[512];
@@ -175,7 +178,7 @@ __device__ __forceinline__ void fetch_arguments_now(const GemmParams& p) {
   asm volatile("" ::"s"(p.a), "s"(p.b), "s"(p.a_scale), "s"(p.b_scale), "s"(p.bias), "s"(p.c), "s"(p.M), "s"(p.N), "s"(p.K),
                "s"(p.lda), "s"(p.ldb), "s"(p.ldc), "s"(p.tiles_m), "s"(p.tiles_n), "s"(p.out_f16));
 }
-// the same for what only the tiled kernel and its second pass read
+
 // Grouped form: zeros into rows first .. M-1 of C, shared out over `of` workgroups of this launch (this one is number `who`).
 // As a fill of all of C in front of the launch it took a launch of its own and a write of everything that the product
 // then writes again (8192 x 4096: 10 us of 115).
@@ -191,6 +194,7 @@ __device__ __forceinline__ void clear_rows(const GemmParams& p, int first, int w
   }
 }
 
+// the same for what only the tiled kernel and its second pass read
 __device__ __forceinline__ void fetch_tiled_arguments_now(const GemmParams& p) {
   asm volatile("" ::"s"(p.splits), "s"(p.steps_per_split), "s"(p.partial), "s"(p.m_sizes), "s"(p.groups), "s"(p.div_tiles_mul),
                "s"(p.div_tiles_shift), "s"(p.div_group_mul), "s"(p.div_group_shift), "s"(p.stamps));
