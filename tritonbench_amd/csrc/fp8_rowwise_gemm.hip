@@ -1454,57 +1454,103 @@ void gemm_block_kernel(GemmParams p) {
   wait_loads<0>();  // (loads into LDS land before it is released)
 }
 
+constexpr int kFinalizeRows = 4;
+
 // Second pass of a split-K launch: sums the splits' partials in a fixed order (results do not
 // depend on scheduling), applies the scales and the bias and rounds to bf16. One thread per
-// 4 consecutive columns.
-__global__ __launch_bounds__(256) void splitk_finalize_kernel(GemmParams p) {
-  fetch_arguments_now(p);
-  fetch_tiled_arguments_now(p);
+// 4 consecutive columns of ROWS consecutive rows.
+// Bound by the partial planes' bytes where it is more than a round of workgroups, which needs loads in flight: every
+// row's loads of two splits (one row: four) are issued before the first is used. (One row a thread, a 64-bit division for its place and
+// two splits' loads one behind the other: 1024x8192, two splits, 22.6 us = 3.7 TB/s; with four
+// rows 15.6 = 5.4 TB/s.)
+template <int ROWS>
+__device__ __forceinline__ void splitk_finalize(const GemmParams& p) {
   const long quads_per_row = (p.N + 3) / 4;
   const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= quads_per_row * p.M) return;
-  const int m = (int)(idx / quads_per_row);
-  const int n = (int)(idx % quads_per_row) * 4;
+  if (idx >= quads_per_row * ((p.M + ROWS - 1) / ROWS)) return;
+  // (the division's factors belong to a quad index below 2^31; larger results divide in 64 bits)
+  const long row_group = p.div_group_mul ? (long)fast_div((int)idx, p.div_group_mul, p.div_group_shift) : idx / quads_per_row;
+  const int m0 = (int)row_group * ROWS;
+  const int n = (int)(idx - row_group * quads_per_row) * 4;
   const size_t plane = (size_t)p.M * p.N;
-  const float* src = p.partial + (size_t)m * p.N + n;
-  const bool vec = (p.N & 3) == 0;  // then n + 3 < N and every row start is 16-byte aligned
-  const float sa_m = p.a_scale[m];  // fetched beside the partial sums, not after them
-  v4f sum = {0.f, 0.f, 0.f, 0.f};
+  // (N a multiple of 4: n + 3 < N and every row start is 16-byte aligned. With several rows a thread it always is.)
+  const bool vec = ROWS > 1 || (p.N & 3) == 0;
+  const float* src[ROWS];
+  float sa[ROWS], sb[4];
+  uint16_t bias[4] = {0, 0, 0, 0};
+  v4f sum[ROWS];
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const int m = min(m0 + i, p.M - 1);  // (rows past the last one read it again)
+    src[i] = p.partial + (size_t)m * p.N + n;
+    sa[i] = p.a_scale[m];  // fetched beside the partial sums, not after them
+    sum[i] = (v4f){0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) sb[e] = p.b_scale[min(n + e, p.N - 1)];
+  if (p.bias)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bias[e] = p.bias[min(n + e, p.N - 1)];
   if (vec) {
-    // four splits' loads in flight at a time; added in split order, as the scalar form does
+    // added in split order, as the scalar form does
+    auto add = [&](int s, auto count) {
+      constexpr int COUNT = decltype(count)::value;
+      v4f part[COUNT][ROWS];
+#pragma unroll
+      for (int u = 0; u < COUNT; ++u)
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) part[u][i] = __builtin_nontemporal_load((const v4f*)(src[i] + (s + u) * plane));
+#pragma unroll
+      for (int u = 0; u < COUNT; ++u)
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) sum[i] += part[u][i];
+    };
     int s = 0;
-    for (; s + 4 <= p.splits; s += 4) {
-      v4f part[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) part[u] = __builtin_nontemporal_load((const v4f*)(src + (s + u) * plane));
-#pragma unroll
-      for (int u = 0; u < 4; ++u) sum += part[u];
-    }
-    for (; s < p.splits; ++s) sum += __builtin_nontemporal_load((const v4f*)(src + s * plane));
+    constexpr int BATCH = ROWS > 1 ? 2 : 4;
+    for (; s + BATCH <= p.splits; s += BATCH) add(s, std::integral_constant<int, BATCH>{});
+    const int rest = p.splits - s;
+    if (BATCH > 3 && rest == 3) add(s, std::integral_constant<int, 3>{});
+    else if (BATCH > 2 && rest == 2) add(s, std::integral_constant<int, 2>{});
+    else if (rest == 1) add(s, std::integral_constant<int, 1>{});
   } else {
     for (int s = 0; s < p.splits; ++s) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (n + e < p.N) sum[e] += src[s * plane + e];
+      for (int i = 0; i < ROWS; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < p.N) sum[i][e] += src[i][s * plane + e];
     }
   }
-  float r[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int ne = min(n + e, p.N - 1);
-    const float t = sum[e] * sa_m;
-    r[e] = p.bias ? __builtin_fmaf(t, p.b_scale[ne], bf16_to_f32(p.bias[ne])) : t * p.b_scale[ne];
+  for (int i = 0; i < ROWS; ++i) {
+    if (m0 + i >= p.M) break;
+    float r[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float t = sum[i][e] * sa[i];
+      r[e] = p.bias ? __builtin_fmaf(t, sb[e], bf16_to_f32(bias[e])) : t * sb[e];
+    }
+    const uint32_t lo = pack_out_x2(r[0], r[1], p.out_f16), hi = pack_out_x2(r[2], r[3], p.out_f16);
+    uint16_t* dst = p.c + (size_t)(m0 + i) * p.ldc + n;
+    if (n + 3 < p.N && ((p.ldc & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.c) & 7) == 0)) {
+      *(v2u*)dst = (v2u){lo, hi};
+    } else {
+      dst[0] = (uint16_t)lo;
+      if (n + 1 < p.N) dst[1] = (uint16_t)(lo >> 16);
+      if (n + 2 < p.N) dst[2] = (uint16_t)hi;
+      if (n + 3 < p.N) dst[3] = (uint16_t)(hi >> 16);
+    }
   }
-  const uint32_t lo = pack_out_x2(r[0], r[1], p.out_f16), hi = pack_out_x2(r[2], r[3], p.out_f16);
-  uint16_t* dst = p.c + (size_t)m * p.ldc + n;
-  if (n + 3 < p.N && ((p.ldc & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.c) & 7) == 0)) {
-    *(v2u*)dst = (v2u){lo, hi};
-  } else {
-    dst[0] = (uint16_t)lo;
-    if (n + 1 < p.N) dst[1] = (uint16_t)(lo >> 16);
-    if (n + 2 < p.N) dst[2] = (uint16_t)hi;
-    if (n + 3 < p.N) dst[3] = (uint16_t)(hi >> 16);
-  }
+}
+__global__ __launch_bounds__(256) void splitk_finalize_kernel(GemmParams p) {
+  fetch_arguments_now(p);
+  fetch_tiled_arguments_now(p);
+  splitk_finalize<1>(p);
+}
+__global__ __launch_bounds__(256) void splitk_finalize_rows_kernel(GemmParams p) {
+  fetch_arguments_now(p);
+  fetch_tiled_arguments_now(p);
+  splitk_finalize<kFinalizeRows>(p);
 }
 
 // ------------------------------------------------------------------------------------
@@ -3776,8 +3822,17 @@ int launch_tiled(GemmParams p, hipStream_t stream) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "tiled kernel launch: %s", hipGetErrorString(e));
   if (EPI == kEpiPartial) {
-    const long quads = (long)p.M * ((p.N + 3) / 4);
-    hipLaunchKernelGGL(splitk_finalize_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, p);
+    // Four rows a thread where one row each would be more workgroups than the chip holds at once (8 of 256 lanes on a
+    // CU): fewer of them to start, more loads in flight each. Below that they would leave CUs idle. (Rows of partials that
+    // start off 16 bytes are read element by element, one row a thread.)
+    const long quads_per_row = ((long)p.N + 3) / 4;
+    const bool many = p.N % 4 == 0 && (quads_per_row * p.M + 255) / 256 > 8L * kNumCu;
+    const long quads = quads_per_row * (many ? ((long)p.M + kFinalizeRows - 1) / kFinalizeRows : p.M);
+    GemmParams f = p;
+    f.div_group_mul = f.div_group_shift = 0;
+    if (quads <= (long)INT32_MAX - 255) make_fast_div((uint32_t)quads_per_row, f.div_group_mul, f.div_group_shift);
+    hipLaunchKernelGGL(many ? splitk_finalize_rows_kernel : splitk_finalize_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0,
+                       stream, f);
     e = hipGetLastError();
     if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "split-K finalize launch: %s", hipGetErrorString(e));
   }
