@@ -76,3 +76,22 @@ def test_streaming_forms_against_float64(gpu_device, m, n, k):
 def test_rotated_walk_against_float64(gpu_device, m, n, k):
     print(f"case m={m} n={n} k={k}", flush=True)
     _check(m, n, k, gpu_device)
+
+
+# An infinite factor (what the block quantiser returns for a block that holds an infinity) in the last K block, against products that
+# are not zero: the result is that infinity in every form, also where a step of K reaches past the last block.
+@pytest.mark.parametrize("side", ["a", "b"])
+@pytest.mark.parametrize("m,n,k", [(16, 130, 96), (33, 515, 1040), (48, 640, 3008), (64, 9999, 4112), (30, 10007, 2000), (16, 5000, 8192),
+                                   (128, 2300, 6656), (200, 1030, 2064), (256, 4090, 528), (77, 26001, 2064), (300, 700, 528),
+                                   (4096, 4096, 96), (4350, 4100, 384)])
+def test_an_infinite_factor_of_the_last_block(gpu_device, m, n, k, side):
+    print(f"case m={m} n={n} k={k} {side}", flush=True)
+    one = torch.ones(1, device=gpu_device).to(torch.float8_e4m3fn)
+    xq, wq = one.expand(m * k).clone().view(m, k), one.expand(n * k).clone().view(n, k)
+    xs = torch.ones((-(-m // 128), -(-k // 128)), device=gpu_device)
+    ws = torch.ones((-(-n // 128), -(-k // 128)), device=gpu_device)
+    (xs if side == "a" else ws)[0, -1] = float("inf")
+    want = torch.full((m, n), float(k), dtype=torch.float64, device=gpu_device)
+    want[(slice(0, 128), slice(None)) if side == "a" else (slice(None), slice(0, 128))] = float("inf")
+    got = ops.fp8_gemm_blockwise(xq, wq, xs, ws)
+    assert torch.equal(got, want.to(torch.bfloat16))

@@ -2497,7 +2497,6 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(GemmParams p) {
         }
       }
     };
-    // (a slab past K: its products are zero, any factor will do)
     auto add_scaled = [&](float fa, const float (&flo)[NB], const float (&fhi)[NB]) {
 #pragma unroll
       for (int jb = 0; jb < NB; ++jb) {
@@ -2518,12 +2517,14 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(GemmParams p) {
     for (int s = 0; s < ksteps; ++s) {
       float f_a = 0.f, f_lo[NB] = {}, f_hi[NB] = {};
       if (BLOCK) {
-        const int kb = min(step_of(s) * 4 + wave, k_blocks - 1);
-        f_a = block_a[kb];
+        // (a slab past K: its products are zero, and so are its factors: the last block's may be infinite)
+        const int block = step_of(s) * 4 + wave, kb = min(block, k_blocks - 1);
+        const bool inside = block < k_blocks;
+        f_a = inside ? block_a[kb] : 0.0f;
 #pragma unroll
         for (int jb = 0; jb < NB; ++jb) {
-          f_lo[jb] = block_lo[jb][kb];
-          f_hi[jb] = block_hi[jb][kb];
+          f_lo[jb] = inside ? block_lo[jb][kb] : 0.0f;
+          f_hi[jb] = inside ? block_hi[jb][kb] : 0.0f;
         }
       }
       read_half(s, 1, fb1, fa1);
