@@ -50,3 +50,15 @@ def test_forms_against_float64(gpu_device, m, n, k, out_dtype):
     guard = canvas.clone()
     guard[1:-1, 2:-3] = 7.0
     assert (guard == 7.0).all()
+
+
+# more columns than a launch of the streaming form holds lanes for (512 lanes for 16 columns, 2^32 lanes)
+@pytest.mark.parametrize("m,n", [(1, 2**27 + 40), (1, 2**27 - 16), (3, 2**27)])
+def test_columns_beyond_the_streaming_forms_grid(gpu_device, m, n):
+    print(f"case m={m} n={n} k=1", flush=True)
+    b = torch.arange(n, device=gpu_device, dtype=torch.int64).remainder_(13).to(torch.uint8).add_(0x38).view(torch.float8_e4m3fn).view(n, 1)
+    a = torch.ones((m, 1), device=gpu_device).to(torch.float8_e4m3fn)
+    sa, sb = torch.ones(m, device=gpu_device), torch.ones(n, device=gpu_device)
+    got = ops.fp8_gemm_rowwise(a, b, sa, sb)
+    torch.cuda.synchronize()
+    assert torch.equal(got, b.to(torch.bfloat16).view(1, n).expand(m, n))

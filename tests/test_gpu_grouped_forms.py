@@ -105,3 +105,14 @@ def test_a_result_made_by_the_call_is_zero_past_the_groups(gpu_device, g, m, n, 
         got = ops.fp8_gemm_rowwise_grouped(x, w, ms, xs, ws, tile_config=config)
         assert torch.equal(got, want), config
         got.fill_(float("nan"))
+
+
+def test_columns_beyond_the_16_row_forms_grid(gpu_device):
+    g, m, n, k = 256, 256, 2200000, 16  # (a column tile of 32 and a row block of 16 are 256 lanes, 2^32 a launch)
+    x = torch.ones((m, k), device=gpu_device).to(torch.float8_e4m3fn)
+    w = torch.full((g * n * k,), 0x38, dtype=torch.uint8, device=gpu_device).view(torch.float8_e4m3fn).view(g * n, k)
+    scale = torch.arange(g, device=gpu_device, dtype=torch.float32).add_(1)
+    ms = torch.ones(g, dtype=torch.int32, device=gpu_device)
+    got = ops.fp8_gemm_rowwise_grouped(x, w, ms, torch.ones(m, device=gpu_device), scale.repeat_interleave(n))
+    torch.cuda.synchronize()
+    assert torch.equal(got, (scale * k).to(torch.bfloat16)[:, None].expand(m, n))

@@ -3379,6 +3379,10 @@ int fail(int code, const char* fmt, ...) {
 
 constexpr int kSkinnyMaxM = 64;
 
+// A launch holds fewer than 2^32 lanes. Kernels whose grid grows with an operand (rather than with the chip) are taken
+// only where theirs does; beyond, the form with the next larger tiles runs.
+constexpr bool grid_fits(int64_t workgroups, int64_t lanes) { return workgroups * lanes <= (int64_t)UINT32_MAX; }
+
 int check_shape(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || N < 1 || K < 1) return fail(MI355X_FP8_EINVAL, "M, N, K must be >= 1 (got %lld, %lld, %lld)",
                                            (long long)M, (long long)N, (long long)K);
@@ -3914,6 +3918,12 @@ int launch_skinny(const GemmParams& p, hipStream_t stream) {
 
 // The grouped form for few rows a group. The most row blocks any sizes can give: every group that has rows at all
 // wastes at most all but one row of a block.
+constexpr int64_t grouped_row_blocks(int64_t G, int64_t M, int bm, bool clear_rest) {
+  // (one more where rows past the groups' are to be cleared, so that there is a surplus to do it)
+  return (M + (int64_t)(bm - 1) * (G < M ? G : M)) / bm + (clear_rest ? 1 : 0);
+}
+constexpr int64_t grouped_column_tiles(int64_t N, int bn) { return ((N + bn - 1) / bn + kNumXcd - 1) / kNumXcd * kNumXcd; }
+
 template <int MT, int NTW, int DEPTH, int KW>
 int launch_grouped_skinny(const GemmParams& p, hipStream_t stream) {
   constexpr int BM = 16 * MT, BN = 16 * NTW;
@@ -3923,10 +3933,8 @@ int launch_grouped_skinny(const GemmParams& p, hipStream_t stream) {
   (void)LdsLimit<kern, lds_bytes>::registered;
   GemmParams q = p;
   q.tiles_n = (p.N + BN - 1) / BN;
-  const long tiles = (q.tiles_n + kNumXcd - 1) / kNumXcd * kNumXcd;
-  // (one more where rows past the groups' are to be cleared, so that there is a surplus to do it)
-  const long row_blocks = ((long)p.M + (long)(BM - 1) * (p.groups < p.M ? p.groups : p.M)) / BM + (p.clear_rest ? 1 : 0);
-  if (tiles * row_blocks > (long)INT32_MAX) return fail(MI355X_FP8_ENOTSUP, "more than 2^31-1 workgroups");
+  const int64_t tiles = grouped_column_tiles(p.N, BN), row_blocks = grouped_row_blocks(p.groups, p.M, BM, p.clear_rest != 0);
+  if (!grid_fits(tiles * row_blocks, KW * 64)) return fail(MI355X_FP8_ENOTSUP, "more lanes than a launch holds");
   if (const int st = ready_device()) return st;
   hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * row_blocks)), dim3(KW * 64), lds_bytes, stream, q);
   hipError_t e = hipGetLastError();
@@ -3951,9 +3959,13 @@ int launch_grouped_skinny(const GemmParams& p, hipStream_t stream) {
 //   with 128 rows 88 -> 73 (128x128 tiles with the streaming policy 99), 8 of 14336x4096 145 -> 109, 16 of 7168x2048
 //   72 -> 63. (Fewer than 128 of them: 8 groups of 2048x7168 42 -> 57.)
 enum GroupedForm { kGroupedTiles, kGroupedRows16, kGroupedRows32, kGroupedRows64, kGroupedStream128, kGroupedStream256 };
+constexpr bool grouped_rows16_fits(int64_t G, int64_t M, int64_t N) {
+  return grid_fits(grouped_column_tiles(N, 32) * grouped_row_blocks(G, M, 16, true), 256);
+}
+static_assert(!grouped_rows16_fits(256, 256, 2200000) && grouped_rows16_fits(256, 2048, 57344), "a column tile and row block are 256 lanes");
 inline GroupedForm grouped_form(int64_t G, int64_t M, int64_t N, int64_t K) {
   const bool rows_forms = G <= 256;  // (a workgroup's look-up goes over 64 groups at a time, the tiled kernel's once a launch)
-  if (M <= 8 * G && rows_forms) return kGroupedRows16;
+  if (M <= 8 * G && rows_forms && grouped_rows16_fits(G, M, N)) return kGroupedRows16;
   const int64_t tiles_128 = G * ((N + 127) / 128), tiles_256 = G * ((N + 255) / 256);
   if (rows_forms && K >= 4096 && tiles_128 <= 128 && M <= 32 * G) return M <= 16 * G ? kGroupedRows32 : kGroupedRows64;
   if (K < 2048 || M > 128 * G) return kGroupedTiles;
@@ -4047,6 +4059,9 @@ int launch_any(GemmParams p, hipStream_t stream) {
   return MI355X_FP8_OK;
 }
 
+// (the streaming kernel's unaligned form: 512 lanes for 16 columns)
+constexpr bool generic_streams(int64_t N) { return grid_fits((N + 15) / 16, 512); }
+static_assert(generic_streams(1 << 27) == false && generic_streams((1 << 27) - 16), "2^27 columns are 2^32 lanes");
 // The generic family: the streaming kernel's unaligned form up to 64 rows (measured cold: 1x8192x8191 14.4 us,
 // 16x8192x8191 19.1, 64x8192x8191 29.7, where 64x64 tiles take 33), tiles beyond. 128x128 tiles from two
 // rounds of the CUs on (4096x8192x8191 563 us = 977 TFLOP/s); below, 64x64 tiles. With at most one of
@@ -4055,9 +4070,11 @@ int launch_any(GemmParams p, hipStream_t stream) {
 // the second step's registers would cost one of them (517x3000x1041 13.9 -> 12.7, 1024x2048x1025 13.7 -> 12.5).
 int launch_generic(const GemmParams& p, hipStream_t s) {
   if (p.M > 65535 * 64) return fail(MI355X_FP8_ENOTSUP, "the generic family takes M <= %d", 65535 * 64);
-  if (p.M <= 16) return launch_skinny<1, 1, 4, 8, true>(p, s);
-  if (p.M <= 32) return launch_skinny<2, 1, 2, 8, true>(p, s);
-  if (p.M <= 64) return launch_skinny<4, 2, 2, 8, true>(p, s);
+  if (p.M <= kSkinnyMaxM && generic_streams(p.N)) {
+    if (p.M <= 16) return launch_skinny<1, 1, 4, 8, true>(p, s);
+    if (p.M <= 32) return launch_skinny<2, 1, 2, 8, true>(p, s);
+    return launch_skinny<4, 2, 2, 8, true>(p, s);
+  }
   auto tiles = [&](long edge) { return ((p.M + edge - 1) / edge) * ((p.N + edge - 1) / edge); };
   if (tiles(128) >= 2 * kNumCu) return launch_any<128, 128, 1>(p, s);
   return tiles(64) <= kNumCu ? launch_any<64, 64, 2>(p, s) : launch_any<64, 64, 1>(p, s);
@@ -4420,6 +4437,10 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
 namespace {
 constexpr int kWaveRows = 4;
 
+// (more rows than a launch of 1024 lanes each holds keep 256 lanes, which read the rest of a long row twice)
+constexpr bool quantize_any_long(int64_t R, int64_t chunks) { return chunks > 4 * 256 && grid_fits(R, 1024); }
+static_assert(quantize_any_long(4194303, 1025) && !quantize_any_long(8388608, 1025), "512 lanes a row reach 2^32 at 8388608 rows");
+
 // The quantiser on rows that do not start 16-byte aligned or do not hold whole 16-byte chunks: the vector kernel's
 // unaligned forms, by the same lines as the aligned ones (fewer of them: this is the rare case). The element-by-element
 // kernel, which ran them all before, is left for rows shorter than one chunk. Measured, sources rotated through memory, before
@@ -4433,11 +4454,12 @@ void launch_quantize_any(const SrcT* x, uint8_t* xq, float* inv_scale, int64_t R
   auto go = [&](auto kern, int64_t grid, int threads) {
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3((unsigned)threads), 0, s, x, xq, inv_scale, (int)K, (long)ldx, (long)ldq, (long)R);
   };
+  const bool long_row = quantize_any_long(R, chunks);
   if (K < epv) {
     hipLaunchKernelGGL(quantize_rows_kernel<SrcT>, dim3((unsigned)R), dim3(256), 0, s, x, xq, inv_scale, (int)K, (long)ldx, (long)ldq);
   } else if (chunks <= 8 * 64 && R > 2048) {
     go(quantize_rows_vec_kernel<SrcT, 8, 64, kWaveRows, true>, (R + kWaveRows - 1) / kWaveRows, 64 * kWaveRows);
-  } else if (chunks <= 4 * 256) {
+  } else if (!long_row) {
     go(quantize_rows_vec_kernel<SrcT, 4, 256, 1, true>, R, 256);
   } else if (chunks <= 8 * 512) {
     go(quantize_rows_vec_kernel<SrcT, 8, 512, 1, true>, R, 512);
