@@ -710,11 +710,16 @@ void gemm_tiled_kernel(GemmParams p) {
     for (int r = 0; r < SC_REGS; ++r) {
       const int kb = min(r * 64 + lane, k_steps - 1);
       sc[r] = factor(kb);
-      rt[r] = factor(kb > 0 ? kb - 1 : k_steps - 1) / sc[r];  // (a rotated walk passes from the last step to the first)
+      if (STREAM_B) rt[r] = factor(kb > 0 ? kb - 1 : k_steps - 1) / sc[r];  // (a rotated walk passes from the last step to the first)
+      else rt[r] = kb > 0 ? factor(kb - 1) / sc[r] : 1.0f;
     }
   };
-  auto lane_value = [&](const float (&regs)[SC_REGS], int kt) -> float {  // (kt at most k_steps past the end)
-    if (kt >= k_steps) kt -= k_steps;
+  // (kt at most k_steps past the end. A walk that wraps around finds the first steps there; what lies past the end of one that
+  // does not is never used, and keeping to the last step costs less scalar work in every step: 721x528x1152 9.85 -> 9.54 us,
+  // 404x3104x464 7.44 -> 7.20.)
+  auto lane_value = [&](const float (&regs)[SC_REGS], int kt) -> float {
+    if (STREAM_B) kt = kt >= k_steps ? kt - k_steps : kt;
+    else kt = min(kt, k_steps - 1);
     const int r = kt >> 6;
     const float v = r == 0 ? regs[0] : r == 1 ? regs[1] : r == 2 ? regs[2] : regs[3];
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), kt & 63));
@@ -1065,7 +1070,7 @@ void gemm_tiled_kernel(GemmParams p) {
       if (t == B_LAST) advance_b(plain_tag);
       if (t == PREP_T) prepare_a_loads();
       if (BLOCKSCALE && t == PREP_T) {
-        n_pend = lane_value(rt, k_steps == 1 ? 0 : kt_c + 2);
+        n_pend = lane_value(rt, STREAM_B && k_steps == 1 ? 0 : kt_c + 2);
         n_last = lane_value(sc, kt_c + 1);
       }
       if (t == PREP_T2) {
@@ -1106,7 +1111,7 @@ void gemm_tiled_kernel(GemmParams p) {
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (BLOCKSCALE) kt_c = kt_c + 1 == k_steps ? 0 : kt_c + 1;
+    if (BLOCKSCALE) kt_c = STREAM_B && kt_c + 1 == k_steps ? 0 : kt_c + 1;
   };
   auto read_first_half = [&]() {
 #pragma unroll
