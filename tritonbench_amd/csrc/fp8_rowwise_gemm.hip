@@ -67,7 +67,10 @@ struct GemmParams {
   int M, N, K;
   long lda, ldb, ldc;
   int tiles_m, tiles_n;
-  int group_m;           // tile rows walked together so an XCD's resident tiles share A and B panels
+  // grouped form: rows of C past the last group's are set to zero (else they are left alone). Here, because the others lie so
+  // that the kernels' argument fetch is a few wide loads: between `groups` and `out_f16` this field took it apart, with a
+  // wait between the pieces (1000x3000x4112, one round of workgroups: 22.67 -> 22.87 us)
+  int clear_rest;
   // split-K: every tile is cut into `splits` work items of `steps_per_split` 128-byte K steps
   // (the last one takes what is left); with splits > 1 the items write fp32 partial sums to
   // partial[split][M][N] and a second kernel adds them up and applies the epilogue
@@ -84,10 +87,6 @@ struct GemmParams {
   // tiled kernel: where every workgroup leaves its start and end readings of the shader clock and of
   // the constant 100 MHz clock (4 values per workgroup), or nullptr
   unsigned long long* stamps;
-  // grouped form: rows of C past the last group's are set to zero (else they are left alone). Last, because the others
-  // lie so that the kernels' argument fetch is a few wide loads: between `groups` and `out_f16` this field took it
-  // apart, with a wait between the pieces (1000x3000x4112, one round of workgroups: 22.67 -> 22.87 us)
-  int clear_rest;
 };
 
 extern thread_local char err[512];
@@ -205,7 +204,7 @@ __device__ __forceinline__ void fetch_tiled_arguments_now(const GemmParams& p) {
 //
 // Hardware hands consecutive workgroup ids to consecutive XCDs, each with a private L2.
 // Workgroup b therefore belongs to XCD b % 8 and is that XCD's slot b / 8. The tile list is
-// cut into 8 contiguous chunks, one per XCD, and walked in "grouped" order (group_m tile
+// cut into 8 contiguous chunks, one per XCD, and walked in "grouped" order (kGroupM tile
 // rows at a time, column-major inside a group) so the tiles an XCD has in flight at any
 // moment form a compact rectangle sharing A row panels and B column panels in its L2.
 // ------------------------------------------------------------------------------------
@@ -399,8 +398,11 @@ constexpr int tiled_waves_per_simd(int BM, int BN, int waves, bool blockscale, i
 // (measured: M=128, N=K=8192 27.6 -> 24.2 us, M=64 22.5 -> 19.6 us; with more tile rows the
 // panels are shared through the L2 and the same policy costs 5-8 %). The grouped form has it for groups of
 // about one tile row (grouped_form).
+// CLEAR: the grouped form that sets the rows of C past the last group's to zero. Instances of their own: with the test
+// and the loop in the others, which a call with a result of its own runs, those were 1-3 % slower (1704x1280x768 in 12 groups
+// 11.46 -> 11.76 us, 450x1024x576 6.47 -> 6.61).
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool KTAIL, int EPI, bool GROUPED = false, bool BLOCKSCALE = false,
-          int DIST = kDefaultDist, bool STREAM_B = false>
+          int DIST = kDefaultDist, bool STREAM_B = false, bool CLEAR = false>
 __global__ __launch_bounds__(WAVES_M* WAVES_N * 64)
 __attribute__((amdgpu_waves_per_eu(tiled_waves_per_simd(BM, BN, WAVES_M * WAVES_N, BLOCKSCALE, DIST),
                                    tiled_waves_per_simd(BM, BN, WAVES_M * WAVES_N, BLOCKSCALE, DIST))))
@@ -408,6 +410,7 @@ void gemm_tiled_kernel(GemmParams p) {
   constexpr int kStagesA = DIST, kStagesB = DIST + 1;
   static_assert(DIST >= 2 && tiled_lds_bytes(BM, BN, DIST) <= 160 * 1024, "the stage rings must fit the LDS");
   static_assert(!GROUPED || EPI == kEpiPlain, "the grouped form has neither bias nor split-K");
+  static_assert(!CLEAR || GROUPED, "only the grouped form has rows past its groups'");
   static_assert(!BLOCKSCALE || (128 % (BM / WAVES_M) == 0 && 128 % (BN / WAVES_N) == 0 && EPI == kEpiPlain && !GROUPED),
                 "a wave's tile must lie inside one 128x128 scale block: one factor per wave and step");
   constexpr bool HAS_BIAS = EPI == kEpiBias;
@@ -471,7 +474,7 @@ void gemm_tiled_kernel(GemmParams p) {
       total_tiles += ((mg + BM - 1) / BM) * p.tiles_n;
       rows += mg;
     }
-    if (p.clear_rest && rows < p.M) clear_rows(p, rows, (int)blockIdx.x, (int)gridDim.x);
+    if (CLEAR && rows < p.M) clear_rows(p, rows, (int)blockIdx.x, (int)gridDim.x);
   }
   const TileWalk walk = make_walk(total_tiles * p.splits);
   if (walk.slot >= walk.chunk_len) return;  // uniform over the workgroup
@@ -3811,21 +3814,20 @@ int mi355x_shared::ready_device(int* dev_out) {
 
 namespace {
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool KTAIL, int EPI, bool GROUPED = false, bool BLOCKSCALE = false,
-          int DIST = kDefaultDist, bool STREAM_B = false>
+          int DIST = kDefaultDist, bool STREAM_B = false, bool CLEAR = false>
 int launch_tiled(GemmParams p, hipStream_t stream) {
   constexpr int threads = WAVES_M * WAVES_N * 64;
   constexpr size_t lds_bytes = tiled_lds_bytes(BM, BN, DIST);
   // grouped: the group sizes live on the device; every group adds at most one partial tile row
   p.tiles_m = GROUPED ? p.M / BM + p.groups : (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
-  p.group_m = kGroupM;
   make_fast_div((uint32_t)p.tiles_m * (uint32_t)p.tiles_n, p.div_tiles_mul, p.div_tiles_shift);
   make_fast_div((uint32_t)kGroupM * (uint32_t)p.tiles_n, p.div_group_mul, p.div_group_shift);
   const long total = (long)p.tiles_m * p.tiles_n * p.splits;
   if (total > (long)INT32_MAX) return fail(MI355X_FP8_ENOTSUP, "more than 2^31-1 work items");
   const long slots = (long)kNumCu * tiled_wgs_per_cu(BM, BN, DIST);
   long grid = total < slots ? ((total + kNumXcd - 1) / kNumXcd) * kNumXcd : slots;
-  constexpr auto kern = gemm_tiled_kernel<BM, BN, WAVES_M, WAVES_N, KTAIL, EPI, GROUPED, BLOCKSCALE, DIST, STREAM_B>;
+  constexpr auto kern = gemm_tiled_kernel<BM, BN, WAVES_M, WAVES_N, KTAIL, EPI, GROUPED, BLOCKSCALE, DIST, STREAM_B, CLEAR>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   if (const int st = ready_device()) return st;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), lds_bytes, stream, p);
@@ -3945,6 +3947,16 @@ int launch_grouped_skinny(const GemmParams& p, hipStream_t stream) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "grouped skinny kernel launch: %s", hipGetErrorString(e));
   return MI355X_FP8_OK;
+}
+
+// The grouped form of the tiled kernel.
+template <int BM, int BN, int DIST, bool STREAM_B>
+int launch_grouped_tiles(const GemmParams& p, hipStream_t s) {
+  if (p.clear_rest)
+    return p.K % kStepK ? launch_tiled<BM, BN, 2, 2, true, kEpiPlain, true, false, DIST, STREAM_B, true>(p, s)
+                        : launch_tiled<BM, BN, 2, 2, false, kEpiPlain, true, false, DIST, STREAM_B, true>(p, s);
+  return p.K % kStepK ? launch_tiled<BM, BN, 2, 2, true, kEpiPlain, true, false, DIST, STREAM_B>(p, s)
+                      : launch_tiled<BM, BN, 2, 2, false, kEpiPlain, true, false, DIST, STREAM_B>(p, s);
 }
 
 // Which form runs a grouped launch whose groups are up to a tile high on average: such a launch is bound by the
@@ -4355,7 +4367,7 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
   p.bias = (const uint16_t*)bias; p.c = (uint16_t*)c;
   p.M = (int)M; p.N = (int)N; p.K = (int)K;
   p.lda = lda; p.ldb = ldb; p.ldc = ldc;
-  p.tiles_m = p.tiles_n = 0; p.group_m = 1;
+  p.tiles_m = p.tiles_n = 0;
   p.splits = 1; p.steps_per_split = k_steps_of(K); p.partial = nullptr;
   p.m_sizes = nullptr; p.groups = 0; p.clear_rest = 0; p.out_f16 = out_type == MI355X_FP8_OUT_F16;
   p.div_tiles_mul = p.div_tiles_shift = p.div_group_mul = p.div_group_shift = 0; p.stamps = stamps;
@@ -4539,22 +4551,17 @@ int mi355x_fp8_rowwise_grouped_gemm_ex(const void* a, const void* b, const float
   p.bias = nullptr; p.c = (uint16_t*)c;
   p.M = (int)M; p.N = (int)N; p.K = (int)K;
   p.lda = lda; p.ldb = ldb; p.ldc = ldc;
-  p.tiles_m = p.tiles_n = 0; p.group_m = 1;
+  p.tiles_m = p.tiles_n = 0;
   p.splits = 1; p.steps_per_split = k_steps_of(K); p.partial = nullptr;
   p.m_sizes = m_sizes; p.groups = (int)G; p.clear_rest = clear_rest != 0; p.out_f16 = 0;
   p.div_tiles_mul = p.div_tiles_shift = p.div_group_mul = p.div_group_shift = 0; p.stamps = nullptr;
   hipStream_t s = (hipStream_t)stream;
-  const bool ktail = K % kStepK;
   switch (tile_config < 0 ? grouped_form(G, M, N, K) : kGroupedTiles) {
     case kGroupedRows16: return launch_grouped_skinny<1, 2, 2, 4>(p, s);
     case kGroupedRows32: return launch_grouped_skinny<2, 2, 2, 8>(p, s);
     case kGroupedRows64: return launch_grouped_skinny<4, 2, 2, 8>(p, s);
-    case kGroupedStream128:
-      return ktail ? launch_tiled<128, 128, 2, 2, true, kEpiPlain, true, false, kDefaultDist, true>(p, s)
-                   : launch_tiled<128, 128, 2, 2, false, kEpiPlain, true, false, kDefaultDist, true>(p, s);
-    case kGroupedStream256:
-      return ktail ? launch_tiled<128, 256, 2, 2, true, kEpiPlain, true, false, kDefaultDist, true>(p, s)
-                   : launch_tiled<128, 256, 2, 2, false, kEpiPlain, true, false, kDefaultDist, true>(p, s);
+    case kGroupedStream128: return launch_grouped_tiles<128, 128, kDefaultDist, true>(p, s);
+    case kGroupedStream256: return launch_grouped_tiles<128, 256, kDefaultDist, true>(p, s);
     default: break;
   }
   // Large tiles when an average group fills most of one and there are enough of them for every
@@ -4568,14 +4575,9 @@ int mi355x_fp8_rowwise_grouped_gemm_ex(const void* a, const void* b, const float
     const int64_t tiles_256 = (M / 256) * (N / 256), tiles_128 = (M / 256) * (N / 128);
     tile_config = rows_fill && tiles_256 >= 192 ? 0 : rows_fill && tiles_128 >= 192 && tiles_128 <= 288 && K >= 4096 ? 2 : 1;
   }
-  if (tile_config == 0)
-    return ktail ? launch_tiled<256, 256, 2, 2, true, kEpiPlain, true>(p, s)
-                 : launch_tiled<256, 256, 2, 2, false, kEpiPlain, true>(p, s);
-  if (tile_config == 2)
-    return ktail ? launch_tiled<256, 128, 2, 2, true, kEpiPlain, true, false, 3>(p, s)
-                 : launch_tiled<256, 128, 2, 2, false, kEpiPlain, true, false, 3>(p, s);
-  return ktail ? launch_tiled<128, 128, 2, 2, true, kEpiPlain, true>(p, s)
-               : launch_tiled<128, 128, 2, 2, false, kEpiPlain, true>(p, s);
+  if (tile_config == 0) return launch_grouped_tiles<256, 256, kDefaultDist, false>(p, s);
+  if (tile_config == 2) return launch_grouped_tiles<256, 128, 3, false>(p, s);
+  return launch_grouped_tiles<128, 128, kDefaultDist, false>(p, s);
 }
 
 int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale, const float* b_scale,
@@ -4603,7 +4605,7 @@ int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale
   p.bias = nullptr; p.c = (uint16_t*)c;
   p.M = (int)M; p.N = (int)N; p.K = (int)K;
   p.lda = lda; p.ldb = ldb; p.ldc = ldc;
-  p.tiles_m = p.tiles_n = 0; p.group_m = 1;
+  p.tiles_m = p.tiles_n = 0;
   p.splits = 1; p.steps_per_split = k_steps_of(K); p.partial = nullptr;
   p.m_sizes = nullptr; p.groups = 0; p.clear_rest = 0; p.out_f16 = 0;
   p.div_tiles_mul = p.div_tiles_shift = p.div_group_mul = p.div_group_shift = 0; p.stamps = nullptr;
