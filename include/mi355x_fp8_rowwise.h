@@ -255,6 +255,17 @@ int mi355x_fp8_rowwise_grouped_gemm_ex(const void* a, const void* b,
                                        int64_t lda, int64_t ldb, int64_t ldc,
                                        int tile_config, int clear_rest, void* stream);
 
+/* The form a grouped call with tile_config -1 runs, or a negative status. Pure host arithmetic: lets tests and timing
+ * audits see the choice. TILES: one of the tile configurations; ROWS_<n>: every group cut into blocks of n rows whose
+ * workgroups stream B; STREAM_<n>: tiles of 128 rows and n columns that fetch B with the streaming cache policy. */
+#define MI355X_FP8_GROUPED_TILES      0
+#define MI355X_FP8_GROUPED_ROWS_16    1
+#define MI355X_FP8_GROUPED_ROWS_32    2
+#define MI355X_FP8_GROUPED_ROWS_64    3
+#define MI355X_FP8_GROUPED_STREAM_128 4
+#define MI355X_FP8_GROUPED_STREAM_256 5
+int mi355x_fp8_rowwise_grouped_form(int64_t G, int64_t M, int64_t N, int64_t K);
+
 /*
  * Block-scaled form: one scale per 128x128 block of A and of B,
  *
@@ -274,6 +285,23 @@ int mi355x_fp8_blockwise_gemm(const void* a, const void* b,
                               const float* a_scale, const float* b_scale, void* c,
                               int64_t M, int64_t N, int64_t K,
                               int64_t lda, int64_t ldb, int64_t ldc, void* stream);
+
+/*
+ * The same with the form pinned (-1: the library's choice, which mi355x_fp8_blockwise_form names without a device):
+ * ONE_TILE (M <= 64) and NARROW (the shapes of MI355X_FP8_SKINNY_NARROW) are the streaming forms of the row-wise product,
+ * TILES_128, TILES_128_STREAM (B fetched with the streaming cache policy) and TILES_256 take any shape. ENOTSUP for a
+ * shape the named form does not take.
+ */
+#define MI355X_FP8_BLOCK_ONE_TILE         0
+#define MI355X_FP8_BLOCK_NARROW           1
+#define MI355X_FP8_BLOCK_TILES_128        2
+#define MI355X_FP8_BLOCK_TILES_128_STREAM 3
+#define MI355X_FP8_BLOCK_TILES_256        4
+int mi355x_fp8_blockwise_form(int64_t M, int64_t N, int64_t K);
+int mi355x_fp8_blockwise_gemm_ex(const void* a, const void* b,
+                                 const float* a_scale, const float* b_scale, void* c,
+                                 int64_t M, int64_t N, int64_t K,
+                                 int64_t lda, int64_t ldb, int64_t ldc, int form, void* stream);
 
 /*
  * Block-wise e4m3fn quantiser, replacing fp8_block_quantize

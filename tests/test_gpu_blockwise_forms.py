@@ -3,7 +3,8 @@ float64. Needs an MI355X."""
 import pytest
 import torch
 
-from tritonbench_amd import ops
+from tritonbench_amd import _lib, ops
+from tritonbench_amd._lib import BLOCK_NARROW, BLOCK_ONE_TILE, BLOCK_TILES_128, BLOCK_TILES_128_STREAM, BLOCK_TILES_256
 
 pytestmark = pytest.mark.gpu
 
@@ -13,7 +14,24 @@ def _expand(codes, scales):
     return codes.double() * s[: codes.shape[0], : codes.shape[1]]
 
 
-def _check(m, n, k, dev, seed=0):
+def _run(xq, wq, xs, ws, out, form):
+    """The product in `form`, whatever the library would choose for the shape (None: its choice, through the wrapper)."""
+    if form is None:
+        return ops.fp8_gemm_blockwise(xq, wq, xs, ws, out=out)
+    m, k = xq.shape
+    st = _lib.load().mi355x_fp8_blockwise_gemm_ex(
+        xq.data_ptr(), wq.data_ptr(), xs.data_ptr(), ws.data_ptr(), out.data_ptr(), m, wq.shape[0], k, xq.stride(0), wq.stride(0),
+        out.stride(0), form, torch.cuda.current_stream().cuda_stream)
+    _lib.check(st, "mi355x_fp8_blockwise_gemm_ex")
+    return out
+
+
+def _streaming_forms(m, n):
+    """The streaming forms that take the shape: one tile a workgroup up to 64 rows, narrow tiles where the row-wise ones go."""
+    return ([BLOCK_ONE_TILE] if m <= 64 else []) + ([BLOCK_NARROW] if _lib.skinny_family_takes(m, n) else [])
+
+
+def _check(m, n, k, dev, form, seed=0):
     g = torch.Generator(device=dev).manual_seed(seed)
     gk = -(-k // 128)
     xq = torch.randn((m, k), generator=g, device=dev).to(torch.float8_e4m3fn)
@@ -28,7 +46,7 @@ def _check(m, n, k, dev, seed=0):
     canvas = torch.full((m + 2, n + 8), 7.0, dtype=torch.bfloat16, device=dev)
     aligned = n % 8 == 0
     out = canvas[1:-1, :n] if aligned else canvas[1:-1, 3 : n + 3]
-    ops.fp8_gemm_blockwise(xq, wq, xs, ws, out=out)
+    _run(xq, wq, xs, ws, out, form)
     torch.cuda.synchronize()
     a, b = _expand(xq, xs), _expand(wq, ws)
     exact = a @ b.t()
@@ -56,7 +74,7 @@ def _check(m, n, k, dev, seed=0):
                                    (4097, 13313, 640), (8200, 4104, 1040)])
 def test_large_tiles_against_float64(gpu_device, m, n, k):
     print(f"case m={m} n={n} k={k}", flush=True)
-    _check(m, n, k, gpu_device)
+    _check(m, n, k, gpu_device, BLOCK_TILES_256)
 
 
 # the streaming forms: rows around 16, 32, 48 and 64, tiles whose columns straddle two column blocks (20 and 40 columns a
@@ -66,8 +84,11 @@ def test_large_tiles_against_float64(gpu_device, m, n, k):
                                    (64, 2050, 1168), (16, 5000, 8192), (30, 10007, 2000), (64, 9999, 4112), (65, 515, 1040),
                                    (128, 2300, 6656), (200, 1030, 2064), (256, 4090, 528)])
 def test_streaming_forms_against_float64(gpu_device, m, n, k):
-    print(f"case m={m} n={n} k={k}", flush=True)
-    _check(m, n, k, gpu_device)
+    forms = _streaming_forms(m, n)
+    assert forms
+    for form in forms:
+        print(f"case m={m} n={n} k={k} form={form}", flush=True)
+        _check(m, n, k, gpu_device, form)
 
 
 # 128x128 tiles whose walk over K starts at a step of its own per tile column and wraps around (one tile row, wide panel): the
@@ -75,7 +96,29 @@ def test_streaming_forms_against_float64(gpu_device, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(100, 24600, 128), (128, 25000, 400), (77, 26001, 2064)])
 def test_rotated_walk_against_float64(gpu_device, m, n, k):
     print(f"case m={m} n={n} k={k}", flush=True)
-    _check(m, n, k, gpu_device)
+    _check(m, n, k, gpu_device, BLOCK_TILES_128_STREAM)
+
+
+# the library's own choice for a shape well inside each form's range, and that it is what runs: the same bits as the pinned form
+@pytest.mark.parametrize("m,n,k,form", [(1, 2304, 2048, BLOCK_ONE_TILE), (32, 8192, 8192, BLOCK_NARROW), (128, 8192, 8192, BLOCK_NARROW),
+                                        (64, 57344, 8192, BLOCK_TILES_128_STREAM), (512, 1024, 1024, BLOCK_TILES_128),
+                                        (4096, 4096, 4096, BLOCK_TILES_256)])
+def test_the_choice_runs_the_form_it_names(gpu_device, m, n, k, form):
+    assert _lib.load().mi355x_fp8_blockwise_form(m, n, k) == form
+    g = torch.Generator(device=gpu_device).manual_seed(7)
+    code = lambda r: torch.randn((r, k), generator=g, device=gpu_device).to(torch.float8_e4m3fn)
+    factors = lambda r: torch.rand((-(-r // 128), -(-k // 128)), generator=g, device=gpu_device) + 0.5
+    x, w, xs, ws = code(m), code(n), factors(m), factors(n)
+    out = torch.zeros((m, n), dtype=torch.bfloat16, device=gpu_device)
+    assert torch.equal(_run(x, w, xs, ws, None, None), _run(x, w, xs, ws, out, form))
+
+
+@pytest.mark.parametrize("m,n,form", [(65, 512, BLOCK_ONE_TILE), (257, 512, BLOCK_NARROW), (128, 20000, BLOCK_NARROW)])
+def test_a_form_refuses_what_it_does_not_take(gpu_device, m, n, form):
+    x, w = (torch.ones((r, 256), device=gpu_device).to(torch.float8_e4m3fn) for r in (m, n))
+    xs, ws = (torch.ones((-(-r // 128), 2), device=gpu_device) for r in (m, n))
+    with pytest.raises(NotImplementedError):
+        _run(x, w, xs, ws, torch.zeros((m, n), dtype=torch.bfloat16, device=gpu_device), form)
 
 
 # An infinite factor (what the block quantiser returns for a block that holds an infinity) in the last K block, against products that
@@ -93,5 +136,7 @@ def test_an_infinite_factor_of_the_last_block(gpu_device, m, n, k, side):
     (xs if side == "a" else ws)[0, -1] = float("inf")
     want = torch.full((m, n), float(k), dtype=torch.float64, device=gpu_device)
     want[(slice(0, 128), slice(None)) if side == "a" else (slice(None), slice(0, 128))] = float("inf")
-    got = ops.fp8_gemm_blockwise(xq, wq, xs, ws)
-    assert torch.equal(got, want.to(torch.bfloat16))
+    want = want.to(torch.bfloat16)
+    for form in [None, BLOCK_TILES_128, BLOCK_TILES_128_STREAM, BLOCK_TILES_256, *_streaming_forms(m, n)]:
+        got = torch.zeros((m, n), dtype=torch.bfloat16, device=gpu_device)
+        assert torch.equal(_run(xq, wq, xs, ws, got, form), want), form

@@ -105,6 +105,13 @@ SIGNATURES = {
         [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
          c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p],
     ),
+    "mi355x_fp8_rowwise_grouped_form": (c_int, [c_int64, c_int64, c_int64, c_int64]),
+    "mi355x_fp8_blockwise_form": (c_int, [c_int64, c_int64, c_int64]),
+    "mi355x_fp8_blockwise_gemm_ex": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+         c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_void_p],
+    ),
     "mi355x_fp8_blockwise_quantize": (
         c_int,
         [c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p],
@@ -125,6 +132,11 @@ SIGNATURES = {
 
 _lock = threading.Lock()
 _lib = None
+
+
+# forms of the block-scaled and of the grouped product, as the library names them
+BLOCK_ONE_TILE, BLOCK_NARROW, BLOCK_TILES_128, BLOCK_TILES_128_STREAM, BLOCK_TILES_256 = range(5)
+GROUPED_TILES, GROUPED_ROWS_16, GROUPED_ROWS_32, GROUPED_ROWS_64, GROUPED_STREAM_128, GROUPED_STREAM_256 = range(6)
 
 
 class LibraryNotBuilt(RuntimeError):

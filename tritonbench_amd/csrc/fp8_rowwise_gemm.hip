@@ -3975,7 +3975,14 @@ int launch_grouped_tiles(const GemmParams& p, hipStream_t s) {
 // * groups of 65 to 128 rows often are two tile rows high; 128x256 tiles then make fewer rounds: 16 groups of 4096x4096
 //   with 128 rows 88 -> 73 (128x128 tiles with the streaming policy 99), 8 of 14336x4096 145 -> 109, 16 of 7168x2048
 //   72 -> 63. (Fewer than 128 of them: 8 groups of 2048x7168 42 -> 57.)
-enum GroupedForm { kGroupedTiles, kGroupedRows16, kGroupedRows32, kGroupedRows64, kGroupedStream128, kGroupedStream256 };
+enum GroupedForm {
+  kGroupedTiles = MI355X_FP8_GROUPED_TILES,
+  kGroupedRows16 = MI355X_FP8_GROUPED_ROWS_16,
+  kGroupedRows32 = MI355X_FP8_GROUPED_ROWS_32,
+  kGroupedRows64 = MI355X_FP8_GROUPED_ROWS_64,
+  kGroupedStream128 = MI355X_FP8_GROUPED_STREAM_128,
+  kGroupedStream256 = MI355X_FP8_GROUPED_STREAM_256
+};
 constexpr bool grouped_rows16_fits(int64_t G, int64_t M, int64_t N) {
   return grid_fits(grouped_column_tiles(N, 32) * grouped_row_blocks(G, M, 16, true), 256);
 }
@@ -4024,7 +4031,13 @@ inline float block_large_cost_us(int64_t M, int64_t N, int64_t K) {
 // share out the K blocks of a tile: measured against 128x128 tiles 1x2304x2048 12.1 -> 3.4 us, 16x8192x8192 40.0 -> 13.6,
 // 16x2048x16384 76.8 -> 13.2, 32x8192x28672 142 -> 46, 64x4096x2048 12.2 -> 6.4, 128x8192x8192 42.9 -> 21.9,
 // 256x4096x4096 19.9 -> 12.2. Their times are those of the row-wise forms within 3 %, and so are the estimates.
-enum BlockForm { kBlockOneTile, kBlockNarrow, kBlockSmall, kBlockSmallStream, kBlockLarge };
+enum BlockForm {
+  kBlockOneTile = MI355X_FP8_BLOCK_ONE_TILE,
+  kBlockNarrow = MI355X_FP8_BLOCK_NARROW,
+  kBlockSmall = MI355X_FP8_BLOCK_TILES_128,
+  kBlockSmallStream = MI355X_FP8_BLOCK_TILES_128_STREAM,
+  kBlockLarge = MI355X_FP8_BLOCK_TILES_256
+};
 inline BlockForm block_form(int64_t M, int64_t N, int64_t K) {
   BlockForm best = block_streams(M, N) ? kBlockSmallStream : kBlockSmall;
   float cost = block_small_cost_us(M, N, K);
@@ -4580,9 +4593,31 @@ int mi355x_fp8_rowwise_grouped_gemm_ex(const void* a, const void* b, const float
   return launch_grouped_tiles<128, 128, kDefaultDist, false>(p, s);
 }
 
+int mi355x_fp8_rowwise_grouped_form(int64_t G, int64_t M, int64_t N, int64_t K) {
+  int st = check_shape(M, N, K);
+  if (st == MI355X_FP8_OK) st = check_fast_shape(K);
+  if (st != MI355X_FP8_OK) return st;
+  if (G < 1 || G > 65536) return fail(MI355X_FP8_EINVAL, "G must be in 1..65536 (got %lld)", (long long)G);
+  return grouped_form(G, M, N, K);
+}
+
+int mi355x_fp8_blockwise_form(int64_t M, int64_t N, int64_t K) {
+  int st = check_shape(M, N, K);
+  if (st == MI355X_FP8_OK) st = check_fast_shape(K);
+  if (st == MI355X_FP8_OK && K > 256 * kStepK)
+    st = fail(MI355X_FP8_ENOTSUP, "block-scaled form handles K <= %d (got %lld)", 256 * kStepK, (long long)K);
+  return st != MI355X_FP8_OK ? st : block_form(M, N, K);
+}
+
 int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale, const float* b_scale,
                               void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                               int64_t ldc, void* stream) {
+  return mi355x_fp8_blockwise_gemm_ex(a, b, a_scale, b_scale, c, M, N, K, lda, ldb, ldc, -1, stream);
+}
+
+int mi355x_fp8_blockwise_gemm_ex(const void* a, const void* b, const float* a_scale, const float* b_scale,
+                                 void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                                 int64_t ldc, int form, void* stream) {
   int st = check_shape(M, N, K);
   if (st == MI355X_FP8_OK) st = check_fast_shape(K);
   if (st != MI355X_FP8_OK) return st;
@@ -4611,7 +4646,10 @@ int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale
   p.div_tiles_mul = p.div_tiles_shift = p.div_group_mul = p.div_group_shift = 0; p.stamps = nullptr;
   hipStream_t s = (hipStream_t)stream;
   const bool ktail = K % kStepK;
-  switch (block_form(M, N, K)) {
+  if (form < 0) form = block_form(M, N, K);
+  else if ((form == kBlockOneTile && M > kSkinnyMaxM) || (form == kBlockNarrow && !narrow_fits(M, N, K)))
+    return fail(MI355X_FP8_ENOTSUP, "block-scaled form %d does not take %lldx%lld", form, (long long)M, (long long)N);
+  switch (form) {
     case kBlockNarrow: return launch_narrow_for<true>(p, s);
     case kBlockOneTile:
       if (M <= 16) return launch_skinny<1, 1, 4, 8, false, true>(p, s);
@@ -4622,9 +4660,10 @@ int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale
     case kBlockSmallStream:
       return ktail ? launch_tiled<128, 128, 2, 2, true, kEpiPlain, false, true, kDefaultDist, true>(p, s)
                    : launch_tiled<128, 128, 2, 2, false, kEpiPlain, false, true, kDefaultDist, true>(p, s);
-    default:
+    case kBlockSmall:
       return ktail ? launch_tiled<128, 128, 2, 2, true, kEpiPlain, false, true>(p, s)
                    : launch_tiled<128, 128, 2, 2, false, kEpiPlain, false, true>(p, s);
+    default: return fail(MI355X_FP8_EINVAL, "unknown block-scaled form %d", form);
   }
 }
 
