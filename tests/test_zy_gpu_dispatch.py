@@ -73,3 +73,60 @@ def test_automatic_choice_is_close_to_the_best_alternative(gpu_device, m, n, k, 
           f"bar {TOLERANCE:.2f}); " + ", ".join(f"{nm} {t:.1f}" for nm, t in times.items()), flush=True)
     assert auto <= TOLERANCE * times[best_name], (
         f"automatic choice takes {auto:.1f} us, '{best_name}' {times[best_name]:.1f} us: the cost tables need recalibrating")
+
+
+def _time_us(call, sets, burst_us=4000.0):
+    """Microseconds per call(i) over operand sets i: a captured graph of 16, the median of three bursts, on a stream of its own."""
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        call(0)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            for i in range(16):
+                call(i % sets)
+
+        def burst(replays):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record(stream)
+            for _ in range(replays):
+                graph.replay()
+            end.record(stream)
+            stream.synchronize()
+            return start.elapsed_time(end) * 1e3 / (16 * replays)
+
+        burst(1)
+        replays = max(1, int(burst_us / (16 * max(burst(1), 1.0))))
+        return sorted(burst(replays) for _ in range(3))[1]
+
+
+# the block-scaled forms: decode and prefill sizes, and wide panels with short rows or rows off the 128-byte lines, where the
+# streaming forms are behind the plain 128x128 tiles
+@pytest.mark.parametrize("m,n,k", [(1, 2304, 2048), (16, 8192, 8192), (32, 8192, 8192), (64, 57344, 8192), (128, 8192, 8192),
+                                   (512, 4096, 4096), (4096, 4096, 4096), (44, 87564, 32), (49, 18200, 64), (128, 100096, 256),
+                                   (128, 40064, 512), (64, 65536, 128), (9, 64149, 3952), (16, 58376, 4112), (1, 58376, 6688)])
+def test_block_scaled_choice_is_close_to_the_best_form(gpu_device, m, n, k):
+    lib = _lib.load()
+    g = torch.Generator(device=gpu_device).manual_seed(m + n + k)
+    codes = lambda r: torch.randn((r, k), generator=g, device=gpu_device, dtype=torch.bfloat16).to(torch.float8_e4m3fn)
+    factors = lambda r: torch.rand((-(-r // 128), -(-k // 128)), generator=g, device=gpu_device) + 0.5
+    count = min(8, max(2, 600_000_000 // (n * k)))
+    sets = [(codes(m), codes(n), factors(m), factors(n), torch.empty((m, n), dtype=torch.bfloat16, device=gpu_device)) for _ in range(count)]
+
+    def call(form):
+        def one(i):
+            x, w, xs, ws, out = sets[i]
+            _lib.check(lib.mi355x_fp8_blockwise_gemm_ex(x.data_ptr(), w.data_ptr(), xs.data_ptr(), ws.data_ptr(), out.data_ptr(), m, n, k,
+                                                        k, k, n, form, torch.cuda.current_stream().cuda_stream), "blockwise_gemm_ex")
+        return one
+    forms = [f for f in range(5) if (f != _lib.BLOCK_ONE_TILE or m <= 64) and (f != _lib.BLOCK_NARROW or _lib.skinny_family_takes(m, n))]
+    times, auto = {f: float("inf") for f in forms}, float("inf")
+    for rnd in range(4):
+        auto = min(auto, _time_us(call(-1), count))
+        for f in forms:
+            times[f] = min(times[f], _time_us(call(f), count))
+        if auto <= TOLERANCE * min(times.values()):
+            break
+    print(f"  {m}x{n}x{k}: form {lib.mi355x_fp8_blockwise_form(m, n, k)} {auto:.1f} us; " +
+          ", ".join(f"{f}: {t:.1f}" for f, t in times.items()), flush=True)
+    assert auto <= TOLERANCE * min(times.values())

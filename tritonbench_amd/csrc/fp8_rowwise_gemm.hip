@@ -4004,10 +4004,17 @@ inline GroupedForm grouped_form(int64_t G, int64_t M, int64_t N, int64_t K) {
 // One tile row against a wide panel is bound by the stream of B and fetches it with the streaming policy: K = 8192,
 // N = 57344 78 / 83 / 98 us with 16 / 64 / 128 rows (96 / 109 / 117 without the policy), N = 28672 48 with 64 rows (63);
 // with fewer workgroups it costs: 24x20480x5120 30.9 -> 31.9, 128x2304x6656 28 -> 34.
-inline bool block_streams(int64_t M, int64_t N) { return M <= 128 && N >= 192 * 128; }
-inline float block_small_cost_us(int64_t M, int64_t N, int64_t K) {
+// It also costs where rows do not start on 128-byte lines, which pieces of two neighbouring steps then share (K = 3952, 9 rows,
+// N = 64149 56 -> 68 us, K = 2640, 23 rows, N = 58574 43 -> 49), and on short rows (N = 65536, 64 rows: K = 128 6.7 -> 8.2, 512
+// 11.2 -> 12.9; 128 rows, K = 1024: 21.4 -> 22.1) against all but the largest panels (one row, K = 768: N = 65536 15.0 -> 13.3,
+// N = 40064 11.35 -> 11.8; 128 rows, N = 100096, K = 768 31.7 -> 29.2). From K = 2048 on it is never behind.
+inline bool block_streams(int64_t M, int64_t N, int64_t K, int64_t ldb) {
+  const int64_t large = (int64_t)(M <= 48 ? 36 : M <= 64 ? 48 : 72) << 20;
+  return M <= 128 && N >= 192 * 128 && ldb % kStepK == 0 && (K >= 2048 || N * K >= large);
+}
+inline float block_small_cost_us(int64_t M, int64_t N, int64_t K, int64_t ldb) {
   const float steps = (float)k_steps_of(K);
-  if (block_streams(M, N)) return fmaxf(5.0f + (float)N * (float)K * (1.0f + (float)M / 400.0f) / 6.4e6f, 6.0f + 0.62f * steps);
+  if (block_streams(M, N, K, ldb)) return fmaxf(5.0f + (float)N * (float)K * (1.0f + (float)M / 400.0f) / 6.4e6f, 6.0f + 0.62f * steps);
   const long tiles = ((M + 127) / 128) * ((N + 127) / 128), full = tiles / (2 * kNumCu), rest = tiles % (2 * kNumCu);
   // (one tile row: its steps wait for HBM, 16x8192x8192 40 us, 16x13312x13312 67)
   const float alone = M <= 128 ? 0.58f : 0.45f + 0.1f * (float)rest / (float)kNumCu;
@@ -4038,9 +4045,18 @@ enum BlockForm {
   kBlockSmallStream = MI355X_FP8_BLOCK_TILES_128_STREAM,
   kBlockLarge = MI355X_FP8_BLOCK_TILES_256
 };
-inline BlockForm block_form(int64_t M, int64_t N, int64_t K) {
-  BlockForm best = block_streams(M, N) ? kBlockSmallStream : kBlockSmall;
-  float cost = block_small_cost_us(M, N, K);
+// (One 16-row tile a workgroup, many of them on short rows: what bounds it is the rate at which they come and go, which the
+// row-wise estimate has too high there. us a workgroup beyond the first 256: 16x24576x256 2.9e-3, 16x24576x384 3.3e-3,
+// 24x31841x16 2.6e-3, 28x66614x208 3.7e-3, 44x87564x32 4.2e-3, 49x18200x64 (32 columns each) 13e-3, 64x65536x128 8.7e-3.)
+inline float block_one_tile_cost_us(int64_t M, int64_t N, int64_t K, float off_lines) {
+  const long wgs = (N + (M > 48 ? 31 : 15)) / (M > 48 ? 32 : 16);
+  const float steps = fminf((float)k_steps_of(K), 8.0f);
+  const float per_wg = (M <= 16 ? 2.4e-3f : M <= 32 ? 2.8e-3f : M <= 48 ? 4.1e-3f : 10.0e-3f) + 0.2e-3f * steps;
+  return fmaxf(off_lines * one_tile_cost_us(M, N, K), 3.0f + (wgs > kNumCu ? (float)(wgs - kNumCu) * per_wg : 0.0f));
+}
+inline BlockForm block_form(int64_t M, int64_t N, int64_t K, int64_t ldb) {
+  BlockForm best = block_streams(M, N, K, ldb) ? kBlockSmallStream : kBlockSmall;
+  float cost = block_small_cost_us(M, N, K, ldb);
   auto weigh = [&](BlockForm form, float us) {
     if (us < cost) {
       best = form;
@@ -4048,8 +4064,20 @@ inline BlockForm block_form(int64_t M, int64_t N, int64_t K) {
     }
   };
   weigh(kBlockLarge, block_large_cost_us(M, N, K));
-  if (M <= kSkinnyMaxM) weigh(kBlockOneTile, one_tile_cost_us(M, N, K));
-  if (narrow_fits(M, N, K)) weigh(kBlockNarrow, narrow_cost_us(M, N, K));
+  // Rows off the 128-byte lines against panels of several rounds of workgroups: every form fetches more than it uses. Times
+  // against the estimates: 128x128 tiles, K = 528 / 1104 / 2064 / 4112, 1.04 / 1.02 / 1.24 / 1.21 with 192 of them, 1.13 / 1.27 /
+  // 1.31 / 1.28 with 313, 1.19 / 1.39 / 1.47 / 1.38 with 457; one 16-row tile a workgroup, K = 2064 and 8240, 1.16 and 1.25
+  // with one row of A, 1.24 and 1.53 with 16; narrow tiles 1.1 whatever the sizes.
+  float one_tile_off = 1.0f, narrow_off = 1.0f;
+  if (ldb % kStepK != 0 && M <= 128 && N > 64 * kNumCu) {
+    const long rest = (N + 127) / 128 % (2 * kNumCu);
+    const float share = rest > kNumCu ? fminf(fmaxf((float)(K - 128) / 1400.0f, 0.0f), 1.0f) : K >= 1536 ? 1.0f : 0.1f;
+    cost *= 1.0f + share * (0.1f + (float)rest / 1300.0f);
+    one_tile_off = 1.2f + 0.035f * (float)(M < 8 ? M : 8) * fminf((float)K / 8192.0f, 1.0f);
+    narrow_off = 1.1f;
+  }
+  if (M <= kSkinnyMaxM) weigh(kBlockOneTile, block_one_tile_cost_us(M, N, K, one_tile_off));
+  if (narrow_fits(M, N, K)) weigh(kBlockNarrow, narrow_off * narrow_cost_us(M, N, K));
   return best;
 }
 
@@ -4606,7 +4634,7 @@ int mi355x_fp8_blockwise_form(int64_t M, int64_t N, int64_t K) {
   if (st == MI355X_FP8_OK) st = check_fast_shape(K);
   if (st == MI355X_FP8_OK && K > 256 * kStepK)
     st = fail(MI355X_FP8_ENOTSUP, "block-scaled form handles K <= %d (got %lld)", 256 * kStepK, (long long)K);
-  return st != MI355X_FP8_OK ? st : block_form(M, N, K);
+  return st != MI355X_FP8_OK ? st : block_form(M, N, K, K);
 }
 
 int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale, const float* b_scale,
@@ -4646,7 +4674,7 @@ int mi355x_fp8_blockwise_gemm_ex(const void* a, const void* b, const float* a_sc
   p.div_tiles_mul = p.div_tiles_shift = p.div_group_mul = p.div_group_shift = 0; p.stamps = nullptr;
   hipStream_t s = (hipStream_t)stream;
   const bool ktail = K % kStepK;
-  if (form < 0) form = block_form(M, N, K);
+  if (form < 0) form = block_form(M, N, K, ldb);
   else if ((form == kBlockOneTile && M > kSkinnyMaxM) || (form == kBlockNarrow && !narrow_fits(M, N, K)))
     return fail(MI355X_FP8_ENOTSUP, "block-scaled form %d does not take %lldx%lld", form, (long long)M, (long long)N);
   switch (form) {
