@@ -18,10 +18,14 @@ def _codes(rows, k, pad, seed, dev):
     return view.view(torch.float8_e4m3fn)
 
 
-# (m, n, k): one K byte to several 128-byte steps; rows and columns around 16, 32, 64 and 128; the last two
-# lie on either side of the 512 tiles of 128x128 from which the large tiles are taken
+# (m, n, k): one K byte to several 128-byte steps; rows and columns around 16, 32, 64 and 128; the two with about 2050
+# rows lie on either side of the 512 tiles of 128x128 from which the large tiles are taken
 SHAPES = [(1, 1, 1), (16, 16, 15), (17, 33, 127), (32, 31, 128), (33, 40, 129), (64, 65, 4099), (65, 63, 17), (128, 129, 256),
-          (129, 257, 1041), (517, 300, 383), (2049, 3840, 145), (2050, 3971, 273)]
+          (129, 257, 1041), (517, 300, 383), (2049, 3840, 145), (2050, 3971, 273),
+          # rows shorter than 16 bytes, in every mix of 8-, 4-, 2- and 1-byte pieces; panels on either side of the lines
+          # between the streaming form and the tiles
+          (3, 40, 2), (70, 33, 3), (5, 66, 5), (64, 20, 7), (16, 17, 8), (33, 70, 11), (66, 65, 13), (7, 31, 14),
+          (16, 8193, 127), (17, 8193, 255), (64, 4097, 255), (64, 4096, 255), (100, 33000, 126)]
 
 
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16])

@@ -1581,6 +1581,7 @@ typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
 typedef uint32_t v2u_any __attribute__((ext_vector_type(2), aligned(1)));
 typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef uint16_t u16_any __attribute__((aligned(1)));
 
 // bytes [k, k + 16) of a row of K bytes; those at or past K count as zero
 __device__ __forceinline__ v4i load16_any(const uint8_t* row, int k, int K) {
@@ -1595,9 +1596,26 @@ __device__ __forceinline__ v4i load16_any(const uint8_t* row, int k, int K) {
       lo = n < 64 ? (lo >> n) | (hi << (64 - n)) : hi >> (n & 63);
       hi = n < 64 ? hi >> n : 0;
     }
-  } else {
-    for (int e = 0; e < kChunk; ++e)
-      if (k + e < K) (e < 8 ? lo : hi) |= (uint64_t)row[k + e] << (8 * (e & 7));
+  } else if (k == 0) {  // the whole row, in pieces of 8, 4, 2 and 1 bytes
+    int at = K & 8, bits = 0;
+    uint64_t rest = 0;
+    if (K & 4) {
+      rest = *(const u32_any*)(row + at);
+      at += 4;
+      bits = 32;
+    }
+    if (K & 2) {
+      rest |= (uint64_t)*(const u16_any*)(row + at) << bits;
+      at += 2;
+      bits += 16;
+    }
+    if (K & 1) rest |= (uint64_t)row[at] << bits;
+    lo = rest;
+    if (K & 8) {
+      const v2u_any first = *(const v2u_any*)row;
+      lo = first[0] | ((uint64_t)first[1] << 32);
+      hi = rest;
+    }
   }
   return (v4i){(int)(uint32_t)lo, (int)(uint32_t)(lo >> 32), (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)};
 }
@@ -1728,8 +1746,8 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
       if (s + d < full) step(d, s + d);
   }
 
-  // lane (l32, half): row l32 of every 32x32 block, columns 8q + 4*half + 0..3
-  const bool vec = ((p.ldc & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.c) & 7) == 0);
+  // lane (l32, half): row l32 of every 32x32 block, columns 8q + 4*half + 0..3, as one 8-byte store wherever it lies
+  // (1795x84399x13, rows of C that start at any 2 bytes: 553 us with a store per element)
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     float sb[4][4], bias[4][4];
@@ -1757,8 +1775,8 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
         }
         const uint32_t lo = pack_out_x2(r[0], r[1], p.out_f16), hi = pack_out_x2(r[2], r[3], p.out_f16);
         uint16_t* dst = p.c + (size_t)m * p.ldc + n;
-        if (vec && n + 3 < p.N) {
-          *(v2u*)dst = (v2u){lo, hi};
+        if (n + 3 < p.N) {
+          *(v2u_any*)dst = (v2u){lo, hi};
         } else {
           if (n < p.N) dst[0] = (uint16_t)lo;
           if (n + 1 < p.N) dst[1] = (uint16_t)(lo >> 16);
@@ -4117,9 +4135,16 @@ int launch_any(GemmParams p, hipStream_t stream) {
   return MI355X_FP8_OK;
 }
 
-// (the streaming kernel's unaligned form: 512 lanes for 16 columns)
-constexpr bool generic_streams(int64_t N) { return grid_fits((N + 15) / 16, 512); }
-static_assert(generic_streams(1 << 27) == false && generic_streams((1 << 27) - 16), "2^27 columns are 2^32 lanes");
+// Up to 64 rows: whether the streaming kernel's unaligned form runs. Its workgroups, one for 16 columns (32 from 33 rows on),
+// share out the K steps among eight waves, so rows of one or two steps leave most of a workgroup idle, and on wide panels what
+// it takes is the rate at which workgroups come and go: 1x30090x1 8.4 us against 4.9 for 64x64 tiles, 34x112402x13 54 against 11,
+// 60x282266x3 156 against 29, 22x116414x94 42 against 19; the other way round 2x10559x202 4.8 against 5.7. (The grid: 512 lanes
+// a workgroup, fewer than 2^32 in all.)
+constexpr bool generic_streams(int64_t M, int64_t N, int64_t K) {
+  if (M > kSkinnyMaxM || !grid_fits((N + 15) / 16, 512)) return false;
+  return !(K <= (M <= 16 ? 128 : 256) && N > (M <= 32 ? 8192 : 4096));
+}
+static_assert(!generic_streams(1, 1 << 27, 1024) && generic_streams(1, (1 << 27) - 16, 1024), "2^27 columns are 2^32 lanes");
 // The generic family: the streaming kernel's unaligned form up to 64 rows (measured cold: 1x8192x8191 14.4 us,
 // 16x8192x8191 19.1, 64x8192x8191 29.7, where 64x64 tiles take 33), tiles beyond. 128x128 tiles from two
 // rounds of the CUs on (4096x8192x8191 563 us = 977 TFLOP/s); below, 64x64 tiles. With at most one of
@@ -4128,13 +4153,15 @@ static_assert(generic_streams(1 << 27) == false && generic_streams((1 << 27) - 1
 // the second step's registers would cost one of them (517x3000x1041 13.9 -> 12.7, 1024x2048x1025 13.7 -> 12.5).
 int launch_generic(const GemmParams& p, hipStream_t s) {
   if (p.M > 65535 * 64) return fail(MI355X_FP8_ENOTSUP, "the generic family takes M <= %d", 65535 * 64);
-  if (p.M <= kSkinnyMaxM && generic_streams(p.N)) {
+  if (generic_streams(p.M, p.N, p.K)) {
     if (p.M <= 16) return launch_skinny<1, 1, 4, 8, true>(p, s);
     if (p.M <= 32) return launch_skinny<2, 1, 2, 8, true>(p, s);
     return launch_skinny<4, 2, 2, 8, true>(p, s);
   }
   auto tiles = [&](long edge) { return ((p.M + edge - 1) / edge) * ((p.N + edge - 1) / edge); };
-  if (tiles(128) >= 2 * kNumCu) return launch_any<128, 128, 1>(p, s);
+  // (one step, or one row of tiles: nothing to gain from the larger tile, 164x39275x3 21.6 us with it, 14.0 with 64x64)
+  if ((tiles(128) >= 2 * kNumCu && p.M > kSkinnyMaxM && p.K > kStepK) || !grid_fits(tiles(64), 256))
+    return launch_any<128, 128, 1>(p, s);
   return tiles(64) <= kNumCu ? launch_any<64, 64, 2>(p, s) : launch_any<64, 64, 1>(p, s);
 }
 
