@@ -29,6 +29,9 @@ def _same(got, want):
     (F32, 2, 16385), (F32, 2, 40001), (F32, 2051, 17), (F32, 2050, 511), (F32, 2049, 2047),
     (BF16, 3, 1), (BF16, 3, 7), (BF16, 3, 8), (BF16, 3, 9), (BF16, 5, 1041), (BF16, 5, 8191), (BF16, 5, 8192), (BF16, 3, 8193),
     (BF16, 2, 32771), (BF16, 2, 70001), (BF16, 2051, 33), (BF16, 2050, 1023), (BF16, 2049, 4095),
+    # a wave each with one or two rounds of loads, and the element-by-element kernel for few short bf16 rows
+    (F32, 7, 63), (F32, 7, 255), (F32, 7, 256), (F32, 7, 257), (F32, 2049, 255), (BF16, 5, 256), (BF16, 5, 257), (BF16, 513, 66),
+    (BF16, 2048, 63), (BF16, 514, 511), (BF16, 6, 512), (BF16, 6, 513), (BF16, 2049, 1023), (BF16, 2049, 1025),
 ])
 @pytest.mark.parametrize("lead,pad", [(0, 0), (1, 2)])
 def test_rows_that_start_anywhere(gpu_device, dtype, rows, cols, lead, pad):
@@ -54,7 +57,7 @@ def test_results_that_start_anywhere_leave_the_rest_alone(gpu_device, dtype, col
     assert torch.all(got[:, cols:] == 0x55) and torch.all(q.cpu()[:lead] == 0x55)
 
 
-@pytest.mark.parametrize("dtype,cols", [(F32, 1041), (BF16, 1041), (BF16, 8199)])
+@pytest.mark.parametrize("dtype,cols", [(F32, 1041), (BF16, 1041), (BF16, 8199), (F32, 101), (BF16, 301), (BF16, 101)])
 def test_non_finite_and_zero_rows(gpu_device, dtype, cols):
     _, x = _source(dtype, 5, cols, 0, 0)
     x = x.clone()

@@ -4528,7 +4528,7 @@ static_assert(quantize_any_long(4194303, 1025) && !quantize_any_long(8388608, 10
 
 // The quantiser on rows that do not start 16-byte aligned or do not hold whole 16-byte chunks: the vector kernel's
 // unaligned forms, by the same lines as the aligned ones (fewer of them: this is the rare case). The element-by-element
-// kernel, which ran them all before, is left for rows shorter than one chunk. Measured, sources rotated through memory, before
+// kernel, which ran them all before, is left for few or very short rows. Measured, sources rotated through memory, before
 // -> now: f32 4096x8191 72 -> 28 us (2.3 -> 6.0 TB/s), 8192x2047 40 -> 15, 2048x20001 99 -> 36, 512x53247 181 -> 30; bf16
 // 4096x8191 73 -> 22 (4.6 TB/s), 8192x2047 40 -> 15, 1024x28671 107 -> 23.
 template <typename SrcT>
@@ -4540,8 +4540,17 @@ void launch_quantize_any(const SrcT* x, uint8_t* xq, float* inv_scale, int64_t R
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3((unsigned)threads), 0, s, x, xq, inv_scale, (int)K, (long)ldx, (long)ldq, (long)R);
   };
   const bool long_row = quantize_any_long(R, chunks);
-  if (K < epv) {
+  // Rows of up to 64 chunks: a wave each with as few rounds of loads as they need. (256 lanes with four rounds, most of them idle,
+  // lose to the element-by-element kernel there, f32 1985x51 3.1 -> 3.5 us, bf16 1624x106 3.3 -> 5.8; and so do eight rounds a
+  // lane, bf16 13772x38 9.5 -> 15.7.) The same for many bf16 rows of up to 128: 2000x700 6.7 us on 256 lanes, 3.8 as waves.
+  // Few very short bf16 rows stay with the latter kernel, which rounds a row's values to bf16 one by one on as many lanes
+  // (115x20 2.7 us, a wave each 3.15).
+  const bool few_short = epv == 8 && ((K <= 256 && R <= 512) || (K <= 64 && R <= 2048));
+  const bool wave_each = chunks <= 64 || (epv == 8 && chunks <= 2 * 64 && R > 512);
+  if (K < epv || few_short) {
     hipLaunchKernelGGL(quantize_rows_kernel<SrcT>, dim3((unsigned)R), dim3(256), 0, s, x, xq, inv_scale, (int)K, (long)ldx, (long)ldq);
+  } else if (wave_each) {
+    go(quantize_rows_vec_kernel<SrcT, 16 / epv, 64, kWaveRows, true>, (R + kWaveRows - 1) / kWaveRows, 64 * kWaveRows);
   } else if (chunks <= 8 * 64 && R > 2048) {
     go(quantize_rows_vec_kernel<SrcT, 8, 64, kWaveRows, true>, (R + kWaveRows - 1) / kWaveRows, 64 * kWaveRows);
   } else if (!long_row) {
