@@ -104,3 +104,31 @@ def test_without_a_device_every_call_is_left_to_the_wrappers():
     assert b.gemm_rowwise() is None and b.row_quantize(x.float()) is None and b.row_quantize("x") is None
     assert b.gemm_rowwise(x, x, x, x, None, None, 0, None, False) is None
     assert b.mark_ready(10**6) is None and b.mark_ready("cuda") is None
+
+
+def _without_binding(monkeypatch, path):
+    monkeypatch.setattr(_lib, "_binding", None)
+    monkeypatch.setattr(_lib, "BINDING_PATH", str(path))
+    with pytest.warns(RuntimeWarning, match="cannot be loaded"):
+        return _lib.binding()
+
+
+@pytest.mark.parametrize("content", [None, b"", b"not a shared object"])
+def test_a_binding_that_cannot_be_loaded_leaves_every_call_to_the_wrappers(monkeypatch, tmp_path, content):
+    path = tmp_path / "mi355x_torch_binding.so"
+    if content is not None:
+        path.write_bytes(content)
+    b = _without_binding(monkeypatch, path)
+    assert b.gemm_rowwise() is None and b.row_quantize(torch.ones(2, 2)) is None and b.mark_ready(0) is None
+    assert _lib.binding() is b  # (one attempt, one warning)
+    with pytest.raises(RuntimeError, match="only runs on a ROCm device"):  # (the wrappers' own check, not the loader's error)
+        ops.fp8_row_quantize(torch.ones(4, 16))
+
+
+@pytest.mark.gpu
+def test_calls_run_without_the_binding(gpu_device, monkeypatch, tmp_path):
+    calls = _calls(gpu_device)
+    want = {name: _bits(call()) for name, call in calls.items()}
+    _without_binding(monkeypatch, tmp_path / "missing.so")
+    for name, call in calls.items():
+        assert all(torch.equal(a, b) for a, b in zip(_bits(call()), want[name])), name

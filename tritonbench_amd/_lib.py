@@ -2,13 +2,14 @@
 
 The shared library is loaded from tritonbench_amd/lib/ (built in-tree by
 tritonbench_amd.build). There is no fallback: if the library is missing or does not
-load, every entry point raises.
+load, every entry point raises. (The native binding beside it is only a shorter way to it.)
 """
 import ctypes
 import importlib.machinery
 import importlib.util
 import os
 import threading
+import warnings
 from ctypes import c_char_p, c_int, c_int64, c_size_t, c_void_p
 
 from .build import BINDING_PATH, LIB_PATH
@@ -181,20 +182,32 @@ def load() -> ctypes.CDLL:
 _binding = None
 
 
+class _NoBinding:
+    """Stands in for the native module: answers None to every call, which the wrappers then take through ctypes."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def binding():
     """The native module that takes everyday calls from PyTorch tensors to the library (csrc/torch_binding.cpp), loaded once,
-    behind the library it calls."""
+    behind the library it calls. It saves a few microseconds a call and nothing else: where it is not there or was built for
+    another PyTorch, a warning says so and every call goes through ctypes."""
     global _binding
     if _binding is None:
         load()
         with _lock:
             if _binding is None:
-                if not os.path.exists(BINDING_PATH):
-                    raise LibraryNotBuilt(f"{BINDING_PATH} does not exist; build it with `python -m tritonbench_amd.build`")
-                loader = importlib.machinery.ExtensionFileLoader("mi355x_torch_binding", BINDING_PATH)
-                module = importlib.util.module_from_spec(importlib.util.spec_from_loader(loader.name, loader))
-                loader.exec_module(module)
-                _binding = module
+                try:
+                    loader = importlib.machinery.ExtensionFileLoader("mi355x_torch_binding", BINDING_PATH)
+                    module = importlib.util.module_from_spec(importlib.util.spec_from_loader(loader.name, loader))
+                    loader.exec_module(module)
+                    _binding = module
+                except (ImportError, OSError) as e:
+                    warnings.warn(f"{BINDING_PATH} cannot be loaded ({e}): every call takes a few microseconds longer through ctypes. "
+                                  "`python -m tritonbench_amd.build` builds it for the PyTorch that is installed.", RuntimeWarning,
+                                  stacklevel=2)
+                    _binding = _NoBinding()
     return _binding
 
 
