@@ -42,7 +42,7 @@ def _run(cmd, verbose):
         print(" ".join(cmd), flush=True)
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if proc.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + " ".join(cmd) + "\n" + proc.stdout)
+        raise RuntimeError(f"{os.path.basename(cmd[0])} failed:\n" + " ".join(cmd) + "\n" + proc.stdout)
 
 
 def _binding_object(verbose):
@@ -67,8 +67,15 @@ def _link_binding(obj, verbose):
     os.replace(tmp, BINDING_PATH)
 
 
+def build_binding(verbose: bool = False) -> None:
+    """Compiles the PyTorch binding and links it to the library, which has to be there."""
+    os.makedirs(BUILD_DIR, exist_ok=True)
+    _link_binding(_binding_object(verbose), verbose)
+
+
 def build_library(verbose: bool = False, jobs: int = 0) -> str:
-    """Compiles the library unconditionally and returns its path.
+    """Compiles the library and the binding unconditionally and returns the library's path. The library does not need PyTorch: it
+    is in place before a binding that cannot be built (no PyTorch, no headers, no g++) raises.
 
     The one source file is compiled as several translation units side by side (the main unit and
     one per tile configuration of the tiled kernel, selected by -DMI355X_SPLIT_MAIN and
@@ -81,8 +88,7 @@ def build_library(verbose: bool = False, jobs: int = 0) -> str:
     if jobs == 1:
         _run([hipcc, *HIPCC_FLAGS, "-o", tmp, *SOURCES], verbose)
         os.replace(tmp, LIB_PATH)
-        os.makedirs(BUILD_DIR, exist_ok=True)
-        _link_binding(_binding_object(verbose), verbose)
+        build_binding(verbose)
         return LIB_PATH
     from concurrent.futures import ThreadPoolExecutor
 
@@ -96,10 +102,9 @@ def build_library(verbose: bool = False, jobs: int = 0) -> str:
         binding = pool.submit(_binding_object, verbose)
         for f in futures:
             f.result()
-        binding_obj = binding.result()
-    _run([hipcc, "--offload-arch=gfx950", "-fPIC", "-shared", "-o", tmp, *objects], verbose)
-    os.replace(tmp, LIB_PATH)
-    _link_binding(binding_obj, verbose)
+        _run([hipcc, "--offload-arch=gfx950", "-fPIC", "-shared", "-o", tmp, *objects], verbose)
+        os.replace(tmp, LIB_PATH)  # (the library is there whatever becomes of the binding)
+        _link_binding(binding.result(), verbose)
     return LIB_PATH
 
 
