@@ -55,6 +55,39 @@ CASES = [
 ]
 
 
+# the form each of these runs, so that the cases above keep reaching what they are there for
+@pytest.mark.parametrize("form,shapes", [
+    (_lib.GROUPED_ROWS_16, [(1, 1, 16, 16), (2, 16, 33, 144), (16, 128, 512, 1040), (65, 200, 40, 128), (256, 256, 32, 128), (8, 64, 128, 512)]),
+    (_lib.GROUPED_ROWS_32, [(2, 32, 128, 4096), (2, 32, 72, 4112)]),
+    (_lib.GROUPED_ROWS_64, [(3, 49, 130, 4096), (2, 64, 128, 4096), (2, 63, 40, 4240)]),
+    (_lib.GROUPED_STREAM_128, [(16, 200, 1024, 2048), (8, 500, 2048, 2048), (16, 700, 1000, 2048)]),
+    (_lib.GROUPED_STREAM_256, [(16, 2048, 2040, 2048), (16, 1500, 2048, 2048), (4, 480, 11584, 9536)]),
+    (_lib.GROUPED_TILES, [(16, 1024, 1000, 2064), (16, 1100, 2048, 2064), (8, 700, 4096, 4112), (4, 8192, 4096, 4096)]),
+])
+def test_the_cases_reach_the_forms(form, shapes):
+    for shape in shapes:
+        assert _lib.load().mi355x_fp8_rowwise_grouped_form(*shape) == form, shape
+
+
+# rows of K bytes in rows of a longer pitch: a partial last step of rows on the 128-byte lines (the streaming tiles with a K tail),
+# and whole steps of rows off them; groups of no, one, two and more tile rows side by side
+@pytest.mark.parametrize("g,m,n,k,pitch", [(16, 700, 1000, 2064, 2176), (16, 1500, 2048, 2064, 2176), (16, 100, 96, 640, 656),
+                                           (16, 700, 1000, 2048, 2064), (4, 450, 11264, 2048, 2064), (2, 64, 128, 4096, 4112)])
+def test_pitches_on_and_off_the_lines(gpu_device, g, m, n, k, pitch):
+    x, w, xs, ws = _operands(gpu_device, g, m, n, k)
+    wide = torch.full((g * n, pitch), 0x7F, dtype=torch.uint8, device=gpu_device).view(torch.float8_e4m3fn)  # (NaN beside the rows)
+    wide[:, :k].copy_(w)
+    sizes = _spread(g, m)
+    hot = max(range(g), key=lambda i: sizes[i])
+    for i in range(g):  # a group of several tile rows, and some of none
+        if i != hot and i % 3 == 0:
+            sizes[hot] += sizes[i]
+            sizes[i] = 0
+    ms = torch.tensor(sizes, dtype=torch.int32, device=gpu_device)
+    got = ops.fp8_gemm_rowwise_grouped(x, wide[:, :k], ms, xs, ws)
+    assert torch.equal(got, ops.fp8_gemm_rowwise_grouped(x, w, ms, xs, ws, tile_config=SMALL_TILES))
+
+
 @pytest.mark.parametrize("g,m,n,k,sizes", CASES)
 def test_forms_equal_the_small_tiles_bit_for_bit(gpu_device, g, m, n, k, sizes):
     x, w, xs, ws = _operands(gpu_device, g, m, n, k)

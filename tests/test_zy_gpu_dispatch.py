@@ -130,3 +130,40 @@ def test_block_scaled_choice_is_close_to_the_best_form(gpu_device, m, n, k):
     print(f"  {m}x{n}x{k}: form {lib.mi355x_fp8_blockwise_form(m, n, k)} {auto:.1f} us; " +
           ", ".join(f"{f}: {t:.1f}" for f, t in times.items()), flush=True)
     assert auto <= TOLERANCE * min(times.values())
+
+
+# the grouped forms against the pinned tile configurations, rows sent to groups at random or half of them to one group, rows of B on
+# and off the 128-byte lines
+@pytest.mark.parametrize("g,m,n,k,hot", [(16, 128, 4096, 4096, False), (16, 128, 4096, 4112, False), (8, 64, 14336, 4112, False),
+                                         (64, 512, 4096, 4096, True), (16, 512, 4096, 4096, True), (8, 256, 14336, 4096, True),
+                                         (16, 400, 4096, 2064, False), (8, 700, 4096, 4112, False), (12, 1200, 6000, 6672, False),
+                                         (16, 939, 1792, 4736, True), (32, 1800, 4096, 4096, True), (4, 8192, 4096, 4096, False)])
+def test_grouped_choice_is_close_to_the_best_tiles(gpu_device, g, m, n, k, hot):
+    lib = _lib.load()
+    gen = torch.Generator(device=gpu_device).manual_seed(m + n + k)
+    codes = lambda r: torch.randn((r, k), generator=gen, device=gpu_device, dtype=torch.bfloat16).to(torch.float8_e4m3fn)
+    count = min(6, max(2, 600_000_000 // (g * n * k)))
+    to = torch.randint(0, g, (m,), generator=gen, device=gpu_device)
+    if hot:
+        to[: m // 2] = g // 2
+    sizes = torch.bincount(to, minlength=g).to(torch.int32)
+    xs, ws = torch.rand(m, generator=gen, device=gpu_device), torch.rand(g * n, generator=gen, device=gpu_device)
+    sets = [(codes(m), codes(g * n), torch.empty((m, n), dtype=torch.bfloat16, device=gpu_device)) for _ in range(count)]
+
+    def call(config):
+        def one(i):
+            x, w, out = sets[i]
+            _lib.check(lib.mi355x_fp8_rowwise_grouped_gemm(x.data_ptr(), w.data_ptr(), xs.data_ptr(), ws.data_ptr(), sizes.data_ptr(),
+                                                           out.data_ptr(), g, m, n, k, k, k, n, config,
+                                                           torch.cuda.current_stream().cuda_stream), "grouped_gemm")
+        return one
+    times, auto = {c: float("inf") for c in range(_lib.NUM_GROUPED_TILE_CONFIGS)}, float("inf")
+    for rnd in range(4):
+        auto = min(auto, _time_us(call(-1), count))
+        for c in times:
+            times[c] = min(times[c], _time_us(call(c), count))
+        if auto <= TOLERANCE * min(times.values()):
+            break
+    print(f"  {g} groups {m}x{n}x{k} hot={hot}: form {lib.mi355x_fp8_rowwise_grouped_form(g, m, n, k)} {auto:.1f} us; " +
+          ", ".join(f"{c}: {t:.1f}" for c, t in times.items()), flush=True)
+    assert auto <= TOLERANCE * min(times.values())

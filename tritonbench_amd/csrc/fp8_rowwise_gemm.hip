@@ -128,6 +128,7 @@ using mi355x_shared::GemmParams;
 // Where a tile sits: rows [m0, m_end) of A and C it may touch, first column, group.
 struct TileLoc {
   int m0, m_end, n0, group;
+  int tiles_m;  // (grouped form: tile rows of the group)
 };
 
 // Cursor over the groups for the grouped form. Tiles are numbered group by group; inside a
@@ -504,7 +505,7 @@ void gemm_tiled_kernel(GemmParams p) {
     if (!GROUPED) {
       int tm, tn;
       tile_coords(tile, p.tiles_m, p.tiles_n, p.div_group_mul, p.div_group_shift, tm, tn);
-      return TileLoc{tm * BM, p.M, tn * BN, 0};
+      return TileLoc{tm * BM, p.M, tn * BN, 0, 0};
     }
     while (tile >= w.tile_end && w.group + 1 < p.groups) {
       w.row_begin += group_rows(w.group, w.row_begin);
@@ -515,7 +516,7 @@ void gemm_tiled_kernel(GemmParams p) {
     }
     const int t = tile - w.tile_begin;
     const int tm = t % max(w.tiles_m, 1), tn = t / max(w.tiles_m, 1);
-    return TileLoc{w.row_begin + tm * BM, w.row_begin + group_rows(w.group, w.row_begin), tn * BN, w.group};
+    return TileLoc{w.row_begin + tm * BM, w.row_begin + group_rows(w.group, w.row_begin), tn * BN, w.group, STREAM_B ? w.tiles_m : 0};
   };
   auto first_group = [&]() -> GroupWalk {
     GroupWalk w = {0, 0, 0, 0, 0};
@@ -537,8 +538,16 @@ void gemm_tiled_kernel(GemmParams p) {
   // share panels of B through the L2 keep the common order: there the sharing needs it. So do
   // plans with more than two splits, whose items are already spread over K (M=128, N=K=8192 with
   // four splits lost 5 % to the rotation; two splits gain 5 %, unsplit plans 11-28 %).
+  // The streaming grouped form decides by group, as its tiles are taken up: those of a group of several tile rows share panels of
+  // B like any others (half of all rows at one of 8 experts, 256x14336x4096 105 -> 84 us, one of 32, 1800x4096x4096 123 -> 112; all
+  // of them 51 -> 38). From two tile rows on with 128 columns a tile, from three on with 256 (1000x14336x4096 in 8 groups, most
+  // of one or two tile rows of those: 105, without streaming those of two 109). Rows off the 128-byte lines are not streamed.
+  constexpr bool STREAM_BY_GROUP = GROUPED && STREAM_B;
+  const int stream_rows = p.ldb % kStepK == 0 ? (BN == 256 ? 2 : 1) : 0;  // tile rows of a group up to which its tiles stream B
+  auto group_streams = [&](const TileLoc& loc) { return loc.tiles_m <= stream_rows; };
   auto first_step = [&](const TileLoc& loc, int begin, int count) {
-    return begin + (STREAM_B && p.splits <= 2 ? (loc.n0 / BN) % count : 0);
+    const bool rotated = STREAM_B && p.splits <= 2 && (!STREAM_BY_GROUP || group_streams(loc));
+    return begin + (rotated ? (loc.n0 / BN) % count : 0);
   };
   auto start_cursor = [&](StepCursor& c, int li, const TileLoc& loc) {
     c.kt_begin = split_begin(item_split(li));
@@ -599,9 +608,11 @@ void gemm_tiled_kernel(GemmParams p) {
     start_cursor(ca, li, loc);
     a_src = make_src(p.a + (size_t)loc.m0 * p.lda, loc.m_end - loc.m0, BM, p.lda);
   };
+  int b_streams = 0;  // whether the loads of B take the streaming policy (STREAM_BY_GROUP: in the tile being loaded)
   auto setup_b = [&](int li) {
     const TileLoc loc = locate(walk_b, li);
     start_cursor(cb, li, loc);
+    if (STREAM_BY_GROUP) b_streams = __builtin_amdgcn_readfirstlane(group_streams(loc));
     b_src = make_src(p.b + ((size_t)loc.group * p.N + loc.n0) * p.ldb, p.N - loc.n0, BN, p.ldb);
   };
   // i-th group of one operand's step kt into the stage at sbase
@@ -1040,7 +1051,7 @@ void gemm_tiled_kernel(GemmParams p) {
   // slots behind which the next phase is prepared (two, so that neither holds more scalar work than
   // an MFMA covers)
   constexpr int PREP_T = NMFMA / 2, PREP_T2 = NMFMA >= 8 ? NMFMA / 2 + 1 : NMFMA / 2;
-  auto step = [&](auto first_tag, auto read_next_tag, auto plain_tag) {
+  auto step = [&](auto first_tag, auto read_next_tag, auto plain_tag, auto stream_tag) {
     constexpr bool FIRST = decltype(first_tag)::value;
     constexpr bool READ_NEXT = decltype(read_next_tag)::value;
     if (BLOCKSCALE) {  // (fetched from the lanes that hold them during the previous step, or at the item's start)
@@ -1066,7 +1077,7 @@ void gemm_tiled_kernel(GemmParams p) {
 #pragma unroll
       for (int l = 0; l < B_GROUPS; ++l)
         if (l * NMFMA / B_GROUPS == t)
-          load_group(std::integral_constant<bool, STREAM_B>{}, b_src, ph_b.lane_off, ph_b.step_off, l, ph_b.stage);
+          load_group(stream_tag, b_src, ph_b.lane_off, ph_b.step_off, l, ph_b.stage);
 #pragma unroll
       for (int u = t * RPS; u < (t + 1) * RPS; ++u)
         if (u < NREAD) read_one(ya, yb, cur_a, cur_b, 1, u);
@@ -1136,17 +1147,29 @@ void gemm_tiled_kernel(GemmParams p) {
       n_pend = lane_value(rt, kt_c + 1);
       n_last = lane_value(sc, kt_c);
     }
-    if (n_steps == 1) {
-      step(std::true_type{}, std::false_type{}, std::false_type{});
+    // step k loads for step k + DIST and then moves the cursors to step k + DIST + 1, which is still this item's for
+    // k < n_steps - DIST - 1. (Text and not a function: as a lambda around `step` it cost every grouped launch 1-2 %, 282x1536x1024
+    // in 30 groups 26.7 -> 27.1 us.)
+#define MI355X_ALL_STEPS(stream_tag)                                                                                           \
+  if (n_steps == 1) {                                                                                                          \
+    step(std::true_type{}, std::false_type{}, std::false_type{}, stream_tag);                                                  \
+  } else {                                                                                                                     \
+    step(std::true_type{}, std::true_type{}, std::false_type{}, stream_tag);                                                   \
+    int k = 1;                                                                                                                 \
+    for (; k < n_steps - DIST - 1; ++k) step(std::false_type{}, std::true_type{}, std::true_type{}, stream_tag);               \
+    for (; k < n_steps - 1; ++k) step(std::false_type{}, std::true_type{}, std::false_type{}, stream_tag);                     \
+    step(std::false_type{}, std::false_type{}, std::false_type{}, stream_tag);                                                 \
+  }
+    if constexpr (STREAM_BY_GROUP) {  // (the cursor of B is a few steps ahead, as a rule in this item; the policy is a hint either way)
+      if (b_streams) {
+        MI355X_ALL_STEPS(std::true_type{})
+      } else {
+        MI355X_ALL_STEPS(std::false_type{})
+      }
     } else {
-      // step k loads for step k + DIST and then moves the cursors to step k + DIST + 1, which is
-      // still this item's for k < n_steps - DIST - 1
-      step(std::true_type{}, std::true_type{}, std::false_type{});
-      int k = 1;
-      for (; k < n_steps - DIST - 1; ++k) step(std::false_type{}, std::true_type{}, std::true_type{});
-      for (; k < n_steps - 1; ++k) step(std::false_type{}, std::true_type{}, std::false_type{});
-      step(std::false_type{}, std::false_type{}, std::false_type{});
+      MI355X_ALL_STEPS((std::integral_constant<bool, STREAM_B>{}))
     }
+#undef MI355X_ALL_STEPS
     {
       const TileLoc loc = locate(walk_c, c_item);
       if (EPI == kEpiPartial) {
@@ -1857,7 +1880,8 @@ __device__ __forceinline__ RowBlock find_row_block(const GemmParams& p, int item
 // a group; the row blocks of one group's columns are neighbours on one XCD (workgroup ids go round the XCDs), so that
 // the group's rows of B come from HBM once. The grid covers the most row blocks that any sizes with these M and G can
 // give; the surplus comes last and returns at once.
-template <int MT, int NTW, int DEPTH, int KW, bool ANY = false, bool BLOCK = false, bool GROUPED = false>
+// OFF_LINES: the grouped form for rows of B that do not start on 128-byte lines: no streaming policy.
+template <int MT, int NTW, int DEPTH, int KW, bool ANY = false, bool BLOCK = false, bool GROUPED = false, bool OFF_LINES = false>
 __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
   static_assert((int)ANY + (int)BLOCK + (int)GROUPED <= 1, "at most one of them");
   using Chunk = std::conditional_t<ANY, v4i_any, v4i>;
@@ -1975,8 +1999,9 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
       for (int h = 0; h < 2; ++h) {
         // B is read once and never again: stream it past the caches; A is shared by everyone. (ANY: an
         // unaligned piece shares its lines with the neighbouring steps, which the streaming policy would
-        // fetch again: 1x8192x8191 19.6 -> 14.4 us without it, 16x8192x8191 25.6 -> 19.1.)
-        if (t < NTW && !ANY) dst[t][h] = __builtin_nontemporal_load((const Chunk*)(src[t][h] + kb));
+        // fetch again: 1x8192x8191 19.6 -> 14.4 us without it, 16x8192x8191 25.6 -> 19.1. The same for rows that start
+        // off a line: 128 rows in 16 groups of 4096x4112 75 -> 60, 64 in 8 of 14336x4112 128 -> 101.)
+        if (t < NTW && !ANY && !OFF_LINES) dst[t][h] = __builtin_nontemporal_load((const Chunk*)(src[t][h] + kb));
         else dst[t][h] = *(const Chunk*)(src[t][h] + kb);
       }
   };
@@ -3953,12 +3978,12 @@ constexpr int64_t grouped_row_blocks(int64_t G, int64_t M, int bm, bool clear_re
 }
 constexpr int64_t grouped_column_tiles(int64_t N, int bn) { return ((N + bn - 1) / bn + kNumXcd - 1) / kNumXcd * kNumXcd; }
 
-template <int MT, int NTW, int DEPTH, int KW>
-int launch_grouped_skinny(const GemmParams& p, hipStream_t stream) {
+template <int MT, int NTW, int DEPTH, int KW, bool OFF_LINES>
+int launch_grouped_rows(const GemmParams& p, hipStream_t stream) {
   constexpr int BM = 16 * MT, BN = 16 * NTW;
   constexpr size_t lds_bytes = (size_t)KW * (NTW + MT) * 16 * kStepK;
   static_assert(lds_bytes <= 160 * 1024, "transpose buffers must fit the 160 KB LDS");
-  constexpr auto kern = gemm_skinny_kernel<MT, NTW, DEPTH, KW, false, false, true>;
+  constexpr auto kern = gemm_skinny_kernel<MT, NTW, DEPTH, KW, false, false, true, OFF_LINES>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   GemmParams q = p;
   q.tiles_n = (p.N + BN - 1) / BN;
@@ -3969,6 +3994,11 @@ int launch_grouped_skinny(const GemmParams& p, hipStream_t stream) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "grouped skinny kernel launch: %s", hipGetErrorString(e));
   return MI355X_FP8_OK;
+}
+
+template <int MT, int NTW, int DEPTH, int KW>
+int launch_grouped_skinny(const GemmParams& p, hipStream_t s) {
+  return p.ldb % kStepK ? launch_grouped_rows<MT, NTW, DEPTH, KW, true>(p, s) : launch_grouped_rows<MT, NTW, DEPTH, KW, false>(p, s);
 }
 
 // The grouped form of the tiled kernel.
@@ -3997,6 +4027,12 @@ int launch_grouped_tiles(const GemmParams& p, hipStream_t s) {
 // * groups of 65 to 128 rows often are two tile rows high; 128x256 tiles then make fewer rounds: 16 groups of 4096x4096
 //   with 128 rows 88 -> 73 (128x128 tiles with the streaming policy 99), 8 of 14336x4096 145 -> 109, 16 of 7168x2048
 //   72 -> 63. (Fewer than 128 of them: 8 groups of 2048x7168 42 -> 57.)
+// * Rows of B off the 128-byte lines: tiles take them without the streaming policy, and so without a reason to be other tiles
+//   (400x4096x2064 in 16 groups 40, streaming 50; 700x4096x4112 in 8 39, 128x256 tiles 60, the same without the policy 55), but for
+//   128x256 tiles that come to one full round (480x11584x9536 in 4 groups 131, now 110).
+// The choice goes by the average. Where one group holds a large share of the rows the forms are still ahead of or level with
+// the plain tiles up to about half of all rows (13 groups, 1076x4608x5120: 82 -> 88, the worst seen), and behind where it holds
+// all of them: 64 groups, 512x4096x4096 34 -> 50, 51 of 346x11584x384 21 -> 43, against 203 -> 174 and 83 -> 74 with rows spread at random.
 enum GroupedForm {
   kGroupedTiles = MI355X_FP8_GROUPED_TILES,
   kGroupedRows16 = MI355X_FP8_GROUPED_ROWS_16,
@@ -4009,12 +4045,13 @@ constexpr bool grouped_rows16_fits(int64_t G, int64_t M, int64_t N) {
   return grid_fits(grouped_column_tiles(N, 32) * grouped_row_blocks(G, M, 16, true), 256);
 }
 static_assert(!grouped_rows16_fits(256, 256, 2200000) && grouped_rows16_fits(256, 2048, 57344), "a column tile and row block are 256 lanes");
-inline GroupedForm grouped_form(int64_t G, int64_t M, int64_t N, int64_t K) {
+inline GroupedForm grouped_form(int64_t G, int64_t M, int64_t N, int64_t K, int64_t ldb) {
   const bool rows_forms = G <= 256;  // (a workgroup's look-up goes over 64 groups at a time, the tiled kernel's once a launch)
   if (M <= 8 * G && rows_forms && grouped_rows16_fits(G, M, N)) return kGroupedRows16;
   const int64_t tiles_128 = G * ((N + 127) / 128), tiles_256 = G * ((N + 255) / 256);
   if (rows_forms && K >= 4096 && tiles_128 <= 128 && M <= 32 * G) return M <= 16 * G ? kGroupedRows32 : kGroupedRows64;
   if (K < 2048 || M > 128 * G) return kGroupedTiles;
+  if (ldb % kStepK != 0) return M > 64 * G && tiles_256 >= 176 && tiles_256 <= kNumCu ? kGroupedStream256 : kGroupedTiles;
   if (M > 64 * G) return tiles_256 >= 128 ? kGroupedStream256 : kGroupedTiles;
   return tiles_128 >= 128 ? kGroupedStream128 : kGroupedTiles;
 }
@@ -4637,7 +4674,7 @@ int mi355x_fp8_rowwise_grouped_gemm_ex(const void* a, const void* b, const float
   p.m_sizes = m_sizes; p.groups = (int)G; p.clear_rest = clear_rest != 0; p.out_f16 = 0;
   p.div_tiles_mul = p.div_tiles_shift = p.div_group_mul = p.div_group_shift = 0; p.stamps = nullptr;
   hipStream_t s = (hipStream_t)stream;
-  switch (tile_config < 0 ? grouped_form(G, M, N, K) : kGroupedTiles) {
+  switch (tile_config < 0 ? grouped_form(G, M, N, K, ldb) : kGroupedTiles) {
     case kGroupedRows16: return launch_grouped_skinny<1, 2, 2, 4>(p, s);
     case kGroupedRows32: return launch_grouped_skinny<2, 2, 2, 8>(p, s);
     case kGroupedRows64: return launch_grouped_skinny<4, 2, 2, 8>(p, s);
@@ -4666,7 +4703,7 @@ int mi355x_fp8_rowwise_grouped_form(int64_t G, int64_t M, int64_t N, int64_t K) 
   if (st == MI355X_FP8_OK) st = check_fast_shape(K);
   if (st != MI355X_FP8_OK) return st;
   if (G < 1 || G > 65536) return fail(MI355X_FP8_EINVAL, "G must be in 1..65536 (got %lld)", (long long)G);
-  return grouped_form(G, M, N, K);
+  return grouped_form(G, M, N, K, K);
 }
 
 int mi355x_fp8_blockwise_form(int64_t M, int64_t N, int64_t K) {
