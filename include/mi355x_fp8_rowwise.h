@@ -54,8 +54,8 @@ extern "C" {
 #define MI355X_FP8_VARIANT_SKINNY  2  /* kernels that own all of K per workgroup and stream B (HBM-bound): M <= 64, \
                                          and M <= 256 where the narrow-tile form below fits */
 #define MI355X_FP8_VARIANT_GENERIC 3  /* unaligned loads and 16-bit MFMA, no requirement on K, the leading dimensions or \
-                                         the alignment of a and b: what AUTO runs for operands the two MFMA families   \
-                                         cannot take (a few TFLOP/s) */
+                                         the alignment of a and b: what AUTO runs for operands the two families above  \
+                                         cannot take (up to 0.98 PFLOP/s; M <= 4194240) */
 
 /*
  * The `variant` argument is a word: bits 0..7 hold the family above; for the tiled family

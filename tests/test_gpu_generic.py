@@ -1,4 +1,4 @@
-"""The generic kernel family (byte loads, f32 multiply-adds): operands the MFMA families cannot take
+"""The generic kernel family (unaligned loads, 16-bit matrix instructions): operands the MFMA families cannot take
 (K, lda or ldb not a multiple of 16, A or B not 16-byte aligned) against the CPU oracle, through
 the C ABI. Needs an MI355X."""
 import numpy as np

@@ -13,7 +13,10 @@
 //                            turned through LDS into 16-byte row stores. Tiles of 256x256,
 //                            128x128 (two ring depths), 256x128, 64x256, 128x256 and 192x256; grouped
 //                            and block-scaled forms.
-//   splitk_finalize_kernel   adds the fp32 partial sums of a split-K launch, applies scales/bias.
+//   gemm_block_kernel        block-scaled form for shapes that fill the chip with 256x256 tiles: two groups of
+//                            four waves take turns between memory and matrix work.
+//   splitk_finalize_kernel   adds the fp32 partial sums of a split-K launch, applies scales/bias
+//                            (splitk_finalize_rows_kernel: four rows a thread, for large results).
 //   gemm_skinny_kernel       M <= 64: every workgroup owns 16 rows of B and all of K, its waves
 //                            split K between them and reduce through LDS; B is streamed once.
 //   gemm_skinny_persistent_kernel  M <= 16 (M <= 32 at K = 4096): one 16-wave workgroup per CU keeps
@@ -25,7 +28,7 @@
 //                            launch); separate waves fetch A and B.
 //   gemm_any_kernel          any K, leading dimension and alignment (more than 64 rows; up to 64 the skinny
 //                            kernel has a form for them): unaligned loads, binary16 MFMA on the widened codes.
-//   quantize_rows_*_kernel   row-wise e4m3fn quantiser (amax, scale, convert), one row per workgroup.
+//   quantize_rows_*_kernel   row-wise e4m3fn quantiser (amax, scale, convert), a row per workgroup or per wave.
 //   quantize_blocks_kernel   128 x 128 block-wise e4m3fn quantiser, one block per workgroup.
 //   fused_rowwise_quant_kernel  RMSNorm or SiLU-mul of bf16 rows followed by the same quantiser, one pass.
 //
@@ -4186,13 +4189,14 @@ constexpr bool generic_streams(int64_t M, int64_t N, int64_t K) {
   return !(K <= (M <= 16 ? 128 : 256) && N > (M <= 32 ? 8192 : 4096));
 }
 static_assert(!generic_streams(1, 1 << 27, 1024) && generic_streams(1, (1 << 27) - 16, 1024), "2^27 columns are 2^32 lanes");
-// The generic family: the streaming kernel's unaligned form up to 64 rows (measured cold: 1x8192x8191 14.4 us,
+// The generic family: the streaming kernel's unaligned form up to 64 rows but for short rows on wide panels (measured cold: 1x8192x8191 14.4 us,
 // 16x8192x8191 19.1, 64x8192x8191 29.7, where 64x64 tiles take 33), tiles beyond. 128x128 tiles from two
 // rounds of the CUs on (4096x8192x8191 563 us = 977 TFLOP/s); below, 64x64 tiles. With at most one of
 // those per CU nothing but its own loads covers a step's latency, and they run two steps ahead
 // (128x8192x8191 61.7 -> 36.7 us, 256x4096x4097 27.9 -> 19.6); with more, the CU's other workgroups do, and
 // the second step's registers would cost one of them (517x3000x1041 13.9 -> 12.7, 1024x2048x1025 13.7 -> 12.5).
 int launch_generic(const GemmParams& p, hipStream_t s) {
+  // (the documented range of the family, which the tests' sizes lie in)
   if (p.M > 65535 * 64) return fail(MI355X_FP8_ENOTSUP, "the generic family takes M <= %d", 65535 * 64);
   if (generic_streams(p.M, p.N, p.K)) {
     if (p.M <= 16) return launch_skinny<1, 1, 4, 8, true>(p, s);
