@@ -90,6 +90,7 @@ struct GemmParams {
   // tiled kernel: where every workgroup leaves its start and end readings of the shader clock and of
   // the constant 100 MHz clock (4 values per workgroup), or nullptr
   unsigned long long* stamps;
+  int store;  // tiles: how their pieces of C are stored (kStoreStream ...)
 };
 
 extern thread_local char err[512];
@@ -121,6 +122,10 @@ typedef float v4f  __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef unsigned short us4 __attribute__((ext_vector_type(4)));
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+// the same in memory at any address (one instruction each on this chip)
+typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t v2u_any __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
 
 constexpr int kNumXcd = 8;       // accelerator complex dies; workgroup ids round-robin over them
 constexpr int kNumCu = 256;
@@ -200,7 +205,7 @@ __device__ __forceinline__ void clear_rows(const GemmParams& p, int first, int w
 // the same for what only the tiled kernel and its second pass read
 __device__ __forceinline__ void fetch_tiled_arguments_now(const GemmParams& p) {
   asm volatile("" ::"s"(p.splits), "s"(p.steps_per_split), "s"(p.partial), "s"(p.m_sizes), "s"(p.groups), "s"(p.div_tiles_mul),
-               "s"(p.div_tiles_shift), "s"(p.div_group_mul), "s"(p.div_group_shift), "s"(p.stamps));
+               "s"(p.div_tiles_shift), "s"(p.div_group_mul), "s"(p.div_group_shift), "s"(p.stamps), "s"(p.store));
 }
 
 // ------------------------------------------------------------------------------------
@@ -319,13 +324,43 @@ __device__ __forceinline__ void store_f32x4_checked(v4f data, __amdgpu_buffer_rs
 #endif
 }
 
-// One wave-wide streaming store of 16 bytes per lane through a buffer descriptor (address = base +
-// lane_off + wave_off): the output is written once and read by a later kernel at best.
-__device__ __forceinline__ void store_chunk_streaming(v4i data, __amdgpu_buffer_rsrc_t rsrc, uint32_t lane_off,
-                                                      uint32_t wave_off) {
+// How tiles store their 16-byte pieces of C (the host decides, store_policy()).
+//   kStoreStream  aligned, with the streaming policy: C is written once and read by a later kernel at best, and what ordinary
+//                 stores leave in the L2s is written back when the kernel ends (2048x4096x4096: 30.9 us, 34.3 with those)
+//   kStoreKeep    aligned, without it (the plain and the block-scaled form)
+//   kStoreAny     at any 2 bytes, without it
+constexpr int kStoreStream = 0, kStoreKeep = 1, kStoreAny = 2;
+
+// One wave-wide store of 16 bytes per lane through a buffer descriptor (address = base + lane_off + wave_off).
+template <bool STREAM>
+__device__ __forceinline__ void store_chunk(v4i data, __amdgpu_buffer_rsrc_t rsrc, uint32_t lane_off, uint32_t wave_off) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  __builtin_amdgcn_raw_buffer_store_b128(data, rsrc, (int)lane_off, (int)wave_off, 2);
+  __builtin_amdgcn_raw_buffer_store_b128(data, rsrc, (int)lane_off, (int)wave_off, STREAM ? 2 : 0);
 #endif
+}
+
+// The first `valid` of 8 consecutive 16-bit results (none below 1, all from 8 on) to a row of C that starts at any 2 bytes: one
+// unaligned store, pieces of 4, 2 and 1 where the row ends.
+// (`valid` is opaque: the comparisons stay here, where as common values of many stores they would live in scalar registers)
+__device__ __forceinline__ void store_columns(uint8_t* dst, v4i out, int valid) {
+  asm volatile("" : "+v"(valid));
+  if (valid >= 8) {
+    *(v4i_any*)dst = out;
+  } else if (valid > 0) {
+    uint32_t first = (uint32_t)out[0], second = (uint32_t)out[1];
+    if (valid & 4) {
+      *(v2u_any*)dst = (v2u){first, second};
+      first = (uint32_t)out[2];
+      second = (uint32_t)out[3];
+      dst += 8;
+    }
+    if (valid & 2) {
+      *(u32_any*)dst = first;
+      first = second;
+      dst += 4;
+    }
+    if (valid & 1) *(uint16_t*)dst = (uint16_t)first;
+  }
 }
 
 // Waits until at most VM of this wave's global loads and none of its LDS operations are
@@ -814,12 +849,11 @@ void gemm_tiled_kernel(GemmParams p) {
   constexpr int ITERS = 32 / ROWS_PER_READ;
   static_assert(B_GROUPS % 4 == 0 && NT % PASS_J == 0 && (CPR == 4 || CPR == 8) && 2 * GROUPS_PER_PASS == B_GROUPS,
                 "turn-table geometry");
-  auto epilogue = [&](const TileLoc& loc, auto vector_tag, auto f16_tag, uint8_t* free_b_stage) {
+  auto epilogue = [&](const TileLoc& loc, auto store_tag, auto f16_tag, uint8_t* free_b_stage) {
     const int m0 = loc.m0, n0 = loc.n0;
-    // VECTOR: C takes 16-byte stores (base and row pitch aligned, N a multiple of 8, so no lane's 8
-    // columns straddle the edge). Edge tiles take it too: rows past the edge fall outside the output
-    // descriptor's extent and lanes past column N are sent there. Anything else stores element by element.
-    constexpr bool VECTOR = decltype(vector_tag)::value;
+    // Aligned stores: no lane's 8 columns straddle the edge. Edge tiles take them too: rows past the edge fall outside the output
+    // descriptor's extent and lanes past column N are sent there.
+    constexpr int STORE = decltype(store_tag)::value;
     constexpr bool OUT_F16 = decltype(f16_tag)::value;      // IEEE binary16 instead of bf16
     // row r of the pass kept in half h of the table
     auto row_addr = [&](int h, int r) -> uint8_t* {
@@ -918,12 +952,14 @@ void gemm_tiled_kernel(GemmParams p) {
     };
     // The wave's part of the tile as a buffer: origin at its first element, extent = its valid rows
     // (none for a wave that lies past the edge); offsets stay below 2^31 by the host's check of ldc.
-    const uint32_t c_row_bytes = (uint32_t)p.ldc * 2u;
+    // (opaque: its multiples are worked out here, not in front of the item loop where the epilogues' common ones would be kept)
+    uint32_t c_row_bytes = (uint32_t)p.ldc * 2u;
+    asm volatile("" : "+s"(c_row_bytes));
     // (pinned to a scalar register: the double clamp exists as a vector instruction only, and a
     // descriptor held in vector registers makes every store a loop)
     const int c_rows = __builtin_amdgcn_readfirstlane(min(max(loc.m_end - (m0 + wm * WTM), 0), WTM));
-    const __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        p.c + ((size_t)(m0 + wm * WTM) * p.ldc + n0 + wn * WTN), 0, (int)((uint32_t)c_rows * c_row_bytes), 0x00020000);
+    uint16_t* const c_wave = p.c + ((size_t)(m0 + wm * WTM) * p.ldc + n0 + wn * WTN);
+    const __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc(c_wave, 0, (int)((uint32_t)c_rows * c_row_bytes), 0x00020000);
     const uint32_t c_lane = (uint32_t)rd_row * c_row_bytes + (uint32_t)rd_col * 2u;
     constexpr int NP = MT * NJP;
     __builtin_amdgcn_sched_barrier(0);
@@ -948,18 +984,13 @@ void gemm_tiled_kernel(GemmParams p) {
       for (int it = 0; it < ITERS; ++it) {
         const int r = it * ROWS_PER_READ + rd_row;
         const v4i out = rows16[it];
-        if (VECTOR) {
+        if (STORE != kStoreAny) {
           // lane part (rd_row, rd_col) + scalar part (block row, read round, pass column)
-          store_chunk_streaming(out, c_rsrc, c_lane_pass,
-                                (uint32_t)(i * 32 + it * ROWS_PER_READ) * c_row_bytes + (uint32_t)(jp * PASS_J * 32 * 2));
+          store_chunk<STORE == kStoreStream>(out, c_rsrc, c_lane_pass,
+                                             (uint32_t)(i * 32 + it * ROWS_PER_READ) * c_row_bytes + (uint32_t)(jp * PASS_J * 32 * 2));
         } else {
-          const int m = m0 + wm * WTM + i * 32 + r;
-          uint16_t* dst = p.c + (size_t)m * p.ldc + n;
-          if (m < loc.m_end) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-              if (n + e < p.N) dst[e] = (uint16_t)((unsigned)out[e / 2] >> (16 * (e & 1)));
-          }
+          store_columns((uint8_t*)c_wave + c_lane + ((uint32_t)(i * 32 + it * ROWS_PER_READ) * c_row_bytes + (uint32_t)(jp * PASS_J * 32 * 2)),
+                        out, i * 32 + r < c_rows ? p.N - n : 0);
         }
       }
     }
@@ -1180,17 +1211,15 @@ void gemm_tiled_kernel(GemmParams p) {
       } else {
         // sb already names the next step's stage; the one before it held this tile's last step
         uint8_t* free_b = lds + LDS_B0 + ((sb + kStagesB - 1) % kStagesB) * STAGE_B;
-        // 16-byte stores need C's base and row pitch aligned and N a multiple of 8 (no lane's 8 columns
-        // straddle the edge); anything else stores element by element
-        const uintptr_t bits = reinterpret_cast<uintptr_t>(p.c) | (uintptr_t)(p.ldc * 2) | (uintptr_t)(p.N * 2);
-        // (the output type is a compile-time property of the epilogue code: one uniform branch per tile)
-        if ((bits & 15) == 0) {
-          if (p.out_f16) epilogue(loc, std::true_type{}, std::true_type{}, free_b);
-          else epilogue(loc, std::true_type{}, std::false_type{}, free_b);
-        } else {
-          if (p.out_f16) epilogue(loc, std::false_type{}, std::true_type{}, free_b);
-          else epilogue(loc, std::false_type{}, std::false_type{}, free_b);
-        }
+        // (kind of store and output type are compile-time properties of the epilogue code: one uniform branch per tile)
+        auto finish = [&](auto store_tag) {
+          if (p.out_f16) epilogue(loc, store_tag, std::true_type{}, free_b);
+          else epilogue(loc, store_tag, std::false_type{}, free_b);
+        };
+        if (p.store == kStoreStream) finish(std::integral_constant<int, kStoreStream>{});
+        // (the grouped form is without kStoreKeep, whose code costs its other launches 1-3 %)
+        else if (!GROUPED && p.store == kStoreKeep) finish(std::integral_constant<int, GROUPED ? kStoreAny : kStoreKeep>{});
+        else finish(std::integral_constant<int, kStoreAny>{});
       }
     }
     read_first_half();  // of the next item's first step (landed before this item's last barrier)
@@ -1407,14 +1436,15 @@ void gemm_block_kernel(GemmParams p) {
 
   // ---- epilogue: each 32-row block of the wave's tile is turned through LDS as 16-bit values, in the four
   // 1 KB groups this wave fetches itself of the B stage the tile's last step was read from
-  auto epilogue = [&](int m0, int n0, uint8_t* table, auto vector_tag) {
-    constexpr bool VECTOR = decltype(vector_tag)::value;
+  auto epilogue = [&](int m0, int n0, uint8_t* table, auto store_tag) {
+    constexpr int STORE = decltype(store_tag)::value;
     int lane_e;  // (an opaque copy: see the tiled kernel's epilogue)
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_e));
     const int row = lane_e & 31, hi = lane_e >> 5, rd_row = lane_e >> 3, rd_c = lane_e & 7;
     auto at = [&](int r, int c) { return table + (wave + NW * (r >> 3)) * 1024 + (r & 7) * 128 + ((c ^ (r & 7)) * 16); };
     const int m_wave = m0 + wm * 128, n_wave = n0 + wn * 64;
-    const uint32_t c_row_bytes = (uint32_t)p.ldc * 2u;
+    uint32_t c_row_bytes = (uint32_t)p.ldc * 2u;
+    asm volatile("" : "+s"(c_row_bytes));
     const int c_rows = __builtin_amdgcn_readfirstlane(min(max(p.M - m_wave, 0), 128));
     const __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc(p.c + ((size_t)m_wave * p.ldc + n_wave), 0,
                                                                             (int)((uint32_t)c_rows * c_row_bytes), 0x00020000);
@@ -1434,16 +1464,11 @@ void gemm_block_kernel(GemmParams p) {
       for (int it = 0; it < 4; ++it) out[it] = *(const v4i*)at(it * 8 + rd_row, rd_c);
 #pragma unroll
       for (int it = 0; it < 4; ++it) {
-        if (VECTOR) {
-          store_chunk_streaming(out[it], c_rsrc, c_lane, (uint32_t)(i * 32 + it * 8) * c_row_bytes);
+        if (STORE != kStoreAny) {
+          store_chunk<STORE == kStoreStream>(out[it], c_rsrc, c_lane, (uint32_t)(i * 32 + it * 8) * c_row_bytes);
         } else {
-          const int m = m_wave + i * 32 + it * 8 + rd_row;
-          uint16_t* dst = p.c + (size_t)m * p.ldc + n;
-          if (m < p.M) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-              if (n + e < p.N) dst[e] = (uint16_t)((unsigned)out[it][e / 2] >> (16 * (e & 1)));
-          }
+          const int r = i * 32 + it * 8 + rd_row;
+          store_columns((uint8_t*)(p.c + ((size_t)(m_wave + r) * p.ldc + n)), out[it], r < c_rows ? p.N - n : 0);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -1466,7 +1491,6 @@ void gemm_block_kernel(GemmParams p) {
     load_step(c_mat);
     __builtin_amdgcn_s_barrier();
   }
-  const bool vec = ((reinterpret_cast<uintptr_t>(p.c) | (uintptr_t)(p.ldc * 2) | (uintptr_t)(p.N * 2)) & 15) == 0;
   for (int item = walk.slot; item < walk.chunk_len; item += walk.slots) {
     int m0, n0;
     tile_of(item, m0, n0);
@@ -1481,8 +1505,9 @@ void gemm_block_kernel(GemmParams p) {
       matrix_phase(std::false_type{}, kt);
     }
     uint8_t* table = lds + LDS_B0 + (sb == 0 ? 2 : sb - 1) * STAGE;
-    if (vec) epilogue(m0, n0, table, std::true_type{});
-    else epilogue(m0, n0, table, std::false_type{});
+    if (p.store == kStoreStream) epilogue(m0, n0, table, std::integral_constant<int, kStoreStream>{});
+    else if (p.store == kStoreKeep) epilogue(m0, n0, table, std::integral_constant<int, kStoreKeep>{});
+    else epilogue(m0, n0, table, std::integral_constant<int, kStoreAny>{});
   }
   if (lead) __builtin_amdgcn_s_barrier();  // the second group's last phase
   wait_loads<0>();  // (loads into LDS land before it is released)
@@ -1604,9 +1629,6 @@ __global__ __launch_bounds__(256) void splitk_finalize_rows_kernel(GemmParams p)
 // ------------------------------------------------------------------------------------
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
-typedef uint32_t v2u_any __attribute__((ext_vector_type(2), aligned(1)));
-typedef uint32_t u32_any __attribute__((aligned(1)));
 typedef uint16_t u16_any __attribute__((aligned(1)));
 
 // bytes [k, k + 16) of a row of K bytes; those at or past K count as zero
@@ -3863,9 +3885,23 @@ int mi355x_shared::ready_device(int* dev_out) {
 #endif
 
 namespace {
+// How a launch of tiles stores C. The streaming policy is for rows on the 128-byte lines, or a C that the L2s hold: off the
+// lines two pieces share a line, which then goes to memory twice in parts. us streaming / ordinary, rows 16 to 32 bytes off
+// the lines: 4924x9808x1024 (97 MB) 80 / 65, 3000x9736x2304 (58) 77 / 61, 6935x5200x1200 (72) 75 / 64.5, block-scaled
+// 4096x8208x1024 (67) 65 / 57, 16384x1040x1024 (34) 32 / 31, 2048x4112x4096 (17) 35.5 / 38.9; on the lines 3122x9728x2304 59 / 63.
+// Pieces that start at any 2 bytes, as one store each where they were eight of 2 bytes: 4924x9807x1024 127 -> 69, 5203x3266x1152
+// 56 -> 31, 1024x5203x1200 23.4 -> 15.4, 16 groups of 8192x4111x1024 112 -> 63 (streaming ones of that kind 97, 38, 17, 73).
+constexpr int64_t kL2Bytes = (int64_t)kNumXcd << 22;
+inline int store_policy(const GemmParams& p) {
+  const uintptr_t base = reinterpret_cast<uintptr_t>(p.c), pitch = (uintptr_t)(p.ldc * 2);
+  if ((base | pitch | (uintptr_t)p.N * 2) & 15) return kStoreAny;
+  return ((base | pitch) & 127) != 0 && (int64_t)p.M * p.N * 2 > kL2Bytes ? kStoreKeep : kStoreStream;
+}
+
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool KTAIL, int EPI, bool GROUPED = false, bool BLOCKSCALE = false,
           int DIST = kDefaultDist, bool STREAM_B = false, bool CLEAR = false>
 int launch_tiled(GemmParams p, hipStream_t stream) {
+  p.store = store_policy(p);
   constexpr int threads = WAVES_M * WAVES_N * 64;
   constexpr size_t lds_bytes = tiled_lds_bytes(BM, BN, DIST);
   // grouped: the group sizes live on the device; every group adds at most one partial tile row
@@ -4147,6 +4183,7 @@ template <bool KTAIL>
 int launch_block_form(GemmParams p, hipStream_t stream) {
   constexpr auto kern = gemm_block_kernel<KTAIL>;
   (void)LdsLimit<kern, kBlockLdsBytes>::registered;
+  p.store = store_policy(p);
   p.tiles_m = (p.M + kBlockTile - 1) / kBlockTile;
   p.tiles_n = (p.N + kBlockTile - 1) / kBlockTile;
   make_fast_div((uint32_t)kGroupM * (uint32_t)p.tiles_n, p.div_group_mul, p.div_group_shift);
