@@ -89,3 +89,35 @@ def test_large_result_off_the_lines(gpu_device, m, n):
         _check(lambda c: ops.fp8_gemm_rowwise(a, b, sa, sb, out=c, out_dtype=dtype, variant=_lib.VARIANT_TILED), m, n, dtype, dev, [(8, 24), (0, 0)])
     xs, ws = torch.rand((-(-m // 128), 2), device=dev) + 0.5, torch.rand((-(-n // 128), 2), device=dev) + 0.5
     _check(lambda c: ops.fp8_gemm_blockwise(a, b, xs, ws, out=c), m, n, torch.bfloat16, dev, [(8, 24), (0, 0)])
+
+
+# split K with rows of partial sums that start on any 4 bytes: the columns of a panel that ends on 4 of them hold the same bits
+@pytest.mark.parametrize("config", range(7))
+@pytest.mark.parametrize("m,n,splits", [(3, 1, 2), (65, 129, 3), (130, 254, 2), (257, 515, 5), (300, 3, 4)])
+def test_partial_rows_off_sixteen_bytes(gpu_device, config, m, n, splits):
+    print(f"case {m}x{n} config {config} splits {splits}", flush=True)
+    dev, k = gpu_device, 1168
+    wide = -(-n // 4) * 4
+    a, b = _codes(m, k, 1, dev), _codes(wide, k, 2, dev)
+    sa, sb = torch.rand(m, device=dev) + 0.5, torch.rand(wide, device=dev) + 0.5
+    bias = torch.randn(wide, device=dev).to(torch.bfloat16)
+    variant = _lib.VARIANT_TILED | ((config + 1) << 8) | (splits << 16)
+    want = ops.fp8_gemm_rowwise(a, b, sa, sb, bias=bias, variant=variant)[:, :n]
+    space = torch.full((splits * m * n + 256,), 7.0, device=dev)
+    canvas, c = _place(m, n, 1, 6, torch.bfloat16, dev)
+    ops.fp8_gemm_rowwise(a, b[:n], sa, sb[:n], bias=bias[:n], out=c, variant=variant, workspace=space[: splits * m * n].view(torch.uint8))
+    torch.cuda.synchronize()
+    assert torch.equal(c.view(torch.int16), want.view(torch.int16))
+    c.fill_(7.0)
+    assert (canvas == 7.0).all() and (space[splits * m * n :] == 7.0).all()
+
+
+# (four rows a thread in the second pass: more than 2048 workgroups of 256 lanes with one)
+def test_second_pass_with_four_rows_off_sixteen_bytes(gpu_device):
+    dev, m, n, k = gpu_device, 1027, 2054, 272
+    a, b = _codes(m, k, 1, dev), _codes(n + 2, k, 2, dev)
+    sa, sb = torch.rand(m, device=dev) + 0.5, torch.rand(n + 2, device=dev) + 0.5
+    variant = _lib.tiled_variant(1, 2)
+    want = ops.fp8_gemm_rowwise(a, b, sa, sb, variant=variant)[:, :n]
+    got = ops.fp8_gemm_rowwise(a, b[:n], sa, sb[:n], variant=variant)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16).contiguous())

@@ -126,6 +126,7 @@ typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
 typedef uint32_t v2u_any __attribute__((ext_vector_type(2), aligned(1)));
 typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef float v4f_by4 __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kNumXcd = 8;       // accelerator complex dies; workgroup ids round-robin over them
 constexpr int kNumCu = 256;
@@ -450,7 +451,7 @@ void gemm_tiled_kernel(GemmParams p) {
   static_assert(DIST >= 2 && tiled_lds_bytes(BM, BN, DIST) <= 160 * 1024, "the stage rings must fit the LDS");
   static_assert(!GROUPED || EPI == kEpiPlain, "the grouped form has neither bias nor split-K");
   static_assert(!CLEAR || GROUPED, "only the grouped form has rows past its groups'");
-  static_assert(!BLOCKSCALE || (128 % (BM / WAVES_M) == 0 && 128 % (BN / WAVES_N) == 0 && EPI == kEpiPlain && !GROUPED),
+  static_assert(!BLOCKSCALE || (128 % (BM / WAVES_M) == 0 && 128 % (BN / WAVES_N) == 0 && EPI != kEpiBias && !GROUPED),
                 "a wave's tile must lie inside one 128x128 scale block: one factor per wave and step");
   constexpr bool HAS_BIAS = EPI == kEpiBias;
   constexpr int NW = WAVES_M * WAVES_N;
@@ -998,48 +999,52 @@ void gemm_tiled_kernel(GemmParams p) {
   };
 
   // ---- split-K: raw fp32 partial sums of this item to partial[split][m][n]: the lane layout the
-  // MFMA leaves (4 consecutive n per lane), one 16-byte buffer store per 4 values when N is a multiple
-  // of 4: rows past M fall outside the descriptor's extent, lanes past N are sent there, and the
-  // values go from the accumulators to memory without passing through other registers.
+  // MFMA leaves (4 consecutive n per lane), one 16-byte buffer store per 4 values (rows of partials start on 4 bytes, which
+  // is all it asks for): rows past M fall outside the descriptor's extent, lanes whose 4 columns are not all below N are sent
+  // there, and the values go from the accumulators to memory without passing through other registers. Where N is no
+  // multiple of 4 the quad at the edge follows value by value. (All of them one by one, as such rows went before, and read one by one by
+  // the second pass: 1042x719x10624 29.4 us, now 22.2; 512x2049x8192 31.2, now 22.0; 128x8194x8192 37.3, now 28.4.)
   auto store_partial = [&](int m0, int n0, int split) {
     int lane_e;  // (inside the opaque statement for the reason given in the epilogue)
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_e));
     const int l32 = lane_e & 31, half = lane_e >> 5;
     float* base = p.partial + (size_t)split * p.M * p.N;
-    if ((p.N & 3) == 0) {
-      const uint32_t row_bytes = (uint32_t)p.N * 4u;  // (N*4*128 < 2^31 by the host's check of the workspace plan)
-      const int rows = __builtin_amdgcn_readfirstlane(min(max(p.M - (m0 + wm * WTM), 0), WTM));  // (scalar: see the epilogue)
-      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-          base + ((size_t)(m0 + wm * WTM) * p.N + n0 + wn * WTN), 0, (int)((uint32_t)rows * row_bytes), 0x00020000);
-      const uint32_t lane_off = (uint32_t)l32 * row_bytes + (uint32_t)(4 * half) * 4u;
+    const uint32_t row_bytes = (uint32_t)p.N * 4u;  // (N*4*128 < 2^31 by the host's check of the workspace plan)
+    const int rows = __builtin_amdgcn_readfirstlane(min(max(p.M - (m0 + wm * WTM), 0), WTM));  // (scalar: see the epilogue)
+    float* const tile = base + ((size_t)(m0 + wm * WTM) * p.N + n0 + wn * WTN);
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(tile, 0, (int)((uint32_t)rows * row_bytes), 0x00020000);
+    const uint32_t lane_off = (uint32_t)l32 * row_bytes + (uint32_t)(4 * half) * 4u;
 #pragma unroll
-      for (int j = 0; j < NT; ++j) {
+    for (int j = 0; j < NT; ++j) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int n = n0 + wn * WTN + j * 32 + 8 * q + 4 * half;
-          const uint32_t lo = n < p.N ? lane_off : 0x80000000u;
+      for (int q = 0; q < 4; ++q) {
+        const int n = n0 + wn * WTN + j * 32 + 8 * q + 4 * half;
+        const uint32_t lo = n + 3 < p.N ? lane_off : 0x80000000u;
 #pragma unroll
-          for (int i = 0; i < MT; ++i) {
-            const v4f v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-            store_f32x4_checked(v, rsrc, lo, (uint32_t)(i * 32) * row_bytes + (uint32_t)(j * 32 + 8 * q) * 4u);
-          }
+        for (int i = 0; i < MT; ++i) {
+          v4f v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+          if (BLOCKSCALE) v = v * s_last;  // (back from the units of the last step's factor)
+          store_f32x4_checked(v, rsrc, lo, (uint32_t)(i * 32) * row_bytes + (uint32_t)(j * 32 + 8 * q) * 4u);
         }
       }
-    } else {
+    }
+    const int n_left = p.N - (n0 + wn * WTN);  // columns of the wave's tile, or more
+    if ((p.N & 3) != 0 && n_left > 0 && n_left < WTN) {
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const int m = m0 + wm * WTM + i * 32 + l32;
+      for (int j = 0; j < NT; ++j) {
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          __builtin_amdgcn_sched_barrier(0);
+        for (int q = 0; q < 4; ++q) {
+          const int n = j * 32 + 8 * q + 4 * half;
+          if (n < n_left && n + 3 >= n_left) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int n = n0 + wn * WTN + j * 32 + 8 * q + 4 * half;
-            if (m < p.M) {
-              float* dst = base + (size_t)m * p.N + n;
+            for (int i = 0; i < MT; ++i) {
+              if (i * 32 + l32 < rows) {
+                float* dst = tile + ((size_t)(i * 32 + l32) * p.N + n);
 #pragma unroll
-              for (int e = 0; e < 4; ++e)
-                if (n + e < p.N) dst[e] = acc[i][j][4 * q + e];
+                for (int e = 0; e < 3; ++e)
+                  if (n + e < n_left) dst[e] = BLOCKSCALE ? acc[i][j][4 * q + e] * s_last : acc[i][j][4 * q + e];
+              }
             }
           }
         }
@@ -1177,7 +1182,7 @@ void gemm_tiled_kernel(GemmParams p) {
     if (BLOCKSCALE) {
       const TileLoc loc = locate(walk_c, c_item);
       load_block_scales(loc);
-      kt_c = first_step(loc, 0, k_steps);
+      kt_c = first_step(loc, split_begin(c_split), n_steps);
       n_pend = lane_value(rt, kt_c + 1);
       n_last = lane_value(sc, kt_c);
     }
@@ -1532,8 +1537,6 @@ __device__ __forceinline__ void splitk_finalize(const GemmParams& p) {
   const int m0 = (int)row_group * ROWS;
   const int n = (int)(idx - row_group * quads_per_row) * 4;
   const size_t plane = (size_t)p.M * p.N;
-  // (N a multiple of 4: n + 3 < N and every row start is 16-byte aligned. With several rows a thread it always is.)
-  const bool vec = ROWS > 1 || (p.N & 3) == 0;
   const float* src[ROWS];
   float sa[ROWS], sb[4];
   uint16_t bias[4] = {0, 0, 0, 0};
@@ -1542,15 +1545,15 @@ __device__ __forceinline__ void splitk_finalize(const GemmParams& p) {
   for (int i = 0; i < ROWS; ++i) {
     const int m = min(m0 + i, p.M - 1);  // (rows past the last one read it again)
     src[i] = p.partial + (size_t)m * p.N + n;
-    sa[i] = p.a_scale[m];  // fetched beside the partial sums, not after them
+    sa[i] = p.a_scale ? p.a_scale[m] : 1.0f;  // fetched beside the partial sums, not after them
     sum[i] = (v4f){0.f, 0.f, 0.f, 0.f};
   }
 #pragma unroll
-  for (int e = 0; e < 4; ++e) sb[e] = p.b_scale[min(n + e, p.N - 1)];
+  for (int e = 0; e < 4; ++e) sb[e] = p.b_scale ? p.b_scale[min(n + e, p.N - 1)] : 1.0f;
   if (p.bias)
 #pragma unroll
     for (int e = 0; e < 4; ++e) bias[e] = p.bias[min(n + e, p.N - 1)];
-  if (vec) {
+  if (n + 3 < p.N) {  // (a row of partials starts on any 4 bytes)
     // added in split order, as the scalar form does
     auto add = [&](int s, auto count) {
       constexpr int COUNT = decltype(count)::value;
@@ -1558,7 +1561,7 @@ __device__ __forceinline__ void splitk_finalize(const GemmParams& p) {
 #pragma unroll
       for (int u = 0; u < COUNT; ++u)
 #pragma unroll
-        for (int i = 0; i < ROWS; ++i) part[u][i] = __builtin_nontemporal_load((const v4f*)(src[i] + (s + u) * plane));
+        for (int i = 0; i < ROWS; ++i) part[u][i] = __builtin_nontemporal_load((const v4f_by4*)(src[i] + (s + u) * plane));
 #pragma unroll
       for (int u = 0; u < COUNT; ++u)
 #pragma unroll
@@ -1576,7 +1579,7 @@ __device__ __forceinline__ void splitk_finalize(const GemmParams& p) {
 #pragma unroll
       for (int i = 0; i < ROWS; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+        for (int e = 0; e < 3; ++e)
           if (n + e < p.N) sum[i][e] += src[i][s * plane + e];
     }
   }
@@ -1591,13 +1594,12 @@ __device__ __forceinline__ void splitk_finalize(const GemmParams& p) {
     }
     const uint32_t lo = pack_out_x2(r[0], r[1], p.out_f16), hi = pack_out_x2(r[2], r[3], p.out_f16);
     uint16_t* dst = p.c + (size_t)(m0 + i) * p.ldc + n;
-    if (n + 3 < p.N && ((p.ldc & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.c) & 7) == 0)) {
-      *(v2u*)dst = (v2u){lo, hi};
+    if (n + 3 < p.N) {
+      *(v2u_any*)dst = (v2u){lo, hi};
     } else {
       dst[0] = (uint16_t)lo;
       if (n + 1 < p.N) dst[1] = (uint16_t)(lo >> 16);
       if (n + 2 < p.N) dst[2] = (uint16_t)hi;
-      if (n + 3 < p.N) dst[3] = (uint16_t)(hi >> 16);
     }
   }
 }
@@ -3921,12 +3923,12 @@ int launch_tiled(GemmParams p, hipStream_t stream) {
   if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "tiled kernel launch: %s", hipGetErrorString(e));
   if (EPI == kEpiPartial) {
     // Four rows a thread where one row each would be more workgroups than the chip holds at once (8 of 256 lanes on a
-    // CU): fewer of them to start, more loads in flight each. Below that they would leave CUs idle. (Rows of partials that
-    // start off 16 bytes are read element by element, one row a thread.)
+    // CU): fewer of them to start, more loads in flight each. Below that they would leave CUs idle.
     const long quads_per_row = ((long)p.N + 3) / 4;
-    const bool many = p.N % 4 == 0 && (quads_per_row * p.M + 255) / 256 > 8L * kNumCu;
+    const bool many = (quads_per_row * p.M + 255) / 256 > 8L * kNumCu;
     const long quads = quads_per_row * (many ? ((long)p.M + kFinalizeRows - 1) / kFinalizeRows : p.M);
     GemmParams f = p;
+    if (BLOCKSCALE) f.a_scale = f.b_scale = nullptr;  // (the factors were applied block by block)
     f.div_group_mul = f.div_group_shift = 0;
     if (quads <= (long)INT32_MAX - 255) make_fast_div((uint32_t)quads_per_row, f.div_group_mul, f.div_group_shift);
     hipLaunchKernelGGL(many ? splitk_finalize_rows_kernel : splitk_finalize_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0,
