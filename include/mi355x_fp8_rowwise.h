@@ -304,6 +304,20 @@ int mi355x_fp8_blockwise_gemm_ex(const void* a, const void* b,
                                  int64_t lda, int64_t ldb, int64_t ldc, int form, void* stream);
 
 /*
+ * The same with a workspace: where the tiles are few and K is long the library cuts K and adds the parts up in a second
+ * launch, in a fixed order, if the workspace (device memory, 16-byte aligned) holds them: as many bytes as
+ * mi355x_fp8_blockwise_workspace_bytes names for the shape (0: it would not). A smaller one takes the best plan that fits it.
+ * With form = TILES_128 + 256 * s the factor is pinned to s (EINVAL without the workspace for it). What is in the workspace
+ * before a call does not matter; two calls that may overlap need one each.
+ */
+size_t mi355x_fp8_blockwise_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int mi355x_fp8_blockwise_gemm_ws(const void* a, const void* b,
+                                 const float* a_scale, const float* b_scale, void* c,
+                                 int64_t M, int64_t N, int64_t K,
+                                 int64_t lda, int64_t ldb, int64_t ldc,
+                                 void* workspace, size_t workspace_bytes, int form, void* stream);
+
+/*
  * Block-wise e4m3fn quantiser, replacing fp8_block_quantize
  * (tritonbench/operators/fp8_gemm_blockwise/operator.py:86-118): one scale per 128 x 128 block,
  *

@@ -79,8 +79,8 @@ def test_block_scaled_tiles_at_any_place(gpu_device, form, m, n):
     _check(run, m, n, torch.bfloat16, dev, PLACES)
 
 
-# a C that the L2s (32 MB) do not hold, on and off the lines: aligned ordinary stores
-@pytest.mark.parametrize("m,n", [(2050, 8328), (4100, 4136)])
+# a C of more than 48 MB, on and off the lines: ordinary stores
+@pytest.mark.parametrize("m,n", [(3070, 8328), (6150, 4136)])
 def test_large_result_off_the_lines(gpu_device, m, n):
     dev, k = gpu_device, 144
     a, b = _codes(m, k, 1, dev), _codes(n, k, 2, dev)

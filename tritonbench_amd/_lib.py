@@ -113,6 +113,12 @@ SIGNATURES = {
         [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
          c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int, c_void_p],
     ),
+    "mi355x_fp8_blockwise_workspace_bytes": (c_size_t, [c_int64, c_int64, c_int64]),
+    "mi355x_fp8_blockwise_gemm_ws": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+         c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p, c_size_t, c_int, c_void_p],
+    ),
     "mi355x_fp8_blockwise_quantize": (
         c_int,
         [c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_void_p],

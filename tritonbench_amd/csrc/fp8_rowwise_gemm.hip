@@ -328,7 +328,7 @@ __device__ __forceinline__ void store_f32x4_checked(v4f data, __amdgpu_buffer_rs
 // How tiles store their 16-byte pieces of C (the host decides, store_policy()).
 //   kStoreStream  aligned, with the streaming policy: C is written once and read by a later kernel at best, and what ordinary
 //                 stores leave in the L2s is written back when the kernel ends (2048x4096x4096: 30.9 us, 34.3 with those)
-//   kStoreKeep    aligned, without it (the plain and the block-scaled form)
+//   kStoreKeep    aligned, without it (gemm_block_kernel)
 //   kStoreAny     at any 2 bytes, without it
 constexpr int kStoreStream = 0, kStoreKeep = 1, kStoreAny = 2;
 
@@ -1221,9 +1221,8 @@ void gemm_tiled_kernel(GemmParams p) {
           if (p.out_f16) epilogue(loc, store_tag, std::true_type{}, free_b);
           else epilogue(loc, store_tag, std::false_type{}, free_b);
         };
+        // (no kStoreKeep here: its code costs all other launches 1-2 %, up to 5 where a tile has few steps)
         if (p.store == kStoreStream) finish(std::integral_constant<int, kStoreStream>{});
-        // (the grouped form is without kStoreKeep, whose code costs its other launches 1-3 %)
-        else if (!GROUPED && p.store == kStoreKeep) finish(std::integral_constant<int, GROUPED ? kStoreAny : kStoreKeep>{});
         else finish(std::integral_constant<int, kStoreAny>{});
       }
     }
@@ -3887,17 +3886,18 @@ int mi355x_shared::ready_device(int* dev_out) {
 #endif
 
 namespace {
-// How a launch of tiles stores C. The streaming policy is for rows on the 128-byte lines, or a C that the L2s hold: off the
-// lines two pieces share a line, which then goes to memory twice in parts. us streaming / ordinary, rows 16 to 32 bytes off
-// the lines: 4924x9808x1024 (97 MB) 80 / 65, 3000x9736x2304 (58) 77 / 61, 6935x5200x1200 (72) 75 / 64.5, block-scaled
-// 4096x8208x1024 (67) 65 / 57, 16384x1040x1024 (34) 32 / 31, 2048x4112x4096 (17) 35.5 / 38.9; on the lines 3122x9728x2304 59 / 63.
-// Pieces that start at any 2 bytes, as one store each where they were eight of 2 bytes: 4924x9807x1024 127 -> 69, 5203x3266x1152
+// How a launch of tiles stores C. The streaming policy is for rows on 64 bytes, or a C that is not much more than the
+// L2s hold (32 MB): with others two pieces share 64 bytes, which then go to memory twice in parts. us streaming / ordinary,
+// rows 16 to 32 bytes off the lines: 4924x9808x1024 (97 MB) 80 / 66, 3000x9736x2304 (58) 77 / 63, 6935x5200x1200 (72) 75 / 68,
+// block-scaled 4096x8208x1024 (67) 65 / 57, 16384x1040x1024 (34) 32 / 33, 2048x4112x4096 (17) 35.5 / 38.9; on the lines
+// 3122x9728x2304 59 / 63; on 64 bytes 5000x9760x1024 68.6 / 70.4, block-scaled 1129x24928x1504 50 / 58.
+// Pieces that start at any 2 bytes, as one store each where they were eight of 2 bytes: 4924x9807x1024 127 -> 68, 5203x3266x1152
 // 56 -> 31, 1024x5203x1200 23.4 -> 15.4, 16 groups of 8192x4111x1024 112 -> 63 (streaming ones of that kind 97, 38, 17, 73).
-constexpr int64_t kL2Bytes = (int64_t)kNumXcd << 22;
+constexpr int64_t kLargeResult = (int64_t)48 << 20;
 inline int store_policy(const GemmParams& p) {
   const uintptr_t base = reinterpret_cast<uintptr_t>(p.c), pitch = (uintptr_t)(p.ldc * 2);
   if ((base | pitch | (uintptr_t)p.N * 2) & 15) return kStoreAny;
-  return ((base | pitch) & 127) != 0 && (int64_t)p.M * p.N * 2 > kL2Bytes ? kStoreKeep : kStoreStream;
+  return ((base | pitch) & 63) != 0 && (int64_t)p.M * p.N * 2 > kLargeResult ? kStoreKeep : kStoreStream;
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool KTAIL, int EPI, bool GROUPED = false, bool BLOCKSCALE = false,
@@ -4154,7 +4154,7 @@ inline float block_one_tile_cost_us(int64_t M, int64_t N, int64_t K, float off_l
   const float per_wg = (M <= 16 ? 2.4e-3f : M <= 32 ? 2.8e-3f : M <= 48 ? 4.1e-3f : 10.0e-3f) + 0.2e-3f * steps;
   return fmaxf(off_lines * one_tile_cost_us(M, N, K), 3.0f + (wgs > kNumCu ? (float)(wgs - kNumCu) * per_wg : 0.0f));
 }
-inline BlockForm block_form(int64_t M, int64_t N, int64_t K, int64_t ldb) {
+inline BlockForm block_form(int64_t M, int64_t N, int64_t K, int64_t ldb, float* cost_us = nullptr) {
   BlockForm best = block_streams(M, N, K, ldb) ? kBlockSmallStream : kBlockSmall;
   float cost = block_small_cost_us(M, N, K, ldb);
   auto weigh = [&](BlockForm form, float us) {
@@ -4178,6 +4178,43 @@ inline BlockForm block_form(int64_t M, int64_t N, int64_t K, int64_t ldb) {
   }
   if (M <= kSkinnyMaxM) weigh(kBlockOneTile, block_one_tile_cost_us(M, N, K, one_tile_off));
   if (narrow_fits(M, N, K)) weigh(kBlockNarrow, narrow_off * narrow_cost_us(M, N, K));
+  if (cost_us) *cost_us = cost;
+  return best;
+}
+
+// K cut in parts where the tiles are few and K is long (with a workspace for the parts). us before, the best form in one piece -> now:
+// 1000x1000x28672 160 -> 49, 312x512x9088 37.3 -> 15.4, 1047x1566x12800 78 -> 43, 92x512x26368 29.5 -> 17.3, 32x1024x28672
+// 27.1 -> 18.1, 500x5120x13824 80 -> 58, 96x16384x16384 96 -> 74, 256x4098x4096 25.5 -> 20.2; behind nowhere by more than 1 %.
+struct BlockPlan {
+  BlockForm form;
+  int splits, steps_per_split;
+};
+// 128x128 tiles with K cut into `splits` parts of `sps` steps: the times of block_small_cost_us over the work items, the second launch
+// and the parts' trip through memory; bound by the stream of B where the tiles are one or two rows (64x28672x8192 in two
+// 68 us, 128x57344x8192 142, where the streaming form takes 45 and 95 in one piece).
+inline float block_split_cost_us(int64_t M, int64_t N, int64_t K, int splits, int sps) {
+  const long items = ((M + 127) / 128) * ((N + 127) / 128) * splits, full = items / (2 * kNumCu), rest = items % (2 * kNumCu);
+  float t = (float)full * ((float)sps + 5.0f);
+  if (rest) t += (float)sps * (rest <= kNumCu ? 0.45f + 0.1f * (float)rest / (float)kNumCu : 1.0f) + 5.0f;
+  t = fmaxf(t, (float)(M + N) * (float)K / 4.4e6f);
+  return t + 4.5f + 2.0f * (float)splits * (float)M * (float)N * 4.0f / 5.0e6f;
+}
+inline BlockPlan block_plan(int64_t M, int64_t N, int64_t K, int64_t ldb, int max_splits) {
+  const int k_steps = k_steps_of(K);
+  float cost = 0.0f;
+  BlockPlan best = {block_form(M, N, K, ldb, &cost), 1, k_steps};
+  for (int want = 2; want <= max_splits; ++want) {
+    int splits, sps;
+    normalise_splits(k_steps, want, splits, sps);
+    if (splits != want || N * 512 > (int64_t)INT32_MAX) continue;
+    // (up to 16 rows the streaming forms are quicker than their estimates on long rows off the lines: 3x1425x24896 17.2 us,
+    // in fifteen parts 23.5, 4x523x22816 21.4 and 22.8)
+    const float us = block_split_cost_us(M, N, K, splits, sps) * (M <= 16 ? 1.5f : 1.0f);
+    if (us < cost) {
+      cost = us;
+      best = {kBlockSmall, splits, sps};
+    }
+  }
   return best;
 }
 
@@ -4760,12 +4797,24 @@ int mi355x_fp8_blockwise_form(int64_t M, int64_t N, int64_t K) {
 int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale, const float* b_scale,
                               void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                               int64_t ldc, void* stream) {
-  return mi355x_fp8_blockwise_gemm_ex(a, b, a_scale, b_scale, c, M, N, K, lda, ldb, ldc, -1, stream);
+  return mi355x_fp8_blockwise_gemm_ws(a, b, a_scale, b_scale, c, M, N, K, lda, ldb, ldc, nullptr, 0, -1, stream);
+}
+
+size_t mi355x_fp8_blockwise_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+  if (check_shape(M, N, K) != MI355X_FP8_OK || check_fast_shape(K) != MI355X_FP8_OK || K > 256 * kStepK) return 0;
+  const BlockPlan plan = block_plan(M, N, K, K, kMaxSplits);
+  return plan.splits > 1 ? (size_t)plan.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
 int mi355x_fp8_blockwise_gemm_ex(const void* a, const void* b, const float* a_scale, const float* b_scale,
                                  void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                                  int64_t ldc, int form, void* stream) {
+  return mi355x_fp8_blockwise_gemm_ws(a, b, a_scale, b_scale, c, M, N, K, lda, ldb, ldc, nullptr, 0, form, stream);
+}
+
+int mi355x_fp8_blockwise_gemm_ws(const void* a, const void* b, const float* a_scale, const float* b_scale,
+                                 void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                                 int64_t ldc, void* workspace, size_t workspace_bytes, int form, void* stream) {
   int st = check_shape(M, N, K);
   if (st == MI355X_FP8_OK) st = check_fast_shape(K);
   if (st != MI355X_FP8_OK) return st;
@@ -4794,8 +4843,30 @@ int mi355x_fp8_blockwise_gemm_ex(const void* a, const void* b, const float* a_sc
   p.div_tiles_mul = p.div_tiles_shift = p.div_group_mul = p.div_group_shift = 0; p.stamps = nullptr;
   hipStream_t s = (hipStream_t)stream;
   const bool ktail = K % kStepK;
-  if (form < 0) form = block_form(M, N, K, ldb);
-  else if ((form == kBlockOneTile && M > kSkinnyMaxM) || (form == kBlockNarrow && !narrow_fits(M, N, K)))
+  // (a split factor pinned to TILES_128)
+  const int want_splits = form < 0 ? 0 : form >> 8;
+  if (form >= 0) form &= 0xff;
+  if (want_splits && form != kBlockSmall) return fail(MI355X_FP8_EINVAL, "only the form of 128x128 tiles is split");
+  const size_t plane = (size_t)M * (size_t)N * sizeof(float);
+  if (form < 0 || want_splits) {
+    // (a workspace that holds fewer planes than the best plan wants takes the best one that it does hold)
+    const size_t planes = workspace ? workspace_bytes / plane : 0;
+    BlockPlan plan = block_plan(M, N, K, ldb, planes < 2 ? 1 : planes > (size_t)kMaxSplits ? kMaxSplits : (int)planes);
+    if (want_splits) {
+      plan.form = kBlockSmall;
+      normalise_splits(p.steps_per_split, want_splits, plan.splits, plan.steps_per_split);
+      if (plan.splits > 1 && ((size_t)plan.splits > planes || N * 512 > (int64_t)INT32_MAX))
+        return fail(MI355X_FP8_EINVAL, "split-K factor %d needs %zu bytes of workspace (got %zu)", plan.splits, plan.splits * plane,
+                    workspace ? workspace_bytes : (size_t)0);
+    }
+    if (plan.splits > 1) {
+      if (reinterpret_cast<uintptr_t>(workspace) & 15) return fail(MI355X_FP8_EINVAL, "workspace must be 16-byte aligned");
+      p.splits = plan.splits;
+      p.steps_per_split = plan.steps_per_split;
+      p.partial = (float*)workspace;
+    }
+    form = plan.form;
+  } else if ((form == kBlockOneTile && M > kSkinnyMaxM) || (form == kBlockNarrow && !narrow_fits(M, N, K)))
     return fail(MI355X_FP8_ENOTSUP, "block-scaled form %d does not take %lldx%lld", form, (long long)M, (long long)N);
   switch (form) {
     case kBlockNarrow: return launch_narrow_for<true>(p, s);
@@ -4808,9 +4879,23 @@ int mi355x_fp8_blockwise_gemm_ex(const void* a, const void* b, const float* a_sc
     case kBlockSmallStream:
       return ktail ? launch_tiled<128, 128, 2, 2, true, kEpiPlain, false, true, kDefaultDist, true>(p, s)
                    : launch_tiled<128, 128, 2, 2, false, kEpiPlain, false, true, kDefaultDist, true>(p, s);
-    case kBlockSmall:
+    case kBlockSmall: {
+      // Loads three steps ahead where a CU has one work item and long rows of it, against two: 1047x1566x12800 in two 49.5 -> 42.7 us,
+      // 1000x1000x28672 in four 54.5 -> 48.9, 64x4096x8192 in four 18.4 -> 17.4, level with fewer steps (unsplit,
+      // 130x16384x16384 95 -> 82, 100x20000x8192 51.5 -> 48.3; 1500x2560x7168 34.6 -> 35.0, 1024^3 9.0 -> 9.2).
+      const bool deep = ((M + 127) / 128) * ((N + 127) / 128) * p.splits <= kNumCu && p.steps_per_split >= (p.splits > 1 ? 16 : 64);
+      if (p.splits > 1 && deep)
+        return ktail ? launch_tiled<128, 128, 2, 2, true, kEpiPartial, false, true, 3>(p, s)
+                     : launch_tiled<128, 128, 2, 2, false, kEpiPartial, false, true, 3>(p, s);
+      if (p.splits > 1)
+        return ktail ? launch_tiled<128, 128, 2, 2, true, kEpiPartial, false, true>(p, s)
+                     : launch_tiled<128, 128, 2, 2, false, kEpiPartial, false, true>(p, s);
+      if (deep)
+        return ktail ? launch_tiled<128, 128, 2, 2, true, kEpiPlain, false, true, 3>(p, s)
+                     : launch_tiled<128, 128, 2, 2, false, kEpiPlain, false, true, 3>(p, s);
       return ktail ? launch_tiled<128, 128, 2, 2, true, kEpiPlain, false, true>(p, s)
                    : launch_tiled<128, 128, 2, 2, false, kEpiPlain, false, true>(p, s);
+    }
     default: return fail(MI355X_FP8_EINVAL, "unknown block-scaled form %d", form);
   }
 }

@@ -181,8 +181,15 @@ PyObject* gemm_blockwise(PyObject* const* a, Py_ssize_t count) {
     made = fresh({m, n}, at::kBFloat16, *xq);
   }
   void* stream = current_stream();
-  const bool ok = enqueue(mi355x_fp8_blockwise_gemm, xq->data_ptr(), wq->data_ptr(), f32(*xs), f32(*ws), out->data_ptr(), m, n, k,
-                                     xq->stride(0), wq->stride(0), out->stride(0), stream);
+  void* space = nullptr;
+  at::Tensor made_space;
+  const size_t space_bytes = mi355x_fp8_blockwise_workspace_bytes(m, n, k);
+  if (space_bytes) {
+    made_space = fresh({(int64_t)space_bytes}, at::kByte, *xq);
+    space = made_space.data_ptr();
+  }
+  const bool ok = enqueue(mi355x_fp8_blockwise_gemm_ws, xq->data_ptr(), wq->data_ptr(), f32(*xs), f32(*ws), out->data_ptr(), m, n, k,
+                          xq->stride(0), wq->stride(0), out->stride(0), space, space_bytes, -1, stream);
   if (!ok) return nullptr;
   if (a[4] == Py_None) return one(made);
   Py_INCREF(a[4]);

@@ -257,7 +257,7 @@ def fp8_gemm_blockwise(
     Same operands as the callables of tritonbench/operators/fp8_gemm_blockwise/operator.py:139-145:
     xq [M,K], wq [N,K] float8_e4m3fn; x_scale [ceil(M/128), ceil(K/128)] and w_scale
     [ceil(N/128), ceil(K/128)] float32 as fp8_block_quantize returns them (:86-118).
-    Only enqueues work on the current stream.
+    Only enqueues work on the current stream. Shapes whose plan cuts K take a workspace of their own (a torch.empty a call).
     """
     done = _lib.binding().gemm_blockwise(xq, wq, x_scale, w_scale, out)
     if done is not None:
@@ -286,9 +286,11 @@ def fp8_gemm_blockwise(
         _require_gpu(out, "out")
         if out.dtype != torch.bfloat16 or tuple(out.shape) != (m, n) or out.stride(1) != 1:
             raise ValueError("out must be bfloat16 [M,N] with unit column stride")
-    st = lib.mi355x_fp8_blockwise_gemm(
+    ws_bytes = lib.mi355x_fp8_blockwise_workspace_bytes(m, n, k)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=xq.device) if ws_bytes else None
+    st = lib.mi355x_fp8_blockwise_gemm_ws(
         xq.data_ptr(), wq.data_ptr(), x_scale.data_ptr(), w_scale.data_ptr(), out.data_ptr(),
-        m, n, k, xq.stride(0), wq.stride(0), out.stride(0), _stream_ptr(),
+        m, n, k, xq.stride(0), wq.stride(0), out.stride(0), ws.data_ptr() if ws is not None else None, ws_bytes, -1, _stream_ptr(),
     )
     _lib.check(st, "mi355x_fp8_blockwise_gemm")
     return out
