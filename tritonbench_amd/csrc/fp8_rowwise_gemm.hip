@@ -441,8 +441,11 @@ constexpr int tiled_waves_per_simd(int BM, int BN, int waves, bool blockscale, i
 // CLEAR: the grouped form that sets the rows of C past the last group's to zero. Instances of their own: with the test
 // and the loop in the others, which a call with a result of its own runs, those were 1-3 % slower (1704x1280x768 in 12 groups
 // 11.46 -> 11.76 us, 450x1024x576 6.47 -> 6.61).
+// OFF_LINES: a STREAM_B launch whose rows of B are off the 128-byte lines keeps the rotated walk but not the policy, with which the
+// line that two steps of a row share would come from memory twice: 119x55346x4112 73.9 -> 62.8 us, 32x57344x4112 68.5 -> 50.2,
+// 128x28672x8256 68.9 -> 63.7, 256x28672x8256 82.0 -> 78.9 (without the rotation 63.6, 51.0, 70.6 and 108).
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool KTAIL, int EPI, bool GROUPED = false, bool BLOCKSCALE = false,
-          int DIST = kDefaultDist, bool STREAM_B = false, bool CLEAR = false>
+          int DIST = kDefaultDist, bool STREAM_B = false, bool CLEAR = false, bool OFF_LINES = false>
 __global__ __launch_bounds__(WAVES_M* WAVES_N * 64)
 __attribute__((amdgpu_waves_per_eu(tiled_waves_per_simd(BM, BN, WAVES_M * WAVES_N, BLOCKSCALE, DIST),
                                    tiled_waves_per_simd(BM, BN, WAVES_M * WAVES_N, BLOCKSCALE, DIST))))
@@ -450,6 +453,7 @@ void gemm_tiled_kernel(GemmParams p) {
   constexpr int kStagesA = DIST, kStagesB = DIST + 1;
   static_assert(DIST >= 2 && tiled_lds_bytes(BM, BN, DIST) <= 160 * 1024, "the stage rings must fit the LDS");
   static_assert(!GROUPED || EPI == kEpiPlain, "the grouped form has neither bias nor split-K");
+  static_assert(!OFF_LINES || (STREAM_B && !GROUPED), "a variant of the streaming launches");
   static_assert(!CLEAR || GROUPED, "only the grouped form has rows past its groups'");
   static_assert(!BLOCKSCALE || (128 % (BM / WAVES_M) == 0 && 128 % (BN / WAVES_N) == 0 && EPI != kEpiBias && !GROUPED),
                 "a wave's tile must lie inside one 128x128 scale block: one factor per wave and step");
@@ -685,7 +689,7 @@ void gemm_tiled_kernel(GemmParams p) {
     const uint32_t lo = lane_part(b_lane, b_lane_tail, cb.kt);
 #pragma unroll
     for (int i = 0; i < B_GROUPS; ++i)
-      load_group(std::integral_constant<bool, STREAM_B>{}, b_src, lo, (uint32_t)cb.kt * kStepK + b_src.wave_off, i,
+      load_group(std::integral_constant<bool, STREAM_B && !OFF_LINES>{}, b_src, lo, (uint32_t)cb.kt * kStepK + b_src.wave_off, i,
                  lds + LDS_B0 + fill_b * STAGE_B);
     next_fill_b();
     ++cb.issued;
@@ -1206,7 +1210,7 @@ void gemm_tiled_kernel(GemmParams p) {
         MI355X_ALL_STEPS(std::false_type{})
       }
     } else {
-      MI355X_ALL_STEPS((std::integral_constant<bool, STREAM_B>{}))
+      MI355X_ALL_STEPS((std::integral_constant<bool, STREAM_B && !OFF_LINES>{}))
     }
 #undef MI355X_ALL_STEPS
     {
@@ -1536,6 +1540,9 @@ __device__ __forceinline__ void splitk_finalize(const GemmParams& p) {
   const int m0 = (int)row_group * ROWS;
   const int n = (int)(idx - row_group * quads_per_row) * 4;
   const size_t plane = (size_t)p.M * p.N;
+  // (the quad at the edge reads the row's last four values and moves its own down: read one by one, split after split, they took
+  // longer than all the others together, 2x707x25888 in sixteen parts 18.9 -> 20.0 us in all)
+  const int first = p.N >= 4 ? min(n, p.N - 4) : n, shift = n - first;
   const float* src[ROWS];
   float sa[ROWS], sb[4];
   uint16_t bias[4] = {0, 0, 0, 0};
@@ -1543,7 +1550,7 @@ __device__ __forceinline__ void splitk_finalize(const GemmParams& p) {
 #pragma unroll
   for (int i = 0; i < ROWS; ++i) {
     const int m = min(m0 + i, p.M - 1);  // (rows past the last one read it again)
-    src[i] = p.partial + (size_t)m * p.N + n;
+    src[i] = p.partial + (size_t)m * p.N + first;
     sa[i] = p.a_scale ? p.a_scale[m] : 1.0f;  // fetched beside the partial sums, not after them
     sum[i] = (v4f){0.f, 0.f, 0.f, 0.f};
   }
@@ -1552,7 +1559,7 @@ __device__ __forceinline__ void splitk_finalize(const GemmParams& p) {
   if (p.bias)
 #pragma unroll
     for (int e = 0; e < 4; ++e) bias[e] = p.bias[min(n + e, p.N - 1)];
-  if (n + 3 < p.N) {  // (a row of partials starts on any 4 bytes)
+  if (p.N >= 4) {  // (a row of partials starts on any 4 bytes)
     // added in split order, as the scalar form does
     auto add = [&](int s, auto count) {
       constexpr int COUNT = decltype(count)::value;
@@ -1573,6 +1580,11 @@ __device__ __forceinline__ void splitk_finalize(const GemmParams& p) {
     if (BATCH > 3 && rest == 3) add(s, std::integral_constant<int, 3>{});
     else if (BATCH > 2 && rest == 2) add(s, std::integral_constant<int, 2>{});
     else if (rest == 1) add(s, std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+      if (shift & 1) sum[i] = (v4f){sum[i][1], sum[i][2], sum[i][3], 0.f};
+      if (shift & 2) sum[i] = (v4f){sum[i][2], sum[i][3], 0.f, 0.f};
+    }
   } else {
     for (int s = 0; s < p.splits; ++s) {
 #pragma unroll
@@ -1906,7 +1918,7 @@ __device__ __forceinline__ RowBlock find_row_block(const GemmParams& p, int item
 // a group; the row blocks of one group's columns are neighbours on one XCD (workgroup ids go round the XCDs), so that
 // the group's rows of B come from HBM once. The grid covers the most row blocks that any sizes with these M and G can
 // give; the surplus comes last and returns at once.
-// OFF_LINES: the grouped form for rows of B that do not start on 128-byte lines: no streaming policy.
+// OFF_LINES: for rows of B that do not start on 128-byte lines: no streaming policy.
 template <int MT, int NTW, int DEPTH, int KW, bool ANY = false, bool BLOCK = false, bool GROUPED = false, bool OFF_LINES = false>
 __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
   static_assert((int)ANY + (int)BLOCK + (int)GROUPED <= 1, "at most one of them");
@@ -2026,7 +2038,8 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
         // B is read once and never again: stream it past the caches; A is shared by everyone. (ANY: an
         // unaligned piece shares its lines with the neighbouring steps, which the streaming policy would
         // fetch again: 1x8192x8191 19.6 -> 14.4 us without it, 16x8192x8191 25.6 -> 19.1. The same for rows that start
-        // off a line: 128 rows in 16 groups of 4096x4112 75 -> 60, 64 in 8 of 14336x4112 128 -> 101.)
+        // off a line: 128 rows in 16 groups of 4096x4112 75 -> 60, 64 in 8 of 14336x4112 128 -> 101, 1x12544x5968 17.4 -> 16.2,
+        // 54x3584x4288 9.0 -> 6.9.)
         if (t < NTW && !ANY && !OFF_LINES) dst[t][h] = __builtin_nontemporal_load((const Chunk*)(src[t][h] + kb));
         else dst[t][h] = *(const Chunk*)(src[t][h] + kb);
       }
@@ -2433,7 +2446,8 @@ __constant__ float kZeroFactor = 0.0f;
 // BLOCK: the block-scaled form. A wave's slab of a step is one K block; the slab's products are scaled by that
 // block's factor as they are added up. A tile's columns may straddle two column blocks of B: every group of 4
 // columns takes the factor of its own.
-template <int MB, int NB, bool BLOCK = false>
+// OFF_LINES: rows of B off the 128-byte lines, without the streaming policy.
+template <int MB, int NB, bool BLOCK = false, bool OFF_LINES = false>
 __global__ __launch_bounds__(512) void gemm_narrow_kernel(GemmParams p) {
   constexpr int BM = 32 * MB, BN = 32 * NB, KS = kNarrowKS;
   constexpr int DA = narrow_a_dist(MB, NB), DB = narrow_b_dist(MB, NB);
@@ -2681,7 +2695,7 @@ __global__ __launch_bounds__(512) void gemm_narrow_kernel(GemmParams p) {
       const uint32_t even = lane_part(b_even, chunk_even, koff), odd = lane_part(b_odd, chunk_even ^ 64u, koff);
 #pragma unroll
       for (int g = 0; g < LB; ++g)
-        load_chunk_to_lds<true>(rb, dst + g * 1024, (g & 1) ? odd : even, (uint32_t)(g * 8) * (uint32_t)p.ldb + koff);
+        load_chunk_to_lds<!OFF_LINES>(rb, dst + g * 1024, (g & 1) ? odd : even, (uint32_t)(g * 8) * (uint32_t)p.ldb + koff);
     };
 #pragma unroll
     for (int s = 0; s < DB; ++s) issue_b(s);
@@ -2728,7 +2742,8 @@ constexpr size_t pair_lds_bytes(int SPW) {
 // predicate per load; HAS_BIAS: a bias vector is added. Both are compile-time properties: this kernel's
 // time hangs on how fast a wave gets its burst of loads out, and the few vector instructions either adds
 // in front of the loads measured 0.3 and 0.1 us at M=16, N=K=8192.
-template <int SPW, bool VEC, bool KTAIL, bool HAS_BIAS>
+// OFF_LINES: rows of B off the 128-byte lines, without the streaming policy (16x8192x4112 12.2 -> 11.0 us, 16x4096x4112 7.1 -> 5.8).
+template <int SPW, bool VEC, bool KTAIL, bool HAS_BIAS, bool OFF_LINES = false>
 __global__ __launch_bounds__(kPersistWaves * 64) void gemm_skinny_pair_kernel(GemmParams p) {
   constexpr int WAVES = kPersistWaves;
   constexpr int STEPS = WAVES * SPW;
@@ -2792,7 +2807,7 @@ __global__ __launch_bounds__(kPersistWaves * 64) void gemm_skinny_pair_kernel(Ge
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
 #if defined(__HIP_DEVICE_COMPILE__)
-      land[t][i][h] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rb, (int)(ok ? b_lane[h] : kOutside), (int)so, 2));
+      land[t][i][h] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rb, (int)(ok ? b_lane[h] : kOutside), (int)so, OFF_LINES ? 0 : 2));
 #else
       land[t][i][h] = (v4i){0, 0, 0, 0};
 #endif
@@ -3901,7 +3916,7 @@ inline int store_policy(const GemmParams& p) {
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool KTAIL, int EPI, bool GROUPED = false, bool BLOCKSCALE = false,
-          int DIST = kDefaultDist, bool STREAM_B = false, bool CLEAR = false>
+          int DIST = kDefaultDist, bool STREAM_B = false, bool CLEAR = false, bool OFF_LINES = false>
 int launch_tiled(GemmParams p, hipStream_t stream) {
   p.store = store_policy(p);
   constexpr int threads = WAVES_M * WAVES_N * 64;
@@ -3915,7 +3930,7 @@ int launch_tiled(GemmParams p, hipStream_t stream) {
   if (total > (long)INT32_MAX) return fail(MI355X_FP8_ENOTSUP, "more than 2^31-1 work items");
   const long slots = (long)kNumCu * tiled_wgs_per_cu(BM, BN, DIST);
   long grid = total < slots ? ((total + kNumXcd - 1) / kNumXcd) * kNumXcd : slots;
-  constexpr auto kern = gemm_tiled_kernel<BM, BN, WAVES_M, WAVES_N, KTAIL, EPI, GROUPED, BLOCKSCALE, DIST, STREAM_B, CLEAR>;
+  constexpr auto kern = gemm_tiled_kernel<BM, BN, WAVES_M, WAVES_N, KTAIL, EPI, GROUPED, BLOCKSCALE, DIST, STREAM_B, CLEAR, OFF_LINES>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   if (const int st = ready_device()) return st;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), lds_bytes, stream, p);
@@ -3939,6 +3954,9 @@ int launch_tiled(GemmParams p, hipStream_t stream) {
   return MI355X_FP8_OK;
 }
 
+// whether rows of B start off the 128-byte lines
+inline bool off_lines(const GemmParams& p) { return ((reinterpret_cast<uintptr_t>(p.b) | (uintptr_t)p.ldb) & (kStepK - 1)) != 0; }
+
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool STREAM_B, bool DEEP = false>
 int launch_tiled_epilogue(const GemmParams& p, hipStream_t s) {
   // 256x128 tiles have the LDS for loads three steps ahead (3 A + 4 B stages = 160 KB): worth 6-10 % where
@@ -3946,6 +3964,15 @@ int launch_tiled_epilogue(const GemmParams& p, hipStream_t s) {
   // K=28672: 220 -> 199 us). The 64x256 tile measured 1-3 % slower that way and stays at two.
   constexpr int D = DEEP || (BM == 256 && BN == 128) ? 3 : kDefaultDist;
   const bool ktail = p.K % kStepK;
+  if constexpr (STREAM_B) {
+    // (mostly because K is no multiple of a step: the kernels for that take the others too. Tiles of 256 rows that are full, in
+    // several parts, whose walk is not rotated, keep the policy: 256x10580x10960 in three 65 us, without 69; 140x10240x10960 50 and 47)
+    if (off_lines(p) && !(BM == 256 && p.M > 192 && p.splits > 2)) {
+      if (p.splits > 1) return launch_tiled<BM, BN, WAVES_M, WAVES_N, true, kEpiPartial, false, false, D, true, false, true>(p, s);
+      return p.bias ? launch_tiled<BM, BN, WAVES_M, WAVES_N, true, kEpiBias, false, false, D, true, false, true>(p, s)
+                    : launch_tiled<BM, BN, WAVES_M, WAVES_N, true, kEpiPlain, false, false, D, true, false, true>(p, s);
+    }
+  }
   if (p.splits > 1)
     return ktail ? launch_tiled<BM, BN, WAVES_M, WAVES_N, true, kEpiPartial, false, false, D, STREAM_B>(p, s)
                  : launch_tiled<BM, BN, WAVES_M, WAVES_N, false, kEpiPartial, false, false, D, STREAM_B>(p, s);
@@ -3997,11 +4024,19 @@ MI355X_DEFINE_TILED_PART(6, 128, 128, 2, 2, false, true)  // (never with the str
 
 #if !defined(MI355X_TILED_PART)  // (everything from here on belongs to the main unit)
 namespace {
-template <int MT, int NTW, int DEPTH, int KW, bool ANY = false, bool BLOCK = false>
+template <int MT, int NTW, int DEPTH, int KW, bool ANY = false, bool BLOCK = false, bool OFF_LINES = false>
 int launch_skinny(const GemmParams& p, hipStream_t stream) {
+  if constexpr (!ANY && !OFF_LINES) {
+    // (up to four rows, up to two workgroups a CU and whole rounds of steps but for the tail, they keep the policy: 1x4096x1040 3.45
+    // us, without 3.64, 1x4096x2064 4.35 and 4.55, 4x8192x1040 4.33 and 4.42; 4x8192x1552 5.22 and 5.04, 1x16384x1040 6.98 and 6.57),
+    // and so do a few workgroups over long rows (2x707x25888 19.0, without 20.3)
+    const bool whole_rounds = p.M <= 4 && p.N <= 2 * kNumCu * 16 * NTW && p.K / kStepK % KW == 0;
+    const bool few_columns = p.N <= 1024 * NTW && p.K > 14336;
+    if (off_lines(p) && !whole_rounds && !few_columns) return launch_skinny<MT, NTW, DEPTH, KW, false, BLOCK, true>(p, stream);
+  }
   constexpr size_t lds_bytes = (size_t)KW * (NTW + MT) * 16 * kStepK;
   static_assert(lds_bytes <= 160 * 1024, "transpose buffers must fit the 160 KB LDS");
-  constexpr auto kern = gemm_skinny_kernel<MT, NTW, DEPTH, KW, ANY, BLOCK>;
+  constexpr auto kern = gemm_skinny_kernel<MT, NTW, DEPTH, KW, ANY, BLOCK, false, OFF_LINES>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   if (const int st = ready_device()) return st;
   const unsigned grid = (unsigned)((p.N + 16 * NTW - 1) / (16 * NTW));
@@ -4192,11 +4227,12 @@ struct BlockPlan {
 // 128x128 tiles with K cut into `splits` parts of `sps` steps: the times of block_small_cost_us over the work items, the second launch
 // and the parts' trip through memory; bound by the stream of B where the tiles are one or two rows (64x28672x8192 in two
 // 68 us, 128x57344x8192 142, where the streaming form takes 45 and 95 in one piece).
-inline float block_split_cost_us(int64_t M, int64_t N, int64_t K, int splits, int sps) {
+inline float block_split_cost_us(int64_t M, int64_t N, int64_t K, int64_t ldb, int splits, int sps) {
   const long items = ((M + 127) / 128) * ((N + 127) / 128) * splits, full = items / (2 * kNumCu), rest = items % (2 * kNumCu);
   float t = (float)full * ((float)sps + 5.0f);
   if (rest) t += (float)sps * (rest <= kNumCu ? 0.45f + 0.1f * (float)rest / (float)kNumCu : 1.0f) + 5.0f;
-  t = fmaxf(t, (float)(M + N) * (float)K / 4.4e6f);
+  // (off the lines: 17x37568x10000 in two 103 us, in one piece 94)
+  t = fmaxf(t, (ldb % kStepK ? 1.25f : 1.0f) * (float)(M + N) * (float)K / 4.4e6f);
   return t + 4.5f + 2.0f * (float)splits * (float)M * (float)N * 4.0f / 5.0e6f;
 }
 inline BlockPlan block_plan(int64_t M, int64_t N, int64_t K, int64_t ldb, int max_splits) {
@@ -4209,7 +4245,8 @@ inline BlockPlan block_plan(int64_t M, int64_t N, int64_t K, int64_t ldb, int ma
     if (splits != want || N * 512 > (int64_t)INT32_MAX) continue;
     // (up to 16 rows the streaming forms are quicker than their estimates on long rows off the lines: 3x1425x24896 17.2 us,
     // in fifteen parts 23.5, 4x523x22816 21.4 and 22.8)
-    const float us = block_split_cost_us(M, N, K, splits, sps) * (M <= 16 ? 1.5f : 1.0f);
+    // (and one row of tiles off the lines: 61x17792x10384 70 us, in two parts 80)
+    const float us = block_split_cost_us(M, N, K, ldb, splits, sps) * (M <= 16 ? 1.5f : M <= 128 && ldb % kStepK ? 1.25f : 1.0f);
     if (us < cost) {
       cost = us;
       best = {kBlockSmall, splits, sps};
@@ -4357,11 +4394,14 @@ int launch_skinny_persistent(const GemmParams& p, hipStream_t stream) {
   return MI355X_FP8_OK;
 }
 
-template <int SPW, bool VEC, bool KTAIL, bool HAS_BIAS>
+template <int SPW, bool VEC, bool KTAIL, bool HAS_BIAS, bool OFF_LINES = false>
 int launch_skinny_pair(const GemmParams& p, hipStream_t stream) {
+  if constexpr (KTAIL && !OFF_LINES) {  // (whole rounds of steps are off the lines with padded rows only)
+    if (off_lines(p)) return launch_skinny_pair<SPW, VEC, KTAIL, HAS_BIAS, true>(p, stream);
+  }
   constexpr size_t lds_bytes = pair_lds_bytes(SPW);
   static_assert(lds_bytes <= 160 * 1024, "A's steps, the transpose buffers and the partial results must fit the LDS");
-  constexpr auto kern = gemm_skinny_pair_kernel<SPW, VEC, KTAIL, HAS_BIAS>;
+  constexpr auto kern = gemm_skinny_pair_kernel<SPW, VEC, KTAIL, HAS_BIAS, OFF_LINES>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   if (const int st = ready_device()) return st;
   const long ntiles = p.N / 16;
@@ -4405,10 +4445,17 @@ int launch_skinny_persistent_steps(const GemmParams& p, hipStream_t s) {
   }
 }
 
-template <int MB, int NB, bool BLOCK>
+template <int MB, int NB, bool BLOCK, bool OFF_LINES = false>
 int launch_narrow(const GemmParams& p, hipStream_t stream) {
+  if constexpr (!OFF_LINES) {
+    // Rows off the lines: 128x8192x4112 17.3 -> 15.8 us without the streaming policy, 256x4096x4112 16.0 -> 12.1, 32x2048x12304
+    // 14.5 -> 10.8, 1x12544x5968 17.4 -> 16.2. Few rows of A, or tiles of up to 20 columns, over long rows keep it: 1x4256x10896
+    // 13.6, without 14.7, 8x4119x17424 20.7 and 22.0, 7x15184x7488 21.6 and 22.3; 32x2048x16448 17.7 and 18.5, 13x2608x22160 21.7 and 24.1.
+    const bool few_columns = p.M <= 32 * MB && narrow_tile_cols(p.N) <= 20;
+    if (off_lines(p) && !(p.M <= 8 && p.K > 7168) && !(few_columns && p.K > 14336)) return launch_narrow<MB, NB, BLOCK, true>(p, stream);
+  }
   constexpr size_t lds_bytes = narrow_lds_bytes(MB, NB);
-  constexpr auto kern = gemm_narrow_kernel<MB, NB, BLOCK>;
+  constexpr auto kern = gemm_narrow_kernel<MB, NB, BLOCK, OFF_LINES>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   if (const int st = ready_device()) return st;
   const unsigned row_blocks = (unsigned)((p.M + 32 * MB - 1) / (32 * MB));
