@@ -4485,6 +4485,34 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
 
 }  // namespace
 
+// What is chosen for a shape depends on its sizes alone and takes 0.7 to 1.5 us of the host to weigh up, two to four times a
+// call, where the whole call is about 4 us and a launch of a few rows 3 us on the GPU: it is the host that such calls wait for. Every
+// thread keeps the choices of the shapes it met last, one per entry of a table of fixed size: workspace_bytes + choice of
+// 1x2304x2048 1.9 us -> 0.02.
+template <typename Value>
+struct Choices {
+  static constexpr int kEntries = 128;
+  struct Entry {
+    int64_t m, n, k, how;  // (m = 0: empty)
+    Value value;
+  } entries[kEntries];
+  template <typename Weigh>
+  const Value& get(int64_t m, int64_t n, int64_t k, int64_t how, Weigh weigh) {
+    const uint64_t h = ((uint64_t)m * 0x9E3779B97F4A7C15u ^ (uint64_t)n) * 0xC2B2AE3D27D4EB4Fu + (uint64_t)k * 0x165667B19E3779F9u + (uint64_t)how;
+    Entry& e = entries[(h * 0x9E3779B97F4A7C15u) >> 57];
+    if (e.m != m || e.n != n || e.k != k || e.how != how) e = {m, n, k, how, weigh()};
+    return e.value;
+  }
+};
+static_assert(Choices<int>::kEntries == 1 << (64 - 57), "the hash's top bits index the table");
+thread_local Choices<TiledPlan> known_plans;
+thread_local Choices<int> known_families;
+
+inline TiledPlan known_plan(int64_t M, int64_t N, int64_t K, int variant, int max_splits) {
+  variant &= ~0xff;  // (the plan does not depend on the family's number)
+  return known_plans.get(M, N, K, (int64_t)variant << 8 | max_splits, [&] { return plan_from_variant(M, N, K, variant, max_splits); });
+}
+
 extern "C" {
 
 int mi355x_fp8_rowwise_abi_version(void) { return MI355X_FP8_ABI_VERSION; }
@@ -4497,17 +4525,19 @@ int mi355x_fp8_rowwise_select_variant(int64_t M, int64_t N, int64_t K) {
   const int st = check_shape(M, N, K);
   if (st != MI355X_FP8_OK) return st;
   if (K % 16 != 0) return MI355X_FP8_VARIANT_GENERIC;
-  // M <= 64: the streaming kernel, unless a tiled plan (64- or 128-row tiles that stream B, split
-  // K where the tiles are few) is expected to beat it: from two 16-row blocks of A up on most
-  // shapes, with one block on the longest weight panels. Up to 8 rows the streaming kernel was
-  // behind on one kind of shape only, few columns with very long rows, where a handful of workgroups
-  // each stream a long tile and split tiles put the whole chip to work (8 x 1024 x 28672: 16.2 us
-  // against 14.5); there a tiled plan has to be expected ahead by a tenth to be taken.
-  // (above 64 rows the family's only member is the narrow-tile kernel in row blocks, where it fits)
   if (M > kSkinnyMaxM && !narrow_fits(M, N, K)) return MI355X_FP8_VARIANT_TILED;
-  const float margin = M <= 8 ? 0.9f : 1.0f;
-  return plan_tiled(M, N, K, -1, 0, kMaxSplits).cost_us < margin * skinny_cost_us(M, N, K) ? MI355X_FP8_VARIANT_TILED
-                                                                                          : MI355X_FP8_VARIANT_SKINNY;
+  return known_families.get(M, N, K, 0, [&] {
+    // M <= 64: the streaming kernel, unless a tiled plan (64- or 128-row tiles that stream B, split
+    // K where the tiles are few) is expected to beat it: from two 16-row blocks of A up on most
+    // shapes, with one block on the longest weight panels. Up to 8 rows the streaming kernel was
+    // behind on one kind of shape only, few columns with very long rows, where a handful of workgroups
+    // each stream a long tile and split tiles put the whole chip to work (8 x 1024 x 28672: 16.2 us
+    // against 14.5); there a tiled plan has to be expected ahead by a tenth to be taken.
+    // (above 64 rows the family's only member is the narrow-tile kernel in row blocks, where it fits)
+    const float margin = M <= 8 ? 0.9f : 1.0f;
+    return known_plan(M, N, K, MI355X_FP8_VARIANT_AUTO, kMaxSplits).cost_us < margin * skinny_cost_us(M, N, K) ? MI355X_FP8_VARIANT_TILED
+                                                                                                              : MI355X_FP8_VARIANT_SKINNY;
+  });
 }
 
 size_t mi355x_fp8_rowwise_workspace_bytes(int64_t M, int64_t N, int64_t K, int variant) {
@@ -4516,7 +4546,7 @@ size_t mi355x_fp8_rowwise_workspace_bytes(int64_t M, int64_t N, int64_t K, int v
     variant = (variant & ~0xff) | mi355x_fp8_rowwise_select_variant(M, N, K);
   // (the skinny kernels reduce on chip, the generic kernel does not split)
   if ((variant & 0xff) != MI355X_FP8_VARIANT_TILED || K % 16 != 0) return 0;
-  const TiledPlan plan = plan_from_variant(M, N, K, variant, kMaxSplits);
+  const TiledPlan plan = known_plan(M, N, K, variant, kMaxSplits);
   return plan.splits > 1 ? (size_t)plan.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
@@ -4585,10 +4615,10 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
     variant = mi355x_fp8_rowwise_select_variant(M, N, K);
     if (variant == MI355X_FP8_VARIANT_TILED && (M <= kSkinnyMaxM || narrow_fits(M, N, K))) {
       // the choice assumed the plan's workspace; without it the plan changes and may lose
-      const TiledPlan plan = plan_from_variant(M, N, K, plan_bits, kMaxSplits);
+      const TiledPlan plan = known_plan(M, N, K, plan_bits, kMaxSplits);
       const size_t need = plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0;
       if (need && (!workspace || workspace_bytes < need) &&
-          plan_from_variant(M, N, K, plan_bits, 1).cost_us >= skinny_cost_us(M, N, K))
+          known_plan(M, N, K, plan_bits, 1).cost_us >= skinny_cost_us(M, N, K))
         variant = MI355X_FP8_VARIANT_SKINNY;
     }
   }
@@ -4614,7 +4644,7 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
       {
         // A caller that brought no (or too little) workspace gets the best plan that needs none,
         // unless it asked for a split factor by name.
-        TiledPlan plan = plan_from_variant(M, N, K, plan_bits, kMaxSplits);
+        TiledPlan plan = known_plan(M, N, K, plan_bits, kMaxSplits);
         const size_t need = plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0;
         if (need && (!workspace || workspace_bytes < need)) {
           if ((plan_bits >> 16) & 0xff)
@@ -4623,10 +4653,10 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
           // the cheapest plan whose partial planes fit what the caller brought (none: the unsplit plans)
           const size_t plane = (size_t)M * (size_t)N * sizeof(float);
           const size_t fit = workspace ? workspace_bytes / plane : 0;
-          plan = plan_from_variant(M, N, K, plan_bits, fit < 1 ? 1 : fit > (size_t)kMaxSplits ? kMaxSplits : (int)fit);
+          plan = known_plan(M, N, K, plan_bits, fit < 1 ? 1 : fit > (size_t)kMaxSplits ? kMaxSplits : (int)fit);
         }
         // (the partial sums of a tile are addressed with 32-bit byte offsets that must stay below 2^31)
-        if (plan.splits > 1 && N * 512 > (int64_t)INT32_MAX) plan = plan_from_variant(M, N, K, plan_bits & 0xff00, 1);
+        if (plan.splits > 1 && N * 512 > (int64_t)INT32_MAX) plan = known_plan(M, N, K, plan_bits & 0xff00, 1);
         if (plan.splits > 1 && (reinterpret_cast<uintptr_t>(workspace) & 15))
           return fail(MI355X_FP8_EINVAL, "workspace must be 16-byte aligned");
         p.splits = plan.splits;
