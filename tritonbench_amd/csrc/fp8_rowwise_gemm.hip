@@ -1699,7 +1699,9 @@ __device__ __forceinline__ v8h e4m3fn_to_f16x8(int lo, int hi) {
 // counts are then exact and DEPTH steps stay in flight).
 constexpr size_t any_lds_bytes(int BM, int BN) { return (size_t)2 * (BM + BN) * kStepK; }
 
-template <int BM, int BN, int DEPTH>
+// PARTIAL: K in p.splits parts of p.steps_per_split steps, each an item of its own that leaves its sums in its plane of p.partial
+// for the second pass. The last part has the partial step.
+template <int BM, int BN, int DEPTH, bool PARTIAL>
 __global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
   constexpr int WTM = BM / 2, WTN = BN / 2, MT = WTM / 32, NT = WTN / 32;
   constexpr int STAGE = (BM + BN) * kStepK;  // A's rows, then B's
@@ -1712,10 +1714,13 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
   const int wm = wave >> 1, wn = wave & 1, l32 = lane & 31, half = lane >> 5;
 
   // each XCD takes a contiguous run of the tile list (kGroupM tile rows at a time, column-major inside)
-  const TileWalk walk = make_walk(p.tiles_m * p.tiles_n);
+  const int tiles = p.tiles_m * p.tiles_n;
+  const TileWalk walk = make_walk(PARTIAL ? tiles * p.splits : tiles);
   if (walk.slot >= walk.chunk_len) return;
+  const int item = walk.chunk_begin + walk.slot;
+  const int part = PARTIAL ? fast_div(item, p.div_tiles_mul, p.div_tiles_shift) : 0;
   int tm, tn;
-  tile_coords(walk.chunk_begin + walk.slot, p.tiles_m, p.tiles_n, p.div_group_mul, p.div_group_shift, tm, tn);
+  tile_coords(item - part * tiles, p.tiles_m, p.tiles_n, p.div_group_mul, p.div_group_shift, tm, tn);
   const long m0 = (long)tm * BM, n0 = (long)tn * BN;
 
   // lane's chunk ld_c of rows ld_row, ld_row + 32, ... (rows past an edge repeat the last one)
@@ -1769,20 +1774,24 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
     }
   };
 
-  const int full = p.K / kStepK;
+  // whole steps of this item from step `first` on, and whether the partial one is its own
+  const int whole = p.K / kStepK;
+  const int first = PARTIAL ? part * p.steps_per_split : 0;
+  const int full = PARTIAL ? min(p.steps_per_split, whole - first) : whole;
+  const bool has_tail = whole * kStepK < p.K && (!PARTIAL || part == p.splits - 1);
   v4i land[DEPTH][LOADS];
   auto fetch = [&](v4i (&to)[LOADS], int s) {  // past the last whole step: that one again, for nobody
-    const int k = min(s, full - 1) * kStepK + ld_c * kChunk;
+    const int k = (first + min(s, full - 1)) * kStepK + ld_c * kChunk;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) to[i] = *(const v4i_any*)(row[i] + k);
   };
   if (full > 0)
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d) fetch(land[d], d);
-  if (full * kStepK < p.K) {
+  if (has_tail) {
     v4i tail[LOADS];
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) tail[i] = load16_any(row[i], full * kStepK + ld_c * kChunk, p.K);
+    for (int i = 0; i < LOADS; ++i) tail[i] = load16_any(row[i], whole * kStepK + ld_c * kChunk, p.K);
     park(tail, 1);
     join();
     multiply(1);
@@ -1807,6 +1816,29 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
       if (s + d < full) step(d, s + d);
   }
 
+  if constexpr (PARTIAL) {
+    float* plane = p.partial + (size_t)part * p.M * p.N;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const long m = m0 + wm * WTM + i * 32 + l32;
+      if (m >= p.M) continue;
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const long n = n0 + wn * WTN + j * 32 + 8 * q + 4 * half;
+          float* dst = plane + (size_t)m * p.N + n;
+          if (n + 3 < p.N) {
+            *(v4f_by4*)dst = (v4f){acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+          } else {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+              if (n + e < p.N) dst[e] = acc[i][j][4 * q + e];
+          }
+        }
+    }
+    return;
+  }
   // lane (l32, half): row l32 of every 32x32 block, columns 8q + 4*half + 0..3, as one 8-byte store wherever it lies
   // (1795x84399x13, rows of C that start at any 2 bytes: 553 us with a store per element)
 #pragma unroll
@@ -3915,6 +3947,22 @@ inline int store_policy(const GemmParams& p) {
   return ((base | pitch) & 63) != 0 && (int64_t)p.M * p.N * 2 > kLargeResult ? kStoreKeep : kStoreStream;
 }
 
+// The second pass of a launch whose items left partial sums.
+int launch_finalize(GemmParams p, hipStream_t stream) {
+  // Four rows a thread where one row each would be more workgroups than the chip holds at once (8 of 256 lanes on a
+  // CU): fewer of them to start, more loads in flight each. Below that they would leave CUs idle.
+  const long quads_per_row = ((long)p.N + 3) / 4;
+  const bool many = (quads_per_row * p.M + 255) / 256 > 8L * kNumCu;
+  const long quads = quads_per_row * (many ? ((long)p.M + kFinalizeRows - 1) / kFinalizeRows : p.M);
+  p.div_group_mul = p.div_group_shift = 0;
+  if (quads <= (long)INT32_MAX - 255) make_fast_div((uint32_t)quads_per_row, p.div_group_mul, p.div_group_shift);
+  hipLaunchKernelGGL(many ? splitk_finalize_rows_kernel : splitk_finalize_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0,
+                     stream, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "split-K finalize launch: %s", hipGetErrorString(e));
+  return MI355X_FP8_OK;
+}
+
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool KTAIL, int EPI, bool GROUPED = false, bool BLOCKSCALE = false,
           int DIST = kDefaultDist, bool STREAM_B = false, bool CLEAR = false, bool OFF_LINES = false>
 int launch_tiled(GemmParams p, hipStream_t stream) {
@@ -3934,22 +3982,11 @@ int launch_tiled(GemmParams p, hipStream_t stream) {
   (void)LdsLimit<kern, lds_bytes>::registered;
   if (const int st = ready_device()) return st;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), lds_bytes, stream, p);
-  hipError_t e = hipGetLastError();
+  const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "tiled kernel launch: %s", hipGetErrorString(e));
   if (EPI == kEpiPartial) {
-    // Four rows a thread where one row each would be more workgroups than the chip holds at once (8 of 256 lanes on a
-    // CU): fewer of them to start, more loads in flight each. Below that they would leave CUs idle.
-    const long quads_per_row = ((long)p.N + 3) / 4;
-    const bool many = (quads_per_row * p.M + 255) / 256 > 8L * kNumCu;
-    const long quads = quads_per_row * (many ? ((long)p.M + kFinalizeRows - 1) / kFinalizeRows : p.M);
-    GemmParams f = p;
-    if (BLOCKSCALE) f.a_scale = f.b_scale = nullptr;  // (the factors were applied block by block)
-    f.div_group_mul = f.div_group_shift = 0;
-    if (quads <= (long)INT32_MAX - 255) make_fast_div((uint32_t)quads_per_row, f.div_group_mul, f.div_group_shift);
-    hipLaunchKernelGGL(many ? splitk_finalize_rows_kernel : splitk_finalize_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0,
-                       stream, f);
-    e = hipGetLastError();
-    if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "split-K finalize launch: %s", hipGetErrorString(e));
+    if (BLOCKSCALE) p.a_scale = p.b_scale = nullptr;  // (the factors were applied block by block)
+    return launch_finalize(p, stream);
   }
   return MI355X_FP8_OK;
 }
@@ -4274,22 +4311,23 @@ int launch_block_form(GemmParams p, hipStream_t stream) {
 }
 int launch_block(const GemmParams& p, hipStream_t s) { return p.K % kStepK ? launch_block_form<true>(p, s) : launch_block_form<false>(p, s); }
 
-template <int BM, int BN, int DEPTH>
+template <int BM, int BN, int DEPTH, bool PARTIAL = false>
 int launch_any(GemmParams p, hipStream_t stream) {
   constexpr size_t lds_bytes = any_lds_bytes(BM, BN);
-  constexpr auto kern = gemm_any_kernel<BM, BN, DEPTH>;
+  constexpr auto kern = gemm_any_kernel<BM, BN, DEPTH, PARTIAL>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
-  const long tiles = (long)p.tiles_m * p.tiles_n;
-  if (tiles > (long)INT32_MAX - kNumXcd || (long)kGroupM * p.tiles_n > (long)INT32_MAX)
+  const long items = (long)p.tiles_m * p.tiles_n * p.splits;
+  if (items > (long)INT32_MAX - kNumXcd || (long)kGroupM * p.tiles_n > (long)INT32_MAX)
     return fail(MI355X_FP8_ENOTSUP, "more than 2^31-1 tiles");
+  make_fast_div((uint32_t)p.tiles_m * (uint32_t)p.tiles_n, p.div_tiles_mul, p.div_tiles_shift);
   make_fast_div((uint32_t)kGroupM * (uint32_t)p.tiles_n, p.div_group_mul, p.div_group_shift);
   if (const int st = ready_device()) return st;
-  hipLaunchKernelGGL(kern, dim3((unsigned)((tiles + kNumXcd - 1) / kNumXcd * kNumXcd)), dim3(256), lds_bytes, stream, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((items + kNumXcd - 1) / kNumXcd * kNumXcd)), dim3(256), lds_bytes, stream, p);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "generic kernel launch: %s", hipGetErrorString(e));
-  return MI355X_FP8_OK;
+  return PARTIAL ? launch_finalize(p, stream) : MI355X_FP8_OK;
 }
 
 // Up to 64 rows: whether the streaming kernel's unaligned form runs. Its workgroups, one for 16 columns (32 from 33 rows on),
@@ -4302,25 +4340,55 @@ constexpr bool generic_streams(int64_t M, int64_t N, int64_t K) {
   return !(K <= (M <= 16 ? 128 : 256) && N > (M <= 32 ? 8192 : 4096));
 }
 static_assert(!generic_streams(1, 1 << 27, 1024) && generic_streams(1, (1 << 27) - 16, 1024), "2^27 columns are 2^32 lanes");
+// Where the tiles are few and K is long, K is cut into parts (128x64 tiles, up to one item a CU): a CU takes in what it can have
+// outstanding, 0.45 us for a step of 64x64 tiles whatever the depth, so a launch is as quick as it has CUs at work. 128x64 tiles
+// take 0.74 us a step for twice the products.
+struct GenericPlan {
+  int splits, steps_per_split;
+};
+inline GenericPlan generic_plan(int64_t M, int64_t N, int64_t K, int max_splits) {
+  const int k_steps = k_steps_of(K);
+  GenericPlan best = {1, k_steps};
+  const int64_t tiles_64 = ((M + 63) / 64) * ((N + 63) / 64), tiles = ((M + 127) / 128) * ((N + 63) / 64);
+  if (generic_streams(M, N, K) || tiles_64 >= kNumCu) return best;
+  float cost = 0.92f * ((float)k_steps * (0.45f + 0.17f * (float)tiles_64 / (float)kNumCu) + 4.0f);
+  for (int want = 2; want <= max_splits && tiles * want <= kNumCu; ++want) {
+    int splits, sps;
+    normalise_splits(k_steps, want, splits, sps);
+    if (splits != want) continue;
+    const float us = (float)sps * 0.74f + 7.0f + 2.0f * (float)splits * (float)M * (float)N * 4.0f / 5.0e6f;
+    if (us < cost) {
+      cost = us;
+      best = {splits, sps};
+    }
+  }
+  return best;
+}
+
 // The generic family: the streaming kernel's unaligned form up to 64 rows but for short rows on wide panels (measured cold: 1x8192x8191 14.4 us,
 // 16x8192x8191 19.1, 64x8192x8191 29.7, where 64x64 tiles take 33), tiles beyond. 128x128 tiles from two
-// rounds of the CUs on (4096x8192x8191 563 us = 977 TFLOP/s); below, 64x64 tiles. With at most one of
+// rounds of the CUs on where K is long enough to pay for their start (2048x4096x4100 78 us, with 128x64 88), 128x64 tiles from
+// somewhat more than one round of those on (against 64x64 or 128x128 before: 7953x1212x847 45.7 -> 38.2 us, 4406x768x6428
+// 74 -> 64, 65x30000x1001 22.6 -> 19.1, 3000x5000x700 44.8 -> 44.0); below, 64x64 tiles (517x3000x1041 13.8 us with 423 of them, 15.7
+// with 235 of 128x64). With at most one of
 // those per CU nothing but its own loads covers a step's latency, and they run two steps ahead
 // (128x8192x8191 61.7 -> 36.7 us, 256x4096x4097 27.9 -> 19.6); with more, the CU's other workgroups do, and
 // the second step's registers would cost one of them (517x3000x1041 13.9 -> 12.7, 1024x2048x1025 13.7 -> 12.5).
 int launch_generic(const GemmParams& p, hipStream_t s) {
   // (the documented range of the family, which the tests' sizes lie in)
   if (p.M > 65535 * 64) return fail(MI355X_FP8_ENOTSUP, "the generic family takes M <= %d", 65535 * 64);
+  if (p.splits > 1) return launch_any<128, 64, 2, true>(p, s);
   if (generic_streams(p.M, p.N, p.K)) {
     if (p.M <= 16) return launch_skinny<1, 1, 4, 8, true>(p, s);
     if (p.M <= 32) return launch_skinny<2, 1, 2, 8, true>(p, s);
     return launch_skinny<4, 2, 2, 8, true>(p, s);
   }
-  auto tiles = [&](long edge) { return ((p.M + edge - 1) / edge) * ((p.N + edge - 1) / edge); };
-  // (one step, or one row of tiles: nothing to gain from the larger tile, 164x39275x3 21.6 us with it, 14.0 with 64x64)
-  if ((tiles(128) >= 2 * kNumCu && p.M > kSkinnyMaxM && p.K > kStepK) || !grid_fits(tiles(64), 256))
-    return launch_any<128, 128, 1>(p, s);
-  return tiles(64) <= kNumCu ? launch_any<64, 64, 2>(p, s) : launch_any<64, 64, 1>(p, s);
+  auto tiles = [&](long bm, long bn) { return ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn); };
+  // (one step, or one row of tiles: nothing to gain from the larger tiles, 164x39275x3 21.6 us with 128x128, 14.0 with 64x64)
+  const bool larger = p.M > kSkinnyMaxM && p.K > kStepK;
+  if ((larger && p.K > 2048 && tiles(128, 128) >= 2 * kNumCu) || !grid_fits(tiles(128, 64), 256)) return launch_any<128, 128, 1>(p, s);
+  if ((larger && tiles(128, 64) >= kNumCu + kNumCu / 4) || !grid_fits(tiles(64, 64), 256)) return launch_any<128, 64, 1>(p, s);
+  return tiles(64, 64) <= kNumCu ? launch_any<64, 64, 2>(p, s) : launch_any<64, 64, 1>(p, s);
 }
 
 // ---- built-in scratch of the entry point that allocates nothing
@@ -4544,7 +4612,11 @@ size_t mi355x_fp8_rowwise_workspace_bytes(int64_t M, int64_t N, int64_t K, int v
   if (check_shape(M, N, K) != MI355X_FP8_OK) return 0;
   if ((variant & 0xff) == MI355X_FP8_VARIANT_AUTO)
     variant = (variant & ~0xff) | mi355x_fp8_rowwise_select_variant(M, N, K);
-  // (the skinny kernels reduce on chip, the generic kernel does not split)
+  if ((variant & 0xff) == MI355X_FP8_VARIANT_GENERIC) {
+    const int splits = generic_plan(M, N, K, kMaxSplits).splits;
+    return splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
+  }
+  // (the skinny kernels reduce on chip)
   if ((variant & 0xff) != MI355X_FP8_VARIANT_TILED || K % 16 != 0) return 0;
   const TiledPlan plan = known_plan(M, N, K, variant, kMaxSplits);
   return plan.splits > 1 ? (size_t)plan.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
@@ -4710,7 +4782,15 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
       if (M <= 48) return launch_skinny<3, 1, 2, 8>(p, s);
       return launch_skinny<4, 2, 2, 8>(p, s);  // 32 rows of B per workgroup: A passes L1 half as often
     case MI355X_FP8_VARIANT_GENERIC:
-      return launch_generic(p, s);
+      {
+        // (as many parts as the workspace holds planes; in one piece without one)
+        const size_t planes = workspace && !(reinterpret_cast<uintptr_t>(workspace) & 15) ? workspace_bytes / ((size_t)M * (size_t)N * sizeof(float)) : 0;
+        const GenericPlan plan = generic_plan(M, N, K, planes < 1 ? 1 : planes > (size_t)kMaxSplits ? kMaxSplits : (int)planes);
+        p.splits = plan.splits;
+        p.steps_per_split = plan.steps_per_split;
+        p.partial = plan.splits > 1 ? (float*)workspace : nullptr;
+        return launch_generic(p, s);
+      }
     default:
       return fail(MI355X_FP8_EINVAL, "unknown variant %d", variant);
   }
