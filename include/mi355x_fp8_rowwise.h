@@ -121,8 +121,8 @@ const char* mi355x_fp8_rowwise_last_error(void);
  * of 16), or a negative status when the shape is not supported. Lets tests pin the dispatch. */
 int mi355x_fp8_rowwise_select_variant(int64_t M, int64_t N, int64_t K);
 
-/* Bytes of device workspace `variant` needs for this shape (0 when none). Pure host
- * arithmetic: callable without a device. */
+/* Bytes of device workspace `variant` needs for this shape (0 when none): the fp32 partial sums of the TILED and GENERIC plans that
+ * cut K. Pure host arithmetic: callable without a device. */
 size_t mi355x_fp8_rowwise_workspace_bytes(int64_t M, int64_t N, int64_t K, int variant);
 
 /*
