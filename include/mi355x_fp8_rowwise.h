@@ -309,6 +309,10 @@ int mi355x_fp8_blockwise_gemm_ex(const void* a, const void* b,
  * mi355x_fp8_blockwise_workspace_bytes names for the shape (0: it would not). A smaller one takes the best plan that fits it.
  * With form = TILES_128 + 256 * s the factor is pinned to s (EINVAL without the workspace for it). What is in the workspace
  * before a call does not matter; two calls that may overlap need one each.
+ *
+ * Factors: the streaming forms and the parts of a cut K take any (each block's products are added with a_scale * b_scale, an f32
+ * product, as it is). The forms of tiles in one piece carry a tile's sum in units of the current block's factor: there the factors along
+ * a row of blocks, but for zeros, have to lie within 2^60 of one another, and not below 2^-60 beside a zero.
  */
 size_t mi355x_fp8_blockwise_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int mi355x_fp8_blockwise_gemm_ws(const void* a, const void* b,

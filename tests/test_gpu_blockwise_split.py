@@ -86,6 +86,42 @@ def test_the_wrapper_cuts_k_and_may_be_captured(gpu_device, m, n, k):
         _within_bounds(got, xq, wq, xs, ws, 16)
 
 
+# Shapes of up to 256 rows that the streaming forms run without a workspace, in parts with one. Those take every factor as it is, and
+# so do the parts: blocks of zeros in both operands (whose factors a quantiser makes very small) among large ones, a factor
+# of zero beside codes that are none and small factors, neighbours up to 2^120 apart, factors of either sign.
+@pytest.mark.parametrize("m,n,k", [(32, 1024, 28672), (92, 515, 26368), (33, 1100, 28656)])
+@pytest.mark.parametrize("factors", ["zero blocks", "zero factors", "far apart", "signs"])
+def test_parts_take_any_factors(gpu_device, m, n, k, factors):
+    print(f"case {m}x{n}x{k} {factors}", flush=True)
+    xq, wq, xs, ws = _inputs(m, n, k, gpu_device, seed=1)
+    gk = xs.shape[1]
+    if factors == "zero blocks":
+        xs *= 2.0**20
+        ws *= 2.0**20
+        for kb in (1, 5, 6, 40, gk - 1):
+            xq[:, kb * 128 : (kb + 1) * 128] = 0
+            wq[:, kb * 128 : (kb + 1) * 128] = 0
+            xs[:, kb] = 1e-12 / 448
+            ws[:, kb] = 1e-12 / 448
+    elif factors == "zero factors":
+        xs *= 2.0**-40
+        ws *= 2.0**-40
+        for kb in (0, 7, 30, 31, gk - 1):
+            xs[:, kb] = 0.0
+    elif factors == "far apart":
+        xs[:, ::2] *= 2.0**60
+        xs[:, 1::2] *= 2.0**-60
+    else:
+        xs *= torch.where(torch.rand(xs.shape, device=gpu_device) < 0.5, -1.0, 1.0)
+        ws *= torch.where(torch.rand(ws.shape, device=gpu_device) < 0.5, -1.0, 1.0)
+    parts = _lib.load().mi355x_fp8_blockwise_workspace_bytes(m, n, k) // (4 * m * n)
+    assert parts >= 2
+    _within_bounds(ops.fp8_gemm_blockwise(xq, wq, xs, ws), xq, wq, xs, ws, parts)
+    streaming = torch.zeros((m, n), dtype=torch.bfloat16, device=gpu_device)
+    _lib.check(_call(xq, wq, xs, ws, streaming, None, _lib.BLOCK_ONE_TILE if m <= 64 else _lib.BLOCK_NARROW), "gemm_ws")
+    _within_bounds(streaming, xq, wq, xs, ws, 1)
+
+
 def test_factors_without_their_workspace_are_refused(gpu_device):
     xq, wq, xs, ws = _inputs(128, 128, 1024, gpu_device)
     out = torch.zeros((128, 128), dtype=torch.bfloat16, device=gpu_device)

@@ -364,6 +364,14 @@ __device__ __forceinline__ void store_columns(uint8_t* dst, v4i out, int valid) 
   }
 }
 
+// A factor f of a block-scaled product in two parts: f = factor_mantissa(f) * 2^(e - 127), e being the biased exponent that the
+// matrix instruction takes as the scale of an operand. Exact; between 2^-23 and 2 in magnitude but for an infinity or NaN, which
+// stays one, and for zero, which counts as one with both operands scaled by 2^-126 (a product of codes is below 2^25: nothing is left).
+__device__ __forceinline__ int factor_exponent(float f) { return min(max((__float_as_int(f) >> 23) & 0xff, 1), 254); }
+__device__ __forceinline__ float factor_mantissa(float f) { return f == 0.0f ? 1.0f : ldexpf(f, 127 - factor_exponent(f)); }
+// the scales of the two operands, a byte each
+__device__ __forceinline__ int factor_scales(float f) { return factor_exponent(f) | (f == 0.0f ? 1 : 127) << 8; }
+
 // Waits until at most VM of this wave's global loads and none of its LDS operations are
 // outstanding, then joins the workgroup barrier. Written with the s_waitcnt builtin (not
 // inline asm) so the compiler's own wait-count bookkeeping knows the LDS queue is empty
@@ -746,29 +754,54 @@ void gemm_tiled_kernel(GemmParams p) {
   // set: the kernel keeps the register budget of the plain 128x128 tile (two workgroups per CU).
   // A factor of exactly zero is replaced by 2^-60 (its block then contributes P_k * 2^-60, nothing
   // at the output's precision); factors are expected to span less than 2^60 within a row of blocks.
+  // ANY_FACTORS: the parts of a split launch, which runs shapes whose form without a workspace adds every block's products with the
+  // factor as it is, and so takes any. There the accumulators are in units of the factor's mantissa, and the matrix
+  // instructions take its exponent as a scale: the same products and ratios times powers of two, hence the same bits where
+  // the other units do not overflow (and 1.6e-3 of the result's norm off float64 either way, nearly all of it the rounding to bf16; the
+  // f32 sums 1.5e-5, what the matrix instruction itself leaves). It costs nothing: a part's steps are half of all at most, and
+  // with two registers to look them up in instead of four 1047x1566x12800 in two parts takes 39.6 us, in units of the factors 41.9,
+  // 32x1024x28672 18.5 and 19.2.
   // Blocks 0 .. n-2 are rescaled in phase [B] of the step before (each under the cover of the next
   // block's MFMA), the last one under the first MFMA of the step itself.
   // s_pend / s_cur: the ratios to the next step / to this one; kt_c: the K step the compute side is
   // at; the lane's share of the item's factors and ratios (sc[r], rt[r] belong to step 64*r + lane).
   float s_pend = 1.0f, s_cur = 1.0f, s_last = 1.0f, n_pend = 1.0f, n_last = 1.0f;
   int kt_c = 0;
-  constexpr int SC_REGS = 4;  // 256 steps = K up to 32768
-  float sc[SC_REGS] = {0.f, 0.f, 0.f, 0.f}, rt[SC_REGS] = {1.f, 1.f, 1.f, 1.f};
-  auto load_block_scales = [&](const TileLoc& loc) {
+  constexpr bool ANY_FACTORS = BLOCKSCALE && EPI == kEpiPartial;
+  int scales = 0, n_scales = 0;  // ANY_FACTORS: of this step's operands, and of the next one's
+  auto unit = [](float f) { return ANY_FACTORS ? factor_mantissa(f) : f; };  // what the accumulators are in units of
+  constexpr int SC_REGS = ANY_FACTORS ? 2 : 4;  // 256 steps = K up to 32768; a part has half of them at most, and its first one is lane 0's
+  float sc[SC_REGS] = {}, rt[SC_REGS] = {};
+  auto load_block_scales = [&](const TileLoc& loc, int first) {
     // the scale block of this wave's tile (clamped for waves that lie past the matrix edge)
     const int mb = min(loc.m0 + wm * WTM, p.M - 1) / 128, nb = min(loc.n0 + wn * WTN, p.N - 1) / 128;
     const float* sa = p.a_scale + (size_t)mb * k_steps;
     const float* sb = p.b_scale + (size_t)nb * k_steps;
     auto factor = [&](int kb) -> float {
       const float f = sa[kb] * sb[kb];
-      return f == 0.0f ? 0x1p-60f : f;
+      return f == 0.0f && !ANY_FACTORS ? 0x1p-60f : f;
     };
+    float before[SC_REGS];  // ANY_FACTORS: the factor of the step before
 #pragma unroll
     for (int r = 0; r < SC_REGS; ++r) {
-      const int kb = min(r * 64 + lane, k_steps - 1);
+      const int kb = min(first + r * 64 + lane, k_steps - 1);
       sc[r] = factor(kb);
       if (STREAM_B) rt[r] = factor(kb > 0 ? kb - 1 : k_steps - 1) / sc[r];  // (a rotated walk passes from the last step to the first)
+      else if (ANY_FACTORS) before[r] = factor(max(kb - 1, 0));
       else rt[r] = kb > 0 ? factor(kb - 1) / sc[r] : 1.0f;
+    }
+    if constexpr (ANY_FACTORS) {
+      bool normal = true;
+#pragma unroll
+      for (int r = 0; r < SC_REGS; ++r) {
+        auto bits = [](float f) { return __int_as_float((__float_as_int(f) & 0x807fffff) | 0x3f800000); };
+        rt[r] = bits(before[r]) / bits(sc[r]);
+        normal = normal && __builtin_isnormal(before[r]) && __builtin_isnormal(sc[r]);
+      }
+      if (!__all(normal)) {  // (zeros, subnormal products, infinities, NaN)
+#pragma unroll
+        for (int r = 0; r < SC_REGS; ++r) rt[r] = unit(before[r]) / unit(sc[r]);
+      }
     }
   };
   // (kt at most k_steps past the end. A walk that wraps around finds the first steps there; what lies past the end of one that
@@ -776,9 +809,9 @@ void gemm_tiled_kernel(GemmParams p) {
   // 404x3104x464 7.44 -> 7.20.)
   auto lane_value = [&](const float (&regs)[SC_REGS], int kt) -> float {
     if (STREAM_B) kt = kt >= k_steps ? kt - k_steps : kt;
-    else kt = min(kt, k_steps - 1);
+    else kt = min(kt, ANY_FACTORS ? 64 * SC_REGS - 1 : k_steps - 1);
     const int r = kt >> 6;
-    const float v = r == 0 ? regs[0] : r == 1 ? regs[1] : r == 2 ? regs[2] : regs[3];
+    const float v = r == 0 ? regs[0] : r == 1 || SC_REGS == 2 ? regs[1] : r == 2 ? regs[SC_REGS - 2] : regs[SC_REGS - 1];
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), kt & 63));
   };
   // brings block t of the accumulators from one step's factor to the next one's
@@ -793,7 +826,10 @@ void gemm_tiled_kernel(GemmParams p) {
   auto mfma_one = [&](const Frag (&fa)[MT], const Frag (&fb)[NT], int t, bool fresh) {
     const int i = t / NT, j = t % NT;
     const v16f zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(as_v8(fb[j]), as_v8(fa[i]), fresh ? zero : acc[i][j], 0, 0, 0, 0, 0, 0);
+    if constexpr (ANY_FACTORS)
+      acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(as_v8(fb[j]), as_v8(fa[i]), fresh ? zero : acc[i][j], 0, 0, 0, scales, 1, scales);
+    else
+      acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(as_v8(fb[j]), as_v8(fa[i]), fresh ? zero : acc[i][j], 0, 0, 0, 0, 0, 0);
   };
   // u-th of the 2*(MT+NT) LDS reads that fill fragment set (fa, fb) with K half s
   auto read_one = [&](Frag (&fa)[MT], Frag (&fb)[NT], const uint8_t* rows_a, const uint8_t* rows_b, int s, int u) {
@@ -1013,6 +1049,7 @@ void gemm_tiled_kernel(GemmParams p) {
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_e));
     const int l32 = lane_e & 31, half = lane_e >> 5;
     float* base = p.partial + (size_t)split * p.M * p.N;
+    const float last_unit = unit(s_last);
     const uint32_t row_bytes = (uint32_t)p.N * 4u;  // (N*4*128 < 2^31 by the host's check of the workspace plan)
     const int rows = __builtin_amdgcn_readfirstlane(min(max(p.M - (m0 + wm * WTM), 0), WTM));  // (scalar: see the epilogue)
     float* const tile = base + ((size_t)(m0 + wm * WTM) * p.N + n0 + wn * WTN);
@@ -1027,7 +1064,7 @@ void gemm_tiled_kernel(GemmParams p) {
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
           v4f v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-          if (BLOCKSCALE) v = v * s_last;  // (back from the units of the last step's factor)
+          if (BLOCKSCALE) v = v * last_unit;  // (back from the units of the last step's factor)
           store_f32x4_checked(v, rsrc, lo, (uint32_t)(i * 32) * row_bytes + (uint32_t)(j * 32 + 8 * q) * 4u);
         }
       }
@@ -1047,7 +1084,7 @@ void gemm_tiled_kernel(GemmParams p) {
                 float* dst = tile + ((size_t)(i * 32 + l32) * p.N + n);
 #pragma unroll
                 for (int e = 0; e < 3; ++e)
-                  if (n + e < n_left) dst[e] = BLOCKSCALE ? acc[i][j][4 * q + e] * s_last : acc[i][j][4 * q + e];
+                  if (n + e < n_left) dst[e] = BLOCKSCALE ? acc[i][j][4 * q + e] * last_unit : acc[i][j][4 * q + e];
               }
             }
           }
@@ -1101,6 +1138,7 @@ void gemm_tiled_kernel(GemmParams p) {
       s_cur = s_pend;    // ratio that brought the accumulators to this step
       s_pend = n_pend;   // ratio to the next step (applied in phase [B])
       s_last = n_last;   // this step's factor: what the epilogue multiplies by after the last step
+      if (ANY_FACTORS) scales = n_scales;
     }
 
     // [A] MFMAs on x* (first K half of this step). Behind them, one per MFMA: the LDS reads
@@ -1129,6 +1167,7 @@ void gemm_tiled_kernel(GemmParams p) {
       if (BLOCKSCALE && t == PREP_T) {
         n_pend = lane_value(rt, STREAM_B && k_steps == 1 ? 0 : kt_c + 2);
         n_last = lane_value(sc, kt_c + 1);
+        if (ANY_FACTORS) n_scales = factor_scales(n_last);
       }
       if (t == PREP_T2) {
         sa = (sa + 1 == kStagesA) ? 0 : sa + 1;
@@ -1185,10 +1224,11 @@ void gemm_tiled_kernel(GemmParams p) {
     const int n_steps = split_end(c_split) - split_begin(c_split);
     if (BLOCKSCALE) {
       const TileLoc loc = locate(walk_c, c_item);
-      load_block_scales(loc);
-      kt_c = first_step(loc, split_begin(c_split), n_steps);
+      load_block_scales(loc, ANY_FACTORS ? split_begin(c_split) : 0);
+      kt_c = ANY_FACTORS ? 0 : first_step(loc, split_begin(c_split), n_steps);
       n_pend = lane_value(rt, kt_c + 1);
       n_last = lane_value(sc, kt_c);
+      if (ANY_FACTORS) n_scales = factor_scales(n_last);
     }
     // step k loads for step k + DIST and then moves the cursors to step k + DIST + 1, which is still this item's for
     // k < n_steps - DIST - 1. (Text and not a function: as a lambda around `step` it cost every grouped launch 1-2 %, 282x1536x1024
