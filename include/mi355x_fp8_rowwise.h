@@ -122,7 +122,9 @@ const char* mi355x_fp8_rowwise_last_error(void);
 int mi355x_fp8_rowwise_select_variant(int64_t M, int64_t N, int64_t K);
 
 /* Bytes of device workspace `variant` needs for this shape (0 when none): the fp32 partial sums of the TILED and GENERIC plans that
- * cut K. Pure host arithmetic: callable without a device. */
+ * cut K. Pure host arithmetic: callable without a device. It knows the sizes only: for AUTO with K a multiple of 16 the answer is that
+ * of the family for operands which meet the alignment requirements. Others run in the GENERIC family, in as many parts as that
+ * many bytes hold for it, or in one piece; ask for VARIANT_GENERIC by name to bring it the workspace of its own plan. */
 size_t mi355x_fp8_rowwise_workspace_bytes(int64_t M, int64_t N, int64_t K, int variant);
 
 /*
@@ -140,6 +142,8 @@ size_t mi355x_fp8_rowwise_workspace_bytes(int64_t M, int64_t N, int64_t K, int v
  * ENOTSUP otherwise. AUTO sends operands that miss any of that to the GENERIC family, which
  * takes every K, leading dimension and alignment (M <= 4194240).
  * `workspace` (16-byte aligned) may be NULL when mi355x_fp8_rowwise_workspace_bytes() is 0.
+ * Calls of the TILED and of the GENERIC family write to it; two calls that may overlap need one each.
+ * (The GENERIC family leaves a workspace that is not 16-byte aligned alone and runs in one piece.)
  * A call whose variant leaves the split-K factor to the library and brings less workspace
  * than that runs the best plan that needs none (same results up to fp32 summation order);
  * a call that names a split factor > 1 without enough workspace fails with EINVAL.
@@ -203,8 +207,8 @@ int mi355x_fp8_rowwise_gemm_stamped(const void* a, const void* b,
  * cheapest plan whose partial sums fit (as the workspace form does with a workspace that is too
  * small); only a call that names a split-K factor the buffer cannot hold is refused with
  * MI355X_FP8_ENOTSUP (use the workspace form for it). All calls on one GPU
- * share that GPU's buffer: calls that may overlap there (different streams, concurrently
- * replayed graphs) race on it and must be ordered by the caller. The buffer's address is looked
+ * share that GPU's buffer (of the GENERIC family too, whose plans for few tiles and long K use it): calls that may overlap
+ * there (different streams, concurrently replayed graphs) race on it and must be ordered by the caller. The buffer's address is looked
  * up by mi355x_fp8_rowwise_init() (or by the first call on a device that was not initialised:
  * make that call outside graph capture).
  */

@@ -134,6 +134,28 @@ def test_no_alloc_entry_runs_a_smaller_plan_when_the_automatic_one_does_not_fit(
     torch.testing.assert_close(got, full, rtol=1e-2, atol=1e-2)
 
 
+# The generic family by the automatic choice: K no multiple of 16 (cut into as many parts as the size query names), and operands off
+# 16 bytes or with an odd pitch on shapes whose size query, which does not see them, names another family's planes or none
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,shift,pitch", [(300, 704, 5001, 0, 0), (123, 512, 9729, 0, 0), (300, 704, 5008, 1, 0), (300, 704, 5008, 0, 3),
+                                               (128, 512, 8192, 1, 0), (246, 1568, 25168, 1, 0)])
+def test_no_alloc_entry_matches_the_workspace_entry_in_the_generic_family(gpu_device, m, n, k, shift, pitch):
+    lib = _lib.load()
+    g = torch.Generator(device=gpu_device).manual_seed(m + n + k)
+    canvas = torch.randn((m * (k + pitch) + shift,), generator=g, device=gpu_device).to(torch.float8_e4m3fn)
+    xq = canvas[shift:].view(m, k + pitch)[:, :k]
+    wq = torch.randn((n, k), generator=g, device=gpu_device).to(torch.float8_e4m3fn)
+    xs, ws = (torch.rand(r, generator=g, device=gpu_device) + 0.5 for r in (m, n))
+    print(f"case {m}x{n}x{k} shift {shift} pitch {pitch}", flush=True)
+    want, got = (torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device) for _ in range(2))
+    _with_workspace(lib, xq, wq, xs, ws, None, want, _lib.VARIANT_AUTO)
+    _no_alloc(lib, xq, wq, xs, ws, None, got, _lib.VARIANT_AUTO)
+    torch.cuda.synchronize()
+    assert np.array_equal(_bits(got), _bits(want))
+    exact = (xq.double() @ wq.double().t()) * xs.double()[:, None] * ws.double()[None, :]
+    assert ((got.double() - exact).norm() / exact.norm()).item() < 2.0**-8  # (one rounding to bf16)
+
+
 def test_no_alloc_entry_refuses_plans_beyond_its_buffer():
     """Host arithmetic only: a split factor the caller named and the buffer cannot hold is turned
     away before any device call."""

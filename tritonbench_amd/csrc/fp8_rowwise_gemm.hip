@@ -4908,8 +4908,11 @@ int mi355x_fp8_rowwise_gemm_noalloc(const void* a, const void* b, const float* a
   }
   // Nothing in the buffer has to start at zero: every split stores its whole plane of partial sums
   // before the finalize kernel (stream-ordered behind it) reads any of it.
+  // As many bytes as the workspace form would bring, though the buffer holds more: operands that send the call to another family than
+  // the shape alone would (misaligned ones, to the generic family, which cuts K into as many parts as it gets planes) have to
+  // find the same plan through both entries.
   return mi355x_fp8_rowwise_gemm_ex(a, b, a_scale, b_scale, bias, c, MI355X_FP8_OUT_BF16, M, N, K, lda, ldb, ldc,
-                                    ws, need ? kScratchBytes : 0, variant, stream);
+                                    ws, need < kScratchBytes ? need : kScratchBytes, variant, stream);
 }
 
 int mi355x_fp8_rowwise_grouped_gemm(const void* a, const void* b, const float* a_scale, const float* b_scale,
