@@ -5011,7 +5011,8 @@ size_t mi355x_fp8_blockwise_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 int mi355x_fp8_blockwise_gemm_ex(const void* a, const void* b, const float* a_scale, const float* b_scale,
                                  void* c, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                                  int64_t ldc, int form, void* stream) {
-  return mi355x_fp8_blockwise_gemm_ws(a, b, a_scale, b_scale, c, M, N, K, lda, ldb, ldc, nullptr, 0, form, stream);
+  // (a form with a factor beside it is the entry's below: here it is none, refused where the others' operands have passed)
+  return mi355x_fp8_blockwise_gemm_ws(a, b, a_scale, b_scale, c, M, N, K, lda, ldb, ldc, nullptr, 0, form > 0xff ? 0xff : form, stream);
 }
 
 int mi355x_fp8_blockwise_gemm_ws(const void* a, const void* b, const float* a_scale, const float* b_scale,
