@@ -40,3 +40,26 @@ def test_answers_do_not_depend_on_the_calls_before():
     for t in threads:
         t.join()
     assert results == [True] * 4
+
+
+def _in_a_thread_of_its_own(question):
+    """The answer of an empty table."""
+    answer = []
+    t = threading.Thread(target=lambda: answer.append(question()))
+    t.start()
+    t.join()
+    return answer[0]
+
+
+def test_block_plans_do_not_depend_on_the_calls_before():
+    lib = _lib.load()
+    rng = random.Random(7)
+    shapes = [(rng.choice((1, 16, 40, 64, 100, 300, 1000)), rng.choice((512, 1000, 2304)) + 16 * rng.randrange(4), 16 * rng.randrange(32, 1800))
+              for _ in range(300)]
+    alone = [_in_a_thread_of_its_own(lambda: lib.mi355x_fp8_blockwise_workspace_bytes(*s)) for s in shapes]
+    assert 50 < sum(a > 0 for a in alone) < 250
+    for _ in range(3):
+        order = list(range(len(shapes)))
+        rng.shuffle(order)
+        for i in order:
+            assert lib.mi355x_fp8_blockwise_workspace_bytes(*shapes[i]) == alone[i], shapes[i]

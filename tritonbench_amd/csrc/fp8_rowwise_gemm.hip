@@ -4222,13 +4222,13 @@ inline GroupedForm grouped_form(int64_t G, int64_t M, int64_t N, int64_t K, int6
 // N = 64149 56 -> 68 us, K = 2640, 23 rows, N = 58574 43 -> 49), and on short rows (N = 65536, 64 rows: K = 128 6.7 -> 8.2, 512
 // 11.2 -> 12.9; 128 rows, K = 1024: 21.4 -> 22.1) against all but the largest panels (one row, K = 768: N = 65536 15.0 -> 13.3,
 // N = 40064 11.35 -> 11.8; 128 rows, N = 100096, K = 768 31.7 -> 29.2). From K = 2048 on it is never behind.
-inline bool block_streams(int64_t M, int64_t N, int64_t K, int64_t ldb) {
+inline bool block_streams(int64_t M, int64_t N, int64_t K, bool off_lines) {
   const int64_t large = (int64_t)(M <= 48 ? 36 : M <= 64 ? 48 : 72) << 20;
-  return M <= 128 && N >= 192 * 128 && ldb % kStepK == 0 && (K >= 2048 || N * K >= large);
+  return M <= 128 && N >= 192 * 128 && !off_lines && (K >= 2048 || N * K >= large);
 }
-inline float block_small_cost_us(int64_t M, int64_t N, int64_t K, int64_t ldb) {
+inline float block_small_cost_us(int64_t M, int64_t N, int64_t K, bool off_lines) {
   const float steps = (float)k_steps_of(K);
-  if (block_streams(M, N, K, ldb)) return fmaxf(5.0f + (float)N * (float)K * (1.0f + (float)M / 400.0f) / 6.4e6f, 6.0f + 0.62f * steps);
+  if (block_streams(M, N, K, off_lines)) return fmaxf(5.0f + (float)N * (float)K * (1.0f + (float)M / 400.0f) / 6.4e6f, 6.0f + 0.62f * steps);
   const long tiles = ((M + 127) / 128) * ((N + 127) / 128), full = tiles / (2 * kNumCu), rest = tiles % (2 * kNumCu);
   // (one tile row: its steps wait for HBM, 16x8192x8192 40 us, 16x13312x13312 67)
   const float alone = M <= 128 ? 0.58f : 0.45f + 0.1f * (float)rest / (float)kNumCu;
@@ -4268,9 +4268,9 @@ inline float block_one_tile_cost_us(int64_t M, int64_t N, int64_t K, float off_l
   const float per_wg = (M <= 16 ? 2.4e-3f : M <= 32 ? 2.8e-3f : M <= 48 ? 4.1e-3f : 10.0e-3f) + 0.2e-3f * steps;
   return fmaxf(off_lines * one_tile_cost_us(M, N, K), 3.0f + (wgs > kNumCu ? (float)(wgs - kNumCu) * per_wg : 0.0f));
 }
-inline BlockForm block_form(int64_t M, int64_t N, int64_t K, int64_t ldb, float* cost_us = nullptr) {
-  BlockForm best = block_streams(M, N, K, ldb) ? kBlockSmallStream : kBlockSmall;
-  float cost = block_small_cost_us(M, N, K, ldb);
+inline BlockForm block_form(int64_t M, int64_t N, int64_t K, bool off_lines, float* cost_us = nullptr) {
+  BlockForm best = block_streams(M, N, K, off_lines) ? kBlockSmallStream : kBlockSmall;
+  float cost = block_small_cost_us(M, N, K, off_lines);
   auto weigh = [&](BlockForm form, float us) {
     if (us < cost) {
       best = form;
@@ -4283,7 +4283,7 @@ inline BlockForm block_form(int64_t M, int64_t N, int64_t K, int64_t ldb, float*
   // 1.31 / 1.28 with 313, 1.19 / 1.39 / 1.47 / 1.38 with 457; one 16-row tile a workgroup, K = 2064 and 8240, 1.16 and 1.25
   // with one row of A, 1.24 and 1.53 with 16; narrow tiles 1.1 whatever the sizes.
   float one_tile_off = 1.0f, narrow_off = 1.0f;
-  if (ldb % kStepK != 0 && M <= 128 && N > 64 * kNumCu) {
+  if (off_lines && M <= 128 && N > 64 * kNumCu) {
     const long rest = (N + 127) / 128 % (2 * kNumCu);
     const float share = rest > kNumCu ? fminf(fmaxf((float)(K - 128) / 1400.0f, 0.0f), 1.0f) : K >= 1536 ? 1.0f : 0.1f;
     cost *= 1.0f + share * (0.1f + (float)rest / 1300.0f);
@@ -4306,18 +4306,18 @@ struct BlockPlan {
 // 128x128 tiles with K cut into `splits` parts of `sps` steps: the times of block_small_cost_us over the work items, the second launch
 // and the parts' trip through memory; bound by the stream of B where the tiles are one or two rows (64x28672x8192 in two
 // 68 us, 128x57344x8192 142, where the streaming form takes 45 and 95 in one piece).
-inline float block_split_cost_us(int64_t M, int64_t N, int64_t K, int64_t ldb, int splits, int sps) {
+inline float block_split_cost_us(int64_t M, int64_t N, int64_t K, bool off_lines, int splits, int sps) {
   const long items = ((M + 127) / 128) * ((N + 127) / 128) * splits, full = items / (2 * kNumCu), rest = items % (2 * kNumCu);
   float t = (float)full * ((float)sps + 5.0f);
   if (rest) t += (float)sps * (rest <= kNumCu ? 0.45f + 0.1f * (float)rest / (float)kNumCu : 1.0f) + 5.0f;
   // (off the lines: 17x37568x10000 in two 103 us, in one piece 94)
-  t = fmaxf(t, (ldb % kStepK ? 1.25f : 1.0f) * (float)(M + N) * (float)K / 4.4e6f);
+  t = fmaxf(t, (off_lines ? 1.25f : 1.0f) * (float)(M + N) * (float)K / 4.4e6f);
   return t + 4.5f + 2.0f * (float)splits * (float)M * (float)N * 4.0f / 5.0e6f;
 }
-inline BlockPlan block_plan(int64_t M, int64_t N, int64_t K, int64_t ldb, int max_splits) {
+inline BlockPlan block_plan(int64_t M, int64_t N, int64_t K, bool off_lines, int max_splits) {
   const int k_steps = k_steps_of(K);
   float cost = 0.0f;
-  BlockPlan best = {block_form(M, N, K, ldb, &cost), 1, k_steps};
+  BlockPlan best = {block_form(M, N, K, off_lines, &cost), 1, k_steps};
   for (int want = 2; want <= max_splits; ++want) {
     int splits, sps;
     normalise_splits(k_steps, want, splits, sps);
@@ -4325,7 +4325,7 @@ inline BlockPlan block_plan(int64_t M, int64_t N, int64_t K, int64_t ldb, int ma
     // (up to 16 rows the streaming forms are quicker than their estimates on long rows off the lines: 3x1425x24896 17.2 us,
     // in fifteen parts 23.5, 4x523x22816 21.4 and 22.8)
     // (and one row of tiles off the lines: 61x17792x10384 70 us, in two parts 80)
-    const float us = block_split_cost_us(M, N, K, ldb, splits, sps) * (M <= 16 ? 1.5f : M <= 128 && ldb % kStepK ? 1.25f : 1.0f);
+    const float us = block_split_cost_us(M, N, K, off_lines, splits, sps) * (M <= 16 ? 1.5f : M <= 128 && off_lines ? 1.25f : 1.0f);
     if (us < cost) {
       cost = us;
       best = {kBlockSmall, splits, sps};
@@ -4617,10 +4617,17 @@ struct Choices {
 static_assert(Choices<int>::kEntries == 1 << (64 - 57), "the hash's top bits index the table");
 thread_local Choices<TiledPlan> known_plans;
 thread_local Choices<int> known_families;
+thread_local Choices<BlockPlan> known_block_plans;
 
 inline TiledPlan known_plan(int64_t M, int64_t N, int64_t K, int variant, int max_splits) {
   variant &= ~0xff;  // (the plan does not depend on the family's number)
   return known_plans.get(M, N, K, (int64_t)variant << 8 | max_splits, [&] { return plan_from_variant(M, N, K, variant, max_splits); });
+}
+
+// (the size query and the call behind it ask for the same entry: 0.2 us for both without it, 0.04 with it, on a call of 4)
+inline BlockPlan known_block_plan(int64_t M, int64_t N, int64_t K, int64_t ldb, int max_splits) {
+  const bool off_lines = ldb % kStepK != 0;  // (all that the plan depends on of ldb)
+  return known_block_plans.get(M, N, K, (int64_t)off_lines << 8 | max_splits, [&] { return block_plan(M, N, K, off_lines, max_splits); });
 }
 
 extern "C" {
@@ -4993,7 +5000,7 @@ int mi355x_fp8_blockwise_form(int64_t M, int64_t N, int64_t K) {
   if (st == MI355X_FP8_OK) st = check_fast_shape(K);
   if (st == MI355X_FP8_OK && K > 256 * kStepK)
     st = fail(MI355X_FP8_ENOTSUP, "block-scaled form handles K <= %d (got %lld)", 256 * kStepK, (long long)K);
-  return st != MI355X_FP8_OK ? st : block_form(M, N, K, K);
+  return st != MI355X_FP8_OK ? st : block_form(M, N, K, K % kStepK != 0);
 }
 
 int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale, const float* b_scale,
@@ -5004,7 +5011,7 @@ int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale
 
 size_t mi355x_fp8_blockwise_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   if (check_shape(M, N, K) != MI355X_FP8_OK || check_fast_shape(K) != MI355X_FP8_OK || K > 256 * kStepK) return 0;
-  const BlockPlan plan = block_plan(M, N, K, K, kMaxSplits);
+  const BlockPlan plan = known_block_plan(M, N, K, K, kMaxSplits);
   return plan.splits > 1 ? (size_t)plan.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
@@ -5054,7 +5061,8 @@ int mi355x_fp8_blockwise_gemm_ws(const void* a, const void* b, const float* a_sc
   if (form < 0 || want_splits) {
     // (a workspace that holds fewer planes than the best plan wants takes the best one that it does hold)
     const size_t planes = workspace ? workspace_bytes / plane : 0;
-    BlockPlan plan = block_plan(M, N, K, ldb, planes < 2 ? 1 : planes > (size_t)kMaxSplits ? kMaxSplits : (int)planes);
+    BlockPlan plan = known_block_plan(M, N, K, ldb, kMaxSplits);
+    if (plan.splits > 1 && (size_t)plan.splits > planes) plan = known_block_plan(M, N, K, ldb, planes < 2 ? 1 : (int)planes);
     if (want_splits) {
       plan.form = kBlockSmall;
       normalise_splits(p.steps_per_split, want_splits, plan.splits, plan.steps_per_split);
