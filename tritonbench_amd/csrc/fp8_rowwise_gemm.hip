@@ -4044,9 +4044,9 @@ int launch_tiled_epilogue(const GemmParams& p, hipStream_t s) {
   constexpr int D = DEEP || (BM == 256 && BN == 128) ? 3 : kDefaultDist;
   const bool ktail = p.K % kStepK;
   if constexpr (STREAM_B) {
-    // (mostly because K is no multiple of a step: the kernels for that take the others too. Tiles of 256 rows that are full, in
-    // several parts, whose walk is not rotated, keep the policy: 256x10580x10960 in three 65 us, without 69; 140x10240x10960 50 and 47)
-    if (off_lines(p) && !(BM == 256 && p.M > 192 && p.splits > 2)) {
+    // (mostly because K is no multiple of a step: the kernels for that take the others too. 120 shapes of 33 to 256 rows: 1.035 times as
+    // fast on average without the policy, 220x12704x17520 100 -> 88 us; at worst 210x8143x24896 78 -> 84)
+    if (off_lines(p)) {
       if (p.splits > 1) return launch_tiled<BM, BN, WAVES_M, WAVES_N, true, kEpiPartial, false, false, D, true, false, true>(p, s);
       return p.bias ? launch_tiled<BM, BN, WAVES_M, WAVES_N, true, kEpiBias, false, false, D, true, false, true>(p, s)
                     : launch_tiled<BM, BN, WAVES_M, WAVES_N, true, kEpiPlain, false, false, D, true, false, true>(p, s);
@@ -4106,12 +4106,11 @@ namespace {
 template <int MT, int NTW, int DEPTH, int KW, bool ANY = false, bool BLOCK = false, bool OFF_LINES = false>
 int launch_skinny(const GemmParams& p, hipStream_t stream) {
   if constexpr (!ANY && !OFF_LINES) {
-    // (up to four rows, up to two workgroups a CU and whole rounds of steps but for the tail, they keep the policy: 1x4096x1040 3.45
-    // us, without 3.64, 1x4096x2064 4.35 and 4.55, 4x8192x1040 4.33 and 4.42; 4x8192x1552 5.22 and 5.04, 1x16384x1040 6.98 and 6.57),
-    // and so do a few workgroups over long rows (2x707x25888 19.0, without 20.3)
-    const bool whole_rounds = p.M <= 4 && p.N <= 2 * kNumCu * 16 * NTW && p.K / kStepK % KW == 0;
-    const bool few_columns = p.N <= 1024 * NTW && p.K > 14336;
-    if (off_lines(p) && !whole_rounds && !few_columns) return launch_skinny<MT, NTW, DEPTH, KW, false, BLOCK, true>(p, stream);
+    // With one step a wave the steps that share lines ask for them at the same time, and the policy stays: 8x714x800 2.96 us, without 3.24,
+    // 2x597x912 2.97 and 3.25, from 2048 columns on within 4 % either way. From the second step on a wave comes back for lines
+    // that went with the policy: 2x1021x3952 5.83 us, without 5.24, 1x6723x8272 14.9 and 13.9, 2x17533x10800 44.6 and 38.7, 3x945x20144
+    // block-scaled 16.1 and 15.0; below 2048 bytes within 0.2 us either way (24x557x1104 3.63 and 3.82, 16x8192x1552 without 0.1 ahead).
+    if (off_lines(p) && k_steps_of(p.K) > KW) return launch_skinny<MT, NTW, DEPTH, KW, false, BLOCK, true>(p, stream);
   }
   constexpr size_t lds_bytes = (size_t)KW * (NTW + MT) * 16 * kStepK;
   static_assert(lds_bytes <= 160 * 1024, "transpose buffers must fit the 160 KB LDS");
@@ -4558,11 +4557,13 @@ int launch_skinny_persistent_steps(const GemmParams& p, hipStream_t s) {
 template <int MB, int NB, bool BLOCK, bool OFF_LINES = false>
 int launch_narrow(const GemmParams& p, hipStream_t stream) {
   if constexpr (!OFF_LINES) {
-    // Rows off the lines: 128x8192x4112 17.3 -> 15.8 us without the streaming policy, 256x4096x4112 16.0 -> 12.1, 32x2048x12304
-    // 14.5 -> 10.8, 1x12544x5968 17.4 -> 16.2. Few rows of A, or tiles of up to 20 columns, over long rows keep it: 1x4256x10896
-    // 13.6, without 14.7, 8x4119x17424 20.7 and 22.0, 7x15184x7488 21.6 and 22.3; 32x2048x16448 17.7 and 18.5, 13x2608x22160 21.7 and 24.1.
-    const bool few_columns = p.M <= 32 * MB && narrow_tile_cols(p.N) <= 20;
-    if (off_lines(p) && !(p.M <= 8 && p.K > 7168) && !(few_columns && p.K > 14336)) return launch_narrow<MB, NB, BLOCK, true>(p, stream);
+    // Rows off the lines: without the streaming policy the wider tiles' launches are quicker (128x8192x4112 17.3 -> 15.8 us,
+    // 256x4096x4112 16.0 -> 12.1, 1x19687x15024 67.4 -> 60.2, 8x5233x12976 18.3 -> 16.5, 24x10179x19168 block-scaled 44.0 -> 40.0). With all rows
+    // in one block and few columns a tile there is so little to fetch that a step's trip is what it takes, and the next step finds the
+    // shared line on its way: 8x714x800 3.52, without 3.78, 2x2177x27472 block-scaled 25.6 and 29.0, 9x2881x21200 21.2 and 24.4,
+    // 7x3468x23088 23.5 and 27.0; row-wise it ends a little earlier, 16x3421x7824 10.9 and 10.3, 16x4274x8176 block-scaled 12.7 and 12.1.
+    const int few_columns = p.M > 32 ? 0 : p.M <= (BLOCK ? 16 : 8) ? (BLOCK ? 20 : 16) : 8;
+    if (off_lines(p) && narrow_tile_cols(p.N) > few_columns) return launch_narrow<MB, NB, BLOCK, true>(p, stream);
   }
   constexpr size_t lds_bytes = narrow_lds_bytes(MB, NB);
   constexpr auto kern = gemm_narrow_kernel<MB, NB, BLOCK, OFF_LINES>;
