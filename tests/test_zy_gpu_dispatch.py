@@ -104,7 +104,8 @@ def _time_us(call, sets, burst_us=4000.0):
 # streaming forms are behind the plain 128x128 tiles
 @pytest.mark.parametrize("m,n,k", [(1, 2304, 2048), (16, 8192, 8192), (32, 8192, 8192), (64, 57344, 8192), (128, 8192, 8192),
                                    (512, 4096, 4096), (4096, 4096, 4096), (44, 87564, 32), (49, 18200, 64), (128, 100096, 256),
-                                   (128, 40064, 512), (64, 65536, 128), (9, 64149, 3952), (16, 58376, 4112), (1, 58376, 6688)])
+                                   (128, 40064, 512), (64, 65536, 128), (9, 64149, 3952), (16, 58376, 4112), (1, 58376, 6688),
+                                   (2, 63172, 4128), (1, 24904, 1424), (64, 19696, 11024)])
 def test_block_scaled_choice_is_close_to_the_best_form(gpu_device, m, n, k):
     lib = _lib.load()
     g = torch.Generator(device=gpu_device).manual_seed(m + n + k)

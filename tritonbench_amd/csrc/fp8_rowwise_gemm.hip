@@ -4277,17 +4277,26 @@ inline BlockForm block_form(int64_t M, int64_t N, int64_t K, bool off_lines, flo
     }
   };
   weigh(kBlockLarge, block_large_cost_us(M, N, K));
-  // Rows off the 128-byte lines against panels of several rounds of workgroups: every form fetches more than it uses. Times
-  // against the estimates: 128x128 tiles, K = 528 / 1104 / 2064 / 4112, 1.04 / 1.02 / 1.24 / 1.21 with 192 of them, 1.13 / 1.27 /
-  // 1.31 / 1.28 with 313, 1.19 / 1.39 / 1.47 / 1.38 with 457; one 16-row tile a workgroup, K = 2064 and 8240, 1.16 and 1.25
-  // with one row of A, 1.24 and 1.53 with 16; narrow tiles 1.1 whatever the sizes.
+  // Rows off the 128-byte lines, K no multiple of a step (832 shapes of 1 to 256 rows, weights from HBM): times against the estimates, which are
+  // of rows on the lines. Panels of several rounds of workgroups: 128x128 tiles 1.25 with 150 of them in the last round, 1.45 with 300, 1.6
+  // with 450, less on short rows; one 16-row tile a workgroup 1.1 to 1.2 with up to four rows of A, 1.2 to 1.35 with 5 to 64; narrow tiles
+  // 0.87 to 1.02 as they are. One round: narrow tiles 1.1 to 1.25 from K = 2048 on and up to 64 rows, 1.0 to 1.2 beyond; one tile a
+  // workgroup 1.25 with 5 to 16 rows, 1.1 with fewer or more (below one a CU its estimate knows of rows off the lines). With the factors
+  // below the form chosen is 0.7 % behind the quickest one on average and 38 of the shapes are more than 5 % behind; with those
+  // of the kernels that fetched such rows with the streaming policy it was 2.4 % and 113: 48x35328x8432 109 us on 128x128 tiles, 88 on
+  // narrow ones, 1x24904x1424 14.3 and 11.3 on one tile each, 5x570x11680 13.1 on narrow tiles and 9.9. (1000 other shapes: 1.016 times
+  // as fast on average, 160 more than 2 % ahead, 23 behind, 32x43552x672 14.6 -> 16.7, 34x16528x8736 56 -> 63 and 59x3388x25840 39 -> 43.)
   float one_tile_off = 1.0f, narrow_off = 1.0f;
-  if (off_lines && M <= 128 && N > 64 * kNumCu) {
-    const long rest = (N + 127) / 128 % (2 * kNumCu);
-    const float share = rest > kNumCu ? fminf(fmaxf((float)(K - 128) / 1400.0f, 0.0f), 1.0f) : K >= 1536 ? 1.0f : 0.1f;
-    cost *= 1.0f + share * (0.1f + (float)rest / 1300.0f);
-    one_tile_off = 1.2f + 0.035f * (float)(M < 8 ? M : 8) * fminf((float)K / 8192.0f, 1.0f);
-    narrow_off = 1.1f;
+  if (off_lines && N > 64 * kNumCu) {
+    if (M <= 128) {
+      const long rest = (N + 127) / 128 % (2 * kNumCu);
+      const float share = rest > kNumCu ? fminf(fmaxf((float)(K - 128) / 1400.0f, 0.0f), 1.0f) : K >= 1536 ? 1.0f : 0.3f;
+      cost *= 1.0f + share * (0.25f + (float)rest / 1300.0f);
+    }
+    one_tile_off = 1.2f + 0.025f * (float)(M < 8 ? M : 8) * fminf((float)K / 8192.0f, 1.0f);
+  } else if (off_lines && K >= 1536 && M <= kSkinnyMaxM) {
+    narrow_off = 1.15f;
+    if ((N + (M > 48 ? 31 : 15)) / (M > 48 ? 32 : 16) >= kNumCu) one_tile_off = M > 4 && M <= 16 ? 1.2f : 1.15f;
   }
   if (M <= kSkinnyMaxM) weigh(kBlockOneTile, block_one_tile_cost_us(M, N, K, one_tile_off));
   if (narrow_fits(M, N, K)) weigh(kBlockNarrow, narrow_off * narrow_cost_us(M, N, K));
@@ -4295,9 +4304,11 @@ inline BlockForm block_form(int64_t M, int64_t N, int64_t K, bool off_lines, flo
   return best;
 }
 
-// K cut in parts where the tiles are few and K is long (with a workspace for the parts). us before, the best form in one piece -> now:
-// 1000x1000x28672 160 -> 49, 312x512x9088 37.3 -> 15.4, 1047x1566x12800 78 -> 43, 92x512x26368 29.5 -> 17.3, 32x1024x28672
-// 27.1 -> 18.1, 500x5120x13824 80 -> 58, 96x16384x16384 96 -> 74, 256x4098x4096 25.5 -> 20.2; behind nowhere by more than 1 %.
+// K cut in parts where the tiles are few and K is long (with a workspace for the parts). us in the quickest form in one piece -> now:
+// 1000x1000x28672 160 -> 47, 312x512x9088 37.3 -> 15.4, 1047x1566x12800 78 -> 40, 92x512x26368 29.5 -> 17.3, 32x1024x28672
+// 27.1 -> 18.5, 500x5120x13824 80 -> 58, 96x16384x16384 96 -> 74. 265 shapes on the lines, 17 to 1500 rows and K from 2048: cut are 116, 0.60
+// of the time on average, 3 of them behind by 2 to 5 %; the plan is 0.6 % behind the quickest one on average, most where it leaves
+// 60 to 130 tiles with K = 4096 to 4700 in one piece (256x4098x4096 27.3, in two 21.7).
 struct BlockPlan {
   BlockForm form;
   int splits, steps_per_split;
@@ -4321,10 +4332,11 @@ inline BlockPlan block_plan(int64_t M, int64_t N, int64_t K, bool off_lines, int
     int splits, sps;
     normalise_splits(k_steps, want, splits, sps);
     if (splits != want || N * 512 > (int64_t)INT32_MAX) continue;
-    // (up to 16 rows the streaming forms are quicker than their estimates on long rows off the lines: 3x1425x24896 17.2 us,
-    // in fifteen parts 23.5, 4x523x22816 21.4 and 22.8)
-    // (and one row of tiles off the lines: 61x17792x10384 70 us, in two parts 80)
-    const float us = block_split_cost_us(M, N, K, off_lines, splits, sps) * (M <= 16 ? 1.5f : M <= 128 && off_lines ? 1.25f : 1.0f);
+    // (Few rows: the estimate of the parts is low against those of the streaming forms. Off the lines, in parts and streaming: 6x1382x26000
+    // 19.6 and 20.8 us, 6x780x20528 17.2 and 17.4, 4x1320x8048 11.9 and 8.1, 34x5029x16048 28.4 and 27.6, 33x894x24624 19.8 and 27.7.
+    // From 65 rows on it is right, where 1.25 left 78x11956x10704 in one piece for 71 us, in two 47, and 110x8845x4592 for 36, in three 25.)
+    const float few_rows = M <= 16 ? (off_lines ? 1.2f : 1.5f) : M <= kSkinnyMaxM && off_lines ? 1.1f : 1.0f;
+    const float us = block_split_cost_us(M, N, K, off_lines, splits, sps) * few_rows;
     if (us < cost) {
       cost = us;
       best = {kBlockSmall, splits, sps};
