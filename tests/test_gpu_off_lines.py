@@ -35,13 +35,12 @@ def _same_and_right(run, xq, wq, exact):
 
 
 ROW_CASES = [
-    # one step a wave and two (the one-tile kernel's eight waves), each of its row counts
-    *[(ONE_TILE, m, 520, k, False) for m in (1, 17, 40, 64) for k in (1024, 1152)],
+    # eight steps and nine, panels of 1.5 MB and more, each of the row counts
+    *[(ONE_TILE, m, n, k, False) for m in (1, 17, 40, 64) for n, k in ((1540, 1024), (1540, 1152), (1364, 1152), (1366, 1152))],
     # tiles of 8, 12, 16 and 20 columns, rows on both sides of the rule's, two row blocks
     *[(NARROW, m, n, 1152, False) for m in (8, 9, 32, 33) for n in (2048, 2052, 4096, 4100)],
-    (NARROW, 100, 512, 1024, False),
-    (RESIDENT, 16, 528, 1152, False),
-    (RESIDENT, 3, 528, 1152, True),
+    *[(NARROW, 100, n, k, False) for n, k in ((400, 1024), (401, 1024), (2000, 1152))],
+    *[(RESIDENT, m, n, k, m == 3) for m in (3, 16) for n, k in ((1600, 1024), (1600, 1152), (528, 1152))],
     # tiles of one and two tile rows whose launch streams B, the kernels for a K tail without one
     *[(_lib.tiled_variant(c, s), 200, 1000, 1152, s == 1) for c in range(_lib.NUM_TILE_CONFIGS) for s in (1, 3)],
     (_lib.tiled_variant(0, 3), 64, 1001, 1024, False),
@@ -67,7 +66,7 @@ def test_row_scaled(gpu_device, variant, m, n, k, with_bias):
     _same_and_right(run, xq, wq, exact)
 
 
-@pytest.mark.parametrize("form,m,n,k", [*[(_lib.BLOCK_ONE_TILE, m, 520, k) for m in (1, 64) for k in (1024, 1152)],
+@pytest.mark.parametrize("form,m,n,k", [*[(_lib.BLOCK_ONE_TILE, m, n, k) for m in (1, 64) for n, k in ((1540, 1024), (1540, 1152), (520, 1152))],
                                         *[(_lib.BLOCK_NARROW, m, n, 1152) for m in (16, 17) for n in (2048, 5120, 5124)],
                                         (_lib.BLOCK_NARROW, 100, 512, 1024), (_lib.BLOCK_TILES_128, 100, 1000, 1152),
                                         (_lib.BLOCK_TILES_128_STREAM, 100, 1000, 1152), (_lib.BLOCK_TILES_256, 100, 1000, 1152)])

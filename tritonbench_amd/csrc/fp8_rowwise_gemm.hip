@@ -4103,14 +4103,18 @@ MI355X_DEFINE_TILED_PART(6, 128, 128, 2, 2, false, true)  // (never with the str
 
 #if !defined(MI355X_TILED_PART)  // (everything from here on belongs to the main unit)
 namespace {
+// Whether the kernels of few rows ask for all of B, or of a row of it, at once: one step a wave, or a panel of at most 1.5 MB. Then both steps
+// that share a line off the 128 bytes have asked for it before it comes, nothing comes twice, and the streaming policy stays:
+// one tile a workgroup 8x714x800 2.96 us, without the policy 3.24, 47x26x3936 7.2 and 8.5, the pair kernel 0.2 to 0.3 us up to
+// 1024 columns; with more columns and K up to 1024 within 4 % either way.
+inline bool asked_for_at_once(const GemmParams& p) { return k_steps_of(p.K) <= 8 || (int64_t)p.N * p.K <= (int64_t)3 << 19; }
+
 template <int MT, int NTW, int DEPTH, int KW, bool ANY = false, bool BLOCK = false, bool OFF_LINES = false>
 int launch_skinny(const GemmParams& p, hipStream_t stream) {
   if constexpr (!ANY && !OFF_LINES) {
-    // With one step a wave the steps that share lines ask for them at the same time, and the policy stays: 8x714x800 2.96 us, without 3.24,
-    // 2x597x912 2.97 and 3.25, from 2048 columns on within 4 % either way. From the second step on a wave comes back for lines
-    // that went with the policy: 2x1021x3952 5.83 us, without 5.24, 1x6723x8272 14.9 and 13.9, 2x17533x10800 44.6 and 38.7, 3x945x20144
-    // block-scaled 16.1 and 15.0; below 2048 bytes within 0.2 us either way (24x557x1104 3.63 and 3.82, 16x8192x1552 without 0.1 ahead).
-    if (off_lines(p) && k_steps_of(p.K) > KW) return launch_skinny<MT, NTW, DEPTH, KW, false, BLOCK, true>(p, stream);
+    // (2x17533x10800 44.6 us with the streaming policy, 38.7 without, 1x6723x8272 14.9 and 13.9, 2x1021x3952 5.83 and 5.24, 3x945x20144
+    // block-scaled 16.1 and 15.0)
+    if (off_lines(p) && !asked_for_at_once(p)) return launch_skinny<MT, NTW, DEPTH, KW, false, BLOCK, true>(p, stream);
   }
   constexpr size_t lds_bytes = (size_t)KW * (NTW + MT) * 16 * kStepK;
   static_assert(lds_bytes <= 160 * 1024, "transpose buffers must fit the 160 KB LDS");
@@ -4518,7 +4522,7 @@ int launch_skinny_persistent(const GemmParams& p, hipStream_t stream) {
 template <int SPW, bool VEC, bool KTAIL, bool HAS_BIAS, bool OFF_LINES = false>
 int launch_skinny_pair(const GemmParams& p, hipStream_t stream) {
   if constexpr (KTAIL && !OFF_LINES) {  // (whole rounds of steps are off the lines with padded rows only)
-    if (off_lines(p)) return launch_skinny_pair<SPW, VEC, KTAIL, HAS_BIAS, true>(p, stream);
+    if (off_lines(p) && !asked_for_at_once(p)) return launch_skinny_pair<SPW, VEC, KTAIL, HAS_BIAS, true>(p, stream);
   }
   constexpr size_t lds_bytes = pair_lds_bytes(SPW);
   static_assert(lds_bytes <= 160 * 1024, "A's steps, the transpose buffers and the partial results must fit the LDS");
@@ -4575,7 +4579,9 @@ int launch_narrow(const GemmParams& p, hipStream_t stream) {
     // shared line on its way: 8x714x800 3.52, without 3.78, 2x2177x27472 block-scaled 25.6 and 29.0, 9x2881x21200 21.2 and 24.4,
     // 7x3468x23088 23.5 and 27.0; row-wise it ends a little earlier, 16x3421x7824 10.9 and 10.3, 16x4274x8176 block-scaled 12.7 and 12.1.
     const int few_columns = p.M > 32 ? 0 : p.M <= (BLOCK ? 16 : 8) ? (BLOCK ? 20 : 16) : 8;
-    if (off_lines(p) && narrow_tile_cols(p.N) > few_columns) return launch_narrow<MB, NB, BLOCK, true>(p, stream);
+    // (row blocks find their neighbours' lines in the L2s: they are level at 0.5 MB, 0.95 with the policy at 1.5; 5 % ahead with it up to 0.4)
+    const bool keep = p.M > 32 * MB ? (int64_t)p.N * p.K <= 400 << 10 : asked_for_at_once(p) || narrow_tile_cols(p.N) <= few_columns;
+    if (off_lines(p) && !keep) return launch_narrow<MB, NB, BLOCK, true>(p, stream);
   }
   constexpr size_t lds_bytes = narrow_lds_bytes(MB, NB);
   constexpr auto kern = gemm_narrow_kernel<MB, NB, BLOCK, OFF_LINES>;
