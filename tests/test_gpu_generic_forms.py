@@ -18,8 +18,8 @@ def _codes(rows, k, pad, seed, dev):
     return view.view(torch.float8_e4m3fn)
 
 
-# (m, n, k): one K byte to several 128-byte steps; rows and columns around 16, 32, 64 and 128; the two with about 2050
-# rows lie on either side of the 512 tiles of 128x128 from which the large tiles are taken
+# (m, n, k): one K byte to several 128-byte steps; rows and columns around 16, 32, 64 and 128; of the two with about
+# 2050 rows the first has 510 tiles of 128x128, which is what it runs, the second 544, where 128x64 tiles are quicker
 SHAPES = [(1, 1, 1), (16, 16, 15), (17, 33, 127), (32, 31, 128), (33, 40, 129), (64, 65, 4099), (65, 63, 17), (128, 129, 256),
           (129, 257, 1041), (517, 300, 383), (2049, 3840, 145), (2050, 3971, 273),
           # rows shorter than 16 bytes, in every mix of 8-, 4-, 2- and 1-byte pieces; panels on either side of the lines

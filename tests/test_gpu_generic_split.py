@@ -50,8 +50,10 @@ def test_parts_against_float64(gpu_device, m, n, k, space):
         assert (canvas == 0xFF).all()
 
 
-# either side of the lines between 64x64, 128x64 and 128x128 tiles (320 and 512 of the larger ones)
-@pytest.mark.parametrize("m,n,k", [(129, 64 * 160 - 1, 131), (129, 64 * 159, 257), (2049, 64 * 20 + 1, 700), (1025, 7200, 2065)])
+# each size of tiles with ragged edges: 64x64 (the first three, 255 of them and 272), 128x64 (1025x7200x2065, 2049x1857x1041),
+# 128x128 (the last)
+@pytest.mark.parametrize("m,n,k", [(129, 64 * 160 - 1, 131), (129, 64 * 159, 257), (2049, 64 * 20 + 1, 700), (1025, 7200, 2065),
+                                   (1025, 897, 1041), (1025, 961, 1041), (2049, 1857, 1041), (2049, 3713, 1041)])
 def test_tile_forms_against_float64(gpu_device, m, n, k):
     print(f"case m={m} n={n} k={k}", flush=True)
     a, b, sa, sb, bias, exact, magnitude = _operands(m, n, k, gpu_device)

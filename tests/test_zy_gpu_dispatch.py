@@ -100,6 +100,19 @@ def _time_us(call, sets, burst_us=4000.0):
         return sorted(burst(replays) for _ in range(3))[1]
 
 
+# the generic family's tiles, which no argument pins: a product with fewer columns or a shorter K takes no longer than the one with
+# more, within 5 % (with lines drawn by tile counts and K 1358x23320x1817 took 199 us and 179 with K = 2051)
+@pytest.mark.parametrize("less,more", [((1024, 8064, 3145), (1024, 8192, 3145)), ((1358, 23320, 1817), (1358, 23320, 2051))])
+def test_generic_tiles_follow_the_work(gpu_device, less, more):
+    times = {}
+    for m, n, k in (less, more):
+        print(f"case {m}x{n}x{k}", flush=True)
+        sets = tuning.make_operand_sets(m, n, k, False, gpu_device)
+        times[m, n, k] = min(tuning.time_variant_us(sets, _lib.VARIANT_GENERIC) for _ in range(3))
+    print("  " + ", ".join(f"{s}: {t:.1f} us" for s, t in times.items()), flush=True)
+    assert times[less] <= 1.05 * times[more]
+
+
 # the block-scaled forms: decode and prefill sizes, and wide panels with short rows or rows off the 128-byte lines, where the
 # streaming forms are behind the plain 128x128 tiles
 @pytest.mark.parametrize("m,n,k", [(1, 2304, 2048), (16, 8192, 8192), (32, 8192, 8192), (64, 57344, 8192), (128, 8192, 8192),

@@ -1043,7 +1043,7 @@ void gemm_tiled_kernel(GemmParams p) {
   // is all it asks for): rows past M fall outside the descriptor's extent, lanes whose 4 columns are not all below N are sent
   // there, and the values go from the accumulators to memory without passing through other registers. Where N is no
   // multiple of 4 the quad at the edge follows value by value. (All of them one by one, as such rows went before, and read one by one by
-  // the second pass: 1042x719x10624 29.4 us, now 22.2; 512x2049x8192 31.2, now 22.0; 128x8194x8192 37.3, now 28.4.)
+  // the second pass: 1042x719x10624 30.5 us, now 21.2; 512x2049x8192 34.8, now 25.3; 128x8194x8192 37.2, now 27.0.)
   auto store_partial = [&](int m0, int n0, int split) {
     int lane_e;  // (inside the opaque statement for the reason given in the epilogue)
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_e));
@@ -4422,13 +4422,30 @@ inline GenericPlan generic_plan(int64_t M, int64_t N, int64_t K, int max_splits)
   return best;
 }
 
+// Tiles of an unsplit launch above 64 rows, estimated from launches of 1 to 110 rounds of the CUs (420 shapes, 65 to 8192 rows, K 131 to
+// 14000): what starts and ends with the tiles, and the rounds times a 128-byte step. 64x64 tiles take 0.55 us a step for one on every
+// CU; 128x64 0.8 for twice the products, but 1.3 alone on their CUs, where nothing covers a step's latency; 128x128 2.3 for two on
+// every CU. The quickest of the three is missed by 0.2 % on average, and by more than 5 % on 5 of the 420. (With 128x128 from 512 tiles and K = 2049 on
+// and 128x64 from 320 tiles on it was 4.4 % and 122: 1154x25158x1493 171 us on 128x64, 144 on 128x128, 1152x6746x3145 92 and 65,
+// 148x51942x1677 95 and 79. What 128x64 are for: 7953x1212x847 38.6, on 128x128 45.4, 4406x768x6428 61 and, on 64x64, 71.)
+enum GenericTiles { kGeneric64, kGeneric128x64, kGeneric128 };
+inline GenericTiles generic_tiles(int64_t M, int64_t N, int64_t K) {
+  auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  auto rounds = [](int64_t tiles, int64_t slots) { return (float)((tiles + slots - 1) / slots); };
+  const int64_t t64 = tiles(64, 64), t128x64 = tiles(128, 64), t128 = tiles(128, 128);
+  const float steps = (float)k_steps_of(K);
+  // (workgroups of 256 lanes: a launch takes fewer than 2^32 lanes)
+  const float us64 = !grid_fits(t64, 256) ? 1e30f : 3.6f + 0.9e-3f * (float)t64 + steps * 0.55f * rounds(t64, kNumCu);
+  const float us128x64 = !grid_fits(t128x64, 256) ? 1e30f : 4.0f + 1.85e-3f * (float)t128x64 + steps * fmaxf(1.3f, 0.8f * rounds(t128x64, kNumCu));
+  const float us128 = 5.8f + 3.6e-3f * (float)t128 + steps * 2.3f * rounds(t128, 2 * kNumCu);
+  // (one step, or one row of tiles: nothing to gain from the larger tiles, 164x39275x3 21.6 us with 128x128, 14.0 with 64x64)
+  if ((M <= kSkinnyMaxM || K <= kStepK) && us64 < 1e30f) return kGeneric64;
+  return us64 <= us128x64 && us64 <= us128 ? kGeneric64 : us128x64 <= us128 ? kGeneric128x64 : kGeneric128;
+}
+
 // The generic family: the streaming kernel's unaligned form up to 64 rows but for short rows on wide panels (measured cold: 1x8192x8191 14.4 us,
-// 16x8192x8191 19.1, 64x8192x8191 29.7, where 64x64 tiles take 33), tiles beyond. 128x128 tiles from two
-// rounds of the CUs on where K is long enough to pay for their start (2048x4096x4100 78 us, with 128x64 88), 128x64 tiles from
-// somewhat more than one round of those on (against 64x64 or 128x128 before: 7953x1212x847 45.7 -> 38.2 us, 4406x768x6428
-// 74 -> 64, 65x30000x1001 22.6 -> 19.1, 3000x5000x700 44.8 -> 44.0); below, 64x64 tiles (517x3000x1041 13.8 us with 423 of them, 15.7
-// with 235 of 128x64). With at most one of
-// those per CU nothing but its own loads covers a step's latency, and they run two steps ahead
+// 16x8192x8191 19.1, 64x8192x8191 29.7, where 64x64 tiles take 33), tiles beyond. With at most one 64x64 tile
+// per CU nothing but its own loads covers a step's latency, and they run two steps ahead
 // (128x8192x8191 61.7 -> 36.7 us, 256x4096x4097 27.9 -> 19.6); with more, the CU's other workgroups do, and
 // the second step's registers would cost one of them (517x3000x1041 13.9 -> 12.7, 1024x2048x1025 13.7 -> 12.5).
 int launch_generic(const GemmParams& p, hipStream_t s) {
@@ -4440,12 +4457,11 @@ int launch_generic(const GemmParams& p, hipStream_t s) {
     if (p.M <= 32) return launch_skinny<2, 1, 2, 8, true>(p, s);
     return launch_skinny<4, 2, 2, 8, true>(p, s);
   }
-  auto tiles = [&](long bm, long bn) { return ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn); };
-  // (one step, or one row of tiles: nothing to gain from the larger tiles, 164x39275x3 21.6 us with 128x128, 14.0 with 64x64)
-  const bool larger = p.M > kSkinnyMaxM && p.K > kStepK;
-  if ((larger && p.K > 2048 && tiles(128, 128) >= 2 * kNumCu) || !grid_fits(tiles(128, 64), 256)) return launch_any<128, 128, 1>(p, s);
-  if ((larger && tiles(128, 64) >= kNumCu + kNumCu / 4) || !grid_fits(tiles(64, 64), 256)) return launch_any<128, 64, 1>(p, s);
-  return tiles(64, 64) <= kNumCu ? launch_any<64, 64, 2>(p, s) : launch_any<64, 64, 1>(p, s);
+  switch (generic_tiles(p.M, p.N, p.K)) {
+    case kGeneric128: return launch_any<128, 128, 1>(p, s);
+    case kGeneric128x64: return launch_any<128, 64, 1>(p, s);
+    default: return ((long)p.M + 63) / 64 * (((long)p.N + 63) / 64) <= kNumCu ? launch_any<64, 64, 2>(p, s) : launch_any<64, 64, 1>(p, s);
+  }
 }
 
 // ---- built-in scratch of the entry point that allocates nothing
