@@ -7,10 +7,11 @@ the headline workload M=N=K=8192 with operands resident in HBM. Prints ONE JSON 
 headline TFLOP/s, the roofline of the dominant kernel measured with HIP events on the launch
 stream, the CPU baseline (the oracle's fp32 dequantise + torch.matmul, timed on this machine's
 host cores), the HBM-bound headline (M=16) with a roofline block of its own, and under
-"configs" one row per benchmark configuration (microseconds, TFLOP/s, GB/s, bound, fraction of
-that bound's peak): the decode shape, all twenty Llama-3-70B projection shapes, the two ragged
-shapes with bias (each of these with its own CPU baseline where that takes seconds), and the
-neighbouring kernels (grouped, block-scaled, quantiser).
+"configs" the microseconds and the fraction of its bound's peak of every benchmark configuration:
+the decode shape, all twenty Llama-3-70B projection shapes, the two ragged shapes with bias, and
+the neighbouring kernels (grouped, block-scaled, quantiser). Their whole rows (TFLOP/s, GB/s,
+bound, a CPU baseline of their own where that takes seconds) go to stderr, one JSON object a line:
+with them the line is 23 KB long, and a log that keeps its last 8 KB loses the headline.
 
 The device runs its first milliseconds of matrix work after an idle spell well below the
 sustained clock, so whatever --warmup says the workload is launched untimed for --preheat-ms
@@ -49,6 +50,13 @@ REFERENCE_BUILTIN_SHAPES = [
     (2048, 13312, 6656), (4096, 2304, 13312), (4096, 13312, 2304), (16384, 4096, 16384),
     (16384, 8192, 13312),
 ]
+
+
+def brief(row: dict):
+    """[microseconds, fraction of the bound's peak] of a configuration's row, of each row inside it, or its error."""
+    if "us" in row:
+        return [float(f"{row['us']:.4g}"), round(row["frac"], 3)]
+    return {k: brief(v) if isinstance(v, dict) else v for k, v in row.items() if k != "cpu_baseline"}
 
 
 def source_sha() -> str:
@@ -679,7 +687,9 @@ def main():
         attempt("quantise_bf16_16384x2048", lambda: time_quantiser(16384, 2048, torch.bfloat16, dev, copies=8))
         attempt("rmsnorm_quantise_bf16_16384x2048", lambda: time_fused_front_end("rmsnorm", 16384, 2048, dev, copies=8))
         attempt("silu_mul_quantise_bf16_16384x2048", lambda: time_fused_front_end("silu_mul", 16384, 2048, dev, copies=4))
-        line["configs"] = configs
+        for name, row in configs.items():
+            print(json.dumps({"config": name, **row}), file=sys.stderr, flush=True)
+        line["configs"] = {name: brief(row) for name, row in configs.items()}
 
     if not args.no_cpu_baseline:
         line["cpu_baseline"] = cpu_baseline(head_sets[0], "M=N=K=8192")
