@@ -1,5 +1,5 @@
 """Rows of B that start off the 128-byte lines: the instances without the streaming policy, on both sides of the rules that choose them.
-The kernels sum in the same order with and without the policy, so rows padded by 16 bytes give the bits that rows on the lines give."""
+The kernels sum in the same order with and without the policy, so rows padded by 16 bytes, or by half a line, give the bits that rows on the lines give."""
 import numpy as np
 import pytest
 import torch
@@ -17,21 +17,21 @@ def _operands(m, n, k, dev):
     return codes(m), codes(n), g
 
 
-def _padded(w):
-    wide = torch.full((w.shape[0], w.shape[1] + 16), 0x7F, dtype=torch.uint8, device=w.device)  # (NaN codes past the rows' ends)
+def _padded(w, pad):
+    wide = torch.full((w.shape[0], w.shape[1] + pad), 0x7F, dtype=torch.uint8, device=w.device)  # (NaN codes past the rows' ends)
     wide[:, : w.shape[1]] = w.view(torch.uint8)
     return wide.view(torch.float8_e4m3fn)[:, : w.shape[1]]
 
 
 def _same_and_right(run, xq, wq, exact):
     bits = []
-    for w in (wq, _padded(wq)):
+    for w in (wq, _padded(wq, 16), _padded(wq, 64)):
         out = torch.full((xq.shape[0], wq.shape[0]), float("nan"), dtype=torch.bfloat16, device=xq.device)
         run(w, out)
         torch.cuda.synchronize()
         assert ((out.double() - exact).norm() / exact.norm()).item() < 2.0**-8  # (one rounding to bf16)
         bits.append(out.view(torch.int16).cpu().numpy())
-    assert np.array_equal(*bits)
+    assert np.array_equal(bits[0], bits[1]) and np.array_equal(bits[0], bits[2])
 
 
 ROW_CASES = [

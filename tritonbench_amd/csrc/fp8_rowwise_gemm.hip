@@ -4037,8 +4037,8 @@ int launch_tiled(GemmParams p, hipStream_t stream) {
   return MI355X_FP8_OK;
 }
 
-// whether rows of B start off the 128-byte lines
-inline bool off_lines(const GemmParams& p) { return ((reinterpret_cast<uintptr_t>(p.b) | (uintptr_t)p.ldb) & (kStepK - 1)) != 0; }
+// whether rows of B start off the 128-byte lines, or off their halves
+inline bool off_lines(const GemmParams& p, int bytes = kStepK) { return ((reinterpret_cast<uintptr_t>(p.b) | (uintptr_t)p.ldb) & (bytes - 1)) != 0; }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool STREAM_B, bool DEEP = false>
 int launch_tiled_epilogue(const GemmParams& p, hipStream_t s) {
@@ -4111,6 +4111,10 @@ namespace {
 // that share a line off the 128 bytes have asked for it before it comes, nothing comes twice, and the streaming policy stays:
 // one tile a workgroup 8x714x800 2.96 us, without the policy 3.24, 47x26x3936 7.2 and 8.5, the pair kernel 0.2 to 0.3 us up to
 // 1024 columns; with more columns and K up to 1024 within 4 % either way.
+// (Rows that start on 64 bytes: memory is read by halves of lines, so no half is fetched twice with the policy, and the pair kernel and the narrow
+// tiles keep it, 1.5 % ahead on 20 and 2 % on 34 shapes: 1x1600x3776 5.01 us, without 5.22, 2x4608x6848 9.36 and 9.69. One tile a workgroup
+// is level, 1 % ahead without.)
+constexpr int kHalfLine = 64;
 inline bool asked_for_at_once(const GemmParams& p) { return k_steps_of(p.K) <= 8 || (int64_t)p.N * p.K <= (int64_t)3 << 19; }
 
 template <int MT, int NTW, int DEPTH, int KW, bool ANY = false, bool BLOCK = false, bool OFF_LINES = false>
@@ -4542,7 +4546,7 @@ int launch_skinny_persistent(const GemmParams& p, hipStream_t stream) {
 template <int SPW, bool VEC, bool KTAIL, bool HAS_BIAS, bool OFF_LINES = false>
 int launch_skinny_pair(const GemmParams& p, hipStream_t stream) {
   if constexpr (KTAIL && !OFF_LINES) {  // (whole rounds of steps are off the lines with padded rows only)
-    if (off_lines(p) && !asked_for_at_once(p)) return launch_skinny_pair<SPW, VEC, KTAIL, HAS_BIAS, true>(p, stream);
+    if (off_lines(p, kHalfLine) && !asked_for_at_once(p)) return launch_skinny_pair<SPW, VEC, KTAIL, HAS_BIAS, true>(p, stream);
   }
   constexpr size_t lds_bytes = pair_lds_bytes(SPW);
   static_assert(lds_bytes <= 160 * 1024, "A's steps, the transpose buffers and the partial results must fit the LDS");
@@ -4600,7 +4604,8 @@ int launch_narrow(const GemmParams& p, hipStream_t stream) {
     // 7x3468x23088 23.5 and 27.0; row-wise it ends a little earlier, 16x3421x7824 10.9 and 10.3, 16x4274x8176 block-scaled 12.7 and 12.1.
     const int few_columns = p.M > 32 ? 0 : p.M <= (BLOCK ? 16 : 8) ? (BLOCK ? 20 : 16) : 8;
     // (row blocks find their neighbours' lines in the L2s: they are level at 0.5 MB, 0.95 with the policy at 1.5; 5 % ahead with it up to 0.4)
-    const bool keep = p.M > 32 * MB ? (int64_t)p.N * p.K <= 400 << 10 : asked_for_at_once(p) || narrow_tile_cols(p.N) <= few_columns;
+    const bool keep = p.M > 32 * MB ? (int64_t)p.N * p.K <= 400 << 10
+                                    : !off_lines(p, kHalfLine) || asked_for_at_once(p) || narrow_tile_cols(p.N) <= few_columns;
     if (off_lines(p) && !keep) return launch_narrow<MB, NB, BLOCK, true>(p, stream);
   }
   constexpr size_t lds_bytes = narrow_lds_bytes(MB, NB);
