@@ -124,6 +124,7 @@ typedef unsigned short us4 __attribute__((ext_vector_type(4)));
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 // the same in memory at any address (one instruction each on this chip)
 typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef int v4i_by4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t v2u_any __attribute__((ext_vector_type(2), aligned(1)));
 typedef uint32_t u32_any __attribute__((aligned(1)));
 typedef float v4f_by4 __attribute__((ext_vector_type(4), aligned(4)));
@@ -1674,17 +1675,17 @@ __global__ __launch_bounds__(256) void splitk_finalize_rows_kernel(GemmParams p)
 // ------------------------------------------------------------------------------------
 // Generic kernels: operands the other families cannot take (K, lda or ldb not a multiple of 16,
 // A or B not 16-byte aligned, leading dimensions beyond a buffer descriptor's range). Rows start at
-// any byte, so a lane's 16 bytes are an unaligned load (one instruction on this chip; the pieces of a
-// row lie across two cache lines more often than not), and the last chunk of a row is put
-// together byte by byte: nothing outside a row's K bytes is ever read.
+// any byte. The streaming form loads a lane's 16 bytes where they lie (one instruction on this chip; the pieces of a
+// row lie across two cache lines more often than not), the tiles in whole dwords, and the last chunk of a row is put
+// together from its last 16 bytes: nothing outside the dwords that a row's K bytes lie in is ever read.
 //
 // The products run on the 16-bit matrix instructions with the codes widened to binary16, which is
 // exact (e4m3fn reaches from 2^-9 to 448), and f32 accumulation that is as accurate as a chain of f32
 // multiply-adds (measured over K = 1024 standard normal codes: 4e-8 of the result's norm for both,
 // 1.5e-5 for the fp8 matrix instructions, which align a group of products before they add). One
-// conversion instruction widens two codes, and the conversions are what bounds the large tiles (a
-// 128x128 tile runs at 0.39 of the 16-bit matrix rate). Against byte loads and f32 multiply-adds on the
-// vector ALU, which this family was before: 517x3000x1041 212 -> 12.7 us.
+// conversion instruction of 8 cycles widens two codes, and the conversions are what bounds the tiles (4096x8192x2047:
+// 840 TFLOP/s, 0.34 of the 16-bit matrix rate). Against byte loads and f32 multiply-adds on the
+// vector ALU, which this family was at first, 517x3000x1041 took 212 us.
 // ------------------------------------------------------------------------------------
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
@@ -1738,26 +1739,47 @@ __device__ __forceinline__ v8h e4m3fn_to_f16x8(int lo, int hi) {
 #endif
 }
 
-// Generic form for more than 64 rows: BM x BN tile per workgroup of 2 x 2 waves, K in 128-byte steps.
+// Generic form for more than 64 rows: BM x BN tile per workgroup of WAVES_M x WAVES_N x WAVES_K waves, K in 128-byte steps.
 // Global memory -> registers (DEPTH steps ahead) -> LDS in the tiled kernel's swizzled layout, two stages,
 // one barrier per step; a fragment's codes are widened as they are read from LDS. The partial step
 // at the end of K is multiplied first, so that the loop over whole steps has no conditional loads (its wait
 // counts are then exact and DEPTH steps stay in flight).
-constexpr size_t any_lds_bytes(int BM, int BN) { return (size_t)2 * (BM + BN) * kStepK; }
+//
+// What bounds it is the vector ALU, which widens every fragment in each wave that multiplies it (an instruction of 8 cycles for two codes):
+// with 2x2 waves of 32x32 on a 64x64 tile 64 of them a step and wave beside 8 MFMAs of 32 cycles. Waves that share out a step's K
+// instead (WAVES_K) widen nothing twice and have wave tiles of twice the size, for one exchange of the sums at the end: 517x3000x1041 with
+// its bias 16.7 -> 14.3 us, 517x3000x4113 36.6 -> 28.4, 1000x3000x4111 52.9 -> 39.4. Where tiles of 64x64 a wave are several rounds
+// of the chip the exchange costs more than it saves and the waves share out the tile (4096x8192x2047 171 us, with WAVES_K 191).
+//
+// The bytes are fetched in whole dwords and moved into place on their way into LDS (load rates a CU from L2, 128-byte pieces of 256 rows: rows on
+// 16 or 4 bytes 83 bytes/ns, on 2 bytes 64, on odd ones 49). The last dword of the chunk in front, which a row that starts
+// off the dwords needs too, is in the lane beside it or was in the step before (a load of its own for it cost more than it gained:
+// 128x8192x8191 33.4 -> 43.0 us). Without that 1000x3000x4111 takes 47.9 us, 517x3000x1041 15.6.
+constexpr size_t any_stage_bytes(int BM, int BN, int WAVES_K, int WAVES_MN) {
+  const size_t stages = (size_t)2 * (BM + BN) * kStepK, sums = (size_t)WAVES_MN * WAVES_K * (WAVES_K - 1) * 32 * 32 * 4;
+  return stages > sums ? stages : sums;
+}
+constexpr size_t any_lds_bytes(int BM, int BN, int WAVES_K, int WAVES_MN) { return any_stage_bytes(BM, BN, WAVES_K, WAVES_MN) + (size_t)(BM + 2 * BN) * 4; }
 
 // PARTIAL: K in p.splits parts of p.steps_per_split steps, each an item of its own that leaves its sums in its plane of p.partial
 // for the second pass. The last part has the partial step.
-template <int BM, int BN, int DEPTH, bool PARTIAL>
-__global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
-  constexpr int WTM = BM / 2, WTN = BN / 2, MT = WTM / 32, NT = WTN / 32;
+template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int DEPTH, bool PARTIAL>
+__global__ __launch_bounds__(WAVES_M* WAVES_N* WAVES_K * 64) void gemm_any_kernel(GemmParams p) {
+  constexpr int THREADS = WAVES_M * WAVES_N * WAVES_K * 64;
+  constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N, MT = WTM / 32, NT = WTN / 32;
   constexpr int STAGE = (BM + BN) * kStepK;  // A's rows, then B's
-  constexpr int LA = BM / 32, LOADS = (BM + BN) / 32;  // chunks of A, and of both, a lane fetches per step
+  constexpr int ROWS = THREADS / 8;          // rows a round of the workgroup's lanes fetches, eight lanes each
+  constexpr int LA = BM / ROWS, LOADS = (BM + BN) / ROWS;  // chunks of A, and of both, a lane fetches per step
+  constexpr int PAIRS = 4 / WAVES_K;         // pairs of chunks of a row's eight that a wave multiplies, one for each half of its lanes
+  constexpr int OWN = MT * NT / WAVES_K;     // 32x32 blocks that a wave finishes
+  static_assert(BM % ROWS == 0 && BN % ROWS == 0 && ROWS % 16 == 0, "whole rounds of rows of one operand, which share their swizzle");
+  static_assert(WAVES_K == 1 || (WAVES_K == 4 && WAVES_K % NT == 0 && OWN * WAVES_K == MT * NT), "each wave finishes blocks of one column");
   fetch_arguments_now(p);
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1, l32 = lane & 31, half = lane >> 5;
+  const int wk = wave % WAVES_K, wmn = wave / WAVES_K, wm = wmn / WAVES_N, wn = wmn % WAVES_N, l32 = lane & 31, half = lane >> 5;
 
   // each XCD takes a contiguous run of the tile list (kGroupM tile rows at a time, column-major inside)
   const int tiles = p.tiles_m * p.tiles_n;
@@ -1769,18 +1791,73 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
   tile_coords(item - part * tiles, p.tiles_m, p.tiles_n, p.div_group_mul, p.div_group_shift, tm, tn);
   const long m0 = (long)tm * BM, n0 = (long)tn * BN;
 
-  // lane's chunk ld_c of rows ld_row, ld_row + 32, ... (rows past an edge repeat the last one)
+  // Steps of this item from step `first` on but for the row's last one, which has 1 to 128 bytes and is its last part's.
+  const int whole = (p.K - 1) / kStepK;
+  const int first = PARTIAL ? part * p.steps_per_split : 0;
+  const int full = PARTIAL ? min(p.steps_per_split, whole - first) : whole;
+  const bool has_tail = !PARTIAL || part == p.splits - 1;
+
+  // Lane's chunk ld_c of rows ld_row, ld_row + ROWS, ... (rows past an edge repeat the last one).
+  // The bytes of a step are fetched as the whole dwords behind the one that its first byte lies in, and moved into place when
+  // they are parked: a chunk begins in the last dword of the chunk in front of it, the lane's beside it, or the step's before.
+  // (Every dword that is fetched holds bytes of its row: the first one byte 0, the last one byte 128 * whole.)
   const int ld_row = tid >> 3, ld_c = tid & 7;
+  const uint8_t* at[LOADS];  // what is fetched next
+  uint32_t shift[LOADS];
+  int before[LOADS];  // the last dword of the step that was parked last
+  v4i land[DEPTH][LOADS];
   const uint8_t* row[LOADS];
 #pragma unroll
   for (int i = 0; i < LOADS; ++i) {
-    const int r = ld_row + 32 * (i < LA ? i : i - LA);
+    const int r = ld_row + ROWS * (i < LA ? i : i - LA);
     row[i] = i < LA ? p.a + (size_t)min(m0 + r, (long)p.M - 1) * p.lda : p.b + (size_t)min(n0 + r, (long)p.N - 1) * p.ldb;
+    shift[i] = (uint32_t)(reinterpret_cast<uintptr_t>(row[i]) & 3);
+    at[i] = row[i] - shift[i] + (long)first * kStepK + ld_c * kChunk + 4;
+    before[i] = full > 0 ? *(const int*)(row[i] - shift[i] + (long)first * kStepK) : 0;
   }
-  const int park_pos = ld_row * kStepK + ((ld_c ^ swz128(ld_row)) * kChunk);  // (32 rows on: the same swizzle)
+  // the factors and the bias of the tile's rows and columns, which wait in LDS behind the stages for the end
+  uint8_t* const ends = lds + any_stage_bytes(BM, BN, WAVES_K, WAVES_M * WAVES_N);
+  float end_a = 0.0f, end_b = 0.0f, end_bias = 0.0f;
+  if constexpr (!PARTIAL) {
+    if (tid < BM) end_a = p.a_scale[min(m0 + tid, (long)p.M - 1)];
+    if (tid < BN) {
+      const long n = min(n0 + tid, (long)p.N - 1);
+      end_b = p.b_scale[n];
+      if (p.bias) end_bias = bf16_to_f32(p.bias[n]);
+    }
+  }
+  auto park_ends = [&]() {  // (after the first steps have been asked for)
+    if constexpr (!PARTIAL) {
+      if (tid < BM) *(float*)(ends + tid * 4) = end_a;
+      if (tid < BN) {
+        *(float*)(ends + (BM + tid) * 4) = end_b;
+        *(float*)(ends + (BM + BN + tid) * 4) = end_bias;
+      }
+    }
+  };
+  int to_fetch = full;  // whole steps that have not been asked for
+  auto fetch = [&](v4i (&to)[LOADS]) {
+    const long on = --to_fetch > 0 ? kStepK : 0;  // past the last whole step: that one again, for nobody
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      to[i] = *(const v4i_by4*)at[i];
+      at[i] += on;
+    }
+  };
+  const int park_pos = ld_row * kStepK + ((ld_c ^ swz128(ld_row)) * kChunk);  // (ROWS rows on: the same swizzle)
+  auto park_one = [&](const v4i& chunk, int i, int stage) { *(v4i*)(lds + park_pos + stage * STAGE + i * ROWS * kStepK) = chunk; };
   auto park = [&](const v4i (&from)[LOADS], int stage) {
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) *(v4i*)(lds + stage * STAGE + i * 32 * kStepK + park_pos) = from[i];
+    for (int i = 0; i < LOADS; ++i) {
+      const v4i x = from[i];
+      // the lane beside it; for the first of a row's eight lanes the last one's of the step before
+      const int left = __builtin_amdgcn_update_dpp(0, x[3], 0x111, 0xf, 0xf, true);       // row_shr:1
+      const int back = __builtin_amdgcn_update_dpp(0, before[i], 0x141, 0xf, 0xf, true);  // row_half_mirror
+      before[i] = x[3];
+      const int front = ld_c == 0 ? back : left;
+      park_one((v4i){(int)__builtin_amdgcn_alignbyte(x[0], front, shift[i]), (int)__builtin_amdgcn_alignbyte(x[1], x[0], shift[i]),
+                     (int)__builtin_amdgcn_alignbyte(x[2], x[1], shift[i]), (int)__builtin_amdgcn_alignbyte(x[3], x[2], shift[i])}, i, stage);
+    }
   };
   auto join = [&]() {  // this wave's LDS accesses are done, then everyone's; global loads stay in flight
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
@@ -1792,137 +1869,157 @@ __global__ __launch_bounds__(256) void gemm_any_kernel(GemmParams p) {
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[i][j] = (v16f){0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  int frag_pos[PAIRS];
+#pragma unroll
+  for (int c = 0; c < PAIRS; ++c) frag_pos[c] = l32 * kStepK + (((2 * (wk * PAIRS + c) + half) ^ swz128(l32)) * kChunk);
+  const int rows_a = wm * WTM * kStepK, rows_b = (BM + wn * WTN) * kStepK;
   auto multiply = [&](int stage) {
-    const uint8_t* rows_a = lds + stage * STAGE + (wm * WTM + l32) * kStepK;
-    const uint8_t* rows_b = lds + stage * STAGE + (BM + wn * WTN + l32) * kStepK;
+    v4i ra[PAIRS][MT], rb[PAIRS][NT];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {  // lane half h multiplies chunk 2c + h of its row: 8 codes per instruction
-      const int off = ((2 * c + half) ^ swz128(l32)) * kChunk;
-      v8h fa[MT][2], fb[NT][2];
+    for (int c = 0; c < PAIRS; ++c) {
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const v4i x = *(const v4i*)(rows_a + i * 32 * kStepK + off);
-        fa[i][0] = e4m3fn_to_f16x8(x[0], x[1]);
-        fa[i][1] = e4m3fn_to_f16x8(x[2], x[3]);
-      }
+      for (int i = 0; i < MT; ++i) ra[c][i] = *(const v4i*)(lds + frag_pos[c] + rows_a + stage * STAGE + i * 32 * kStepK);
 #pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        const v4i x = *(const v4i*)(rows_b + j * 32 * kStepK + off);
-        fb[j][0] = e4m3fn_to_f16x8(x[0], x[1]);
-        fb[j][1] = e4m3fn_to_f16x8(x[2], x[3]);
-      }
+      for (int j = 0; j < NT; ++j) rb[c][j] = *(const v4i*)(lds + frag_pos[c] + rows_b + stage * STAGE + j * 32 * kStepK);
+    }
+    if (PAIRS > 1) __builtin_amdgcn_sched_barrier(0);  // (left alone, the reads of a pair wait for the products of the one before)
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
+    for (int c = 0; c < PAIRS; ++c) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {  // 8 codes of a lane per instruction
+        v8h fa[MT], fb[NT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) fa[i] = e4m3fn_to_f16x8(ra[c][i][2 * u], ra[c][i][2 * u + 1]);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) fb[j] = e4m3fn_to_f16x8(rb[c][j][2 * u], rb[c][j][2 * u + 1]);
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-          for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[j][u], fa[i][u], acc[i][j], 0, 0, 0);
+          for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+      }
     }
   };
 
-  // whole steps of this item from step `first` on, and whether the partial one is its own
-  const int whole = p.K / kStepK;
-  const int first = PARTIAL ? part * p.steps_per_split : 0;
-  const int full = PARTIAL ? min(p.steps_per_split, whole - first) : whole;
-  const bool has_tail = whole * kStepK < p.K && (!PARTIAL || part == p.splits - 1);
-  v4i land[DEPTH][LOADS];
-  auto fetch = [&](v4i (&to)[LOADS], int s) {  // past the last whole step: that one again, for nobody
-    const int k = (first + min(s, full - 1)) * kStepK + ld_c * kChunk;
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) to[i] = *(const v4i_any*)(row[i] + k);
-  };
   if (full > 0)
 #pragma unroll
-    for (int d = 0; d < DEPTH; ++d) fetch(land[d], d);
+    for (int d = 0; d < DEPTH; ++d) fetch(land[d]);
+  park_ends();
   if (has_tail) {
     v4i tail[LOADS];
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) tail[i] = load16_any(row[i], whole * kStepK + ld_c * kChunk, p.K);
-    park(tail, 1);
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) park_one(tail[i], i, 1);
     join();
     multiply(1);
+    if (full <= 0) join();
   }
   if (full > 0) {
-    // step s on the stage it was parked in; its registers take step s + DEPTH, the other stage step s + 1
-    auto step = [&](int d, int s) {
-      fetch(land[d], s + DEPTH);
+    // a step on the stage it was parked in; its registers take the step DEPTH on, the other stage the next one
+    auto step = [&](int d, int stage) {
+      fetch(land[d]);
       __builtin_amdgcn_sched_barrier(0);
-      multiply(s & 1);
-      park(land[(d + 1) % DEPTH], (s + 1) & 1);
+      multiply(stage);
+      park(land[(d + 1) % DEPTH], stage ^ 1);
       join();
     };
     park(land[0], 0);
     join();
+    constexpr int TURN = DEPTH % 2 ? 2 * DEPTH : DEPTH;  // steps after which registers and stages are the same again
     int s = 0;
-    for (; s + DEPTH <= full; s += DEPTH)
+    for (; s + TURN <= full; s += TURN)
 #pragma unroll
-      for (int d = 0; d < DEPTH; ++d) step(d, s + d);
+      for (int d = 0; d < TURN; ++d) step(d % DEPTH, d & 1);
 #pragma unroll
-    for (int d = 0; d < DEPTH - 1; ++d)
-      if (s + d < full) step(d, s + d);
+    for (int d = 0; d < TURN - 1; ++d)
+      if (s + d < full) step(d % DEPTH, d & 1);
   }
 
-  if constexpr (PARTIAL) {
-    float* plane = p.partial + (size_t)part * p.M * p.N;
+  // Lane (l32, half) holds row l32 of a block, columns 8q + 4*half + 0..3: each four as one piece wherever it lies
+  // (1795x84399x13, rows of C that start at any 2 bytes: 553 us with a store per element).
+  auto finish = [&](const v16f& sum, int i, int j) {
+    const int m_tile = wm * WTM + i * 32 + l32, n_tile = wn * WTN + j * 32 + 4 * half;
+    const long m = m0 + m_tile;
+    const float sa_m = PARTIAL ? 0.0f : *(const float*)(ends + m_tile * 4);
+    v4f sb[4], bias[4];
+    if constexpr (!PARTIAL) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const long m = m0 + wm * WTM + i * 32 + l32;
-      if (m >= p.M) continue;
+      for (int q = 0; q < 4; ++q) {
+        sb[q] = *(const v4f*)(ends + (BM + n_tile + 8 * q) * 4);
+        bias[q] = *(const v4f*)(ends + (BM + BN + n_tile + 8 * q) * 4);
+      }
+    }
+    if (m < p.M) {
 #pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const long n = n0 + wn * WTN + j * 32 + 8 * q + 4 * half;
-          float* dst = plane + (size_t)m * p.N + n;
+      for (int q = 0; q < 4; ++q) {
+        const long n = n0 + n_tile + 8 * q;
+        if constexpr (PARTIAL) {
+          float* dst = p.partial + ((size_t)part * p.M + m) * p.N + n;
           if (n + 3 < p.N) {
-            *(v4f_by4*)dst = (v4f){acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+            *(v4f_by4*)dst = (v4f){sum[4 * q], sum[4 * q + 1], sum[4 * q + 2], sum[4 * q + 3]};
           } else {
 #pragma unroll
             for (int e = 0; e < 3; ++e)
-              if (n + e < p.N) dst[e] = acc[i][j][4 * q + e];
+              if (n + e < p.N) dst[e] = sum[4 * q + e];
+          }
+        } else {
+          float v[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float t = sum[4 * q + e] * sa_m;
+            v[e] = p.bias ? __builtin_fmaf(t, sb[q][e], bias[q][e]) : t * sb[q][e];
+          }
+          const uint32_t lo = pack_out_x2(v[0], v[1], p.out_f16), hi = pack_out_x2(v[2], v[3], p.out_f16);
+          uint16_t* dst = p.c + (size_t)m * p.ldc + n;
+          if (n + 3 < p.N) {
+            *(v2u_any*)dst = (v2u){lo, hi};
+          } else {
+            if (n < p.N) dst[0] = (uint16_t)lo;
+            if (n + 1 < p.N) dst[1] = (uint16_t)(lo >> 16);
+            if (n + 2 < p.N) dst[2] = (uint16_t)hi;
           }
         }
+      }
     }
-    return;
-  }
-  // lane (l32, half): row l32 of every 32x32 block, columns 8q + 4*half + 0..3, as one 8-byte store wherever it lies
-  // (1795x84399x13, rows of C that start at any 2 bytes: 553 us with a store per element)
+  };
+  if constexpr (WAVES_K == 1) {
 #pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    float sb[4][4], bias[4][4];
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+      for (int i = 0; i < MT; ++i) finish(acc[i][j], i, j);
+  } else {
+    // The sums of the waves that shared out K meet in LDS, where the stages were, a block for each of them at a time: the wave that
+    // finishes it adds what the others left to its own, in their order.
+    constexpr int kBlockBytes = 32 * 32 * 4;
+    uint8_t* const slots = lds + wmn * (WAVES_K * (WAVES_K - 1) * kBlockBytes) + lane * 16;
+    auto slot = [&](int writer, int owner) { return slots + (owner * (WAVES_K - 1) + (writer < owner ? writer : writer - 1)) * kBlockBytes; };
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const long ne = min(n0 + wn * WTN + j * 32 + 8 * q + 4 * half + e, (long)p.N - 1);
-        sb[q][e] = p.b_scale[ne];
-        bias[q][e] = p.bias ? bf16_to_f32(p.bias[ne]) : 0.0f;
-      }
+    for (int r = 0; r < OWN; ++r) {
+      v16f mine;
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const long m = m0 + wm * WTM + i * 32 + l32;
-      if (m >= p.M) continue;
-      const float sa_m = p.a_scale[m];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const long n = n0 + wn * WTN + j * 32 + 8 * q + 4 * half;
-        float r[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float t = acc[i][j][4 * q + e] * sa_m;
-          r[e] = p.bias ? __builtin_fmaf(t, sb[q][e], bias[q][e]) : t * sb[q][e];
-        }
-        const uint32_t lo = pack_out_x2(r[0], r[1], p.out_f16), hi = pack_out_x2(r[2], r[3], p.out_f16);
-        uint16_t* dst = p.c + (size_t)m * p.ldc + n;
-        if (n + 3 < p.N) {
-          *(v2u_any*)dst = (v2u){lo, hi};
+      for (int o = 0; o < WAVES_K; ++o) {
+        const v16f& block = acc[o / NT * OWN + r][o % NT];
+        if (wk == o) {
+          mine = block;
         } else {
-          if (n < p.N) dst[0] = (uint16_t)lo;
-          if (n + 1 < p.N) dst[1] = (uint16_t)(lo >> 16);
-          if (n + 2 < p.N) dst[2] = (uint16_t)hi;
-          if (n + 3 < p.N) dst[3] = (uint16_t)(hi >> 16);
+          uint8_t* const to = slot(wk, o);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) *(v4f*)(to + q * 1024) = (v4f){block[4 * q], block[4 * q + 1], block[4 * q + 2], block[4 * q + 3]};
         }
       }
+      join();
+#pragma unroll
+      for (int o = 0; o < WAVES_K - 1; ++o) {
+        const uint8_t* const from = slot(o < wk ? o : o + 1, wk);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const v4f x = *(const v4f*)(from + q * 1024);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) mine[4 * q + e] += x[e];
+        }
+      }
+      if (r + 1 < OWN) join();
+      finish(mine, wk / NT * OWN + r, wk % NT);
     }
   }
 }
@@ -4376,10 +4473,10 @@ int launch_block_form(GemmParams p, hipStream_t stream) {
 }
 int launch_block(const GemmParams& p, hipStream_t s) { return p.K % kStepK ? launch_block_form<true>(p, s) : launch_block_form<false>(p, s); }
 
-template <int BM, int BN, int DEPTH, bool PARTIAL = false>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int DEPTH, bool PARTIAL = false>
 int launch_any(GemmParams p, hipStream_t stream) {
-  constexpr size_t lds_bytes = any_lds_bytes(BM, BN);
-  constexpr auto kern = gemm_any_kernel<BM, BN, DEPTH, PARTIAL>;
+  constexpr size_t lds_bytes = any_lds_bytes(BM, BN, WAVES_K, WAVES_M * WAVES_N);
+  constexpr auto kern = gemm_any_kernel<BM, BN, WAVES_M, WAVES_N, WAVES_K, DEPTH, PARTIAL>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
@@ -4389,7 +4486,7 @@ int launch_any(GemmParams p, hipStream_t stream) {
   make_fast_div((uint32_t)p.tiles_m * (uint32_t)p.tiles_n, p.div_tiles_mul, p.div_tiles_shift);
   make_fast_div((uint32_t)kGroupM * (uint32_t)p.tiles_n, p.div_group_mul, p.div_group_shift);
   if (const int st = ready_device()) return st;
-  hipLaunchKernelGGL(kern, dim3((unsigned)((items + kNumXcd - 1) / kNumXcd * kNumXcd)), dim3(256), lds_bytes, stream, p);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((items + kNumXcd - 1) / kNumXcd * kNumXcd)), dim3(WAVES_M * WAVES_N * WAVES_K * 64), lds_bytes, stream, p);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "generic kernel launch: %s", hipGetErrorString(e));
   return PARTIAL ? launch_finalize(p, stream) : MI355X_FP8_OK;
@@ -4405,9 +4502,39 @@ constexpr bool generic_streams(int64_t M, int64_t N, int64_t K) {
   return !(K <= (M <= 16 ? 128 : 256) && N > (M <= 32 ? 8192 : 4096));
 }
 static_assert(!generic_streams(1, 1 << 27, 1024) && generic_streams(1, (1 << 27) - 16, 1024), "2^27 columns are 2^32 lanes");
-// Where the tiles are few and K is long, K is cut into parts (128x64 tiles, up to one item a CU): a CU takes in what it can have
-// outstanding, 0.45 us for a step of 64x64 tiles whatever the depth, so a launch is as quick as it has CUs at work. 128x64 tiles
-// take 0.74 us a step for twice the products.
+// Tiles of a launch above 64 rows, estimated from launches of 1 to 70 rounds of the CUs (180 shapes, 65 to 12000 rows, K 100 to 16000): what
+// starts and ends with the launch and with each tile, and the rounds of the CUs times a 128-byte step. Waves that share out K (64x64, 128x64 and 128x128
+// tiles) are ahead while the tiles are few rounds, waves that share out the tile (64x64 and 128x128) on short rows and over many rounds: us in that
+// order 463x1440x2101 14.2, 17.0, 23.9, 31.4 and 18.6; 362x5040x4907 39.8, 35.0, 45.6, 63.5 and 42.4; 243x15469x7535 105.6, 96.7, 76.8, 97.0 and 106.3;
+// 707x19781x241 38.8, 51.8, 40.4, 33.1 and 35.8; 134x20332x519 19.9, 25.5, 26.0, 21.4 and 16.6. The quickest of the five is missed by 0.3 % on
+// average, and by more than 7 % on 3 of the 180.
+enum GenericTiles { kGeneric64Shared, kGeneric128x64Shared, kGeneric128Shared, kGeneric128, kGeneric64 };
+struct GenericChoice {
+  GenericTiles tiles;
+  float us;
+};
+inline GenericChoice generic_tiles(int64_t M, int64_t N, int64_t K) {
+  auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  auto rounds = [](int64_t tiles, int64_t slots) { return (float)((tiles + slots - 1) / slots); };
+  const int64_t t64 = tiles(64, 64), t128x64 = tiles(128, 64), t128 = tiles(128, 128);
+  const float steps = (float)k_steps_of(K);
+  // (workgroups of 256 or 512 lanes: a launch takes fewer than 2^32 lanes)
+  const float us[] = {grid_fits(t64, 256) ? 4.4f + 7.05e-3f * (float)t64 + steps * 0.40f * rounds(t64, kNumCu) : 1e30f,
+                      grid_fits(t128x64, 512) ? 4.0f + 15.3e-3f * (float)t128x64 + steps * 0.53f * rounds(t128x64, kNumCu) : 1e30f,
+                      grid_fits(t128, 512) ? 6.3f + 23.3e-3f * (float)t128 + steps * 0.89f * rounds(t128, kNumCu) : 1e30f,
+                      5.4f + 22.9e-3f * (float)t128 + steps * 1.39f * rounds(t128, 2 * kNumCu),
+                      grid_fits(t64, 256) ? 3.2f + 6.0e-3f * (float)t64 + steps * fmaxf(0.90f, 0.37f * rounds(t64, kNumCu)) : 1e30f};
+  // (one step, or one row of tiles: nothing to gain from the larger tiles, 164x39275x3 21.6 us with 128x128, 14.0 with 64x64)
+  GenericChoice best = {(M <= kSkinnyMaxM || K <= kStepK) && us[kGeneric64] < 1e30f ? kGeneric64 : kGeneric128, 1e30f};
+  best.us = us[best.tiles];
+  if (best.tiles == kGeneric128)
+    for (int f = kGeneric64Shared; f <= kGeneric64; ++f)
+      if (us[f] < best.us) best = {(GenericTiles)f, us[f]};
+  return best;
+}
+
+// Where the tiles are few and K is long, K is cut into parts (128x64 tiles, up to one item a CU): a launch is as quick as it has CUs at
+// work. What the second pass adds is a launch and the planes' way through memory.
 struct GenericPlan {
   int splits, steps_per_split;
 };
@@ -4416,12 +4543,12 @@ inline GenericPlan generic_plan(int64_t M, int64_t N, int64_t K, int max_splits)
   GenericPlan best = {1, k_steps};
   const int64_t tiles_64 = ((M + 63) / 64) * ((N + 63) / 64), tiles = ((M + 127) / 128) * ((N + 63) / 64);
   if (generic_streams(M, N, K) || tiles_64 >= kNumCu) return best;
-  float cost = 0.92f * ((float)k_steps * (0.45f + 0.17f * (float)tiles_64 / (float)kNumCu) + 4.0f);
+  float cost = generic_tiles(M, N, K).us;
   for (int want = 2; want <= max_splits && tiles * want <= kNumCu; ++want) {
     int splits, sps;
     normalise_splits(k_steps, want, splits, sps);
     if (splits != want) continue;
-    const float us = (float)sps * 0.74f + 7.0f + 2.0f * (float)splits * (float)M * (float)N * 4.0f / 5.0e6f;
+    const float us = (float)sps * 0.62f + 7.5f + 2.0f * (float)splits * (float)M * (float)N * 4.0f / 5.0e6f;
     if (us < cost) {
       cost = us;
       best = {splits, sps};
@@ -4430,45 +4557,24 @@ inline GenericPlan generic_plan(int64_t M, int64_t N, int64_t K, int max_splits)
   return best;
 }
 
-// Tiles of an unsplit launch above 64 rows, estimated from launches of 1 to 110 rounds of the CUs (420 shapes, 65 to 8192 rows, K 131 to
-// 14000): what starts and ends with the tiles, and the rounds times a 128-byte step. 64x64 tiles take 0.55 us a step for one on every
-// CU; 128x64 0.8 for twice the products, but 1.3 alone on their CUs, where nothing covers a step's latency; 128x128 2.3 for two on
-// every CU. The quickest of the three is missed by 0.2 % on average, and by more than 5 % on 5 of the 420. (With 128x128 from 512 tiles and K = 2049 on
-// and 128x64 from 320 tiles on it was 4.4 % and 122: 1154x25158x1493 171 us on 128x64, 144 on 128x128, 1152x6746x3145 92 and 65,
-// 148x51942x1677 95 and 79. What 128x64 are for: 7953x1212x847 38.6, on 128x128 45.4, 4406x768x6428 61 and, on 64x64, 71.)
-enum GenericTiles { kGeneric64, kGeneric128x64, kGeneric128 };
-inline GenericTiles generic_tiles(int64_t M, int64_t N, int64_t K) {
-  auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  auto rounds = [](int64_t tiles, int64_t slots) { return (float)((tiles + slots - 1) / slots); };
-  const int64_t t64 = tiles(64, 64), t128x64 = tiles(128, 64), t128 = tiles(128, 128);
-  const float steps = (float)k_steps_of(K);
-  // (workgroups of 256 lanes: a launch takes fewer than 2^32 lanes)
-  const float us64 = !grid_fits(t64, 256) ? 1e30f : 3.6f + 0.9e-3f * (float)t64 + steps * 0.55f * rounds(t64, kNumCu);
-  const float us128x64 = !grid_fits(t128x64, 256) ? 1e30f : 4.0f + 1.85e-3f * (float)t128x64 + steps * fmaxf(1.3f, 0.8f * rounds(t128x64, kNumCu));
-  const float us128 = 5.8f + 3.6e-3f * (float)t128 + steps * 2.3f * rounds(t128, 2 * kNumCu);
-  // (one step, or one row of tiles: nothing to gain from the larger tiles, 164x39275x3 21.6 us with 128x128, 14.0 with 64x64)
-  if ((M <= kSkinnyMaxM || K <= kStepK) && us64 < 1e30f) return kGeneric64;
-  return us64 <= us128x64 && us64 <= us128 ? kGeneric64 : us128x64 <= us128 ? kGeneric128x64 : kGeneric128;
-}
-
 // The generic family: the streaming kernel's unaligned form up to 64 rows but for short rows on wide panels (measured cold: 1x8192x8191 14.4 us,
-// 16x8192x8191 19.1, 64x8192x8191 29.7, where 64x64 tiles take 33), tiles beyond. With at most one 64x64 tile
-// per CU nothing but its own loads covers a step's latency, and they run two steps ahead
-// (128x8192x8191 61.7 -> 36.7 us, 256x4096x4097 27.9 -> 19.6); with more, the CU's other workgroups do, and
-// the second step's registers would cost one of them (517x3000x1041 13.9 -> 12.7, 1024x2048x1025 13.7 -> 12.5).
+// 16x8192x8191 19.1, 64x8192x8191 29.7, where 64x64 tiles take 33), tiles beyond. Tiles whose waves share out K run two steps ahead
+// (61.1 -> 41.8 us on 128x8192x8191), the others, of which a CU has several, one.
 int launch_generic(const GemmParams& p, hipStream_t s) {
   // (the documented range of the family, which the tests' sizes lie in)
   if (p.M > 65535 * 64) return fail(MI355X_FP8_ENOTSUP, "the generic family takes M <= %d", 65535 * 64);
-  if (p.splits > 1) return launch_any<128, 64, 2, true>(p, s);
+  if (p.splits > 1) return launch_any<128, 64, 2, 1, 4, 2, true>(p, s);
   if (generic_streams(p.M, p.N, p.K)) {
     if (p.M <= 16) return launch_skinny<1, 1, 4, 8, true>(p, s);
     if (p.M <= 32) return launch_skinny<2, 1, 2, 8, true>(p, s);
     return launch_skinny<4, 2, 2, 8, true>(p, s);
   }
-  switch (generic_tiles(p.M, p.N, p.K)) {
-    case kGeneric128: return launch_any<128, 128, 1>(p, s);
-    case kGeneric128x64: return launch_any<128, 64, 1>(p, s);
-    default: return ((long)p.M + 63) / 64 * (((long)p.N + 63) / 64) <= kNumCu ? launch_any<64, 64, 2>(p, s) : launch_any<64, 64, 1>(p, s);
+  switch (generic_tiles(p.M, p.N, p.K).tiles) {
+    case kGeneric64Shared: return launch_any<64, 64, 1, 1, 4, 2>(p, s);
+    case kGeneric128x64Shared: return launch_any<128, 64, 2, 1, 4, 2>(p, s);
+    case kGeneric128Shared: return launch_any<128, 128, 2, 1, 4, 2>(p, s);
+    case kGeneric64: return launch_any<64, 64, 2, 2, 1, 1>(p, s);
+    default: return launch_any<128, 128, 2, 2, 1, 1>(p, s);
   }
 }
 
