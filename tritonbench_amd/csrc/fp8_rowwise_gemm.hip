@@ -3139,6 +3139,29 @@ __device__ __forceinline__ uint8_t f32_to_e4m3fn_rne(float f) {
   return (uint8_t)(sign | v);
 }
 
+// A reduction over the wave, in every lane: each lane's value with that of the lane whose number differs in one bit, from bit 5 down to bit 0. In the
+// register file: __shfl_xor goes through LDS, six round trips in a row (0.1 to 0.3 us of a call of few rows: RMSNorm 32x8192, which has two
+// reductions, 4.95 -> 4.64 us in four rounds of 256 lanes, SiLU-mul 32x8192 3.76 -> 3.63).
+template <typename Op>
+__device__ __forceinline__ float wave_reduce(float v, Op op) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  auto dpp = [](float from, float old, auto ctrl, auto banks) -> float {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(from), decltype(ctrl)::value, 0xf, decltype(banks)::value, false));
+  };
+  using std::integral_constant;
+  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+  v = op(__int_as_float(halves[0]), __int_as_float(halves[1]));
+  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+  v = op(__int_as_float(rows[0]), __int_as_float(rows[1]));
+  v = op(v, dpp(v, v, integral_constant<int, 0x128>{}, integral_constant<int, 0xf>{}));  // row_ror:8
+  const float up = dpp(v, v, integral_constant<int, 0x104>{}, integral_constant<int, 0x5>{});  // row_shl:4 into the even fours
+  v = op(v, dpp(v, up, integral_constant<int, 0x114>{}, integral_constant<int, 0xa>{}));       // row_shr:4 into the odd ones
+  v = op(v, dpp(v, v, integral_constant<int, 0x4E>{}, integral_constant<int, 0xf>{}));         // quad_perm [2, 3, 0, 1]
+  v = op(v, dpp(v, v, integral_constant<int, 0xB1>{}, integral_constant<int, 0xf>{}));         // quad_perm [1, 0, 3, 2]
+#endif
+  return v;
+}
+
 template <typename SrcT>
 struct SrcTraits;
 // fp32 source: every step rounds to fp32 once, as the eager PyTorch program does.
@@ -3194,8 +3217,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(const SrcT* x, uint8
 
   float amax = 0.0f;
   for (int k = threadIdx.x; k < K; k += 256) amax = max_keep_nan(amax, fabsf(T::load(xr + k)));
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) amax = max_keep_nan(amax, __shfl_xor(amax, o));
+  amax = wave_reduce(amax, [](float a, float b) { return max_keep_nan(a, b); });
   if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = amax;
   __syncthreads();
   amax = max_keep_nan(max_keep_nan(wave_max[0], wave_max[1]), max_keep_nan(wave_max[2], wave_max[3]));
@@ -3282,8 +3304,7 @@ __global__ __launch_bounds__(THREADS* ROWS) void quantize_rows_vec_kernel(const 
 #pragma unroll
   for (int i = 0; i < CACHE; ++i) fold(cache[i]);
   for (int c = tid + THREADS * CACHE; c < nchunks; c += THREADS) fold(load(c));
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) amax = max_keep_nan(amax, __shfl_xor(amax, o));
+  amax = wave_reduce(amax, [](float a, float b) { return max_keep_nan(a, b); });
   if (THREADS > 64) {
     if ((tid & 63) == 0) wave_max[tid >> 6] = amax;
     __syncthreads();
@@ -3325,18 +3346,17 @@ __global__ __launch_bounds__(THREADS* ROWS) void quantize_rows_vec_kernel(const 
   // a wave-private LDS strip (LDS executes a wave's operations in order: no barrier) and
   // leave as one 16-byte store per lane, BATCH runs of 1024 / BATCH contiguous bytes each.
   constexpr int BATCH = 16 / EPV;
-  static_assert(CACHE % BATCH == 0, "cached rounds must split into whole batches");
   __shared__ __attribute__((aligned(16))) uint8_t strip[THREADS * ROWS / 64][1024];
   uint8_t* mine = strip[threadIdx.x >> 6];
   const int lane = tid & 63;
   constexpr int LPR = 64 / BATCH;  // lanes that store one round's bytes of this wave
 #pragma unroll
   for (int i0 = 0; i0 < CACHE; i0 += BATCH) {
-    if (THREADS * (i0 + BATCH) <= K / EPV) {  // uniform: every lane of every wave has all BATCH rounds
+    if (i0 + BATCH <= CACHE && THREADS * (i0 + BATCH) <= K / EPV) {  // uniform: every lane of every wave has all BATCH rounds
 #pragma unroll
       for (int b = 0; b < BATCH; ++b) {
         uint32_t out[EPV / 4];
-        convert(cache[i0 + b], out);
+        convert(cache[min(i0 + b, CACHE - 1)], out);
         if (EPV == 4) *(uint32_t*)(mine + b * 256 + lane * 4) = out[0];
         else *(v2u*)(mine + b * 512 + lane * 8) = (v2u){out[0], out[EPV / 4 - 1]};
       }
@@ -3346,7 +3366,7 @@ __global__ __launch_bounds__(THREADS* ROWS) void quantize_rows_vec_kernel(const 
       *(Codes*)(qr + ((size_t)THREADS * (i0 + b) + (tid & ~63)) * EPV + piece * 16) = bytes;
     } else {
 #pragma unroll
-      for (int b = 0; b < BATCH; ++b) {
+      for (int b = 0; b < BATCH && i0 + b < CACHE; ++b) {
         const int c = tid + THREADS * (i0 + b);
         if (c < nchunks) convert_store(cache[i0 + b], c);
       }
@@ -3418,8 +3438,7 @@ __global__ __launch_bounds__(256) void quantize_blocks_kernel(const SrcT* x, uin
       if (r < M && c < K) amax = max_keep_nan(amax, fabsf(T::load(x + (long)r * ldx + c)));
     }
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) amax = max_keep_nan(amax, __shfl_xor(amax, o));
+  amax = wave_reduce(amax, [](float a, float b) { return max_keep_nan(a, b); });
   if ((tid & 63) == 0) wave_max[tid >> 6] = amax;
   __syncthreads();
   amax = max_keep_nan(max_keep_nan(wave_max[0], wave_max[1]), max_keep_nan(wave_max[2], wave_max[3]));
@@ -3499,8 +3518,7 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
 
   // sums (or maxima) of one value per lane over the row's lanes; every lane gets the result
   auto block_reduce = [&](int set, float v, auto op) -> float {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = op(v, __shfl_xor(v, o));
+    v = wave_reduce(v, op);
     if (THREADS == 64) return v;
     if ((tid & 63) == 0) wave_part[set][tid >> 6] = v;
     __syncthreads();
@@ -3602,15 +3620,14 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
   __shared__ __attribute__((aligned(16))) uint8_t strip[THREADS * ROWS / 64][1024];
   uint8_t* mine = strip[threadIdx.x >> 6];
   const int lane = tid & 63;
-  static_assert(CACHE % 2 == 0, "cached rounds are stored in pairs");
 #pragma unroll
   for (int i0 = 0; i0 < CACHE; i0 += 2) {
-    if (finite_row && THREADS * (i0 + 2) <= nchunks) {  // uniform: every lane of every wave has both rounds
+    if (i0 + 2 <= CACHE && finite_row && THREADS * (i0 + 2) <= nchunks) {  // uniform: every lane of every wave has both rounds
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         float f[EPV];
 #pragma unroll
-        for (int e = 0; e < EPV; ++e) f[e] = fminf(fmaxf(vals[i0 + b][e] * scale, -448.0f), 448.0f);
+        for (int e = 0; e < EPV; ++e) f[e] = fminf(fmaxf(vals[min(i0 + b, CACHE - 1)][e] * scale, -448.0f), 448.0f);
         int lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
         lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], lo, true);
         int hi = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], 0, false);
@@ -3622,7 +3639,7 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
       *(v4i*)(qr + ((size_t)THREADS * (i0 + b) + (tid & ~63)) * EPV + piece * 16) = bytes;
     } else {
 #pragma unroll
-      for (int b = 0; b < 2; ++b) {
+      for (int b = 0; b < 2 && i0 + b < CACHE; ++b) {
         const int c = tid + THREADS * (i0 + b);
         if (c < nchunks) convert_store(vals[i0 + b], c);
       }
@@ -4999,9 +5016,78 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
 namespace {
 constexpr int kWaveRows = 4;
 
+// How a row's chunks of 16 bytes are dealt out by the quantiser and the fused front ends (rows that start 16-byte aligned): `lanes` of them,
+// `chunks` rounds each that stay in registers; 64 lanes are a wave, kWaveRows rows a workgroup. Any form takes any row (what the registers don't
+// hold is read again), so the rule is about speed alone:
+//  - no round is idle if it can be helped, for it loads and computes like any other: rows just above a power of two had up to half of them
+//    idle (RMSNorm 8192x8960 56.5 us as 4 rounds of 512, 42.8 as 5 of 256; SiLU-mul 2048x19904 41.4 and 34.7; f32 8192x9472 72.7 and 60.6);
+//  - up to one row a CU, what counts is the chain of a single row, and one round of as many lanes as that takes is the shortest (RMSNorm
+//    32x8192 4.64 us as 4 rounds of 256, 3.50 as one of 1024; SiLU-mul 32x4096 4.89 as 8 of 64, 2.69 as one of 512);
+//  - with more rows, fewer lanes with more rounds: 256x4 against 1024x1 is 36.3 and 48.4 us on 8192x8192, waves of 4 rounds against 256x1
+//    12.9 and 14.1 on 8192x2048, but 6.2 and 5.6 on 2048x2048.
+// Measured on 21 row lengths from 512 to 28672 with 1 to 8192 rows, every form whose rounds hold the row.
+enum RowSource { kRowF32, kRowBf16, kRowRmsNorm, kRowSiluMul };
+struct RowForm {
+  int lanes, chunks;
+};
+constexpr bool row_form_exists(RowSource source, int lanes, int chunks) {
+  if (lanes == 64) return chunks <= 4 || (source == kRowF32 && (chunks == 6 || chunks == 8));
+  if (lanes == 256) return chunks <= 5;
+  if (lanes == 512) return chunks <= 8 && (chunks < 7 || source != kRowSiluMul) && (chunks != 7 || source != kRowRmsNorm);
+  return chunks <= 4 || chunks == 8 || (source == kRowF32 && chunks <= 7);
+}
+constexpr RowForm row_form_of(RowSource source, int64_t R, int64_t chunks) {
+  if (chunks > 4096) {  // (bf16 rows hold half the values in as many registers as f32 ones: more rounds than 4 halve their rate)
+    if (source == kRowBf16) return {1024, 4};
+    if (source == kRowF32 && chunks <= 7168) return {1024, (int)((chunks + 1023) / 1024)};
+    return {1024, 8};
+  }
+  if (chunks <= 64) return {64, 1};
+  if (R <= kNumCu) {
+    if (chunks <= 256) return {256, 1};
+    if (chunks <= 512) return {512, 1};
+    return {1024, (int)((chunks + 1023) / 1024)};
+  }
+  const bool many = R > 2048;
+  if (chunks <= 192) return {64, chunks <= 128 ? 2 : 3};
+  if (chunks <= 256) return many ? RowForm{64, 4} : RowForm{256, 1};
+  if (chunks <= 512) return many && source == kRowF32 ? RowForm{64, chunks <= 384 ? 6 : 8} : RowForm{256, 2};
+  if (chunks <= 768) return {256, 3};
+  if (chunks <= 1024) return many ? RowForm{256, 4} : RowForm{512, 2};
+  if (chunks <= 1280 && many) return {256, 5};
+  if (chunks <= 3072) return {512, (int)((chunks + 511) / 512)};
+  if (source == kRowSiluMul) return {1024, 4};
+  return {512, chunks <= 3584 && source != kRowRmsNorm ? 7 : 8};
+}
+// (a launch holds fewer than 2^32 lanes: beyond, 256 of them read the rest of a row twice)
+constexpr RowForm row_form(RowSource source, int64_t R, int64_t chunks) {
+  const RowForm f = row_form_of(source, R, chunks);
+  return f.lanes > 256 && !grid_fits(R, f.lanes) ? RowForm{256, 5} : f;
+}
+static_assert(row_form(kRowBf16, 8388607, 2000).lanes == 512 && row_form(kRowBf16, 8388608, 2000).lanes == 256, "512 lanes a row reach 2^32 at 8388608 rows");
+
+// Calls launch(lanes, chunks), as integral constants, for the form.
+template <RowSource SOURCE, int LANES = 64, int CHUNKS = 1, typename Launch>
+void with_row_form(RowForm f, Launch&& launch) {
+  if constexpr (row_form_exists(SOURCE, LANES, CHUNKS)) {
+    if (f.lanes == LANES && f.chunks == CHUNKS) return launch(std::integral_constant<int, LANES>{}, std::integral_constant<int, CHUNKS>{});
+  }
+  if constexpr (CHUNKS < 8) with_row_form<SOURCE, LANES, CHUNKS + 1>(f, launch);
+  else if constexpr (LANES < 1024) with_row_form<SOURCE, LANES == 64 ? 256 : LANES * 2, 1>(f, launch);
+}
+
 // (more rows than a launch of 1024 lanes each holds keep 256 lanes, which read the rest of a long row twice)
 constexpr bool quantize_any_long(int64_t R, int64_t chunks) { return chunks > 4 * 256 && grid_fits(R, 1024); }
 static_assert(quantize_any_long(4194303, 1025) && !quantize_any_long(8388608, 1025), "512 lanes a row reach 2^32 at 8388608 rows");
+
+template <RowSource SOURCE, typename SrcT>
+void launch_quantize_rows(const SrcT* x, uint8_t* xq, float* inv_scale, int64_t R, int64_t K, int64_t ldx, int64_t ldq, hipStream_t s) {
+  with_row_form<SOURCE>(row_form(SOURCE, R, K / VecTraits<SrcT>::EPV), [&](auto lanes, auto chunks) {
+    constexpr int LANES = decltype(lanes)::value, ROWS = LANES == 64 ? kWaveRows : 1;
+    hipLaunchKernelGGL((quantize_rows_vec_kernel<SrcT, decltype(chunks)::value, LANES, ROWS>), dim3((unsigned)((R + ROWS - 1) / ROWS)),
+                       dim3(LANES * ROWS), 0, s, x, xq, inv_scale, (int)K, (long)ldx, (long)ldq, (long)R);
+  });
+}
 
 // The quantiser on rows that do not start 16-byte aligned or do not hold whole 16-byte chunks: the vector kernel's
 // unaligned forms, by the same lines as the aligned ones (fewer of them: this is the rare case). The element-by-element
@@ -5030,8 +5116,10 @@ void launch_quantize_any(const SrcT* x, uint8_t* xq, float* inv_scale, int64_t R
     go(quantize_rows_vec_kernel<SrcT, 16 / epv, 64, kWaveRows, true>, (R + kWaveRows - 1) / kWaveRows, 64 * kWaveRows);
   } else if (chunks <= 8 * 64 && R > 2048) {
     go(quantize_rows_vec_kernel<SrcT, 8, 64, kWaveRows, true>, (R + kWaveRows - 1) / kWaveRows, 64 * kWaveRows);
-  } else if (!long_row) {
-    go(quantize_rows_vec_kernel<SrcT, 4, 256, 1, true>, R, 256);
+  } else if (!long_row) {  // (no idle rounds where that is had without more forms than these)
+    if (chunks <= 256) go(quantize_rows_vec_kernel<SrcT, 1, 256, 1, true>, R, 256);
+    else if (chunks <= 512) go(quantize_rows_vec_kernel<SrcT, 2, 256, 1, true>, R, 256);
+    else go(quantize_rows_vec_kernel<SrcT, 4, 256, 1, true>, R, 256);
   } else if (chunks <= 8 * 512) {
     go(quantize_rows_vec_kernel<SrcT, 8, 512, 1, true>, R, 512);
   } else {
@@ -5261,18 +5349,6 @@ int mi355x_fp8_blockwise_gemm_ws(const void* a, const void* b, const float* a_sc
   }
 }
 
-namespace {
-// Rows of at most 64 x 8 16-byte chunks are quantised by one wave each, kWaveRows rows per workgroup:
-// the number of chunks a lane keeps in registers (4 or 8), or 0 for longer rows. (Measured, bf16 rows,
-// workgroup per row -> wave per row: 16384 x 2048 quantiser 28.7 -> 19.9 us, RMSNorm form 40.8 -> 21.0,
-// SiLU-mul form 49.0 -> 27.9; 65536 x 512 75 -> 27, 132 -> 29, 170 -> 32; eight rows per workgroup
-// instead of four changed nothing.)
-inline int row_chunks_per_lane(int64_t chunks) { return chunks <= 64 * 4 ? 4 : chunks <= 64 * 8 ? 8 : 0; }
-// (bf16 rows of up to 1024 elements: two rounds per lane instead of four, of which at least two would be idle)
-inline int bf16_row_chunks_per_lane(int64_t chunks) { return chunks <= 64 * 2 ? 2 : row_chunks_per_lane(chunks); }
-
-}  // namespace
-
 int mi355x_fp8_rowwise_quantize(const void* x, int src_type, void* xq, float* inv_scale, int64_t R,
                                 int64_t K, int64_t ldx, int64_t ldq, void* stream) {
   if (!x || !xq || !inv_scale) return fail(MI355X_FP8_EINVAL, "null pointer");
@@ -5285,44 +5361,10 @@ int mi355x_fp8_rowwise_quantize(const void* x, int src_type, void* xq, float* in
   const int epv = 16 / esz;
   const bool vec = (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (ldx * esz) % 16 == 0 && K % epv == 0 &&
                    (reinterpret_cast<uintptr_t>(xq) & 15) == 0 && ldq % 16 == 0;
-  const bool long_row = K / epv > 8 * 256;  // more chunks than 256 lanes keep in registers
-  const bool short_row = K / epv <= 4 * 256;  // (bf16 source: half the registers, more workgroups per CU)
-  const int wave_cache = row_chunks_per_lane(K / epv);  // > 0: a wave per row, that many chunks per lane
-  const unsigned wave_grid = (unsigned)((R + kWaveRows - 1) / kWaveRows);
   if (vec && src_type == MI355X_FP8_SRC_F32) {
-    if (wave_cache) {
-      auto kern = wave_cache == 4 ? quantize_rows_vec_kernel<float, 4, 64, kWaveRows> : quantize_rows_vec_kernel<float, 8, 64, kWaveRows>;
-      hipLaunchKernelGGL(kern, dim3(wave_grid), dim3(64 * kWaveRows), 0, s, (const float*)x, (uint8_t*)xq, inv_scale, (int)K,
-                         (long)ldx, (long)ldq, (long)R);
-    } else {
-      auto kern = long_row ? quantize_rows_vec_kernel<float, 8, 1024> : quantize_rows_vec_kernel<float, 8, 256>;
-      hipLaunchKernelGGL(kern, dim3((unsigned)R), dim3(long_row ? 1024 : 256), 0, s, (const float*)x,
-                         (uint8_t*)xq, inv_scale, (int)K, (long)ldx, (long)ldq, (long)R);
-    }
+    launch_quantize_rows<kRowF32>((const float*)x, (uint8_t*)xq, inv_scale, R, K, ldx, ldq, s);
   } else if (vec && src_type == MI355X_FP8_SRC_BF16) {
-    // (A wave per row is the form for many rows. With few, a row spread over a workgroup's 256 lanes is back sooner:
-    // 16 x 4096 3.3 us against 5.2, 2048 x 4096 9.2 against 10.2, 512 x 2048 3.3 against 3.9; from 8192 rows up the wave
-    // form is ahead, 16384 x 4096 37.4 against 40.1.)
-    const int lanes_cache = bf16_row_chunks_per_lane(K / epv);
-    const bool few_rows = (lanes_cache == 8 && R <= 2048) || (lanes_cache == 4 && R <= 512);
-    if (const int wave_cache = few_rows ? 0 : lanes_cache) {
-      auto kern = wave_cache == 2   ? quantize_rows_vec_kernel<uint16_t, 2, 64, kWaveRows>
-                  : wave_cache == 4 ? quantize_rows_vec_kernel<uint16_t, 4, 64, kWaveRows>
-                                    : quantize_rows_vec_kernel<uint16_t, 8, 64, kWaveRows>;
-      hipLaunchKernelGGL(kern, dim3(wave_grid), dim3(64 * kWaveRows), 0, s, (const uint16_t*)x, (uint8_t*)xq, inv_scale, (int)K,
-                         (long)ldx, (long)ldq, (long)R);
-    } else {
-      // (Long rows: 512 lanes with 8 chunks each up to 4096 chunks, 1024 lanes with 4 beyond. 1024 lanes with 8 chunks
-      // each, the f32 form, reach half the rate here: 16384 x 28672 397.6 us against 235.4, 4096 x 28672 104.6 against 64.0;
-      // 16384 x 53248 600 against 469.)
-      const bool very_long_row = K / epv > 8 * 512;
-      auto kern = very_long_row ? quantize_rows_vec_kernel<uint16_t, 4, 1024>
-                  : long_row    ? quantize_rows_vec_kernel<uint16_t, 8, 512>
-                  : short_row   ? quantize_rows_vec_kernel<uint16_t, 4, 256>
-                                : quantize_rows_vec_kernel<uint16_t, 8, 256>;
-      hipLaunchKernelGGL(kern, dim3((unsigned)R), dim3(very_long_row ? 1024 : long_row ? 512 : 256), 0, s,
-                         (const uint16_t*)x, (uint8_t*)xq, inv_scale, (int)K, (long)ldx, (long)ldq, (long)R);
-    }
+    launch_quantize_rows<kRowBf16>((const uint16_t*)x, (uint8_t*)xq, inv_scale, R, K, ldx, ldq, s);
   } else if (src_type == MI355X_FP8_SRC_F32) {
     launch_quantize_any<float>((const float*)x, (uint8_t*)xq, inv_scale, R, K, ldx, ldq, s);
   } else if (src_type == MI355X_FP8_SRC_BF16) {
@@ -5379,45 +5421,17 @@ int launch_fused_quant(int op, const void* x1, const void* x2, float eps, void* 
     return fail(MI355X_FP8_ENOTSUP, "rows must hold whole 16-byte chunks and start 16-byte aligned");
   if (!(eps >= 0.0f)) return fail(MI355X_FP8_EINVAL, "eps must be >= 0");
   hipStream_t s = (hipStream_t)stream;
-  // chunks a lane keeps in registers: 4 for rows up to 8192 elements (half the registers, twice the
-  // workgroups per CU), 8 up to 16384, beyond that 1024 lanes per row
-  const int64_t chunks = K / 8;
-  const bool long_row = chunks > 8 * 256;
-  const bool short_row = chunks <= 4 * 256;
-  // > 0: a wave per row, that many chunks per lane (RMSNorm with eight chunks and their weights per lane
-  // measured behind the workgroup-per-row form: 50.1 against 47.8 us on 16384 x 4096)
-  int wave_cache = bf16_row_chunks_per_lane(chunks);
-  if (op == kFusedRmsNorm && wave_cache == 8) wave_cache = 0;
-  const dim3 grid(wave_cache ? (unsigned)((R + kWaveRows - 1) / kWaveRows) : (unsigned)R);
-  // (Long rows up to 32768 elements: 512 lanes with 8 chunks each. With 1024 lanes they reach two thirds of that rate:
-  // SiLU-mul 4096 x 28672 146.6 -> 100.6 us, 1024 x 28672 44.5 -> 29.5; RMSNorm 4096 x 28672 115.8 -> 83.8. Beyond,
-  // 1024 lanes: 4096 x 53248 199.5 us against 218.)
-  const bool mid_row = long_row && chunks <= 8 * 512;
-  // (Rows of 8193 to 16384 elements: 512 lanes with 4 chunks each instead of 256 with 8. RMSNorm 8192 x 16384 96.0 ->
-  // 78.6 us, 32768 x 16384 370 -> 302, 8192 x 11008 85.1 -> 67.1; SiLU-mul 8192 x 11008 80.6 -> 79.6, 8192 x 16384
-  // 109.1 -> 107.6.)
-  const bool half_row = !wave_cache && !long_row && !short_row;
-  const dim3 block(wave_cache ? 64 * kWaveRows : mid_row || half_row ? 512 : long_row ? 1024 : 256);
-  const uint16_t* a = (const uint16_t*)x1;
-  const uint16_t* b = (const uint16_t*)x2;
-  if (op == kFusedRmsNorm) {
-    auto kern = wave_cache == 2 ? fused_rowwise_quant_kernel<kFusedRmsNorm, 2, 64, kWaveRows>
-                : wave_cache == 4 ? fused_rowwise_quant_kernel<kFusedRmsNorm, 4, 64, kWaveRows>
-                : wave_cache  ? fused_rowwise_quant_kernel<kFusedRmsNorm, 8, 64, kWaveRows>
-                : mid_row     ? fused_rowwise_quant_kernel<kFusedRmsNorm, 8, 512>
-                : long_row    ? fused_rowwise_quant_kernel<kFusedRmsNorm, 8, 1024>
-                : chunks <= 2 * 256 ? fused_rowwise_quant_kernel<kFusedRmsNorm, 2, 256>  // (no idle rounds: 16384 x 4096 47.8 -> 35.5 us)
-                : short_row   ? fused_rowwise_quant_kernel<kFusedRmsNorm, 4, 256> : fused_rowwise_quant_kernel<kFusedRmsNorm, 4, 512>;
-    hipLaunchKernelGGL(kern, grid, block, 0, s, a, b, eps, (uint8_t*)xq, inv_scale, (int)K, (long)ld1, (long)ld2, (long)ldq, (long)R);
-  } else {
-    auto kern = wave_cache == 2 ? fused_rowwise_quant_kernel<kFusedSiluMul, 2, 64, kWaveRows>
-                : wave_cache == 4 ? fused_rowwise_quant_kernel<kFusedSiluMul, 4, 64, kWaveRows>
-                : wave_cache  ? fused_rowwise_quant_kernel<kFusedSiluMul, 8, 64, kWaveRows>
-                : mid_row     ? fused_rowwise_quant_kernel<kFusedSiluMul, 8, 512>
-                : long_row    ? fused_rowwise_quant_kernel<kFusedSiluMul, 8, 1024>
-                : short_row   ? fused_rowwise_quant_kernel<kFusedSiluMul, 4, 256> : fused_rowwise_quant_kernel<kFusedSiluMul, 4, 512>;
-    hipLaunchKernelGGL(kern, grid, block, 0, s, a, b, eps, (uint8_t*)xq, inv_scale, (int)K, (long)ld1, (long)ld2, (long)ldq, (long)R);
-  }
+  auto launch = [&](auto op_tag, RowForm form) {
+    constexpr int OP = decltype(op_tag)::value;
+    with_row_form<OP == kFusedRmsNorm ? kRowRmsNorm : kRowSiluMul>(form, [&](auto lanes, auto chunks) {
+      constexpr int LANES = decltype(lanes)::value, ROWS = LANES == 64 ? kWaveRows : 1;
+      hipLaunchKernelGGL((fused_rowwise_quant_kernel<OP, decltype(chunks)::value, LANES, ROWS>), dim3((unsigned)((R + ROWS - 1) / ROWS)),
+                         dim3(LANES * ROWS), 0, s, (const uint16_t*)x1, (const uint16_t*)x2, eps, (uint8_t*)xq, inv_scale, (int)K,
+                         (long)ld1, (long)ld2, (long)ldq, (long)R);
+    });
+  };
+  if (op == kFusedRmsNorm) launch(std::integral_constant<int, kFusedRmsNorm>{}, row_form(kRowRmsNorm, R, K / 8));
+  else launch(std::integral_constant<int, kFusedSiluMul>{}, row_form(kRowSiluMul, R, K / 8));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(MI355X_FP8_ELAUNCH, "fused quantise kernel launch: %s", hipGetErrorString(e));
   return MI355X_FP8_OK;
