@@ -98,7 +98,7 @@ struct LdsKernel {
   const void* kernel;
   size_t lds_bytes;
 };
-constexpr int kMaxLdsKernels = 256;
+constexpr int kMaxLdsKernels = 512;
 extern LdsKernel lds_kernels[kMaxLdsKernels];
 extern int num_lds_kernels;
 extern bool lds_table_overflow;
@@ -2918,8 +2918,12 @@ constexpr size_t pair_lds_bytes(int SPW) {
 // time hangs on how fast a wave gets its burst of loads out, and the few vector instructions either adds
 // in front of the loads measured 0.3 and 0.1 us at M=16, N=K=8192.
 // OFF_LINES: rows of B off the 128-byte lines, without the streaming policy (16x8192x4112 12.2 -> 11.0 us, 16x4096x4112 7.1 -> 5.8).
-template <int SPW, bool VEC, bool KTAIL, bool HAS_BIAS, bool OFF_LINES = false>
+// BLOCK: the block-scaled product. A step's product is multiplied by its a_scale[0][kb] * b_scale[nb][kb] before it is added up; a wave's
+// factors, one for each of its steps of either tile, lie in its first lanes (16x8192x8192 15.4 us with narrow tiles, 14.1 here, 16x8192x8176 18.9 and
+// 16.7, 16x8192x4096 10.9 and 9.2, with one tile a workgroup 9.6).
+template <int SPW, bool VEC, bool KTAIL, bool HAS_BIAS, bool OFF_LINES = false, bool BLOCK = false>
 __global__ __launch_bounds__(kPersistWaves * 64) void gemm_skinny_pair_kernel(GemmParams p) {
+  static_assert(!BLOCK || !HAS_BIAS, "the block-scaled product has no bias");
   constexpr int WAVES = kPersistWaves;
   constexpr int STEPS = WAVES * SPW;
   constexpr int A_LDS = SPW - 1;  // steps of A per wave that live in LDS
@@ -3008,7 +3012,23 @@ __global__ __launch_bounds__(kPersistWaves * 64) void gemm_skinny_pair_kernel(Ge
   const int fin_n = (tile0 + min(wave, count - 1)) * 16 + 4 * g4;
   float fin_sa = 0.f, sb_raw[4] = {0.f, 0.f, 0.f, 0.f};
   uint16_t bias_raw[4] = {0, 0, 0, 0};
-  if constexpr (VEC) {
+  if constexpr (BLOCK) {
+    // lane t * SPW + i: step i of tile t (a step past K has no block: its factors are outside both vectors and read as zeros)
+    const uint32_t blocks = (uint32_t)(p.K + kStepK - 1) / kStepK;
+    uint32_t kb = (uint32_t)(base_step + WAVES * (lane % SPW));
+    if (kb >= STEPS) kb -= STEPS;
+    const uint32_t nb = (uint32_t)(tile0 + min(lane / SPW, 1)) / (kStepK / 16);
+    const bool inside = kb < blocks && nb < ((uint32_t)p.N + kStepK - 1) / kStepK;
+#if defined(__HIP_DEVICE_COMPILE__)
+    const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.a_scale), 0, (int)(blocks * 4u), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rsb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(p.b_scale), 0, (int)(((uint32_t)p.N + kStepK - 1) / kStepK * blocks * 4u), 0x00020000);
+    fin_sa = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsa, (int)(inside ? kb * 4u : kOutside), 0, 0));
+    sb_raw[0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsb, (int)(inside ? (nb * blocks + kb) * 4u : kOutside), 0, 0));
+#endif
+    __builtin_amdgcn_sched_barrier(0);
+    wait_loads<2>();
+  } else if constexpr (VEC) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.a_scale), 0, p.M * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsb = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p.b_scale), 0, p.N * 4, 0x00020000);
@@ -3050,14 +3070,21 @@ __global__ __launch_bounds__(kPersistWaves * 64) void gemm_skinny_pair_kernel(Ge
       const v4i ahi = *(const v4i*)(a_mine + i * 2048 + rd1);
       fa = (v8i){alo[0], alo[1], alo[2], alo[3], ahi[0], ahi[1], ahi[2], ahi[3]};
     }
-    acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb, fa, acc, 0, 0, 0, 0, 0, 0);
+    if constexpr (BLOCK) {
+      const v4f product = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb, fa, (v4f){0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+      const float factor = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(fin_sa * sb_raw[0]), t * SPW + i));
+#pragma unroll
+      for (int x = 0; x < 4; ++x) acc[x] = __builtin_fmaf(product[x], factor, acc[x]);
+    } else {
+      acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb, fa, acc, 0, 0, 0, 0, 0, 0);
+    }
   };
   // tile 0: the rest of its loads in one burst, the first step of tile 1 behind them
 #pragma unroll
   for (int i = 1; i < SPW; ++i) fetch(0, i);
   fetch(1, 0);
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (!VEC) {  // (element by element: a count the compiler may change, so behind the burst)
+  if constexpr (!VEC && !BLOCK) {  // (element by element: a count the compiler may change, so behind the burst)
     fin_sa = p.a_scale[min(r16, p.M - 1)];
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
@@ -3083,7 +3110,9 @@ __global__ __launch_bounds__(kPersistWaves * 64) void gemm_skinny_pair_kernel(Ge
         float r[4];
 #pragma unroll
         for (int x = 0; x < 4; ++x)
-          r[x] = HAS_BIAS ? __builtin_fmaf(sum[x] * fin_sa, sb_raw[x], bf16_to_f32(bias_raw[x])) : sum[x] * fin_sa * sb_raw[x];
+          r[x] = BLOCK      ? sum[x]
+                 : HAS_BIAS ? __builtin_fmaf(sum[x] * fin_sa, sb_raw[x], bf16_to_f32(bias_raw[x]))
+                            : sum[x] * fin_sa * sb_raw[x];
         const uint32_t lo = pack_out_x2(r[0], r[1], p.out_f16), hi = pack_out_x2(r[2], r[3], p.out_f16);
         uint16_t* dst = p.c + (size_t)r16 * p.ldc + (tile0 + j) * 16 + 4 * g4;
         if (VEC) {
@@ -4382,7 +4411,8 @@ enum BlockForm {
   kBlockNarrow = MI355X_FP8_BLOCK_NARROW,
   kBlockSmall = MI355X_FP8_BLOCK_TILES_128,
   kBlockSmallStream = MI355X_FP8_BLOCK_TILES_128_STREAM,
-  kBlockLarge = MI355X_FP8_BLOCK_TILES_256
+  kBlockLarge = MI355X_FP8_BLOCK_TILES_256,
+  kBlockResident  // the pair kernel: the library's choice only, which is ONE_TILE to callers
 };
 // (One 16-row tile a workgroup, many of them on short rows: what bounds it is the rate at which they come and go, which the
 // row-wise estimate has too high there. us a workgroup beyond the first 256: 16x24576x256 2.9e-3, 16x24576x384 3.3e-3,
@@ -4426,6 +4456,7 @@ inline BlockForm block_form(int64_t M, int64_t N, int64_t K, bool off_lines, flo
   }
   if (M <= kSkinnyMaxM) weigh(kBlockOneTile, block_one_tile_cost_us(M, N, K, one_tile_off));
   if (narrow_fits(M, N, K)) weigh(kBlockNarrow, narrow_off * narrow_cost_us(M, N, K));
+  if (pair_skinny_fits(M, N, K)) weigh(kBlockResident, one_tile_off * pair_cost_us(M, N, K));
   if (cost_us) *cost_us = cost;
   return best;
 }
@@ -4666,14 +4697,14 @@ int launch_skinny_persistent(const GemmParams& p, hipStream_t stream) {
   return MI355X_FP8_OK;
 }
 
-template <int SPW, bool VEC, bool KTAIL, bool HAS_BIAS, bool OFF_LINES = false>
+template <int SPW, bool VEC, bool KTAIL, bool HAS_BIAS, bool OFF_LINES = false, bool BLOCK = false>
 int launch_skinny_pair(const GemmParams& p, hipStream_t stream) {
   if constexpr (KTAIL && !OFF_LINES) {  // (whole rounds of steps are off the lines with padded rows only)
-    if (off_lines(p, kHalfLine) && !asked_for_at_once(p)) return launch_skinny_pair<SPW, VEC, KTAIL, HAS_BIAS, true>(p, stream);
+    if (off_lines(p, kHalfLine) && !asked_for_at_once(p)) return launch_skinny_pair<SPW, VEC, KTAIL, HAS_BIAS, true, BLOCK>(p, stream);
   }
   constexpr size_t lds_bytes = pair_lds_bytes(SPW);
   static_assert(lds_bytes <= 160 * 1024, "A's steps, the transpose buffers and the partial results must fit the LDS");
-  constexpr auto kern = gemm_skinny_pair_kernel<SPW, VEC, KTAIL, HAS_BIAS, OFF_LINES>;
+  constexpr auto kern = gemm_skinny_pair_kernel<SPW, VEC, KTAIL, HAS_BIAS, OFF_LINES, BLOCK>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   if (const int st = ready_device()) return st;
   const long ntiles = p.N / 16;
@@ -4687,15 +4718,15 @@ int launch_skinny_pair(const GemmParams& p, hipStream_t stream) {
   return MI355X_FP8_OK;
 }
 
-template <bool VEC, bool KTAIL, bool HAS_BIAS>
+template <bool VEC, bool KTAIL, bool HAS_BIAS, bool BLOCK = false>
 int launch_skinny_pair_steps(const GemmParams& p, hipStream_t s) {
   const int steps = (p.K + kStepK - 1) / kStepK;
   const int spw = (steps + kPersistWaves - 1) / kPersistWaves;
   switch (spw) {
-    case 1: return launch_skinny_pair<1, VEC, KTAIL, HAS_BIAS>(p, s);
-    case 2: return launch_skinny_pair<2, VEC, KTAIL, HAS_BIAS>(p, s);
-    case 3: return launch_skinny_pair<3, VEC, KTAIL, HAS_BIAS>(p, s);
-    default: return launch_skinny_pair<4, VEC, KTAIL, HAS_BIAS>(p, s);
+    case 1: return launch_skinny_pair<1, VEC, KTAIL, HAS_BIAS, false, BLOCK>(p, s);
+    case 2: return launch_skinny_pair<2, VEC, KTAIL, HAS_BIAS, false, BLOCK>(p, s);
+    case 3: return launch_skinny_pair<3, VEC, KTAIL, HAS_BIAS, false, BLOCK>(p, s);
+    default: return launch_skinny_pair<4, VEC, KTAIL, HAS_BIAS, false, BLOCK>(p, s);
   }
 }
 template <bool VEC>
@@ -4703,6 +4734,13 @@ int launch_skinny_pair_form(const GemmParams& p, hipStream_t s) {
   const bool ktail = p.K % (kPersistWaves * kStepK) != 0;
   if (p.bias) return ktail ? launch_skinny_pair_steps<VEC, true, true>(p, s) : launch_skinny_pair_steps<VEC, false, true>(p, s);
   return ktail ? launch_skinny_pair_steps<VEC, true, false>(p, s) : launch_skinny_pair_steps<VEC, false, false>(p, s);
+}
+
+int launch_skinny_pair_block(const GemmParams& p, hipStream_t s) {
+  const bool vec = (reinterpret_cast<uintptr_t>(p.c) & 7) == 0 && (p.ldc & 3) == 0;  // (8-byte stores of C)
+  const bool ktail = p.K % (kPersistWaves * kStepK) != 0;
+  if (vec) return ktail ? launch_skinny_pair_steps<true, true, false, true>(p, s) : launch_skinny_pair_steps<true, false, false, true>(p, s);
+  return ktail ? launch_skinny_pair_steps<false, true, false, true>(p, s) : launch_skinny_pair_steps<false, false, false, true>(p, s);
 }
 
 template <bool VEC>
@@ -5238,7 +5276,9 @@ int mi355x_fp8_blockwise_form(int64_t M, int64_t N, int64_t K) {
   if (st == MI355X_FP8_OK) st = check_fast_shape(K);
   if (st == MI355X_FP8_OK && K > 256 * kStepK)
     st = fail(MI355X_FP8_ENOTSUP, "block-scaled form handles K <= %d (got %lld)", 256 * kStepK, (long long)K);
-  return st != MI355X_FP8_OK ? st : block_form(M, N, K, K % kStepK != 0);
+  if (st != MI355X_FP8_OK) return st;
+  const BlockForm form = block_form(M, N, K, K % kStepK != 0);
+  return form == kBlockResident ? kBlockOneTile : form;
 }
 
 int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale, const float* b_scale,
@@ -5315,10 +5355,16 @@ int mi355x_fp8_blockwise_gemm_ws(const void* a, const void* b, const float* a_sc
       p.partial = (float*)workspace;
     }
     form = plan.form;
+  } else if (form > kBlockLarge) {
+    return fail(MI355X_FP8_EINVAL, "unknown block-scaled form %d", form);
   } else if ((form == kBlockOneTile && M > kSkinnyMaxM) || (form == kBlockNarrow && !narrow_fits(M, N, K)))
     return fail(MI355X_FP8_ENOTSUP, "block-scaled form %d does not take %lldx%lld", form, (long long)M, (long long)N);
   switch (form) {
     case kBlockNarrow: return launch_narrow_for<true>(p, s);
+    case kBlockResident:
+      // (the pair kernel addresses a workgroup's rows of B with 32-bit offsets below 2^31)
+      if (ldb * 32 <= (int64_t)INT32_MAX) return launch_skinny_pair_block(p, s);
+      [[fallthrough]];
     case kBlockOneTile:
       if (M <= 16) return launch_skinny<1, 1, 4, 8, false, true>(p, s);
       if (M <= 32) return launch_skinny<2, 1, 2, 8, false, true>(p, s);
