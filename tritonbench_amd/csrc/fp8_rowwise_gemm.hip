@@ -453,8 +453,14 @@ constexpr int tiled_waves_per_simd(int BM, int BN, int waves, bool blockscale, i
 // OFF_LINES: a STREAM_B launch whose rows of B are off the 128-byte lines keeps the rotated walk but not the policy, with which the
 // line that two steps of a row share would come from memory twice: 119x55346x4112 73.9 -> 62.8 us, 32x57344x4112 68.5 -> 50.2,
 // 128x28672x8256 68.9 -> 63.7, 256x28672x8256 82.0 -> 78.9 (without the rotation 63.6, 51.0, 70.6 and 108).
+// LINES: rows off the 128-byte lines (their base or pitch no multiple of 128) are fetched in whole lines all the same. A row's windows start
+// at the line that its first byte lies in, so its chunks sit up to seven places further back than its neighbour's: chunk c of step g is
+// chunk c + shift of window g, or of window g + 1, whatever of the next row or of the one before lies in a window is never read, and an item
+// has one window more than steps. Eight rows on, the shift is the same (pitches are multiples of 16), so it is one number a lane for
+// the loads and one for the operand reads. For launches of at most one item a workgroup (a second one would start in another place of the
+// ring). From L2 a CU takes in 123 bytes/ns in whole lines and 83 in 128-byte pieces 16 bytes off them.
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool KTAIL, int EPI, bool GROUPED = false, bool BLOCKSCALE = false,
-          int DIST = kDefaultDist, bool STREAM_B = false, bool CLEAR = false, bool OFF_LINES = false>
+          int DIST = kDefaultDist, bool STREAM_B = false, bool CLEAR = false, bool OFF_LINES = false, bool LINES = false>
 __global__ __launch_bounds__(WAVES_M* WAVES_N * 64)
 __attribute__((amdgpu_waves_per_eu(tiled_waves_per_simd(BM, BN, WAVES_M * WAVES_N, BLOCKSCALE, DIST),
                                    tiled_waves_per_simd(BM, BN, WAVES_M * WAVES_N, BLOCKSCALE, DIST))))
@@ -464,6 +470,7 @@ void gemm_tiled_kernel(GemmParams p) {
   static_assert(!GROUPED || EPI == kEpiPlain, "the grouped form has neither bias nor split-K");
   static_assert(!OFF_LINES || (STREAM_B && !GROUPED), "a variant of the streaming launches");
   static_assert(!CLEAR || GROUPED, "only the grouped form has rows past its groups'");
+  static_assert(!LINES || (KTAIL && DIST >= 3 && !GROUPED && !BLOCKSCALE && !STREAM_B), "a window more has to have landed; the walk over K starts at its beginning");
   static_assert(!BLOCKSCALE || (128 % (BM / WAVES_M) == 0 && 128 % (BN / WAVES_N) == 0 && EPI != kEpiBias && !GROUPED),
                 "a wave's tile must lie inside one 128x128 scale block: one factor per wave and step");
   constexpr bool HAS_BIAS = EPI == kEpiBias;
@@ -511,6 +518,22 @@ void gemm_tiled_kernel(GemmParams p) {
 #pragma unroll
     for (int j = 0; j < 2; ++j)
       rd_off[s][j] = l32 * kStepK + (((4 * half + 2 * s + j) ^ swz128(l32)) * kChunk);
+  // LINES: a row's shift in chunks, by its number modulo 8; the reads of either operand, and whether they are the next window's
+  auto row_shift = [](const uint8_t* base, long ld, int row) { return (int)(((uint32_t)reinterpret_cast<uintptr_t>(base) + (uint32_t)row * (uint32_t)ld) & 127u) / kChunk; };
+  int rd_off_a[2][2], rd_off_b[2][2];
+  bool rd_next_a[2][2], rd_next_b[2][2];
+  if constexpr (LINES) {
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int ca = 4 * half + 2 * s + j + row_shift(p.a, p.lda, l32 & 7), cb = 4 * half + 2 * s + j + row_shift(p.b, p.ldb, l32 & 7);
+        rd_off_a[s][j] = l32 * kStepK + (((ca & 7) ^ swz128(l32)) * kChunk);
+        rd_off_b[s][j] = l32 * kStepK + (((cb & 7) ^ swz128(l32)) * kChunk);
+        rd_next_a[s][j] = ca >= 8;
+        rd_next_b[s][j] = cb >= 8;
+      }
+  }
   const int a_rd_base = (wm * WTM) * kStepK;
   const int b_rd_base = LDS_B0 + (wn * WTN) * kStepK;
 
@@ -548,7 +571,7 @@ void gemm_tiled_kernel(GemmParams p) {
   auto split_end = [&](int sp) { return min((sp + 1) * p.steps_per_split, k_steps); };
   int total_steps = 0;
   for (int li = walk.slot; li < walk.chunk_len; li += walk.slots)
-    total_steps += split_end(item_split(li)) - split_begin(item_split(li));
+    total_steps += split_end(item_split(li)) - split_begin(item_split(li)) + (LINES ? 1 : 0);
 
   // item -> tile location. Plain form: grouped walk order over the tile grid. Grouped form:
   // the walker steps through m_sizes until it reaches the group that holds the tile.
@@ -603,7 +626,7 @@ void gemm_tiled_kernel(GemmParams p) {
   };
   auto start_cursor = [&](StepCursor& c, int li, const TileLoc& loc) {
     c.kt_begin = split_begin(item_split(li));
-    c.kt_end = split_end(item_split(li));
+    c.kt_end = split_end(item_split(li)) + (LINES ? 1 : 0);
     c.left = c.kt_end - c.kt_begin;
     c.kt = first_step(loc, c.kt_begin, c.left);
   };
@@ -623,17 +646,18 @@ void gemm_tiled_kernel(GemmParams p) {
     uint32_t wave_off, group_stride;  // 8*wave*ld and 8*NW*ld
   };
   constexpr int kRsrcFlags = 0x00020000;  // raw buffer, 32-bit data format: plain byte addressing with range check
+  constexpr uint32_t kLead = LINES ? 7 * kChunk : 0;  // (the most that a window starts in front of its row: offsets stay positive)
   auto make_src = [&](const uint8_t* base, int rows_valid, int rows_tile, long ld) -> OperandSrc {
     // (a tile always starts on a valid row, so rows_valid >= 1; clamping at zero as well would turn
     // the pair into a three-operand median, which exists as a vector instruction only and would
     // pull the descriptor out of the scalar registers)
-    const uint32_t extent = (uint32_t)min(rows_valid, rows_tile) * (uint32_t)ld;
+    const uint32_t extent = (uint32_t)min(rows_valid, rows_tile) * (uint32_t)ld + kLead;
     // Base and extent are the same for every lane; they are pinned to scalar registers because a
     // descriptor that the compiler takes for lane-dependent (the grouped form derives these from
     // sizes it loads, through a clamp that only exists as a vector instruction) makes every load a
     // loop over the distinct descriptors of the wave.
     OperandSrc o;
-    const uintptr_t b = reinterpret_cast<uintptr_t>(base);
+    const uintptr_t b = reinterpret_cast<uintptr_t>(base) - kLead;
     o.base = reinterpret_cast<const uint8_t*>(
         ((uintptr_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)) << 32) |
         (uintptr_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b));
@@ -644,16 +668,22 @@ void gemm_tiled_kernel(GemmParams p) {
   };
   // 24-bit multiplies (row < 8, leading dimension < 2^24 by the host's check)
   const uint32_t lane_chunk = (uint32_t)ld_chunk_off(wave);
-  const uint32_t a_lane = __umul24((uint32_t)ld_row, (uint32_t)p.lda) + lane_chunk;
-  const uint32_t b_lane = __umul24((uint32_t)ld_row, (uint32_t)p.ldb) + lane_chunk;
+  const int a_shift = LINES ? row_shift(p.a, p.lda, ld_row) : 0, b_shift = LINES ? row_shift(p.b, p.ldb, ld_row) : 0;
+  const uint32_t a_lane = __umul24((uint32_t)ld_row, (uint32_t)p.lda) + lane_chunk + kLead - (uint32_t)(a_shift * kChunk);
+  const uint32_t b_lane = __umul24((uint32_t)ld_row, (uint32_t)p.ldb) + lane_chunk + kLead - (uint32_t)(b_shift * kChunk);
   // K tail (KTAIL kernels only): in the partial last step, lanes whose chunk lies at or past K
   // must fetch zeros (whatever follows a row in memory could decode to NaN): their lane part is
   // pushed past every extent for that step. A lane's logical chunk is the same for all its
   // groups.
   const bool tail_chunk_ok = ((ld_pc ^ swz128(wave * 8 + ld_row)) * kChunk) < k_tail;
   constexpr uint32_t kPastExtent = 0x80000000u;  // extents and scalar parts stay below 2^31
-  const uint32_t a_lane_tail = tail_chunk_ok ? a_lane : kPastExtent;
-  const uint32_t b_lane_tail = tail_chunk_ok ? b_lane : kPastExtent;
+  // LINES: the lane's chunk of window w is chunk 8w + c - shift of its row, which a window at either end need not have
+  const int chunk_c = (int)lane_chunk / kChunk, chunks_left = k_tail / kChunk;  // of the row, past its whole steps
+  const uint32_t a_lane_tail = (LINES ? chunk_c - a_shift < chunks_left : tail_chunk_ok) ? a_lane : kPastExtent;
+  const uint32_t b_lane_tail = (LINES ? chunk_c - b_shift < chunks_left : tail_chunk_ok) ? b_lane : kPastExtent;
+  const uint32_t a_lane_end = 8 + chunk_c - a_shift < chunks_left ? a_lane : kPastExtent;
+  const uint32_t b_lane_end = 8 + chunk_c - b_shift < chunks_left ? b_lane : kPastExtent;
+  const uint32_t a_lane_head = chunk_c >= a_shift ? a_lane : kPastExtent, b_lane_head = chunk_c >= b_shift ? b_lane : kPastExtent;
   OperandSrc a_src = {nullptr, 0, 0, 0}, b_src = {nullptr, 0, 0, 0};
   auto setup_a = [&](int li) {
     const TileLoc loc = locate(walk_a, li);
@@ -676,8 +706,14 @@ void gemm_tiled_kernel(GemmParams p) {
     load_chunk_to_lds<decltype(stream_tag)::value>(rsrc, sbase + (wave + NW * i) * 1024, lane_off,
                                                    step_off + (uint32_t)i * src.group_stride);
   };
-  auto lane_part = [&](uint32_t whole, uint32_t tail, int kt) -> uint32_t {
+  auto lane_part = [&](uint32_t whole, uint32_t tail, uint32_t end, int kt) -> uint32_t {
+    if (LINES && kt > k_full) return end;
     return KTAIL && kt >= k_full ? tail : whole;
+  };
+  // (the first windows of an item; a row of one step has both its ends in window 0)
+  auto first_lane_part = [&](uint32_t whole, uint32_t tail, uint32_t end, uint32_t head, int kt) -> uint32_t {
+    const uint32_t part = lane_part(whole, tail, end, kt);
+    return LINES && kt == 0 ? max(part, head) : part;
   };
   // Ring positions the next loads of A and of B go to (= issued % stages, kept as counters that wrap).
   int fill_a = 0, fill_b = 0;
@@ -687,7 +723,7 @@ void gemm_tiled_kernel(GemmParams p) {
   // last step it re-issues the last one into a stage nobody reads again, which keeps the
   // path free of branches.
   auto issue_a = [&]() {
-    const uint32_t lo = lane_part(a_lane, a_lane_tail, ca.kt);
+    const uint32_t lo = first_lane_part(a_lane, a_lane_tail, a_lane_end, a_lane_head, ca.kt);
 #pragma unroll
     for (int i = 0; i < A_GROUPS; ++i)
       load_group(std::false_type{}, a_src, lo, (uint32_t)ca.kt * kStepK + a_src.wave_off, i, lds + fill_a * STAGE_A);
@@ -695,7 +731,7 @@ void gemm_tiled_kernel(GemmParams p) {
     ++ca.issued;
   };
   auto issue_b = [&]() {
-    const uint32_t lo = lane_part(b_lane, b_lane_tail, cb.kt);
+    const uint32_t lo = first_lane_part(b_lane, b_lane_tail, b_lane_end, b_lane_head, cb.kt);
 #pragma unroll
     for (int i = 0; i < B_GROUPS; ++i)
       load_group(std::integral_constant<bool, STREAM_B && !OFF_LINES>{}, b_src, lo, (uint32_t)cb.kt * kStepK + b_src.wave_off, i,
@@ -737,11 +773,14 @@ void gemm_tiled_kernel(GemmParams p) {
     v4i lo, hi;
   };
   Frag xa[MT], xb[NT], ya[MT], yb[NT];
-  auto read_lo = [&](const uint8_t* rows, int s, int i) -> v4i {
-    return *(const v4i*)(rows + i * 32 * kStepK + rd_off[s][0]);
+  // (next: where the same rows' next window lies, LINES only)
+  auto read_a = [&](const uint8_t* rows, const uint8_t* next, int s, int j, int i) -> v4i {
+    if constexpr (LINES) return *(const v4i*)((rd_next_a[s][j] ? next : rows) + rd_off_a[s][j] + i * 32 * kStepK);
+    else return *(const v4i*)(rows + i * 32 * kStepK + rd_off[s][j]);
   };
-  auto read_hi = [&](const uint8_t* rows, int s, int i) -> v4i {
-    return *(const v4i*)(rows + i * 32 * kStepK + rd_off[s][1]);
+  auto read_b = [&](const uint8_t* rows, const uint8_t* next, int s, int j, int i) -> v4i {
+    if constexpr (LINES) return *(const v4i*)((rd_next_b[s][j] ? next : rows) + rd_off_b[s][j] + i * 32 * kStepK);
+    else return *(const v4i*)(rows + i * 32 * kStepK + rd_off[s][j]);
   };
   auto as_v8 = [](const Frag& f) -> v8i {
     return (v8i){f.lo[0], f.lo[1], f.lo[2], f.lo[3], f.hi[0], f.hi[1], f.hi[2], f.hi[3]};
@@ -833,16 +872,18 @@ void gemm_tiled_kernel(GemmParams p) {
       acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(as_v8(fb[j]), as_v8(fa[i]), fresh ? zero : acc[i][j], 0, 0, 0, 0, 0, 0);
   };
   // u-th of the 2*(MT+NT) LDS reads that fill fragment set (fa, fb) with K half s
-  auto read_one = [&](Frag (&fa)[MT], Frag (&fb)[NT], const uint8_t* rows_a, const uint8_t* rows_b, int s, int u) {
+  auto read_one = [&](Frag (&fa)[MT], Frag (&fb)[NT], const uint8_t* rows_a, const uint8_t* next_a, const uint8_t* rows_b,
+                      const uint8_t* next_b, int s, int u) {
     const int f = u >> 1;
     if (f < MT) {
-      if (u & 1) fa[f].hi = read_hi(rows_a, s, f);
-      else fa[f].lo = read_lo(rows_a, s, f);
+      if (u & 1) fa[f].hi = read_a(rows_a, next_a, s, 1, f);
+      else fa[f].lo = read_a(rows_a, next_a, s, 0, f);
     } else {
-      if (u & 1) fb[f - MT].hi = read_hi(rows_b, s, f - MT);
-      else fb[f - MT].lo = read_lo(rows_b, s, f - MT);
+      if (u & 1) fb[f - MT].hi = read_b(rows_b, next_b, s, 1, f - MT);
+      else fb[f - MT].lo = read_b(rows_b, next_b, s, 0, f - MT);
     }
   };
+  constexpr int AHEAD = LINES ? 1 : 0;  // windows behind a step's own that have to have landed for it
   // Per half step: NMFMA MFMAs, NREAD LDS reads, A_GROUPS or B_GROUPS global->LDS loads, the
   // memory instructions placed behind the MFMAs: load l in slot l*NMFMA/GROUPS, the reads RPS
   // per slot in the first half of the slots. The reads have then returned while the last
@@ -859,9 +900,9 @@ void gemm_tiled_kernel(GemmParams p) {
     issue_a(); advance_a(std::false_type{});
     issue_b(); advance_b(std::false_type{});
   }
-  wait_loads_and_barrier<(DIST - 1) * (A_GROUPS + B_GROUPS)>();
+  wait_loads_and_barrier<(DIST - 1 - AHEAD) * (A_GROUPS + B_GROUPS)>();
 #pragma unroll
-  for (int u = 0; u < NREAD; ++u) read_one(xa, xb, lds + a_rd_base, lds + b_rd_base, 0, u);
+  for (int u = 0; u < NREAD; ++u) read_one(xa, xb, lds + a_rd_base, lds + a_rd_base + STAGE_A, lds + b_rd_base, lds + b_rd_base + STAGE_B, 0, u);
 
   // ---- epilogue. The MFMA leaves lane (l32, half) with row l32 of every 32x32 block and the
   // columns 8*q + 4*half + e (register 4*q + e): storing from there would touch 32 rows per
@@ -1098,8 +1139,9 @@ void gemm_tiled_kernel(GemmParams p) {
   int sa = 0, sb = 0;  // stages holding the step being computed
   const uint8_t* cur_a = lds + a_rd_base;  // where this wave reads the step being computed ...
   const uint8_t* cur_b = lds + b_rd_base;
-  const uint8_t* nxt_a = cur_a;            // ... and the step after it
-  const uint8_t* nxt_b = cur_b;
+  const uint8_t* nxt_a = LINES ? cur_a + STAGE_A : cur_a;  // ... and the step after it
+  const uint8_t* nxt_b = LINES ? cur_b + STAGE_B : cur_b;
+  const uint8_t *then_a = nxt_a, *then_b = nxt_b;  // (LINES: and the window after that)
   // What a phase's loads need, put together while the previous phase's last MFMAs run: between
   // the last MFMA of one phase and the first of the next a wave, which issues its instructions in
   // order, should find as little as possible (every scalar instruction there is time the matrix
@@ -1110,14 +1152,14 @@ void gemm_tiled_kernel(GemmParams p) {
   };
   LoadPhase ph_a = {0, 0, lds}, ph_b = {0, 0, lds};  // loads of A (issued in phase [B]) / of B (issued in phase [A])
   auto prepare_b_loads = [&]() {
-    ph_b.lane_off = lane_part(b_lane, b_lane_tail, cb.kt);
+    ph_b.lane_off = lane_part(b_lane, b_lane_tail, b_lane_end, cb.kt);
     ph_b.step_off = (uint32_t)cb.kt * kStepK + b_src.wave_off;
     ph_b.stage = lds + LDS_B0 + fill_b * STAGE_B;
     next_fill_b();
     ++cb.issued;
   };
   auto prepare_a_loads = [&]() {
-    ph_a.lane_off = lane_part(a_lane, a_lane_tail, ca.kt);
+    ph_a.lane_off = lane_part(a_lane, a_lane_tail, a_lane_end, ca.kt);
     ph_a.step_off = (uint32_t)ca.kt * kStepK + a_src.wave_off;
     ph_a.stage = lds + fill_a * STAGE_A;
     next_fill_a();
@@ -1162,7 +1204,7 @@ void gemm_tiled_kernel(GemmParams p) {
           load_group(stream_tag, b_src, ph_b.lane_off, ph_b.step_off, l, ph_b.stage);
 #pragma unroll
       for (int u = t * RPS; u < (t + 1) * RPS; ++u)
-        if (u < NREAD) read_one(ya, yb, cur_a, cur_b, 1, u);
+        if (u < NREAD) read_one(ya, yb, cur_a, nxt_a, cur_b, nxt_b, 1, u);
       if (t == B_LAST) advance_b(plain_tag);
       if (t == PREP_T) prepare_a_loads();
       if (BLOCKSCALE && t == PREP_T) {
@@ -1173,8 +1215,13 @@ void gemm_tiled_kernel(GemmParams p) {
       if (t == PREP_T2) {
         sa = (sa + 1 == kStagesA) ? 0 : sa + 1;
         sb = (sb + 1 == kStagesB) ? 0 : sb + 1;
-        nxt_a = lds + a_rd_base + sa * STAGE_A;
-        nxt_b = lds + b_rd_base + sb * STAGE_B;
+        if constexpr (LINES) {  // (this phase's reads, which end in front of this slot or behind it, have the next window's place in nxt_*)
+          then_a = lds + a_rd_base + (sa + 1 == kStagesA ? 0 : sa + 1) * STAGE_A;
+          then_b = lds + b_rd_base + (sb + 1 == kStagesB ? 0 : sb + 1) * STAGE_B;
+        } else {
+          nxt_a = lds + a_rd_base + sa * STAGE_A;
+          nxt_b = lds + b_rd_base + sb * STAGE_B;
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -1182,7 +1229,7 @@ void gemm_tiled_kernel(GemmParams p) {
     // own loads of A(g+1) and B(g+1) have landed (the younger B(g+2) .. B(g+DIST) and
     // A(g+2) .. A(g+DIST-1) may still be in flight); past the barrier everyone's have, and
     // every wave is done reading this step's stages
-    wait_loads_and_barrier<(DIST - 1) * B_GROUPS + (DIST - 2) * A_GROUPS>();
+    wait_loads_and_barrier<(DIST - 1 - AHEAD) * B_GROUPS + (DIST - 2 - AHEAD) * A_GROUPS>();
 
     // [B] MFMAs on y* (second K half); behind them the loads of A(g+DIST) into the A stage just
     //     released and the LDS reads of step g+1's first half (-> x*; at the end of a tile
@@ -1199,7 +1246,7 @@ void gemm_tiled_kernel(GemmParams p) {
         if (l * NMFMA / A_GROUPS == t) load_group(std::false_type{}, a_src, ph_a.lane_off, ph_a.step_off, l, ph_a.stage);
 #pragma unroll
       for (int u = t * RPS; u < (t + 1) * RPS; ++u)
-        if (READ_NEXT && u < NREAD) read_one(xa, xb, nxt_a, nxt_b, 0, u);
+        if (READ_NEXT && u < NREAD) read_one(xa, xb, nxt_a, then_a, nxt_b, then_b, 0, u);
       if (t == A_LAST) advance_a(plain_tag);
       if (t == PREP_T) {
         prepare_b_loads();
@@ -1208,11 +1255,15 @@ void gemm_tiled_kernel(GemmParams p) {
       }
       __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (LINES) {
+      nxt_a = then_a;
+      nxt_b = then_b;
+    }
     if (BLOCKSCALE) kt_c = STREAM_B && kt_c + 1 == k_steps ? 0 : kt_c + 1;
   };
   auto read_first_half = [&]() {
 #pragma unroll
-    for (int u = 0; u < NREAD; ++u) read_one(xa, xb, cur_a, cur_b, 0, u);
+    for (int u = 0; u < NREAD; ++u) read_one(xa, xb, cur_a, nxt_a, cur_b, nxt_b, 0, u);
   };
 
   // Item loop around the K loop. The first step of an item is its own copy of the step code
@@ -3980,7 +4031,11 @@ inline float plan_cost_us(int64_t M, int64_t N, int64_t K, int config, int split
   // (128x256 tiles over fewer than 8 steps: what a launch costs before its first step is not in the table's 2.6 us a
   // tile, 2129 x 32 x 512 7.2 us with 17 tiles where 128x128 tiles take 5.2: such launches are left to those)
   const float us_per_item = config == 5 && items <= 2 * slots ? 7.0f : short_c3 ? 5.0f : config == 4 && sps < 8 ? 10.0f : c.us_per_item;
-  const float us_step = short_c3 ? 0.54f : c.us_per_step, us_step_alone = short_c3 ? 0.54f : c.us_per_step_alone;
+  // (Rows off the lines, K standing in for the pitch: the deep form fetches them in whole lines, the others' steps take a fifth longer. In the deep
+  // form and in what came out ahead without this: 1317 x 1808 x 13392 51.7 and 66.1 us, 1323 x 1692 x 10352 43.3 and 57.3, 1504 x 943 x 14896 44.7 and
+  // 54.0, 458 x 3993 x 11456 41.0 and 47.1. Above the rows of the narrow tiles, whose own estimate knows of no pitch.)
+  const float off_lines = K % kStepK != 0 && config != kDeepSmallConfig && M > 256 ? 1.2f : 1.0f;
+  const float us_step = off_lines * (short_c3 ? 0.54f : c.us_per_step), us_step_alone = off_lines * (short_c3 ? 0.54f : c.us_per_step_alone);
   float t = full_rounds * (sps * us_step * step_scale + us_per_item);
   if (rest) t += sps * (rest <= kNumCu ? us_step_alone : us_step) * step_scale + us_per_item;
   // (the deep 128x128 form is for one round only; beyond 128 workgroups its steps slow down with the chip's
@@ -4153,7 +4208,7 @@ int launch_finalize(GemmParams p, hipStream_t stream) {
 }
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, bool KTAIL, int EPI, bool GROUPED = false, bool BLOCKSCALE = false,
-          int DIST = kDefaultDist, bool STREAM_B = false, bool CLEAR = false, bool OFF_LINES = false>
+          int DIST = kDefaultDist, bool STREAM_B = false, bool CLEAR = false, bool OFF_LINES = false, bool LINES = false>
 int launch_tiled(GemmParams p, hipStream_t stream) {
   p.store = store_policy(p);
   constexpr int threads = WAVES_M * WAVES_N * 64;
@@ -4167,7 +4222,7 @@ int launch_tiled(GemmParams p, hipStream_t stream) {
   if (total > (long)INT32_MAX) return fail(MI355X_FP8_ENOTSUP, "more than 2^31-1 work items");
   const long slots = (long)kNumCu * tiled_wgs_per_cu(BM, BN, DIST);
   long grid = total < slots ? ((total + kNumXcd - 1) / kNumXcd) * kNumXcd : slots;
-  constexpr auto kern = gemm_tiled_kernel<BM, BN, WAVES_M, WAVES_N, KTAIL, EPI, GROUPED, BLOCKSCALE, DIST, STREAM_B, CLEAR, OFF_LINES>;
+  constexpr auto kern = gemm_tiled_kernel<BM, BN, WAVES_M, WAVES_N, KTAIL, EPI, GROUPED, BLOCKSCALE, DIST, STREAM_B, CLEAR, OFF_LINES, LINES>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   if (const int st = ready_device()) return st;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), lds_bytes, stream, p);
@@ -4190,6 +4245,19 @@ int launch_tiled_epilogue(const GemmParams& p, hipStream_t s) {
   // K=28672: 220 -> 199 us). The 64x256 tile measured 1-3 % slower that way and stays at two.
   constexpr int D = DEEP || (BM == 256 && BN == 128) ? 3 : kDefaultDist;
   const bool ktail = p.K % kStepK;
+  // The deep form, rows off the lines: in whole lines where the steps of an item pay for the window more that has to land before the first.
+  // us so and as they lie, by items and steps of each: 1000x3000x4112 (192, 33) 24.5 and 28.9, 512x4096x4112 (128, 33) 24.4 and 31.4, 539x4260x6480
+  // (170, 51) 30.8 and 39.6, 252x2688x13840 (in six) 26.3 and 31.7, 2048x2048x2064 (256, 17) 16.2 and 18.8, 1693x663x1488 (84, 12)
+  // 12.2 and 13.1; with 10 steps 699x3051x1216 (144) 12.8 and 12.6, with 9 535x2440x1056 (100) 10.2 and 9.6.
+  if constexpr (DEEP) {
+    const long items = (long)((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN) * p.splits;
+    const uintptr_t off = reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.b) | (uintptr_t)p.lda | (uintptr_t)p.ldb;
+    if (off % kStepK != 0 && items <= kNumCu && p.steps_per_split >= 12) {
+      if (p.splits > 1) return launch_tiled<BM, BN, WAVES_M, WAVES_N, true, kEpiPartial, false, false, D + 1, false, false, false, true>(p, s);
+      return p.bias ? launch_tiled<BM, BN, WAVES_M, WAVES_N, true, kEpiBias, false, false, D + 1, false, false, false, true>(p, s)
+                    : launch_tiled<BM, BN, WAVES_M, WAVES_N, true, kEpiPlain, false, false, D + 1, false, false, false, true>(p, s);
+    }
+  }
   if constexpr (STREAM_B) {
     // (mostly because K is no multiple of a step: the kernels for that take the others too. 120 shapes of 33 to 256 rows: 1.035 times as
     // fast on average without the policy, 220x12704x17520 100 -> 88 us; at worst 210x8143x24896 78 -> 84)
