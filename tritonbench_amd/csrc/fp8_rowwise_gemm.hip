@@ -2326,49 +2326,12 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
     multiply(bf, af, factors);
   };
 
-  // The loop is unrolled DEPTH times so every register set has a fixed name; the compiler's
-  // own wait counts then make each consume() wait for exactly its set's loads (they return
-  // in issue order, so the younger sets stay in flight). That only works on paths without
-  // conditional fetches: where paths with different numbers of younger loads meet, the
-  // compiler has to assume the fewest and ends up draining the whole queue once per round.
-  // So the rounds in which every consume is followed by a fetch form their own loop, the
-  // last full round (consumes only) is straight-line code, and only ragged step counts take
-  // the conditional form. (Measured: worth 2 % with four steps in flight; with two steps in
-  // flight the drained form is 8-11 % faster, so those configurations keep it.)
-  constexpr bool kSteadyLoop = DEPTH >= 4;
-  int i = 0;
-  if (kSteadyLoop && my_steps >= DEPTH) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) fetch(d, land[d], land_f[d]);
-    for (; i + 2 * DEPTH <= my_steps; i += DEPTH) {
-#pragma unroll
-      for (int d = 0; d < DEPTH; ++d) {
-        consume(land[d], land_f[d]);
-        fetch(i + d + DEPTH, land[d], land_f[d]);
-      }
-    }
-    if (i + DEPTH == my_steps) {
-#pragma unroll
-      for (int d = 0; d < DEPTH; ++d) consume(land[d], land_f[d]);
-      i += DEPTH;
-    }
-  } else {
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d)
-      if (d < my_steps) fetch(d, land[d], land_f[d]);
-  }
-  for (; i < my_steps; i += DEPTH) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) {
-      if (i + d < my_steps) {
-        consume(land[d], land_f[d]);
-        if (i + d + DEPTH < my_steps) fetch(i + d + DEPTH, land[d], land_f[d]);
-      }
-    }
-  }
   // K tail (K % 128 != 0): one partial step, taken by the wave whose turn it would be; the
-  // lanes fetch their own 16-byte chunks and chunks (ANY: bytes) at or past K count as zero
-  if (k_tail && (k_full % KW) == wave) {
+  // lanes fetch their own 16-byte chunks and chunks (ANY: bytes) at or past K count as zero. Behind the first steps' loads and in front of
+  // their products: at the end its trip to memory is on its own (2x6400x3008 7.46 -> 7.03 us, 12x1916x752 3.37 -> 3.16). ANY: at the end after all, where
+  // the one wave that has it holds the others' lines up less (42x33317x2297 57.4 us so, 52.2 at the end).
+  auto multiply_tail = [&]() {
+    if (!k_tail || (k_full % KW) != wave) return;
     const int kb = k_full * kStepK;
     auto chunk_of = [&](const uint8_t* row, int c) -> v4i {
       if constexpr (ANY) return load16_any(row, kb + c * kChunk, p.K);
@@ -2390,7 +2353,51 @@ __global__ __launch_bounds__(KW * 64) void gemm_skinny_kernel(GemmParams p) {
     Factors f;
     fetch_factors(k_full, f);
     multiply(bf, af, f);
+  };
+
+  // The loop is unrolled DEPTH times so every register set has a fixed name; the compiler's
+  // own wait counts then make each consume() wait for exactly its set's loads (they return
+  // in issue order, so the younger sets stay in flight). That only works on paths without
+  // conditional fetches: where paths with different numbers of younger loads meet, the
+  // compiler has to assume the fewest and ends up draining the whole queue once per round.
+  // So the rounds in which every consume is followed by a fetch form their own loop, the
+  // last full round (consumes only) is straight-line code, and only ragged step counts take
+  // the conditional form. (Measured: worth 2 % with four steps in flight; with two steps in
+  // flight the drained form is 8-11 % faster, so those configurations keep it.)
+  constexpr bool kSteadyLoop = DEPTH >= 4;
+  int i = 0;
+  if (kSteadyLoop && my_steps >= DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) fetch(d, land[d], land_f[d]);
+    if (!ANY) multiply_tail();
+    for (; i + 2 * DEPTH <= my_steps; i += DEPTH) {
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+        consume(land[d], land_f[d]);
+        fetch(i + d + DEPTH, land[d], land_f[d]);
+      }
+    }
+    if (i + DEPTH == my_steps) {
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) consume(land[d], land_f[d]);
+      i += DEPTH;
+    }
+  } else {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d)
+      if (d < my_steps) fetch(d, land[d], land_f[d]);
+    if (!ANY) multiply_tail();
   }
+  for (; i < my_steps; i += DEPTH) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      if (i + d < my_steps) {
+        consume(land[d], land_f[d]);
+        if (i + d + DEPTH < my_steps) fetch(i + d + DEPTH, land[d], land_f[d]);
+      }
+    }
+  }
+  if (ANY) multiply_tail();
 
   // ---- cross-wave reduction through each wave's own (now idle) buffer
   v4f* mine = (v4f*)buf;
