@@ -63,7 +63,7 @@ def _link_binding(obj, verbose):
 
     tmp = BINDING_PATH + ".tmp"
     _run(["g++", "-shared", "-o", tmp, obj, f"-L{LIB_DIR}", "-l:" + os.path.basename(LIB_PATH), "-Wl,-rpath,$ORIGIN",
-          f"-L{os.path.join(os.path.dirname(torch.__file__), 'lib')}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"], verbose)
+          f"-L{os.path.join(os.path.dirname(torch.__file__), 'lib')}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"], verbose)
     os.replace(tmp, BINDING_PATH)
 
 
