@@ -5177,6 +5177,17 @@ constexpr RowForm row_form(RowSource source, int64_t R, int64_t chunks) {
   const RowForm f = row_form_of(source, R, chunks);
   return f.lanes > 256 && !grid_fits(R, f.lanes) ? RowForm{256, 5} : f;
 }
+constexpr bool every_row_form_exists() {  // (the rule's lines lie at multiples of 64 chunks)
+  for (int source = kRowF32; source <= kRowSiluMul; ++source)
+    for (int64_t R : {int64_t(1), int64_t(kNumCu), int64_t(kNumCu + 1), int64_t(2048), int64_t(2049), int64_t(1) << 24})
+      for (int64_t chunks = 64; chunks <= 8192; chunks += 64)
+        for (int64_t c : {chunks, chunks + 1}) {
+          const RowForm f = row_form((RowSource)source, R, c);
+          if (!row_form_exists((RowSource)source, f.lanes, f.chunks)) return false;
+        }
+  return true;
+}
+static_assert(every_row_form_exists(), "a row without a kernel would not be quantised");
 static_assert(row_form(kRowBf16, 8388607, 2000).lanes == 512 && row_form(kRowBf16, 8388608, 2000).lanes == 256, "512 lanes a row reach 2^32 at 8388608 rows");
 
 // Calls launch(lanes, chunks), as integral constants, for the form.
