@@ -383,7 +383,8 @@ int mi355x_fp8_rowwise_quantize(const void* x, int src_type,
  *   SiLU-mul   y[r,k] = (x1[r,k] / (1 + exp(-x1[r,k]))) * x2[r,k]
  *
  * all in f32 on the bf16 inputs, followed by the row-wise quantiser's arithmetic on y as on an
- * f32 tensor (see mi355x_fp8_rowwise_quantize): xq, inv_scale feed mi355x_fp8_rowwise_gemm.
+ * f32 tensor (see mi355x_fp8_rowwise_quantize): xq, inv_scale feed mi355x_fp8_rowwise_gemm. A row's codes and scale
+ * hang on that row alone: RMSNorm's sum is added up in an order that only K decides.
  *
  *   x, x1, x2  bf16 [R, K], row strides ldx / ldx1 / ldx2 (elements, multiples of 8)
  *   weight     bf16 [K]                    xq  e4m3fn [R, K], row stride ldq (multiple of 16)

@@ -3230,16 +3230,12 @@ __device__ __forceinline__ uint8_t f32_to_e4m3fn_rne(float f) {
 // register file: __shfl_xor goes through LDS, six round trips in a row (0.1 to 0.3 us of a call of few rows: RMSNorm 32x8192, which has two
 // reductions, 4.95 -> 4.64 us in four rounds of 256 lanes, SiLU-mul 32x8192 3.76 -> 3.63).
 template <typename Op>
-__device__ __forceinline__ float wave_reduce(float v, Op op) {
+__device__ __forceinline__ float row_reduce(float v, Op op) {  // bits 3 to 0: within each row of 16 lanes
 #if defined(__HIP_DEVICE_COMPILE__)
   auto dpp = [](float from, float old, auto ctrl, auto banks) -> float {
     return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(from), decltype(ctrl)::value, 0xf, decltype(banks)::value, false));
   };
   using std::integral_constant;
-  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
-  v = op(__int_as_float(halves[0]), __int_as_float(halves[1]));
-  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
-  v = op(__int_as_float(rows[0]), __int_as_float(rows[1]));
   v = op(v, dpp(v, v, integral_constant<int, 0x128>{}, integral_constant<int, 0xf>{}));  // row_ror:8
   const float up = dpp(v, v, integral_constant<int, 0x104>{}, integral_constant<int, 0x5>{});  // row_shl:4 into the even fours
   v = op(v, dpp(v, up, integral_constant<int, 0x114>{}, integral_constant<int, 0xa>{}));       // row_shr:4 into the odd ones
@@ -3247,6 +3243,33 @@ __device__ __forceinline__ float wave_reduce(float v, Op op) {
   v = op(v, dpp(v, v, integral_constant<int, 0xB1>{}, integral_constant<int, 0xf>{}));         // quad_perm [1, 0, 3, 2]
 #endif
   return v;
+}
+// Either half of a wave, and either row of two, in both: {lower, lower} and {upper, upper}.
+struct Halves {
+  float lower, upper;
+};
+__device__ __forceinline__ Halves halves_of_wave(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto both = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+  return {__int_as_float(both[0]), __int_as_float(both[1])};
+#else
+  return {v, v};
+#endif
+}
+__device__ __forceinline__ Halves rows_of_pair(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto both = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+  return {__int_as_float(both[0]), __int_as_float(both[1])};
+#else
+  return {v, v};
+#endif
+}
+template <typename Op>
+__device__ __forceinline__ float wave_reduce(float v, Op op) {
+  const Halves halves = halves_of_wave(v);
+  v = op(halves.lower, halves.upper);
+  const Halves rows = rows_of_pair(v);
+  return row_reduce(op(rows.lower, rows.upper), op);
 }
 
 template <typename SrcT>
@@ -3586,6 +3609,12 @@ __global__ __launch_bounds__(256) void quantize_blocks_kernel(const SrcT* x, uin
 // ------------------------------------------------------------------------------------
 constexpr int kFusedRmsNorm = 0, kFusedSiluMul = 1;
 
+// A row's sum of squares is added up in an order that hangs on the row's length alone (in another order rstd can move by a unit in its last
+// place, which sends exact ties between two codes the other way), so a row has the same codes however many rows the call has:
+// as by this many lanes, of which lane o adds up chunks o, o + S, o + 2 S, ... element by element in one chain, then the lanes of each
+// 64 pairwise from bit 5 of their numbers down to bit 0, then the 64s one after another.
+constexpr int rms_sum_lanes(int64_t chunks) { return chunks <= 256 ? 64 : chunks <= 1024 ? 256 : chunks <= 4096 ? 512 : 1024; }
+
 template <int OP, int CACHE, int THREADS, int ROWS = 1>
 __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(const uint16_t* x1, const uint16_t* x2,
                                                                              float eps, uint8_t* xq, float* inv_scale,
@@ -3593,7 +3622,15 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
   static_assert(ROWS == 1 || THREADS == 64, "several rows per workgroup: one wave each (as in the quantiser)");
   using V = VecTraits<uint16_t>;
   constexpr int EPV = 8;
-  __shared__ float wave_part[2][THREADS / 64];  // one set per reduction: neither waits for the other's readers
+  // A form with more lanes than the sum's order has (HANDS times as many) hands a chain on from lane to lane, and one with fewer has CHAINS
+  // of them in each lane. (A chain's lanes are in one wave, a row of 16 or a half each, where handing on is one instruction. All of them
+  // add at each turn, which costs 0.2 us: 32x8192 with 1024 lanes 3.58 us cold in an order of its own, 3.79 in this one, where the 256 lanes
+  // of the order take 5.11.)
+  constexpr int SUM_LANES = OP == kFusedRmsNorm ? rms_sum_lanes((int64_t)THREADS * CACHE) : THREADS;
+  constexpr int HANDS = THREADS > SUM_LANES ? THREADS / SUM_LANES : 1, CHAINS = SUM_LANES > THREADS ? SUM_LANES / THREADS : 1;
+  static_assert(HANDS <= 2 || (HANDS == 4 && CACHE == 1), "a chain starts in the first row or half, and with two hands it comes back to it");
+  __shared__ float wave_part[THREADS / 64];
+  __shared__ __attribute__((aligned(16))) float sum_part[HANDS > 1 ? SUM_LANES : THREADS / 64 * CHAINS];  // (of its own: no wait for the other's readers)
   const long row = (long)blockIdx.x * ROWS + (ROWS > 1 ? (long)(threadIdx.x >> 6) : 0);
   if (ROWS > 1 && row >= rows) return;  // (whole waves; this form has no barrier)
   const v4i* r1 = (const v4i*)(x1 + row * ld1);
@@ -3602,18 +3639,14 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
   uint8_t* qr = xq + row * ldq;
   const int nchunks = K / EPV;
   const int tid = ROWS > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
-
-  // sums (or maxima) of one value per lane over the row's lanes; every lane gets the result
-  auto block_reduce = [&](int set, float v, auto op) -> float {
-    v = wave_reduce(v, op);
-    if (THREADS == 64) return v;
-    if ((tid & 63) == 0) wave_part[set][tid >> 6] = v;
-    __syncthreads();
-    float r = wave_part[set][0];
-#pragma unroll
-    for (int w = 1; w < THREADS / 64; ++w) r = op(r, wave_part[set][w]);
-    return r;
-  };
+  const int lane = tid & 63;
+  // Round i of lane t is chunk first_chunk(t) + THREADS * i. Four hands: the turns of a wave's rows are 0, 1, 3, 2, so that each has its
+  // neighbour's in the other row of its pair or in the other half.
+  constexpr int WAVE_CHAINS = 64 / HANDS;
+  auto turn_of = [](int t) { return HANDS == 4 ? (t & 63) / 16 ^ (t & 63) / 32 : (t & 63) / WAVE_CHAINS; };
+  auto chain_of = [](int t) { return (t >> 6) * WAVE_CHAINS + t % WAVE_CHAINS; };
+  auto first_chunk = [&](int t) { return HANDS == 1 ? t : chain_of(t) + SUM_LANES * turn_of(t); };
+  const int at = first_chunk(tid);
   // (hardware exponential and reciprocal, about one ulp each: the result is rounded to 4 significant
   // bits next; the library exponential costs six times the instructions and a correctly rounded
   // quotient ten, which together made the kernel compute-bound)
@@ -3629,27 +3662,66 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
     // pass 1: x to registers, sum of squares (lanes past the row's end re-read the last chunk and
     // leave it out of the sum). The weights of the cached chunks are asked for here as well: fetched
     // after the reduction they would put a second trip to the L2 on every row's critical path.
-    float ss = 0.0f;
     if (EARLY_WEIGHTS) {
 #pragma unroll
-      for (int i = 0; i < CACHE; ++i) wts[EARLY_WEIGHTS ? i : 0] = r2[min(tid + THREADS * i, nchunks - 1)];
+      for (int i = 0; i < CACHE; ++i) wts[EARLY_WEIGHTS ? i : 0] = r2[min(at + THREADS * i, nchunks - 1)];
     }
+#pragma unroll
+    for (int i = 0; i < CACHE; ++i) V::unpack(__builtin_nontemporal_load(r1 + min(at + THREADS * i, nchunks - 1)), vals[i]);
+    auto add_squares = [](const float (&f)[EPV], float s) -> float {
+#pragma unroll
+      for (int e = 0; e < EPV; ++e) s = __builtin_fmaf(f[e], f[e], s);
+      return s;
+    };
+    float sums[CHAINS] = {};
 #pragma unroll
     for (int i = 0; i < CACHE; ++i) {
-      const int c = tid + THREADS * i;
-      V::unpack(__builtin_nontemporal_load(r1 + min(c, nchunks - 1)), vals[i]);
-      if (c < nchunks) {
+      float& s = sums[i % CHAINS];
 #pragma unroll
-        for (int e = 0; e < EPV; ++e) ss = __builtin_fmaf(vals[i][e], vals[i][e], ss);
+      for (int turn = 0; turn < HANDS; ++turn) {
+        if (HANDS == 2 && i + turn > 0) s = turn == 1 ? halves_of_wave(s).lower : halves_of_wave(s).upper;
+        if (HANDS == 4 && turn > 0) s = turn == 1 ? rows_of_pair(s).lower : turn == 2 ? halves_of_wave(s).lower : rows_of_pair(s).upper;
+        const float with = add_squares(vals[i], s);
+        s = at + THREADS * i < nchunks ? with : s;
       }
     }
-    for (int c = tid + THREADS * CACHE; c < nchunks; c += THREADS) {
-      float f[EPV];
-      V::unpack(r1[c], f);
+    auto add = [](float a, float b) { return a + b; };
+    float ss = 0.0f;
+    if constexpr (HANDS > 1) {
+      // the chains' sums, those of the lanes that are added first beside one another: a row of lanes takes 64 of them
+      const int chain = chain_of(tid);
+      if (turn_of(tid) == HANDS - 1) sum_part[chain / 64 * 64 + chain % 16 * 4 + chain % 64 / 16] = sums[0];
+      __syncthreads();
+      constexpr int GROUPS = SUM_LANES / 64;
 #pragma unroll
-      for (int e = 0; e < EPV; ++e) ss = __builtin_fmaf(f[e], f[e], ss);
+      for (int g = 0; g < GROUPS; g += 4) {
+        const v4f four = *(const v4f*)(sum_part + min(g + lane / 16, GROUPS - 1) * 64 + lane % 16 * 4);
+        const float group = row_reduce((four[0] + four[2]) + (four[1] + four[3]), add);
+#pragma unroll
+        for (int r = 0; r < 4 && g + r < GROUPS; ++r) {
+          const float one = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(group), 16 * r));
+          ss = g + r == 0 ? one : ss + one;
+        }
+      }
+    } else {
+      for (int c = tid + THREADS * CACHE; c < nchunks; c += THREADS) {
+        float f[EPV];
+        V::unpack(r1[c], f);
+        sums[0] = add_squares(f, sums[0]);
+      }
+      ss = wave_reduce(sums[0], add);
+      if constexpr (THREADS > 64) {
+#pragma unroll
+        for (int chain = 0; chain < CHAINS; ++chain) {
+          const float of_wave = chain == 0 ? ss : wave_reduce(sums[chain], add);
+          if (lane == 0) sum_part[chain * (THREADS / 64) + (tid >> 6)] = of_wave;
+        }
+        __syncthreads();
+        ss = sum_part[0];
+#pragma unroll
+        for (int w = 1; w < THREADS / 64 * CHAINS; ++w) ss += sum_part[w];
+      }
     }
-    ss = block_reduce(0, ss, [](float a, float b) { return a + b; });
     rstd = 1.0f / sqrtf(ss / (float)K + eps);
   }
   // value of chunk c from its raw operands
@@ -3661,7 +3733,7 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
   float amax = 0.0f;
 #pragma unroll
   for (int i = 0; i < CACHE; ++i) {
-    const int c = min(tid + THREADS * i, nchunks - 1);
+    const int c = min(at + THREADS * i, nchunks - 1);
     float a[EPV], b[EPV];
     if (OP == kFusedRmsNorm) {
 #pragma unroll
@@ -3674,7 +3746,9 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
 #pragma unroll
     for (int e = 0; e < EPV; ++e) amax = max_keep_nan(amax, fabsf(vals[i][e]));
   }
-  for (int c = tid + THREADS * CACHE; c < nchunks; c += THREADS) {
+  // (what the registers do not hold: rows of a form with HANDS never have any)
+  const int rest = HANDS == 1 ? tid + THREADS * CACHE : nchunks;
+  for (int c = rest; c < nchunks; c += THREADS) {
     float a[EPV], b[EPV], y[EPV];
     V::unpack(r1[c], a);
     V::unpack(r2[c], b);
@@ -3682,7 +3756,14 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
 #pragma unroll
     for (int e = 0; e < EPV; ++e) amax = max_keep_nan(amax, fabsf(y[e]));
   }
-  amax = block_reduce(1, amax, [](float a, float b) { return max_keep_nan(a, b); });
+  amax = wave_reduce(amax, [](float a, float b) { return max_keep_nan(a, b); });
+  if (THREADS > 64) {
+    if (lane == 0) wave_part[tid >> 6] = amax;
+    __syncthreads();
+    amax = wave_part[0];
+#pragma unroll
+    for (int w = 1; w < THREADS / 64; ++w) amax = max_keep_nan(amax, wave_part[w]);
+  }
 
   const float scale = row_scale<float>(amax);
   if (tid == 0) inv_scale[row] = 1.0f / scale;
@@ -3706,7 +3787,6 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
   // leave as one 16-byte store per lane (LDS executes a wave's operations in order: no barrier).
   __shared__ __attribute__((aligned(16))) uint8_t strip[THREADS * ROWS / 64][1024];
   uint8_t* mine = strip[threadIdx.x >> 6];
-  const int lane = tid & 63;
 #pragma unroll
   for (int i0 = 0; i0 < CACHE; i0 += 2) {
     if (i0 + 2 <= CACHE && finite_row && THREADS * (i0 + 2) <= nchunks) {  // uniform: every lane of every wave has both rounds
@@ -3723,16 +3803,16 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
       }
       const int b = lane / 32, piece = lane % 32;
       const v4i bytes = *(const v4i*)(mine + lane * 16);
-      *(v4i*)(qr + ((size_t)THREADS * (i0 + b) + (tid & ~63)) * EPV + piece * 16) = bytes;
+      *(v4i*)(qr + (size_t)(THREADS * (i0 + b) + first_chunk((tid & ~63) + 2 * piece)) * EPV) = bytes;
     } else {
 #pragma unroll
       for (int b = 0; b < 2 && i0 + b < CACHE; ++b) {
-        const int c = tid + THREADS * (i0 + b);
+        const int c = at + THREADS * (i0 + b);
         if (c < nchunks) convert_store(vals[i0 + b], c);
       }
     }
   }
-  for (int c = tid + THREADS * CACHE; c < nchunks; c += THREADS) {
+  for (int c = rest; c < nchunks; c += THREADS) {
     float a[EPV], b[EPV], y[EPV];
     V::unpack(r1[c], a);
     V::unpack(r2[c], b);
@@ -5177,17 +5257,18 @@ constexpr RowForm row_form(RowSource source, int64_t R, int64_t chunks) {
   const RowForm f = row_form_of(source, R, chunks);
   return f.lanes > 256 && !grid_fits(R, f.lanes) ? RowForm{256, 5} : f;
 }
-constexpr bool every_row_form_exists() {  // (the rule's lines lie at multiples of 64 chunks)
+constexpr bool row_forms_are_sound() {  // (the rule's lines lie at multiples of 64 chunks)
   for (int source = kRowF32; source <= kRowSiluMul; ++source)
     for (int64_t R : {int64_t(1), int64_t(kNumCu), int64_t(kNumCu + 1), int64_t(2048), int64_t(2049), int64_t(1) << 24})
       for (int64_t chunks = 64; chunks <= 8192; chunks += 64)
         for (int64_t c : {chunks, chunks + 1}) {
           const RowForm f = row_form((RowSource)source, R, c);
           if (!row_form_exists((RowSource)source, f.lanes, f.chunks)) return false;
+          if (source == kRowRmsNorm && grid_fits(R, 1024) && rms_sum_lanes((int64_t)f.lanes * f.chunks) != rms_sum_lanes(c)) return false;
         }
   return true;
 }
-static_assert(every_row_form_exists(), "a row without a kernel would not be quantised");
+static_assert(row_forms_are_sound(), "a row without a kernel would not be quantised, and in another order of its sum not as among other rows");
 static_assert(row_form(kRowBf16, 8388607, 2000).lanes == 512 && row_form(kRowBf16, 8388608, 2000).lanes == 256, "512 lanes a row reach 2^32 at 8388608 rows");
 
 // Calls launch(lanes, chunks), as integral constants, for the form.
