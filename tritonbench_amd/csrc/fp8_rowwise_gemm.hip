@@ -5211,7 +5211,7 @@ constexpr int kWaveRows = 4;
 
 // How a row's chunks of 16 bytes are dealt out by the quantiser and the fused front ends (rows that start 16-byte aligned): `lanes` of them,
 // `chunks` rounds each that stay in registers; 64 lanes are a wave, kWaveRows rows a workgroup. Any form takes any row (what the registers don't
-// hold is read again), so the rule is about speed alone:
+// hold is read again; RMSNorm: a row of its order of the sum, if it has other lanes than that), so the rule is about speed alone:
 //  - no round is idle if it can be helped, for it loads and computes like any other: rows just above a power of two had up to half of them
 //    idle (RMSNorm 8192x8960 56.5 us as 4 rounds of 512, 42.8 as 5 of 256; SiLU-mul 2048x19904 41.4 and 34.7; f32 8192x9472 72.7 and 60.6);
 //  - up to one row a CU, what counts is the chain of a single row, and one round of as many lanes as that takes is the shortest (RMSNorm
@@ -5229,7 +5229,7 @@ constexpr bool row_form_exists(RowSource source, int lanes, int chunks) {
   if (lanes == 512) return chunks <= 8 && (chunks < 7 || source != kRowSiluMul) && (chunks != 7 || source != kRowRmsNorm);
   return chunks <= 4 || chunks == 8 || (source == kRowF32 && chunks <= 7);
 }
-constexpr RowForm row_form_of(RowSource source, int64_t R, int64_t chunks) {
+constexpr RowForm row_form(RowSource source, int64_t R, int64_t chunks) {
   if (chunks > 4096) {  // (bf16 rows hold half the values in as many registers as f32 ones: more rounds than 4 halve their rate)
     if (source == kRowBf16) return {1024, 4};
     if (source == kRowF32 && chunks <= 7168) return {1024, (int)((chunks + 1023) / 1024)};
@@ -5252,24 +5252,27 @@ constexpr RowForm row_form_of(RowSource source, int64_t R, int64_t chunks) {
   if (source == kRowSiluMul) return {1024, 4};
   return {512, chunks <= 3584 && source != kRowRmsNorm ? 7 : 8};
 }
-// (a launch holds fewer than 2^32 lanes: beyond, 256 of them read the rest of a row twice)
-constexpr RowForm row_form(RowSource source, int64_t R, int64_t chunks) {
-  const RowForm f = row_form_of(source, R, chunks);
-  return f.lanes > 256 && !grid_fits(R, f.lanes) ? RowForm{256, 5} : f;
+// Rows of a launch, which holds fewer than 2^32 lanes (256 a row: 16777212 rows). More of them are several launches of the same form.
+constexpr int64_t rows_per_launch(int64_t lanes) { return (int64_t)UINT32_MAX / lanes / kWaveRows * kWaveRows; }
+template <typename Launch>
+void launch_by_rows(int64_t R, int64_t lanes, Launch&& launch) {
+  for (int64_t row = 0; row < R; row += rows_per_launch(lanes)) launch(row, R - row < rows_per_launch(lanes) ? R - row : rows_per_launch(lanes));
 }
 constexpr bool row_forms_are_sound() {  // (the rule's lines lie at multiples of 64 chunks)
   for (int source = kRowF32; source <= kRowSiluMul; ++source)
-    for (int64_t R : {int64_t(1), int64_t(kNumCu), int64_t(kNumCu + 1), int64_t(2048), int64_t(2049), int64_t(1) << 24})
+    for (int64_t R : {int64_t(1), int64_t(kNumCu), int64_t(kNumCu + 1), int64_t(2048), int64_t(2049)})
       for (int64_t chunks = 64; chunks <= 8192; chunks += 64)
         for (int64_t c : {chunks, chunks + 1}) {
           const RowForm f = row_form((RowSource)source, R, c);
           if (!row_form_exists((RowSource)source, f.lanes, f.chunks)) return false;
-          if (source == kRowRmsNorm && grid_fits(R, 1024) && rms_sum_lanes((int64_t)f.lanes * f.chunks) != rms_sum_lanes(c)) return false;
+          if (!grid_fits(rows_per_launch(f.lanes), f.lanes)) return false;
+          const int64_t held = (int64_t)f.lanes * f.chunks;
+          if (source == kRowRmsNorm && c > held && rms_sum_lanes(held) != f.lanes) return false;
+          if (source == kRowRmsNorm && rms_sum_lanes(held) != rms_sum_lanes(c)) return false;
         }
   return true;
 }
 static_assert(row_forms_are_sound(), "a row without a kernel would not be quantised, and in another order of its sum not as among other rows");
-static_assert(row_form(kRowBf16, 8388607, 2000).lanes == 512 && row_form(kRowBf16, 8388608, 2000).lanes == 256, "512 lanes a row reach 2^32 at 8388608 rows");
 
 // Calls launch(lanes, chunks), as integral constants, for the form.
 template <RowSource SOURCE, int LANES = 64, int CHUNKS = 1, typename Launch>
@@ -5289,8 +5292,10 @@ template <RowSource SOURCE, typename SrcT>
 void launch_quantize_rows(const SrcT* x, uint8_t* xq, float* inv_scale, int64_t R, int64_t K, int64_t ldx, int64_t ldq, hipStream_t s) {
   with_row_form<SOURCE>(row_form(SOURCE, R, K / VecTraits<SrcT>::EPV), [&](auto lanes, auto chunks) {
     constexpr int LANES = decltype(lanes)::value, ROWS = LANES == 64 ? kWaveRows : 1;
-    hipLaunchKernelGGL((quantize_rows_vec_kernel<SrcT, decltype(chunks)::value, LANES, ROWS>), dim3((unsigned)((R + ROWS - 1) / ROWS)),
-                       dim3(LANES * ROWS), 0, s, x, xq, inv_scale, (int)K, (long)ldx, (long)ldq, (long)R);
+    launch_by_rows(R, LANES, [&](int64_t row, int64_t rows) {
+      hipLaunchKernelGGL((quantize_rows_vec_kernel<SrcT, decltype(chunks)::value, LANES, ROWS>), dim3((unsigned)((rows + ROWS - 1) / ROWS)),
+                         dim3(LANES * ROWS), 0, s, x + row * ldx, xq + row * ldq, inv_scale + row, (int)K, (long)ldx, (long)ldq, (long)rows);
+    });
   });
 }
 
@@ -5638,9 +5643,12 @@ int launch_fused_quant(int op, const void* x1, const void* x2, float eps, void* 
     constexpr int OP = decltype(op_tag)::value;
     with_row_form<OP == kFusedRmsNorm ? kRowRmsNorm : kRowSiluMul>(form, [&](auto lanes, auto chunks) {
       constexpr int LANES = decltype(lanes)::value, ROWS = LANES == 64 ? kWaveRows : 1;
-      hipLaunchKernelGGL((fused_rowwise_quant_kernel<OP, decltype(chunks)::value, LANES, ROWS>), dim3((unsigned)((R + ROWS - 1) / ROWS)),
-                         dim3(LANES * ROWS), 0, s, (const uint16_t*)x1, (const uint16_t*)x2, eps, (uint8_t*)xq, inv_scale, (int)K,
-                         (long)ld1, (long)ld2, (long)ldq, (long)R);
+      launch_by_rows(R, LANES, [&](int64_t row, int64_t rows) {
+        const uint16_t* second = (const uint16_t*)x2 + (OP == kFusedRmsNorm ? 0 : row * ld2);  // (RMSNorm: the weights of every row)
+        hipLaunchKernelGGL((fused_rowwise_quant_kernel<OP, decltype(chunks)::value, LANES, ROWS>), dim3((unsigned)((rows + ROWS - 1) / ROWS)),
+                           dim3(LANES * ROWS), 0, s, (const uint16_t*)x1 + row * ld1, second, eps, (uint8_t*)xq + row * ldq, inv_scale + row,
+                           (int)K, (long)ld1, (long)ld2, (long)ldq, (long)rows);
+      });
     });
   };
   if (op == kFusedRmsNorm) launch(std::integral_constant<int, kFusedRmsNorm>{}, row_form(kRowRmsNorm, R, K / 8));
