@@ -28,7 +28,9 @@ def _same_rows(t, period):
 @pytest.mark.parametrize("source", [torch.bfloat16, torch.float32])
 def test_quantiser(gpu_device, rows, source):
     for chunks in CHUNKS + ([7168, 7169] if source == torch.float32 else []):
-        k = chunks * 16 // source.itemsize // 16 * 16 + 16  # (whole 16-byte chunks of codes too)
+        k = chunks * 16 // source.itemsize
+        k += -k % 16  # (whole 16-byte chunks of codes too: the longest row of a form stays what it is)
+        assert chunks % 2 or k * source.itemsize == chunks * 16
         print(f"case {rows}x{k} {source}", flush=True)
         x = torch.randn((4, k), generator=torch.Generator().manual_seed(k)).to(source)
         x[1, k - 1], x[2, 0], x[3, k // 2] = 300.0, float("nan"), float("-inf")  # (the first two rows' largest wherever they fall)
