@@ -293,8 +293,8 @@ int mi355x_fp8_blockwise_gemm(const void* a, const void* b,
 /*
  * The same with the form pinned (-1: the library's choice, which mi355x_fp8_blockwise_form names without a device; it is that of the
  * calls without a workspace, with one the library may cut K instead, see below):
- * ONE_TILE (M <= 64) and NARROW (the shapes of MI355X_FP8_SKINNY_NARROW) are the streaming forms of the row-wise product (the
- * library's choice is named ONE_TILE also where it keeps A on chip, M <= 16 with N a multiple of 16 up to 8192 and K up to 8192),
+ * ONE_TILE (M <= 64), NARROW (the shapes of MI355X_FP8_SKINNY_NARROW) and RESIDENT (A on chip: M <= 16, N a multiple of 16
+ * up to 8192, K up to 8192) are the streaming forms of the row-wise product,
  * TILES_128, TILES_128_STREAM (B fetched with the streaming cache policy) and TILES_256 take any shape. ENOTSUP for a
  * shape the named form does not take.
  */
@@ -303,6 +303,7 @@ int mi355x_fp8_blockwise_gemm(const void* a, const void* b,
 #define MI355X_FP8_BLOCK_TILES_128        2
 #define MI355X_FP8_BLOCK_TILES_128_STREAM 3
 #define MI355X_FP8_BLOCK_TILES_256        4
+#define MI355X_FP8_BLOCK_RESIDENT         6  /* (5 names no form) */
 int mi355x_fp8_blockwise_form(int64_t M, int64_t N, int64_t K);
 int mi355x_fp8_blockwise_gemm_ex(const void* a, const void* b,
                                  const float* a_scale, const float* b_scale, void* c,

@@ -4,12 +4,11 @@ import pytest
 import torch
 
 from tritonbench_amd import ops
+from tritonbench_amd._lib import BLOCK_RESIDENT
 
 from test_gpu_blockwise_forms import _check, _expand, _run
 
 pytestmark = pytest.mark.gpu
-
-CHOICE = None  # the library's own: by its estimates this form, for the shapes below
 
 # one tile, tiles for some CUs, one each, one more than that, two each but for one CU, two each; one to four rounds of steps, whole and with a
 # last step that is partial; tiles of either side of a scale block's edge in one workgroup
@@ -18,7 +17,7 @@ CHOICE = None  # the library's own: by its estimates this form, for the shapes b
                                    (9, 8192, 8176)])
 def test_against_float64(gpu_device, m, n, k):
     print(f"case m={m} n={n} k={k}", flush=True)
-    _check(m, n, k, gpu_device, CHOICE)
+    _check(m, n, k, gpu_device, BLOCK_RESIDENT)
 
 
 @pytest.mark.parametrize("side", ["a", "b"])
@@ -31,10 +30,10 @@ def test_an_infinite_factor_of_the_last_block(gpu_device, m, n, k, side):
     want = torch.full((m, n), float(k), dtype=torch.float64, device=gpu_device)
     want[:, slice(None) if side == "a" else slice(0, 128)] = float("inf")
     got = torch.zeros((m, n), dtype=torch.bfloat16, device=gpu_device)
-    assert torch.equal(_run(xq, wq, xs, ws, got, CHOICE), want.to(torch.bfloat16))
+    assert torch.equal(_run(xq, wq, xs, ws, got, BLOCK_RESIDENT), want.to(torch.bfloat16))
 
 
-# rows of C on any 2 bytes, factors 2^120 apart between neighbouring blocks and of zero; the choice, which is this form, and a replay of it
+# rows of C on any 2 bytes, factors 2^120 apart between neighbouring blocks and of zero; a replay of the library's choice, which is this form
 def test_odd_rows_of_c_any_factors_and_capture(gpu_device):
     m, n, k = 11, 8000, 6000
     g = torch.Generator(device=gpu_device).manual_seed(5)
@@ -45,7 +44,7 @@ def test_odd_rows_of_c_any_factors_and_capture(gpu_device):
     xs[:, 3] = 0.0
     canvas = torch.full((m + 2, n + 5), 7.0, dtype=torch.bfloat16, device=gpu_device)
     out = canvas[1:-1, 3:-2]
-    _run(xq, wq, xs, ws, out, CHOICE)
+    _run(xq, wq, xs, ws, out, BLOCK_RESIDENT)
     exact = _expand(xq, xs) @ _expand(wq, ws).t()
     assert ((out.double() - exact).norm() / exact.norm()).item() < 2.0**-8  # (one rounding to bf16)
     graph = torch.cuda.CUDAGraph()

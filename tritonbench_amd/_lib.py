@@ -143,6 +143,7 @@ _lib = None
 
 # forms of the block-scaled and of the grouped product, as the library names them
 BLOCK_ONE_TILE, BLOCK_NARROW, BLOCK_TILES_128, BLOCK_TILES_128_STREAM, BLOCK_TILES_256 = range(5)
+BLOCK_RESIDENT = 6
 GROUPED_TILES, GROUPED_ROWS_16, GROUPED_ROWS_32, GROUPED_ROWS_64, GROUPED_STREAM_128, GROUPED_STREAM_256 = range(6)
 
 

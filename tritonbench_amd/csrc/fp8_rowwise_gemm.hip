@@ -4567,7 +4567,7 @@ enum BlockForm {
   kBlockSmall = MI355X_FP8_BLOCK_TILES_128,
   kBlockSmallStream = MI355X_FP8_BLOCK_TILES_128_STREAM,
   kBlockLarge = MI355X_FP8_BLOCK_TILES_256,
-  kBlockResident  // the pair kernel: the library's choice only, which is ONE_TILE to callers
+  kBlockResident = MI355X_FP8_BLOCK_RESIDENT  // the pair kernel
 };
 // (One 16-row tile a workgroup, many of them on short rows: what bounds it is the rate at which they come and go, which the
 // row-wise estimate has too high there. us a workgroup beyond the first 256: 16x24576x256 2.9e-3, 16x24576x384 3.3e-3,
@@ -5448,9 +5448,7 @@ int mi355x_fp8_blockwise_form(int64_t M, int64_t N, int64_t K) {
   if (st == MI355X_FP8_OK) st = check_fast_shape(K);
   if (st == MI355X_FP8_OK && K > 256 * kStepK)
     st = fail(MI355X_FP8_ENOTSUP, "block-scaled form handles K <= %d (got %lld)", 256 * kStepK, (long long)K);
-  if (st != MI355X_FP8_OK) return st;
-  const BlockForm form = block_form(M, N, K, K % kStepK != 0);
-  return form == kBlockResident ? kBlockOneTile : form;
+  return st != MI355X_FP8_OK ? st : block_form(M, N, K, K % kStepK != 0);
 }
 
 int mi355x_fp8_blockwise_gemm(const void* a, const void* b, const float* a_scale, const float* b_scale,
@@ -5527,9 +5525,8 @@ int mi355x_fp8_blockwise_gemm_ws(const void* a, const void* b, const float* a_sc
       p.partial = (float*)workspace;
     }
     form = plan.form;
-  } else if (form > kBlockLarge) {
-    return fail(MI355X_FP8_EINVAL, "unknown block-scaled form %d", form);
-  } else if ((form == kBlockOneTile && M > kSkinnyMaxM) || (form == kBlockNarrow && !narrow_fits(M, N, K)))
+  } else if ((form == kBlockOneTile && M > kSkinnyMaxM) || (form == kBlockNarrow && !narrow_fits(M, N, K)) ||
+             (form == kBlockResident && !pair_skinny_fits(M, N, K)))
     return fail(MI355X_FP8_ENOTSUP, "block-scaled form %d does not take %lldx%lld", form, (long long)M, (long long)N);
   switch (form) {
     case kBlockNarrow: return launch_narrow_for<true>(p, s);
