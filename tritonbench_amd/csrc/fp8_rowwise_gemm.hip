@@ -5227,7 +5227,7 @@ constexpr bool row_form_exists(RowSource source, int lanes, int chunks) {
   if (lanes == 64) return chunks <= 4 || (source == kRowF32 && (chunks == 6 || chunks == 8));
   if (lanes == 256) return chunks <= 5;
   if (lanes == 512) return chunks <= 8 && (chunks < 7 || source != kRowSiluMul) && (chunks != 7 || source != kRowRmsNorm);
-  return chunks <= 4 || chunks == 8 || (source == kRowF32 && chunks <= 7);
+  return chunks <= 4 || (source == kRowF32 && chunks <= 7) || (source != kRowBf16 && chunks == 8);
 }
 constexpr RowForm row_form(RowSource source, int64_t R, int64_t chunks) {
   if (chunks > 4096) {  // (bf16 rows hold half the values in as many registers as f32 ones: more rounds than 4 halve their rate)
@@ -5259,20 +5259,27 @@ void launch_by_rows(int64_t R, int64_t lanes, Launch&& launch) {
   for (int64_t row = 0; row < R; row += rows_per_launch(lanes)) launch(row, R - row < rows_per_launch(lanes) ? R - row : rows_per_launch(lanes));
 }
 constexpr bool row_forms_are_sound() {  // (the rule's lines lie at multiples of 64 chunks)
-  for (int source = kRowF32; source <= kRowSiluMul; ++source)
+  for (int source = kRowF32; source <= kRowSiluMul; ++source) {
+    bool chosen[17][9] = {};  // by 64 lanes and rounds
     for (int64_t R : {int64_t(1), int64_t(kNumCu), int64_t(kNumCu + 1), int64_t(2048), int64_t(2049)})
       for (int64_t chunks = 64; chunks <= 8192; chunks += 64)
         for (int64_t c : {chunks, chunks + 1}) {
           const RowForm f = row_form((RowSource)source, R, c);
           if (!row_form_exists((RowSource)source, f.lanes, f.chunks)) return false;
+          chosen[f.lanes / 64][f.chunks] = true;
           if (!grid_fits(rows_per_launch(f.lanes), f.lanes)) return false;
           const int64_t held = (int64_t)f.lanes * f.chunks;
           if (source == kRowRmsNorm && c > held && rms_sum_lanes(held) != f.lanes) return false;
           if (source == kRowRmsNorm && rms_sum_lanes(held) != rms_sum_lanes(c)) return false;
         }
+    for (int lanes : {64, 256, 512, 1024})
+      for (int chunks = 1; chunks <= 8; ++chunks)
+        if (row_form_exists((RowSource)source, lanes, chunks) && !chosen[lanes / 64][chunks]) return false;
+  }
   return true;
 }
-static_assert(row_forms_are_sound(), "a row without a kernel would not be quantised, and in another order of its sum not as among other rows");
+static_assert(row_forms_are_sound(), "a row without a kernel would not be quantised, and in another order of its sum not as among other rows; "
+                                     "a kernel without a row is code that nothing runs");
 
 // Calls launch(lanes, chunks), as integral constants, for the form.
 template <RowSource SOURCE, int LANES = 64, int CHUNKS = 1, typename Launch>
@@ -5530,10 +5537,7 @@ int mi355x_fp8_blockwise_gemm_ws(const void* a, const void* b, const float* a_sc
     return fail(MI355X_FP8_ENOTSUP, "block-scaled form %d does not take %lldx%lld", form, (long long)M, (long long)N);
   switch (form) {
     case kBlockNarrow: return launch_narrow_for<true>(p, s);
-    case kBlockResident:
-      // (the pair kernel addresses a workgroup's rows of B with 32-bit offsets below 2^31)
-      if (ldb * 32 <= (int64_t)INT32_MAX) return launch_skinny_pair_block(p, s);
-      [[fallthrough]];
+    case kBlockResident: return launch_skinny_pair_block(p, s);
     case kBlockOneTile:
       if (M <= 16) return launch_skinny<1, 1, 4, 8, false, true>(p, s);
       if (M <= 32) return launch_skinny<2, 1, 2, 8, false, true>(p, s);
