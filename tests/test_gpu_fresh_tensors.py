@@ -1,4 +1,6 @@
 """Results that the native binding allocates: the same kind of tensor, and seen by whoever watches, whichever way they were made."""
+import ctypes
+
 import pytest
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
@@ -54,3 +56,31 @@ def test_results_are_the_same_whoever_watches(gpu_device):
     assert torch.cuda.memory_allocated(gpu_device) > before
     del more
     assert torch.cuda.memory_allocated(gpu_device) == before
+
+
+def _nodes(call):
+    """What a captured call consists of: its launches and whatever its allocations add."""
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        call()
+    count = ctypes.c_size_t()
+    assert ctypes.CDLL(path).hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    return count.value
+
+
+def test_new_memory_is_filled_where_that_is_asked_for(gpu_device):
+    x = torch.randn((5, 512), device=gpu_device, dtype=torch.bfloat16)
+    plain = ops.fp8_row_quantize(x)
+    alone = _nodes(lambda: ops.fp8_row_quantize(x))
+    try:
+        torch.use_deterministic_algorithms(True)
+        filled = _nodes(lambda: ops.fp8_row_quantize(x))
+        other = ops.fp8_row_quantize(x)
+        torch.utils.deterministic.fill_uninitialized_memory = False
+        not_filled = _nodes(lambda: ops.fp8_row_quantize(x))
+    finally:
+        torch.use_deterministic_algorithms(False)
+        torch.utils.deterministic.fill_uninitialized_memory = True
+    assert filled >= alone + 2 and not_filled == alone  # (codes and scales)
+    assert all(torch.equal(a.view(torch.uint8), b.view(torch.uint8)) for a, b in zip(plain, other))

@@ -8,6 +8,7 @@
 // What it is for: launches of a few microseconds. A product of one row against a 2304 x 2048 weight takes 3.3 us on the
 // GPU and took 12.2 us a call, the rest of it attribute look-ups, conversions of 18 arguments and wrapper objects.
 #include <Python.h>
+#include <ATen/Context.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/ops/empty.h>
@@ -46,10 +47,12 @@ bool result(const at::Tensor* t, at::ScalarType type, int64_t m, int64_t n) {
 }
 // Straight from the device's allocator, without the dispatcher, which is half of what a tensor of a few kilobytes costs (a quantiser and a product of
 // 5 x 512 x 2560, three tensors and two launches: 9.8 -> 9.1 us a call) - where nothing would see the difference: no dispatch mode, tracer,
-// transform, inference mode or autocast in this thread, nobody who records operators.
+// transform, inference mode or autocast in this thread, nobody who records operators, and no filling of new memory, which the operator does
+// under deterministic algorithms.
 bool dispatch_is_plain() {
   const auto keys = c10::impl::tls_local_dispatch_key_set();
-  return keys.included_ == c10::default_included_set && keys.excluded_ == c10::default_excluded_set && !at::hasCallbacks();
+  return keys.included_ == c10::default_included_set && keys.excluded_ == c10::default_excluded_set && !at::hasCallbacks() &&
+         !(at::globalContext().deterministicAlgorithms() && at::globalContext().deterministicFillUninitializedMemory());
 }
 at::Tensor fresh(at::IntArrayRef shape, at::ScalarType type, const at::Tensor& like) {
   if (!dispatch_is_plain()) return at::empty(shape, at::TensorOptions().dtype(type).device(like.device()));
