@@ -4089,11 +4089,22 @@ inline void normalise_splits(int k_steps, int want, int& splits, int& sps) {
   splits = (k_steps + sps - 1) / sps;
 }
 
+// What a step takes on rows off the 128-byte lines against rows on them, by configuration: the deep 128x128 form fetches them in whole lines from
+// kWindowSteps steps an item on, the others' pieces lie across two. Fitted to what the choice then costs: 1120 shapes of more than 256 rows,
+// every configuration in one to eight parts, operands from HBM. With one factor of 1.2 for all but the deep form, whatever its steps, the
+// choice is 3.9 % behind the quickest on average, with these 1.9, without any 6.2. (Medians of the launches alone 1.21, 1.14,
+// 1.34, 1.37, 1.38, 1.29 and, deep, 1.06: what a factor also makes up for is where a configuration's estimate on the lines is off.)
+// 3846x1656x2384 31.1 us with the one factor, 27.2 with these or none; 411x4682x10848 51.6 with the one or none, 46.3 with these.
+// Not on rows of fewer steps than kOffLinesMinSteps, where parts of few steps look like a gain that they are not: 563x64x752 in six 1.34 times
+// as long as in one.
+constexpr int kWindowSteps = 12, kOffLinesMinSteps = 16;
+constexpr float kOffLinesStep[kNumTileConfigs] = {1.2f, 1.4f, 1.34f, 1.3f, 1.23f, 1.2f, 1.08f}, kOffLinesWindowStep = 0.96f;
+
 // Estimated run time of a plan. Work items are dealt to 256 * wgs_per_cu workgroup slots in
 // rounds; a last round that fills at most one slot per CU runs at the faster stand-alone
 // rate. The operands cannot arrive faster than the configuration streams from HBM. Split
 // plans add a launch and the partial sums' trip through memory (written once, read once).
-inline float plan_cost_us(int64_t M, int64_t N, int64_t K, int config, int splits, int sps) {
+inline float plan_cost_us(int64_t M, int64_t N, int64_t K, bool off_lines, int config, int splits, int sps) {
   const TileConfig& c = kTileConfigs[config];
   const long tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
   const long items = tiles * splits;
@@ -4118,11 +4129,10 @@ inline float plan_cost_us(int64_t M, int64_t N, int64_t K, int config, int split
   // (128x256 tiles over fewer than 8 steps: what a launch costs before its first step is not in the table's 2.6 us a
   // tile, 2129 x 32 x 512 7.2 us with 17 tiles where 128x128 tiles take 5.2: such launches are left to those)
   const float us_per_item = config == 5 && items <= 2 * slots ? 7.0f : short_c3 ? 5.0f : config == 4 && sps < 8 ? 10.0f : c.us_per_item;
-  // (Rows off the lines, K standing in for the pitch: the deep form fetches them in whole lines, the others' steps take a fifth longer. In the deep
-  // form and in what came out ahead without this: 1317 x 1808 x 13392 51.7 and 66.1 us, 1323 x 1692 x 10352 43.3 and 57.3, 1504 x 943 x 14896 44.7 and
-  // 54.0, 458 x 3993 x 11456 41.0 and 47.1. Above the rows of the narrow tiles, whose own estimate knows of no pitch.)
-  const float off_lines = K % kStepK != 0 && config != kDeepSmallConfig && M > 256 ? 1.2f : 1.0f;
-  const float us_step = off_lines * (short_c3 ? 0.54f : c.us_per_step), us_step_alone = off_lines * (short_c3 ? 0.54f : c.us_per_step_alone);
+  // (Rows off the lines: see kOffLinesStep. Above the rows of the narrow tiles, whose own estimate has K stand in for the pitch.)
+  const bool windows = config == kDeepSmallConfig && sps >= kWindowSteps;
+  const float off = off_lines && M > kNarrowMaxM && k_steps_of(K) >= kOffLinesMinSteps ? (windows ? kOffLinesWindowStep : kOffLinesStep[config]) : 1.0f;
+  const float us_step = off * (short_c3 ? 0.54f : c.us_per_step), us_step_alone = off * (short_c3 ? 0.54f : c.us_per_step_alone);
   float t = full_rounds * (sps * us_step * step_scale + us_per_item);
   if (rest) t += sps * (rest <= kNumCu ? us_step_alone : us_step) * step_scale + us_per_item;
   // (the deep 128x128 form is for one round only; beyond 128 workgroups its steps slow down with the chip's
@@ -4158,7 +4168,7 @@ inline float plan_cost_us(int64_t M, int64_t N, int64_t K, int config, int split
 }
 
 // Cheapest plan by the model above; `max_splits` = 1 restricts it to plans without workspace.
-inline TiledPlan plan_tiled(int64_t M, int64_t N, int64_t K, int force_config, int force_splits,
+inline TiledPlan plan_tiled(int64_t M, int64_t N, int64_t K, bool off_lines, int force_config, int force_splits,
                             int max_splits) {
   const int k_steps = k_steps_of(K);
   TiledPlan best = {0, 1, k_steps, 0.0f};
@@ -4184,7 +4194,7 @@ inline TiledPlan plan_tiled(int64_t M, int64_t N, int64_t K, int force_config, i
       // 128 x 13312 x 2048 10.0 against 13.9; from HBM level with the 128x128 form), on large ones the policy wins
       // (64 x 28672 x 8192 from HBM: 51.7 us against 42.7).)
       if (c == kDeepSmallConfig && force_config < 0 && M <= 2 * 128 && N * K > (int64_t)48 << 20) continue;
-      const float cost = plan_cost_us(M, N, K, c, splits, sps);
+      const float cost = plan_cost_us(M, N, K, off_lines, c, splits, sps);
       if (best_cost < 0.0f || cost < best_cost) {
         best_cost = cost;
         best = {c, splits, sps, cost};
@@ -4196,10 +4206,10 @@ inline TiledPlan plan_tiled(int64_t M, int64_t N, int64_t K, int force_config, i
 
 // variant word: bits 0..7 kernel family, bits 8..15 tile configuration + 1 (0 = automatic),
 // bits 16..23 split-K factor (0 = automatic)
-inline TiledPlan plan_from_variant(int64_t M, int64_t N, int64_t K, int variant, int max_splits) {
+inline TiledPlan plan_from_variant(int64_t M, int64_t N, int64_t K, bool off_lines, int variant, int max_splits) {
   const int cfg = ((variant >> 8) & 0xff) - 1;
   const int spl = (variant >> 16) & 0xff;
-  return plan_tiled(M, N, K, cfg, spl, spl > 0 ? spl : max_splits);
+  return plan_tiled(M, N, K, off_lines, cfg, spl, spl > 0 ? spl : max_splits);
 }
 
 constexpr int kMaxDevices = 64;
@@ -4339,7 +4349,7 @@ int launch_tiled_epilogue(const GemmParams& p, hipStream_t s) {
   if constexpr (DEEP) {
     const long items = (long)((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN) * p.splits;
     const uintptr_t off = reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.b) | (uintptr_t)p.lda | (uintptr_t)p.ldb;
-    if (off % kStepK != 0 && items <= kNumCu && p.steps_per_split >= 12) {
+    if (off % kStepK != 0 && items <= kNumCu && p.steps_per_split >= kWindowSteps) {
       if (p.splits > 1) return launch_tiled<BM, BN, WAVES_M, WAVES_N, true, kEpiPartial, false, false, D + 1, false, false, false, true>(p, s);
       return p.bias ? launch_tiled<BM, BN, WAVES_M, WAVES_N, true, kEpiBias, false, false, D + 1, false, false, false, true>(p, s)
                     : launch_tiled<BM, BN, WAVES_M, WAVES_N, true, kEpiPlain, false, false, D + 1, false, false, false, true>(p, s);
@@ -4974,14 +4984,18 @@ struct Choices {
     return e.value;
   }
 };
+static_assert(kMaxSplits < 1 << 7, "the factor has seven bits of a plan's key");
 static_assert(Choices<int>::kEntries == 1 << (64 - 57), "the hash's top bits index the table");
 thread_local Choices<TiledPlan> known_plans;
 thread_local Choices<int> known_families;
 thread_local Choices<BlockPlan> known_block_plans;
 
-inline TiledPlan known_plan(int64_t M, int64_t N, int64_t K, int variant, int max_splits) {
+// (`pitch`: lda | ldb; the size queries, which know of no pitch, pass K)
+inline TiledPlan known_plan(int64_t M, int64_t N, int64_t K, int64_t pitch, int variant, int max_splits) {
   variant &= ~0xff;  // (the plan does not depend on the family's number)
-  return known_plans.get(M, N, K, (int64_t)variant << 8 | max_splits, [&] { return plan_from_variant(M, N, K, variant, max_splits); });
+  const bool off_lines = pitch % kStepK != 0;
+  return known_plans.get(M, N, K, (int64_t)variant << 8 | (int64_t)off_lines << 7 | max_splits,
+                         [&] { return plan_from_variant(M, N, K, off_lines, variant, max_splits); });
 }
 
 // (the size query and the call behind it ask for the same entry: 0.2 us for both without it, 0.04 with it, on a call of 4)
@@ -5012,7 +5026,7 @@ int mi355x_fp8_rowwise_select_variant(int64_t M, int64_t N, int64_t K) {
     // against 14.5); there a tiled plan has to be expected ahead by a tenth to be taken.
     // (above 64 rows the family's only member is the narrow-tile kernel in row blocks, where it fits)
     const float margin = M <= 8 ? 0.9f : 1.0f;
-    return known_plan(M, N, K, MI355X_FP8_VARIANT_AUTO, kMaxSplits).cost_us < margin * skinny_cost_us(M, N, K) ? MI355X_FP8_VARIANT_TILED
+    return known_plan(M, N, K, K, MI355X_FP8_VARIANT_AUTO, kMaxSplits).cost_us < margin * skinny_cost_us(M, N, K) ? MI355X_FP8_VARIANT_TILED
                                                                                                               : MI355X_FP8_VARIANT_SKINNY;
   });
 }
@@ -5027,7 +5041,7 @@ size_t mi355x_fp8_rowwise_workspace_bytes(int64_t M, int64_t N, int64_t K, int v
   }
   // (the skinny kernels reduce on chip)
   if ((variant & 0xff) != MI355X_FP8_VARIANT_TILED || K % 16 != 0) return 0;
-  const TiledPlan plan = known_plan(M, N, K, variant, kMaxSplits);
+  const TiledPlan plan = known_plan(M, N, K, K, variant, kMaxSplits);
   return plan.splits > 1 ? (size_t)plan.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
@@ -5096,10 +5110,10 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
     variant = mi355x_fp8_rowwise_select_variant(M, N, K);
     if (variant == MI355X_FP8_VARIANT_TILED && (M <= kSkinnyMaxM || narrow_fits(M, N, K))) {
       // the choice assumed the plan's workspace; without it the plan changes and may lose
-      const TiledPlan plan = known_plan(M, N, K, plan_bits, kMaxSplits);
+      const TiledPlan plan = known_plan(M, N, K, lda | ldb, plan_bits, kMaxSplits);
       const size_t need = plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0;
       if (need && (!workspace || workspace_bytes < need) &&
-          known_plan(M, N, K, plan_bits, 1).cost_us >= skinny_cost_us(M, N, K))
+          known_plan(M, N, K, lda | ldb, plan_bits, 1).cost_us >= skinny_cost_us(M, N, K))
         variant = MI355X_FP8_VARIANT_SKINNY;
     }
   }
@@ -5125,7 +5139,7 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
       {
         // A caller that brought no (or too little) workspace gets the best plan that needs none,
         // unless it asked for a split factor by name.
-        TiledPlan plan = known_plan(M, N, K, plan_bits, kMaxSplits);
+        TiledPlan plan = known_plan(M, N, K, lda | ldb, plan_bits, kMaxSplits);
         const size_t need = plan.splits > 1 ? (size_t)plan.splits * M * N * sizeof(float) : 0;
         if (need && (!workspace || workspace_bytes < need)) {
           if ((plan_bits >> 16) & 0xff)
@@ -5134,10 +5148,10 @@ int run_gemm(const void* a, const void* b, const float* a_scale, const float* b_
           // the cheapest plan whose partial planes fit what the caller brought (none: the unsplit plans)
           const size_t plane = (size_t)M * (size_t)N * sizeof(float);
           const size_t fit = workspace ? workspace_bytes / plane : 0;
-          plan = known_plan(M, N, K, plan_bits, fit < 1 ? 1 : fit > (size_t)kMaxSplits ? kMaxSplits : (int)fit);
+          plan = known_plan(M, N, K, lda | ldb, plan_bits, fit < 1 ? 1 : fit > (size_t)kMaxSplits ? kMaxSplits : (int)fit);
         }
         // (the partial sums of a tile are addressed with 32-bit byte offsets that must stay below 2^31)
-        if (plan.splits > 1 && N * 512 > (int64_t)INT32_MAX) plan = known_plan(M, N, K, plan_bits & 0xff00, 1);
+        if (plan.splits > 1 && N * 512 > (int64_t)INT32_MAX) plan = known_plan(M, N, K, lda | ldb, plan_bits & 0xff00, 1);
         if (plan.splits > 1 && (reinterpret_cast<uintptr_t>(workspace) & 15))
           return fail(MI355X_FP8_EINVAL, "workspace must be 16-byte aligned");
         p.splits = plan.splits;
