@@ -7,15 +7,21 @@ from tritonbench_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
-# By the estimates 64x64, 128x64 and 128x128 tiles whose waves share out K, then 128x128 and 64x64 tiles whose waves share out the tile
-SHAPES = [(130, 190, 640), (130, 190, 641), (130, 190, 767), (517, 3001, 896), (517, 3001, 897), (517, 3001, 1023), (900, 2990, 3968),
-          (900, 2990, 3969), (900, 2990, 4095), (1100, 20011, 256), (1100, 20011, 257), (1100, 20011, 383), (130, 3000, 128),
-          (130, 3000, 129), (130, 3000, 255), (130, 3000, 256)]
+# 64x64, 128x64 and 128x128 tiles whose waves share out K, then 128x128 and 64x64 tiles whose waves share out the tile
+FORMS = {
+    _lib.GENERIC_TILES_64_K: [(130, 190, 640), (130, 190, 641), (130, 190, 767)],
+    _lib.GENERIC_TILES_128X64_K: [(517, 3001, 896), (517, 3001, 897), (517, 3001, 1023)],
+    _lib.GENERIC_TILES_128_K: [(900, 2990, 3968), (900, 2990, 3969), (900, 2990, 4095)],
+    _lib.GENERIC_TILES_128: [(1100, 20011, 256), (1100, 20011, 257), (1100, 20011, 383)],
+    _lib.GENERIC_TILES_64: [(130, 3000, 128), (130, 3000, 129), (130, 3000, 255), (130, 3000, 256)],
+}
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("m,n,k,form", [(*s, form) for form, shapes in FORMS.items() for s in shapes])
 @pytest.mark.parametrize("shift,pitch", [(1, 0), (2, 3), (3, 2), (0, 1)])
-def test_rows_at_any_byte(gpu_device, m, n, k, shift, pitch):
+def test_rows_at_any_byte(gpu_device, m, n, k, form, shift, pitch):
+    assert _lib.load().mi355x_fp8_rowwise_generic_form(m, n, k) == form
+    assert _lib.load().mi355x_fp8_rowwise_workspace_bytes(m, n, k, _lib.VARIANT_GENERIC) == 0  # (in one piece)
     print(f"case m={m} n={n} k={k} shift={shift} pitch={pitch}", flush=True)
     g = torch.Generator(device=gpu_device).manual_seed(m + n + k)
 

@@ -4722,6 +4722,9 @@ static_assert(!generic_streams(1, 1 << 27, 1024) && generic_streams(1, (1 << 27)
 // 707x19781x241 38.8, 51.8, 40.4, 33.1 and 35.8; 134x20332x519 19.9, 25.5, 26.0, 21.4 and 16.6. The quickest of the five is missed by 0.3 % on
 // average, and by more than 7 % on 3 of the 180.
 enum GenericTiles { kGeneric64Shared, kGeneric128x64Shared, kGeneric128Shared, kGeneric128, kGeneric64 };
+static_assert(kGeneric64Shared + 1 == MI355X_FP8_GENERIC_TILES_64_K && kGeneric128x64Shared + 1 == MI355X_FP8_GENERIC_TILES_128X64_K &&
+              kGeneric128Shared + 1 == MI355X_FP8_GENERIC_TILES_128_K && kGeneric128 + 1 == MI355X_FP8_GENERIC_TILES_128 &&
+              kGeneric64 + 1 == MI355X_FP8_GENERIC_TILES_64, "the query's names, behind the streaming form's");
 struct GenericChoice {
   GenericTiles tiles;
   float us;
@@ -5462,6 +5465,12 @@ int mi355x_fp8_rowwise_grouped_form(int64_t G, int64_t M, int64_t N, int64_t K) 
   if (st != MI355X_FP8_OK) return st;
   if (G < 1 || G > 65536) return fail(MI355X_FP8_EINVAL, "G must be in 1..65536 (got %lld)", (long long)G);
   return grouped_form(G, M, N, K, K);
+}
+
+int mi355x_fp8_rowwise_generic_form(int64_t M, int64_t N, int64_t K) {
+  const int st = check_shape(M, N, K);
+  if (st != MI355X_FP8_OK) return st;
+  return generic_streams(M, N, K) ? MI355X_FP8_GENERIC_STREAM : generic_tiles(M, N, K).tiles + 1;
 }
 
 int mi355x_fp8_blockwise_form(int64_t M, int64_t N, int64_t K) {
