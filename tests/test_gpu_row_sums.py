@@ -12,7 +12,7 @@ from test_gpu_row_forms import _repeated, _same_rows
 pytestmark = pytest.mark.gpu
 
 # rows of 16-byte chunks on both sides of each line of the order and of the forms
-CHUNKS = [2, 64, 66, 128, 130, 192, 194, 256, 258, 512, 514, 768, 770, 1024, 1026, 1280, 1282, 1536, 1538, 2048, 2050, 3072, 3074, 4096, 4098, 8192, 8194]
+CHUNKS = [2, 64, 66, 128, 130, 192, 194, 256, 258, 512, 514, 768, 770, 1024, 1026, 1280, 1282, 1536, 1538, 2048, 2050, 2560, 2562, 3072, 3074, 3584, 3586, 4096, 4098, 8192, 8194]
 
 
 def _sum_of_squares(x):

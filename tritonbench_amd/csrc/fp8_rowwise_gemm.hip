@@ -3614,6 +3614,9 @@ constexpr int kFusedRmsNorm = 0, kFusedSiluMul = 1;
 // as by this many lanes, of which lane o adds up chunks o, o + S, o + 2 S, ... element by element in one chain, then the lanes of each
 // 64 pairwise from bit 5 of their numbers down to bit 0, then the 64s one after another.
 constexpr int rms_sum_lanes(int64_t chunks) { return chunks <= 256 ? 64 : chunks <= 1024 ? 256 : chunks <= 4096 ? 512 : 1024; }
+// Whether a form of the RMSNorm kernel asks for the weights beside x. (With 512 lanes and 8 chunks each the weights' registers cost more than
+// the second trip, 8192 x 28672 245 us with them, 167 without, and 1024 lanes have 128 registers each and none to spare.)
+constexpr bool rms_early_weights(int lanes, int chunks) { return lanes <= 256 || (lanes == 512 && chunks <= 4); }
 
 template <int OP, int CACHE, int THREADS, int ROWS = 1>
 __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(const uint16_t* x1, const uint16_t* x2,
@@ -3622,15 +3625,13 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
   static_assert(ROWS == 1 || THREADS == 64, "several rows per workgroup: one wave each (as in the quantiser)");
   using V = VecTraits<uint16_t>;
   constexpr int EPV = 8;
-  // A form with more lanes than the sum's order has (HANDS times as many) hands a chain on from lane to lane, and one with fewer has CHAINS
-  // of them in each lane. (A chain's lanes are in one wave, a row of 16 or a half each, where handing on is one instruction. All of them
-  // add at each turn, which costs 0.2 us: 32x8192 with 1024 lanes 3.58 us cold in an order of its own, 3.79 in this one, where the 256 lanes
-  // of the order take 5.11.)
+  // Rows of up to 256 chunks on 256 lanes, with one chunk each: the order's 64 lanes are 64 chains that four lanes of a wave hand on, one in each
+  // row of 16, where that is one instruction. (All of them add at each turn. 32x2048 2.71 us, on 64 lanes with four chunks 3.26.)
   constexpr int SUM_LANES = OP == kFusedRmsNorm ? rms_sum_lanes((int64_t)THREADS * CACHE) : THREADS;
-  constexpr int HANDS = THREADS > SUM_LANES ? THREADS / SUM_LANES : 1, CHAINS = SUM_LANES > THREADS ? SUM_LANES / THREADS : 1;
-  static_assert(HANDS <= 2 || (HANDS == 4 && CACHE == 1), "a chain starts in the first row or half, and with two hands it comes back to it");
+  constexpr bool HANDED_ON = SUM_LANES != THREADS;
+  static_assert(!HANDED_ON || (SUM_LANES == 64 && THREADS == 256 && CACHE == 1), "the other forms have the lanes of the order");
   __shared__ float wave_part[THREADS / 64];
-  __shared__ __attribute__((aligned(16))) float sum_part[HANDS > 1 ? SUM_LANES : THREADS / 64 * CHAINS];  // (of its own: no wait for the other's readers)
+  __shared__ __attribute__((aligned(16))) float sum_part[HANDED_ON ? SUM_LANES : THREADS / 64];  // (of its own: no wait for the other's readers)
   const long row = (long)blockIdx.x * ROWS + (ROWS > 1 ? (long)(threadIdx.x >> 6) : 0);
   if (ROWS > 1 && row >= rows) return;  // (whole waves; this form has no barrier)
   const v4i* r1 = (const v4i*)(x1 + row * ld1);
@@ -3640,22 +3641,19 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
   const int nchunks = K / EPV;
   const int tid = ROWS > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
   const int lane = tid & 63;
-  // Round i of lane t is chunk first_chunk(t) + THREADS * i. Four hands: the turns of a wave's rows are 0, 1, 3, 2, so that each has its
-  // neighbour's in the other row of its pair or in the other half.
-  constexpr int WAVE_CHAINS = 64 / HANDS;
-  auto turn_of = [](int t) { return HANDS == 4 ? (t & 63) / 16 ^ (t & 63) / 32 : (t & 63) / WAVE_CHAINS; };
-  auto chain_of = [](int t) { return (t >> 6) * WAVE_CHAINS + t % WAVE_CHAINS; };
-  auto first_chunk = [&](int t) { return HANDS == 1 ? t : chain_of(t) + SUM_LANES * turn_of(t); };
+  // Round i of lane t is chunk first_chunk(t) + THREADS * i. (Handed on: the rows of a wave have turns 0, 1, 3, 2, so that each finds what it goes
+  // on with in the other row of its pair or in the other half.)
+  auto turn_of = [](int t) { return (t & 63) / 16 ^ (t & 63) / 32; };
+  auto first_chunk = [&](int t) { return HANDED_ON ? (t >> 6) * 16 + t % 16 + SUM_LANES * turn_of(t) : t; };
   const int at = first_chunk(tid);
+  const int rest = HANDED_ON ? nchunks : tid + THREADS * CACHE;  // what the registers do not hold (0.1 us of a call of 2 where there never is any)
   // (hardware exponential and reciprocal, about one ulp each: the result is rounded to 4 significant
   // bits next; the library exponential costs six times the instructions and a correctly rounded
   // quotient ten, which together made the kernel compute-bound)
   auto silu_mul = [](float a, float b) -> float { return (a * __builtin_amdgcn_rcpf(1.0f + __expf(-a))) * b; };
 
   float vals[CACHE][EPV];
-  // (the 1024-lane form has 128 registers per lane and none to spare for them; with 512 lanes and 8 chunks each the
-  // weights' registers cost more than the second trip: 8192 x 28672 245 us with them, 167 without)
-  constexpr bool EARLY_WEIGHTS = OP == kFusedRmsNorm && (THREADS <= 256 || (THREADS == 512 && CACHE <= 4));
+  constexpr bool EARLY_WEIGHTS = OP == kFusedRmsNorm && rms_early_weights(THREADS, CACHE);
   v4i wts[EARLY_WEIGHTS ? CACHE : 1];
   float rstd = 0.0f;
   if (OP == kFusedRmsNorm) {
@@ -3673,53 +3671,38 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
       for (int e = 0; e < EPV; ++e) s = __builtin_fmaf(f[e], f[e], s);
       return s;
     };
-    float sums[CHAINS] = {};
-#pragma unroll
-    for (int i = 0; i < CACHE; ++i) {
-      float& s = sums[i % CHAINS];
-#pragma unroll
-      for (int turn = 0; turn < HANDS; ++turn) {
-        if (HANDS == 2 && i + turn > 0) s = turn == 1 ? halves_of_wave(s).lower : halves_of_wave(s).upper;
-        if (HANDS == 4 && turn > 0) s = turn == 1 ? rows_of_pair(s).lower : turn == 2 ? halves_of_wave(s).lower : rows_of_pair(s).upper;
-        const float with = add_squares(vals[i], s);
-        s = at + THREADS * i < nchunks ? with : s;
-      }
-    }
-    auto add = [](float a, float b) { return a + b; };
     float ss = 0.0f;
-    if constexpr (HANDS > 1) {
-      // the chains' sums, those of the lanes that are added first beside one another: a row of lanes takes 64 of them
-      const int chain = chain_of(tid);
-      if (turn_of(tid) == HANDS - 1) sum_part[chain / 64 * 64 + chain % 16 * 4 + chain % 64 / 16] = sums[0];
-      __syncthreads();
-      constexpr int GROUPS = SUM_LANES / 64;
+    auto add = [](float a, float b) { return a + b; };
+    if constexpr (HANDED_ON) {
 #pragma unroll
-      for (int g = 0; g < GROUPS; g += 4) {
-        const v4f four = *(const v4f*)(sum_part + min(g + lane / 16, GROUPS - 1) * 64 + lane % 16 * 4);
-        const float group = row_reduce((four[0] + four[2]) + (four[1] + four[3]), add);
-#pragma unroll
-        for (int r = 0; r < 4 && g + r < GROUPS; ++r) {
-          const float one = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(group), 16 * r));
-          ss = g + r == 0 ? one : ss + one;
-        }
+      for (int turn = 0; turn < 4; ++turn) {
+        if (turn > 0) ss = turn == 1 ? rows_of_pair(ss).lower : turn == 2 ? halves_of_wave(ss).lower : rows_of_pair(ss).upper;
+        const float with = add_squares(vals[0], ss);
+        ss = at < nchunks ? with : ss;
       }
+      // the chains' sums, those of the lanes that are added first beside one another
+      if (turn_of(tid) == 3) sum_part[lane % 16 * 4 + (tid >> 6)] = ss;
+      __syncthreads();
+      const v4f four = *(const v4f*)(sum_part + lane % 16 * 4);
+      ss = row_reduce((four[0] + four[2]) + (four[1] + four[3]), add);
     } else {
-      for (int c = tid + THREADS * CACHE; c < nchunks; c += THREADS) {
+#pragma unroll
+      for (int i = 0; i < CACHE; ++i) {
+        const float with = add_squares(vals[i], ss);
+        ss = at + THREADS * i < nchunks ? with : ss;
+      }
+      for (int c = rest; c < nchunks; c += THREADS) {
         float f[EPV];
         V::unpack(r1[c], f);
-        sums[0] = add_squares(f, sums[0]);
+        ss = add_squares(f, ss);
       }
-      ss = wave_reduce(sums[0], add);
-      if constexpr (THREADS > 64) {
-#pragma unroll
-        for (int chain = 0; chain < CHAINS; ++chain) {
-          const float of_wave = chain == 0 ? ss : wave_reduce(sums[chain], add);
-          if (lane == 0) sum_part[chain * (THREADS / 64) + (tid >> 6)] = of_wave;
-        }
+      ss = wave_reduce(ss, add);
+      if (THREADS > 64) {
+        if (lane == 0) sum_part[tid >> 6] = ss;
         __syncthreads();
         ss = sum_part[0];
 #pragma unroll
-        for (int w = 1; w < THREADS / 64 * CHAINS; ++w) ss += sum_part[w];
+        for (int w = 1; w < THREADS / 64; ++w) ss += sum_part[w];
       }
     }
     rstd = 1.0f / sqrtf(ss / (float)K + eps);
@@ -3746,8 +3729,6 @@ __global__ __launch_bounds__(THREADS* ROWS) void fused_rowwise_quant_kernel(cons
 #pragma unroll
     for (int e = 0; e < EPV; ++e) amax = max_keep_nan(amax, fabsf(vals[i][e]));
   }
-  // (what the registers do not hold: rows of a form with HANDS never have any)
-  const int rest = HANDS == 1 ? tid + THREADS * CACHE : nchunks;
   for (int c = rest; c < nchunks; c += THREADS) {
     float a[EPV], b[EPV], y[EPV];
     V::unpack(r1[c], a);
@@ -5228,25 +5209,41 @@ constexpr int kWaveRows = 4;
 
 // How a row's chunks of 16 bytes are dealt out by the quantiser and the fused front ends (rows that start 16-byte aligned): `lanes` of them,
 // `chunks` rounds each that stay in registers; 64 lanes are a wave, kWaveRows rows a workgroup. Any form takes any row (what the registers don't
-// hold is read again; RMSNorm: a row of its order of the sum, if it has other lanes than that), so the rule is about speed alone:
+// hold is read again), so the rule is about speed alone, but for RMSNorm, whose lanes are those of the order of its sum or hand its chains on:
 //  - no round is idle if it can be helped, for it loads and computes like any other: rows just above a power of two had up to half of them
-//    idle (RMSNorm 8192x8960 56.5 us as 4 rounds of 512, 42.8 as 5 of 256; SiLU-mul 2048x19904 41.4 and 34.7; f32 8192x9472 72.7 and 60.6);
-//  - up to one row a CU, what counts is the chain of a single row, and one round of as many lanes as that takes is the shortest (RMSNorm
-//    32x8192 4.64 us as 4 rounds of 256, 3.50 as one of 1024; SiLU-mul 32x4096 4.89 as 8 of 64, 2.69 as one of 512);
-//  - with more rows, fewer lanes with more rounds: 256x4 against 1024x1 is 36.3 and 48.4 us on 8192x8192, waves of 4 rounds against 256x1
-//    12.9 and 14.1 on 8192x2048, but 6.2 and 5.6 on 2048x2048.
+//    idle (SiLU-mul 2048x19904 41.4 and 34.7; f32 8192x9472 72.7 and 60.6);
+//  - up to one row a CU, what counts is the chain of a single row, and one round of as many lanes as that takes is the shortest (SiLU-mul
+//    32x4096 4.89 as 8 of 64, 2.69 as one of 512). RMSNorm's second reduction makes that as long: cold 32x8192 3.49 us as 4 rounds of 256, 3.51
+//    as 2 of 512 that hand on, 3.75 as one of 1024, 32x10240 3.78 as 3 of 512, 4.23 as 2 of 1024, so it keeps the lanes of its order;
+//  - with more rows, fewer lanes with more rounds: RMSNorm 256x4 against 1024x1 is 35.5 and 53.0 us on 8192x8192, waves of 4 rounds against
+//    256x1 11.0 and 14.3 on 8192x2048.
 // Measured on 21 row lengths from 512 to 28672 with 1 to 8192 rows, every form whose rounds hold the row.
 enum RowSource { kRowF32, kRowBf16, kRowRmsNorm, kRowSiluMul };
 struct RowForm {
   int lanes, chunks;
 };
 constexpr bool row_form_exists(RowSource source, int lanes, int chunks) {
+  if (source == kRowRmsNorm) return lanes <= 256 ? chunks <= 4 : lanes == 512 ? chunks == 8 || (chunks >= 3 && chunks <= 6) : chunks == 8;
   if (lanes == 64) return chunks <= 4 || (source == kRowF32 && (chunks == 6 || chunks == 8));
   if (lanes == 256) return chunks <= 5;
-  if (lanes == 512) return chunks <= 8 && (chunks < 7 || source != kRowSiluMul) && (chunks != 7 || source != kRowRmsNorm);
+  if (lanes == 512) return chunks <= 8 && (chunks < 7 || source != kRowSiluMul);
   return chunks <= 4 || (source == kRowF32 && chunks <= 7) || (source != kRowBf16 && chunks == 8);
 }
+constexpr RowForm rms_row_form(int64_t R, int64_t chunks) {
+  if (chunks > 4096) return {1024, 8};
+  if (chunks > 256) {
+    const int lanes = rms_sum_lanes(chunks), rounds = (int)((chunks + lanes - 1) / lanes);
+    // (a round of its own at the end costs few rows more than an idle one, cold 32x20480 5.48 us as five, 4.78 as six, 32x28672 6.55 as seven, 5.42 as
+    // eight; many rows not, 2048x20480 27.2 and 27.8, but for seven, 38.8 and 37.1)
+    return {lanes, rounds == 7 || (rounds == 5 && R <= kNumCu) ? rounds + 1 : rounds};
+  }
+  if (chunks <= 64) return {64, 1};
+  // (256x1 and 64x4 on rows of 2048: 512 rows 3.27 and 3.56 us, 1024 4.02 and 3.93, 2048 5.42 and 5.16; on rows of 1536 level with 512)
+  if (R <= kNumCu || (chunks > 192 && R <= 2 * kNumCu)) return {256, 1};
+  return {64, (int)((chunks + 63) / 64)};
+}
 constexpr RowForm row_form(RowSource source, int64_t R, int64_t chunks) {
+  if (source == kRowRmsNorm) return rms_row_form(R, chunks);
   if (chunks > 4096) {  // (bf16 rows hold half the values in as many registers as f32 ones: more rounds than 4 halve their rate)
     if (source == kRowBf16) return {1024, 4};
     if (source == kRowF32 && chunks <= 7168) return {1024, (int)((chunks + 1023) / 1024)};
@@ -5267,7 +5264,7 @@ constexpr RowForm row_form(RowSource source, int64_t R, int64_t chunks) {
   if (chunks <= 1280 && many) return {256, 5};
   if (chunks <= 3072) return {512, (int)((chunks + 511) / 512)};
   if (source == kRowSiluMul) return {1024, 4};
-  return {512, chunks <= 3584 && source != kRowRmsNorm ? 7 : 8};
+  return {512, chunks <= 3584 ? 7 : 8};
 }
 // Rows of a launch, which holds fewer than 2^32 lanes (256 a row: 16777212 rows). More of them are several launches of the same form.
 constexpr int64_t rows_per_launch(int64_t lanes) { return (int64_t)UINT32_MAX / lanes / kWaveRows * kWaveRows; }
@@ -5288,6 +5285,7 @@ constexpr bool row_forms_are_sound() {  // (the rule's lines lie at multiples of
           const int64_t held = (int64_t)f.lanes * f.chunks;
           if (source == kRowRmsNorm && c > held && rms_sum_lanes(held) != f.lanes) return false;
           if (source == kRowRmsNorm && rms_sum_lanes(held) != rms_sum_lanes(c)) return false;
+          if (source == kRowRmsNorm && c <= 2048 && !rms_early_weights(f.lanes, f.chunks)) return false;
         }
     for (int lanes : {64, 256, 512, 1024})
       for (int chunks = 1; chunks <= 8; ++chunks)
@@ -5295,8 +5293,8 @@ constexpr bool row_forms_are_sound() {  // (the rule's lines lie at multiples of
   }
   return true;
 }
-static_assert(row_forms_are_sound(), "a row without a kernel would not be quantised, and in another order of its sum not as among other rows; "
-                                     "a kernel without a row is code that nothing runs");
+static_assert(row_forms_are_sound(), "a row without a kernel would not be quantised, and in another order of its sum not as among other rows; without "
+                                     "its weights beside x it takes a second trip; a kernel without a row is code that nothing runs");
 
 // Calls launch(lanes, chunks), as integral constants, for the form.
 template <RowSource SOURCE, int LANES = 64, int CHUNKS = 1, typename Launch>
