@@ -25,9 +25,15 @@ def test_the_entry_with_a_workspace_refuses_other_forms_and_factors_without_spac
 
 
 # what the query names can be pinned, and is what the library's choice runs: the form that keeps A on chip has a name of its own
-@pytest.mark.parametrize("m,n,k", [(16, 8192, 8192), (1, 16, 8192), (16, 144, 8192), (9, 160, 6160), (16, 4240, 2000), (16, 8176, 4096)])
+@pytest.mark.parametrize("m,n,k", [(16, 8192, 8192), (16, 144, 8192), (9, 160, 6160), (16, 4240, 2000), (16, 8192, 3600), (11, 8000, 6000)])
 def test_the_form_that_keeps_a_on_chip_is_named(m, n, k):
     assert _lib.load().mi355x_fp8_blockwise_form(m, n, k) == _lib.BLOCK_RESIDENT
+
+
+# (where it is 7 to 15 % behind one tile a workgroup)
+@pytest.mark.parametrize("m,n,k", [(2, 1600, 3648), (16, 2528, 3264), (4, 336, 3376), (8, 1088, 4592), (4, 5376, 3584), (2, 256, 3600), (8, 320, 3536)])
+def test_the_form_that_keeps_a_on_chip_is_left_where_it_is_behind(m, n, k):
+    assert _lib.load().mi355x_fp8_blockwise_form(m, n, k) == _lib.BLOCK_ONE_TILE
 
 
 @pytest.mark.parametrize("shape", [(17, 64, 1024), (16, 72, 1024), (16, 8208, 64), (16, 16, 8208)])
