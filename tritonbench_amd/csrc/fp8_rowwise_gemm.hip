@@ -4071,15 +4071,21 @@ inline void normalise_splits(int k_steps, int want, int& splits, int& sps) {
 }
 
 // What a step takes on rows off the 128-byte lines against rows on them, by configuration: the deep 128x128 form fetches them in whole lines from
-// kWindowSteps steps an item on, the others' pieces lie across two. Fitted to what the choice then costs: 1120 shapes of more than 256 rows,
+// kWindowSteps steps an item on, the others' pieces lie across two. Fitted to what the choice then costs: 1380 shapes of more than 256 rows,
 // every configuration in one to eight parts, operands from HBM. With one factor of 1.2 for all but the deep form, whatever its steps, the
-// choice is 3.9 % behind the quickest on average, with these 1.9, without any 6.2. (Medians of the launches alone 1.21, 1.14,
+// choice is 3.5 % behind the quickest on average, with these 1.7, without any 5.6. (Medians of the launches alone 1.21, 1.14,
 // 1.34, 1.37, 1.38, 1.29 and, deep, 1.06: what a factor also makes up for is where a configuration's estimate on the lines is off.)
 // 3846x1656x2384 31.1 us with the one factor, 27.2 with these or none; 411x4682x10848 51.6 with the one or none, 46.3 with these.
 // Not on rows of fewer steps than kOffLinesMinSteps, where parts of few steps look like a gain that they are not: 563x64x752 in six 1.34 times
 // as long as in one.
 constexpr int kWindowSteps = 12, kOffLinesMinSteps = 16;
-constexpr float kOffLinesStep[kNumTileConfigs] = {1.2f, 1.4f, 1.34f, 1.3f, 1.23f, 1.2f, 1.08f}, kOffLinesWindowStep = 0.96f;
+inline float off_lines_step(int config, int64_t M, int splits, int sps) {
+  static const float step[kNumTileConfigs] = {1.14f, 1.4f, 1.3f, 1.3f, 1.17f, 1.2f, 1.08f};
+  if (config == kDeepSmallConfig && sps >= kWindowSteps) return 0.96f;
+  if (config == 0 && splits > 1) return 1.22f;  // (512x10884x8096 in two 1.17 times as long as 256x128 tiles in one)
+  if (config == 4 && M <= 512) return 1.29f;    // (484x12572x5520 60.2 us, on 256x128 tiles, whose second row is not full, 52.8)
+  return step[config];
+}
 
 // Estimated run time of a plan. Work items are dealt to 256 * wgs_per_cu workgroup slots in
 // rounds; a last round that fills at most one slot per CU runs at the faster stand-alone
@@ -4110,9 +4116,8 @@ inline float plan_cost_us(int64_t M, int64_t N, int64_t K, bool off_lines, int c
   // (128x256 tiles over fewer than 8 steps: what a launch costs before its first step is not in the table's 2.6 us a
   // tile, 2129 x 32 x 512 7.2 us with 17 tiles where 128x128 tiles take 5.2: such launches are left to those)
   const float us_per_item = config == 5 && items <= 2 * slots ? 7.0f : short_c3 ? 5.0f : config == 4 && sps < 8 ? 10.0f : c.us_per_item;
-  // (Rows off the lines: see kOffLinesStep. Above the rows of the narrow tiles, whose own estimate has K stand in for the pitch.)
-  const bool windows = config == kDeepSmallConfig && sps >= kWindowSteps;
-  const float off = off_lines && M > kNarrowMaxM && k_steps_of(K) >= kOffLinesMinSteps ? (windows ? kOffLinesWindowStep : kOffLinesStep[config]) : 1.0f;
+  // (Rows off the lines: see off_lines_step. Above the rows of the narrow tiles, whose own estimate has K stand in for the pitch.)
+  const float off = off_lines && M > kNarrowMaxM && k_steps_of(K) >= kOffLinesMinSteps ? off_lines_step(config, M, splits, sps) : 1.0f;
   const float us_step = off * (short_c3 ? 0.54f : c.us_per_step), us_step_alone = off * (short_c3 ? 0.54f : c.us_per_step_alone);
   float t = full_rounds * (sps * us_step * step_scale + us_per_item);
   if (rest) t += sps * (rest <= kNumCu ? us_step_alone : us_step) * step_scale + us_per_item;
