@@ -122,7 +122,8 @@ const char* mi355x_fp8_rowwise_last_error(void);
 int mi355x_fp8_rowwise_select_variant(int64_t M, int64_t N, int64_t K);
 
 /* Bytes of device workspace `variant` needs for this shape (0 when none): the fp32 partial sums of the TILED and GENERIC plans that
- * cut K. Pure host arithmetic: callable without a device. It knows the sizes only: for AUTO with K a multiple of 16 the answer is that
+ * cut K. Pure host arithmetic: callable without a device. It knows the sizes only: with K no multiple of 128 the answer is enough for rows of
+ * K bytes and for rows padded to whole 128-byte lines, of which either may use less; for AUTO with K a multiple of 16 it is that
  * of the family for operands which meet the alignment requirements. Others run in the GENERIC family, in as many parts as that
  * many bytes hold for it, or in one piece; ask for VARIANT_GENERIC by name to bring it the workspace of its own plan. */
 size_t mi355x_fp8_rowwise_workspace_bytes(int64_t M, int64_t N, int64_t K, int variant);

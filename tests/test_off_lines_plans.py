@@ -17,23 +17,38 @@ def test_short_rows_stay_whole(m, n, k):
     assert _planes(m, n, k) == _planes(m, n, -(-k // 128) * 128) == 0
 
 
+# (cut into more parts on the lines than off them)
+@pytest.mark.parametrize("m,n,k", [(10605, 243, 10720), (1196, 205, 11840), (522, 3880, 10208), (265, 9949, 17568), (6219, 248, 12656), (515, 818, 2256),
+                                   (303, 142, 9328), (1568, 2132, 19312), (4805, 553, 23088), (283, 3747, 26224), (8276, 300, 21536)])
+def test_the_query_is_enough_for_padded_rows(m, n, k):
+    """The query knows of no pitch: it names as many planes as rows want that are padded onto the lines."""
+    assert _planes(m, n, k) >= _planes(m, n, -(-k // 128) * 128) > 0
+
+
+# (`other`: on the lines another number of parts than off them)
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k", [(1447, 3247, 6864), (2052, 1168, 14048), (1000, 3000, 4112), (317, 825, 3312), (6603, 16, 1440), (1447, 3247, 6912)])
-@pytest.mark.parametrize("side", ["on", "off"])
-def test_the_plan_is_by_the_pitch(gpu_device, m, n, k, side):
-    """As many parts as for rows that fill the pitch, off the lines as the query says, and the product is right."""
-    lines = -(-k // 128) * 128
-    ld = lines if side == "on" else k if k % 128 else k + 16
-    want = _planes(m, n, lines) if side == "on" else _planes(m, n, k if k % 128 else k + 16 - 128)  # (a step's worth: off the lines, as many steps)
-    print(f"case {m}x{n}x{k} pitch {ld}: {want} planes", flush=True)
+@pytest.mark.parametrize("m,n,k,other", [(1447, 3247, 6864, True), (2052, 1168, 14048, True), (522, 3880, 10208, True), (317, 825, 3312, True),
+                                         (1000, 3000, 4112, False), (6603, 16, 1440, False), (1447, 3247, 6912, True)])
+def test_the_plan_is_by_the_pitch(gpu_device, m, n, k, other):
+    """With the workspace that the query names: rows that are or are padded onto the lines in as many parts as rows that fill the pitch, and
+    the product is right on either pitch."""
     g = torch.Generator(device=gpu_device).manual_seed(m)
-    a, b = (torch.randn((r, ld), generator=g, device=gpu_device).to(torch.float8_e4m3fn)[:, :k] for r in (m, n))
-    sa, sb = (torch.rand(r, generator=g, device=gpu_device) + 0.5 for r in (m, n))
-    space = torch.full((16, m, n), float("nan"), device=gpu_device)
-    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
-    _lib.check(_lib.load().mi355x_fp8_rowwise_gemm(a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), None, out.data_ptr(), m, n, k, ld, ld, n,
-                                                   space.data_ptr(), 64 * m * n, AUTO, torch.cuda.current_stream().cuda_stream), "gemm")
-    torch.cuda.synchronize()
-    assert int(torch.isfinite(space).flatten(1).all(1).sum()) == want
-    exact = (a.double() @ b.double().t()) * sa.double()[:, None] * sb.double()[None, :]
-    assert ((out.double() - exact).norm() / exact.norm()).item() < 2.0**-8  # (one rounding to bf16)
+    on = -(-k // 128) * 128
+    written = {}
+    for ld in (on, k if k % 128 else k + 16):
+        print(f"case {m}x{n}x{k} pitch {ld}", flush=True)
+        a, b = (torch.randn((r, ld), generator=g, device=gpu_device).to(torch.float8_e4m3fn)[:, :k] for r in (m, n))
+        sa, sb = (torch.rand(r, generator=g, device=gpu_device) + 0.5 for r in (m, n))
+        need = 4 * m * n * _planes(m, n, k)
+        space = torch.full((16, m, n), float("nan"), device=gpu_device)
+        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+        _lib.check(_lib.load().mi355x_fp8_rowwise_gemm(a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), None, out.data_ptr(), m, n, k,
+                                                       ld, ld, n, space.data_ptr(), need if k % 128 else space.nbytes, AUTO,
+                                                       torch.cuda.current_stream().cuda_stream), "gemm")
+        torch.cuda.synchronize()
+        written[ld] = int(torch.isfinite(space).flatten(1).all(1).sum())
+        exact = (a.double() @ b.double().t()) * sa.double()[:, None] * sb.double()[None, :]
+        assert ((out.double() - exact).norm() / exact.norm()).item() < 2.0**-8  # (one rounding to bf16)
+    parts_on = written.pop(on)
+    assert parts_on == _planes(m, n, on)
+    assert (written.popitem()[1] != parts_on) == other

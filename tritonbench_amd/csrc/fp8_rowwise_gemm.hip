@@ -4989,7 +4989,7 @@ thread_local Choices<TiledPlan> known_plans;
 thread_local Choices<int> known_families;
 thread_local Choices<BlockPlan> known_block_plans;
 
-// (`pitch`: lda | ldb; the size queries, which know of no pitch, pass K)
+// (`pitch`: lda | ldb)
 inline TiledPlan known_plan(int64_t M, int64_t N, int64_t K, int64_t pitch, int variant, int max_splits) {
   variant &= ~0xff;  // (the plan does not depend on the family's number)
   const bool off_lines = pitch % kStepK != 0;
@@ -5040,8 +5040,10 @@ size_t mi355x_fp8_rowwise_workspace_bytes(int64_t M, int64_t N, int64_t K, int v
   }
   // (the skinny kernels reduce on chip)
   if ((variant & 0xff) != MI355X_FP8_VARIANT_TILED || K % 16 != 0) return 0;
-  const TiledPlan plan = known_plan(M, N, K, K, variant, kMaxSplits);
-  return plan.splits > 1 ? (size_t)plan.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
+  // (the pitch is not known here: enough for rows of K bytes and for rows padded onto the lines, whose plan can have more parts)
+  int splits = known_plan(M, N, K, K, variant, kMaxSplits).splits;
+  if (K % kStepK != 0) splits = std::max(splits, known_plan(M, N, K, 0, variant, kMaxSplits).splits);
+  return splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
 int mi355x_fp8_rowwise_gemm(const void* a, const void* b, const float* a_scale, const float* b_scale,
