@@ -42,6 +42,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 #include <string.h>
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -1734,8 +1735,8 @@ __global__ __launch_bounds__(256) void splitk_finalize_rows_kernel(GemmParams p)
 // exact (e4m3fn reaches from 2^-9 to 448), and f32 accumulation that is as accurate as a chain of f32
 // multiply-adds (measured over K = 1024 standard normal codes: 4e-8 of the result's norm for both,
 // 1.5e-5 for the fp8 matrix instructions, which align a group of products before they add). One
-// conversion instruction of 8 cycles widens two codes, and the conversions are what bounds the tiles (4096x8192x2047:
-// 840 TFLOP/s, 0.34 of the 16-bit matrix rate). Against byte loads and f32 multiply-adds on the
+// conversion instruction of 8 cycles widens two codes, and over many rounds of tiles the conversions are what bounds them (4096x8192x2047:
+// 810 TFLOP/s, 0.32 of the 16-bit matrix rate). Against byte loads and f32 multiply-adds on the
 // vector ALU, which this family was at first, 517x3000x1041 took 212 us.
 // ------------------------------------------------------------------------------------
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
@@ -1796,8 +1797,11 @@ __device__ __forceinline__ v8h e4m3fn_to_f16x8(int lo, int hi) {
 // at the end of K is multiplied first, so that the loop over whole steps has no conditional loads (its wait
 // counts are then exact and DEPTH steps stay in flight).
 //
-// What bounds it is the vector ALU, which widens every fragment in each wave that multiplies it (an instruction of 8 cycles for two codes):
-// with 2x2 waves of 32x32 on a 64x64 tile 64 of them a step and wave beside 8 MFMAs of 32 cycles. Waves that share out a step's K
+// What bounds it over many rounds of tiles is the vector ALU, which widens every fragment in each wave that multiplies it (an instruction of 8 cycles
+// for two codes), beside MFMAs that it hardly overlaps with: of the 340000 cycles of 4096x8192x2047 on 128x128 tiles a SIMD converts for 133000, has
+// 57000 of other vector instructions and 131000 of MFMAs. One round on short rows waits instead, for its first data and at its few barriers: waves of
+// 517x3000x1041 are in s_waitcnt for half of their time. With 2x2 waves of 32x32 on a 64x64 tile it is 64 conversions a step and wave beside 8 MFMAs of
+// 32 cycles. Waves that share out a step's K
 // instead (WAVES_K) widen nothing twice and have wave tiles of twice the size, for one exchange of the sums at the end: 517x3000x1041 with
 // its bias 16.7 -> 14.3 us, 517x3000x4113 36.6 -> 28.4, 1000x3000x4111 52.9 -> 39.4. Where tiles of 64x64 a wave are several rounds
 // of the chip the exchange costs more than it saves and the waves share out the tile (4096x8192x2047 171 us, with WAVES_K 191).
