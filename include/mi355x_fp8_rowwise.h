@@ -273,14 +273,15 @@ int mi355x_fp8_rowwise_grouped_form(int64_t G, int64_t M, int64_t N, int64_t K);
 
 /* The form a call of the GENERIC family runs in one piece (where K is cut, see the size query, its parts are tiles of
  * their own), or a negative status. Pure host arithmetic, for tests and timing audits. STREAM: a workgroup streams 16 or 32 rows of
- * B; TILES_<rows>[x<columns>]: tiles whose waves share out the tile, with _K each step's K. */
+ * B; TILES_<rows>[x<columns>]: tiles whose waves share out the tile, with _K each step's K. `dwords`: whether all rows of A and of B start on 4 bytes. */
 #define MI355X_FP8_GENERIC_STREAM         0
 #define MI355X_FP8_GENERIC_TILES_64_K     1
 #define MI355X_FP8_GENERIC_TILES_128X64_K 2
 #define MI355X_FP8_GENERIC_TILES_128_K    3
 #define MI355X_FP8_GENERIC_TILES_128      4
 #define MI355X_FP8_GENERIC_TILES_64       5
-int mi355x_fp8_rowwise_generic_form(int64_t M, int64_t N, int64_t K);
+#define MI355X_FP8_GENERIC_TILES_128X64   6  /* (with `dwords` only) */
+int mi355x_fp8_rowwise_generic_form(int64_t M, int64_t N, int64_t K, int dwords);
 
 /*
  * Block-scaled form: one scale per 128x128 block of A and of B,

@@ -1,5 +1,5 @@
-"""Tiles of the generic family on rows that start at each byte of a dword: the bytes are fetched in whole dwords and moved into place, so
-what lies in front of, between and behind the rows must not show. Each form of the tiles, K at both ends of a 128-byte step."""
+"""Tiles of the generic family on rows that start at each byte of a dword: the bytes are fetched in whole dwords and, where not all rows start on
+one, moved into place, so what lies in front of, between and behind the rows must not show. Each form of the tiles, K at both ends of a 128-byte step."""
 import pytest
 import torch
 
@@ -17,10 +17,30 @@ FORMS = {
 }
 
 
+# where all rows start on a dword: 64x64, 128x64 and 128x128 tiles whose waves share out K, then 128x128, 64x64 and 128x64 whose waves share out the tile
+FORMS_ON_DWORDS = {
+    **{f: FORMS[f] for f in (_lib.GENERIC_TILES_64_K, _lib.GENERIC_TILES_128X64_K, _lib.GENERIC_TILES_128, _lib.GENERIC_TILES_64)},
+    _lib.GENERIC_TILES_128_K: [(193, 13249, 640), (193, 13249, 641), (193, 13249, 767)],
+    _lib.GENERIC_TILES_128X64: [(745, 5384, 640), (745, 5384, 641), (745, 5384, 767)],
+}
+
+
 @pytest.mark.parametrize("m,n,k,form", [(*s, form) for form, shapes in FORMS.items() for s in shapes])
 @pytest.mark.parametrize("shift,pitch", [(1, 0), (2, 3), (3, 2), (0, 1)])
 def test_rows_at_any_byte(gpu_device, m, n, k, form, shift, pitch):
-    assert _lib.load().mi355x_fp8_rowwise_generic_form(m, n, k) == form
+    if shift or (k + pitch) % 4:
+        assert _lib.load().mi355x_fp8_rowwise_generic_form(m, n, k, 0) == form
+    _check(gpu_device, m, n, k, shift, pitch)
+
+
+@pytest.mark.parametrize("m,n,k,form", [(*s, form) for form, shapes in FORMS_ON_DWORDS.items() for s in shapes])
+@pytest.mark.parametrize("shift,pad", [(0, 0), (4, 4), (8, 20)])
+def test_rows_on_dwords(gpu_device, m, n, k, form, shift, pad):
+    assert _lib.load().mi355x_fp8_rowwise_generic_form(m, n, k, 1) == form
+    _check(gpu_device, m, n, k, shift, -k % 4 + pad)
+
+
+def _check(gpu_device, m, n, k, shift, pitch):
     assert _lib.load().mi355x_fp8_rowwise_workspace_bytes(m, n, k, _lib.VARIANT_GENERIC) == 0  # (in one piece)
     print(f"case m={m} n={n} k={k} shift={shift} pitch={pitch}", flush=True)
     g = torch.Generator(device=gpu_device).manual_seed(m + n + k)

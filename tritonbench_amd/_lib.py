@@ -107,7 +107,7 @@ SIGNATURES = {
          c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p],
     ),
     "mi355x_fp8_rowwise_grouped_form": (c_int, [c_int64, c_int64, c_int64, c_int64]),
-    "mi355x_fp8_rowwise_generic_form": (c_int, [c_int64, c_int64, c_int64]),
+    "mi355x_fp8_rowwise_generic_form": (c_int, [c_int64, c_int64, c_int64, c_int]),
     "mi355x_fp8_blockwise_form": (c_int, [c_int64, c_int64, c_int64]),
     "mi355x_fp8_blockwise_gemm_ex": (
         c_int,
@@ -145,7 +145,8 @@ _lib = None
 # forms of the block-scaled and of the grouped product, as the library names them
 BLOCK_ONE_TILE, BLOCK_NARROW, BLOCK_TILES_128, BLOCK_TILES_128_STREAM, BLOCK_TILES_256 = range(5)
 BLOCK_RESIDENT = 6
-(GENERIC_STREAM, GENERIC_TILES_64_K, GENERIC_TILES_128X64_K, GENERIC_TILES_128_K, GENERIC_TILES_128, GENERIC_TILES_64) = range(6)
+(GENERIC_STREAM, GENERIC_TILES_64_K, GENERIC_TILES_128X64_K, GENERIC_TILES_128_K, GENERIC_TILES_128, GENERIC_TILES_64,
+ GENERIC_TILES_128X64) = range(7)
 GROUPED_TILES, GROUPED_ROWS_16, GROUPED_ROWS_32, GROUPED_ROWS_64, GROUPED_STREAM_128, GROUPED_STREAM_256 = range(6)
 
 

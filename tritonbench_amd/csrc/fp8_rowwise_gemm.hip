@@ -1810,6 +1810,9 @@ __device__ __forceinline__ v8h e4m3fn_to_f16x8(int lo, int hi) {
 // 16 or 4 bytes 83 bytes/ns, on 2 bytes 64, on odd ones 49). The last dword of the chunk in front, which a row that starts
 // off the dwords needs too, is in the lane beside it or was in the step before (a load of its own for it cost more than it gained:
 // 128x8192x8191 33.4 -> 43.0 us). Without that 1000x3000x4111 takes 47.9 us, 517x3000x1041 15.6.
+// DWORDS: rows that all start on a dword lie in place already: their chunks go into LDS as they are (64x64 tiles 0.89 of the time on average with waves that
+// share out K and 0.95 with waves that share out the tile, 128x64 0.97 and 0.90, 128x128 0.98 and 0.96; 423 shapes. Moved like the others, 152x24457x820 took
+// 26.4 us where 22.4 are had).
 constexpr size_t any_stage_bytes(int BM, int BN, int WAVES_K, int WAVES_MN) {
   const size_t stages = (size_t)2 * (BM + BN) * kStepK, sums = (size_t)WAVES_MN * WAVES_K * (WAVES_K - 1) * 32 * 32 * 4;
   return stages > sums ? stages : sums;
@@ -1818,7 +1821,7 @@ constexpr size_t any_lds_bytes(int BM, int BN, int WAVES_K, int WAVES_MN) { retu
 
 // PARTIAL: K in p.splits parts of p.steps_per_split steps, each an item of its own that leaves its sums in its plane of p.partial
 // for the second pass. The last part has the partial step.
-template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int DEPTH, bool PARTIAL>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int DEPTH, bool PARTIAL, bool DWORDS>
 __global__ __launch_bounds__(WAVES_M* WAVES_N* WAVES_K * 64) void gemm_any_kernel(GemmParams p) {
   constexpr int THREADS = WAVES_M * WAVES_N * WAVES_K * 64;
   constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N, MT = WTM / 32, NT = WTN / 32;
@@ -1853,7 +1856,7 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* WAVES_K * 64) void gemm_any_kerne
   const bool has_tail = !PARTIAL || part == p.splits - 1;
 
   // Lane's chunk ld_c of rows ld_row, ld_row + ROWS, ... (rows past an edge repeat the last one).
-  // The bytes of a step are fetched as the whole dwords behind the one that its first byte lies in, and moved into place when
+  // The bytes of a step are fetched as the whole dwords behind the one that its first byte lies in (DWORDS: from that one on), and moved into place when
   // they are parked: a chunk begins in the last dword of the chunk in front of it, the lane's beside it, or the step's before.
   // (Every dword that is fetched holds bytes of its row: the first one byte 0, the last one byte 128 * whole.)
   const int ld_row = tid >> 3, ld_c = tid & 7;
@@ -1866,9 +1869,9 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* WAVES_K * 64) void gemm_any_kerne
   for (int i = 0; i < LOADS; ++i) {
     const int r = ld_row + ROWS * (i < LA ? i : i - LA);
     row[i] = i < LA ? p.a + (size_t)min(m0 + r, (long)p.M - 1) * p.lda : p.b + (size_t)min(n0 + r, (long)p.N - 1) * p.ldb;
-    shift[i] = (uint32_t)(reinterpret_cast<uintptr_t>(row[i]) & 3);
-    at[i] = row[i] - shift[i] + (long)first * kStepK + ld_c * kChunk + 4;
-    before[i] = full > 0 ? *(const int*)(row[i] - shift[i] + (long)first * kStepK) : 0;
+    shift[i] = DWORDS ? 0 : (uint32_t)(reinterpret_cast<uintptr_t>(row[i]) & 3);
+    at[i] = row[i] - shift[i] + (long)first * kStepK + ld_c * kChunk + (DWORDS ? 0 : 4);
+    before[i] = !DWORDS && full > 0 ? *(const int*)(row[i] - shift[i] + (long)first * kStepK) : 0;
   }
   // the factors and the bias of the tile's rows and columns, which wait in LDS behind the stages for the end
   uint8_t* const ends = lds + any_stage_bytes(BM, BN, WAVES_K, WAVES_M * WAVES_N);
@@ -1905,6 +1908,10 @@ __global__ __launch_bounds__(WAVES_M* WAVES_N* WAVES_K * 64) void gemm_any_kerne
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       const v4i x = from[i];
+      if constexpr (DWORDS) {
+        park_one(x, i, stage);
+        continue;
+      }
       // the lane beside it; for the first of a row's eight lanes the last one's of the step before
       const int left = __builtin_amdgcn_update_dpp(0, x[3], 0x111, 0xf, 0xf, true);       // row_shr:1
       const int back = __builtin_amdgcn_update_dpp(0, before[i], 0x141, 0xf, 0xf, true);  // row_half_mirror
@@ -4686,10 +4693,10 @@ int launch_block_form(GemmParams p, hipStream_t stream) {
 }
 int launch_block(const GemmParams& p, hipStream_t s) { return p.K % kStepK ? launch_block_form<true>(p, s) : launch_block_form<false>(p, s); }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int DEPTH, bool PARTIAL = false>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int WAVES_K, int DEPTH, bool PARTIAL, bool DWORDS>
 int launch_any(GemmParams p, hipStream_t stream) {
   constexpr size_t lds_bytes = any_lds_bytes(BM, BN, WAVES_K, WAVES_M * WAVES_N);
-  constexpr auto kern = gemm_any_kernel<BM, BN, WAVES_M, WAVES_N, WAVES_K, DEPTH, PARTIAL>;
+  constexpr auto kern = gemm_any_kernel<BM, BN, WAVES_M, WAVES_N, WAVES_K, DEPTH, PARTIAL, DWORDS>;
   (void)LdsLimit<kern, lds_bytes>::registered;
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
@@ -4715,37 +4722,46 @@ constexpr bool generic_streams(int64_t M, int64_t N, int64_t K) {
   return !(K <= (M <= 16 ? 128 : 256) && N > (M <= 32 ? 8192 : 4096));
 }
 static_assert(!generic_streams(1, 1 << 27, 1024) && generic_streams(1, (1 << 27) - 16, 1024), "2^27 columns are 2^32 lanes");
-// Tiles of a launch above 64 rows, estimated from launches of 1 to 70 rounds of the CUs (180 shapes, 65 to 12000 rows, K 100 to 16000): what
+// Tiles of a launch above 64 rows, estimated from launches of 1 to 70 rounds of the CUs (1297 shapes, 65 to 8192 rows, K 100 to 16000): what
 // starts and ends with the launch and with each tile, and the rounds of the CUs times a 128-byte step. Waves that share out K (64x64, 128x64 and 128x128
-// tiles) are ahead while the tiles are few rounds, waves that share out the tile (64x64 and 128x128) on short rows and over many rounds: us in that
+// tiles) are ahead while the tiles are few rounds, waves that share out the tile (128x128 and 64x64) on short rows and over many rounds: us in that
 // order 463x1440x2101 14.2, 17.0, 23.9, 31.4 and 18.6; 362x5040x4907 39.8, 35.0, 45.6, 63.5 and 42.4; 243x15469x7535 105.6, 96.7, 76.8, 97.0 and 106.3;
-// 707x19781x241 38.8, 51.8, 40.4, 33.1 and 35.8; 134x20332x519 19.9, 25.5, 26.0, 21.4 and 16.6. The quickest of the five is missed by 0.3 % on
-// average, and by more than 7 % on 3 of the 180.
-enum GenericTiles { kGeneric64Shared, kGeneric128x64Shared, kGeneric128Shared, kGeneric128, kGeneric64 };
+// 707x19781x241 38.8, 51.8, 40.4, 33.1 and 35.8; 134x20332x519 19.9, 25.5, 26.0, 21.4 and 16.6. Rows on dwords have a sixth form, 128x64 tiles that
+// the waves share out: 449x18784x3624 102.3, 107.4, 105.4, 105.2, 110.1 and 90.7; 152x24457x820 24.2, 28.2, 29.3, 23.9, 24.8 and 22.4. (Off the dwords it is
+// never the quickest by more than noise.) The quickest is missed by 0.4 % on average off the dwords and by 0.5 % on them, and by more than 7 % on 4 of 674
+// and 11 of 623. (With constants from 180 shapes for either 0.8 and 1.3 %: 210x193x356 8.04 us on 128x64, 6.60 on 64x64.)
+enum GenericTiles { kGeneric64Shared, kGeneric128x64Shared, kGeneric128Shared, kGeneric128, kGeneric64, kGeneric128x64 };
 static_assert(kGeneric64Shared + 1 == MI355X_FP8_GENERIC_TILES_64_K && kGeneric128x64Shared + 1 == MI355X_FP8_GENERIC_TILES_128X64_K &&
               kGeneric128Shared + 1 == MI355X_FP8_GENERIC_TILES_128_K && kGeneric128 + 1 == MI355X_FP8_GENERIC_TILES_128 &&
-              kGeneric64 + 1 == MI355X_FP8_GENERIC_TILES_64, "the query's names, behind the streaming form's");
+              kGeneric64 + 1 == MI355X_FP8_GENERIC_TILES_64 && kGeneric128x64 + 1 == MI355X_FP8_GENERIC_TILES_128X64, "the query's names, behind the streaming form's");
 struct GenericChoice {
   GenericTiles tiles;
   float us;
 };
-inline GenericChoice generic_tiles(int64_t M, int64_t N, int64_t K) {
-  auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  auto rounds = [](int64_t tiles, int64_t slots) { return (float)((tiles + slots - 1) / slots); };
-  const int64_t t64 = tiles(64, 64), t128x64 = tiles(128, 64), t128 = tiles(128, 128);
+struct GenericCost {
+  int bm, bn, lanes, slots;  // slots: tiles of a round
+  float start, tile, step, alone;  // us: of a launch, of each tile, of a step of a round, of a step at least
+};
+inline GenericChoice generic_tiles(int64_t M, int64_t N, int64_t K, bool dwords) {
+  static const GenericCost any[] = {{64, 64, 256, kNumCu, 4.16f, 5.45e-3f, 0.433f, 0.0f},     {128, 64, 512, kNumCu, 3.64f, 9.56e-3f, 0.771f, 0.0f},
+                                    {128, 128, 512, kNumCu, 3.86f, 21.1e-3f, 1.135f, 0.0f},    {128, 128, 256, 2 * kNumCu, 4.32f, 17.9e-3f, 1.682f, 0.0f},
+                                    {64, 64, 256, kNumCu, 1.85f, 5.15e-3f, 0.385f, 1.371f}};
+  static const GenericCost on_dwords[] = {{64, 64, 256, kNumCu, 3.86f, 3.28e-3f, 0.443f, 0.0f},  {128, 64, 512, kNumCu, 3.72f, 11.3e-3f, 0.629f, 0.0f},
+                                          {128, 128, 512, kNumCu, 3.85f, 16.7e-3f, 1.086f, 0.0f}, {128, 128, 256, 2 * kNumCu, 5.06f, 12.1e-3f, 1.787f, 0.0f},
+                                          {64, 64, 256, kNumCu, 1.81f, 4.46e-3f, 0.380f, 1.123f}, {128, 64, 256, kNumCu, 5.38f, 5.36e-3f, 0.568f, 0.769f}};
+  const GenericCost* const forms = dwords ? on_dwords : any;
   const float steps = (float)k_steps_of(K);
-  // (workgroups of 256 or 512 lanes: a launch takes fewer than 2^32 lanes)
-  const float us[] = {grid_fits(t64, 256) ? 4.4f + 7.05e-3f * (float)t64 + steps * 0.40f * rounds(t64, kNumCu) : 1e30f,
-                      grid_fits(t128x64, 512) ? 4.0f + 15.3e-3f * (float)t128x64 + steps * 0.53f * rounds(t128x64, kNumCu) : 1e30f,
-                      grid_fits(t128, 512) ? 6.3f + 23.3e-3f * (float)t128 + steps * 0.89f * rounds(t128, kNumCu) : 1e30f,
-                      5.4f + 22.9e-3f * (float)t128 + steps * 1.39f * rounds(t128, 2 * kNumCu),
-                      grid_fits(t64, 256) ? 3.2f + 6.0e-3f * (float)t64 + steps * fmaxf(0.90f, 0.37f * rounds(t64, kNumCu)) : 1e30f};
+  auto us = [&](int form) {
+    const GenericCost& c = forms[form];
+    const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+    if (form != kGeneric128 && !grid_fits(tiles, c.lanes)) return 1e30f;  // (a launch takes fewer than 2^32 lanes)
+    return c.start + c.tile * (float)tiles + steps * fmaxf(c.alone, c.step * (float)((tiles + c.slots - 1) / c.slots));
+  };
   // (one step, or one row of tiles: nothing to gain from the larger tiles, 164x39275x3 21.6 us with 128x128, 14.0 with 64x64)
-  GenericChoice best = {(M <= kSkinnyMaxM || K <= kStepK) && us[kGeneric64] < 1e30f ? kGeneric64 : kGeneric128, 1e30f};
-  best.us = us[best.tiles];
-  if (best.tiles == kGeneric128)
-    for (int f = kGeneric64Shared; f <= kGeneric64; ++f)
-      if (us[f] < best.us) best = {(GenericTiles)f, us[f]};
+  if ((M <= kSkinnyMaxM || K <= kStepK) && us(kGeneric64) < 1e30f) return {kGeneric64, us(kGeneric64)};
+  GenericChoice best = {kGeneric128, us(kGeneric128)};
+  for (int f = kGeneric64Shared; f <= (dwords ? kGeneric128x64 : kGeneric64); ++f)
+    if (us(f) < best.us) best = {(GenericTiles)f, us(f)};
   return best;
 }
 
@@ -4759,7 +4775,7 @@ inline GenericPlan generic_plan(int64_t M, int64_t N, int64_t K, int max_splits)
   GenericPlan best = {1, k_steps};
   const int64_t tiles_64 = ((M + 63) / 64) * ((N + 63) / 64), tiles = ((M + 127) / 128) * ((N + 63) / 64);
   if (generic_streams(M, N, K) || tiles_64 >= kNumCu) return best;
-  float cost = generic_tiles(M, N, K).us;
+  float cost = generic_tiles(M, N, K, K % 4 == 0).us;  // (by the sizes alone, like the query)
   for (int want = 2; want <= max_splits && tiles * want <= kNumCu; ++want) {
     int splits, sps;
     normalise_splits(k_steps, want, splits, sps);
@@ -4776,22 +4792,30 @@ inline GenericPlan generic_plan(int64_t M, int64_t N, int64_t K, int max_splits)
 // The generic family: the streaming kernel's unaligned form up to 64 rows but for short rows on wide panels (measured cold: 1x8192x8191 14.4 us,
 // 16x8192x8191 19.1, 64x8192x8191 29.7, where 64x64 tiles take 33), tiles beyond. Tiles whose waves share out K run two steps ahead
 // (61.1 -> 41.8 us on 128x8192x8191), the others, of which a CU has several, one.
+template <bool DWORDS>
+int launch_generic_tiles(const GemmParams& p, hipStream_t s) {
+  switch (generic_tiles(p.M, p.N, p.K, DWORDS).tiles) {
+    case kGeneric64Shared: return launch_any<64, 64, 1, 1, 4, 2, false, DWORDS>(p, s);
+    case kGeneric128x64Shared: return launch_any<128, 64, 2, 1, 4, 2, false, DWORDS>(p, s);
+    case kGeneric128Shared: return launch_any<128, 128, 2, 1, 4, 2, false, DWORDS>(p, s);
+    case kGeneric64: return launch_any<64, 64, 2, 2, 1, 1, false, DWORDS>(p, s);
+    case kGeneric128x64:
+      if constexpr (DWORDS) return launch_any<128, 64, 2, 2, 1, 1, false, true>(p, s);
+      [[fallthrough]];
+    default: return launch_any<128, 128, 2, 2, 1, 1, false, DWORDS>(p, s);
+  }
+}
 int launch_generic(const GemmParams& p, hipStream_t s) {
   // (the documented range of the family, which the tests' sizes lie in)
   if (p.M > 65535 * 64) return fail(MI355X_FP8_ENOTSUP, "the generic family takes M <= %d", 65535 * 64);
-  if (p.splits > 1) return launch_any<128, 64, 2, 1, 4, 2, true>(p, s);
+  const bool dwords = ((reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.b) | (uintptr_t)p.lda | (uintptr_t)p.ldb) & 3) == 0;
+  if (p.splits > 1) return dwords ? launch_any<128, 64, 2, 1, 4, 2, true, true>(p, s) : launch_any<128, 64, 2, 1, 4, 2, true, false>(p, s);
   if (generic_streams(p.M, p.N, p.K)) {
     if (p.M <= 16) return launch_skinny<1, 1, 4, 8, true>(p, s);
     if (p.M <= 32) return launch_skinny<2, 1, 2, 8, true>(p, s);
     return launch_skinny<4, 2, 2, 8, true>(p, s);
   }
-  switch (generic_tiles(p.M, p.N, p.K).tiles) {
-    case kGeneric64Shared: return launch_any<64, 64, 1, 1, 4, 2>(p, s);
-    case kGeneric128x64Shared: return launch_any<128, 64, 2, 1, 4, 2>(p, s);
-    case kGeneric128Shared: return launch_any<128, 128, 2, 1, 4, 2>(p, s);
-    case kGeneric64: return launch_any<64, 64, 2, 2, 1, 1>(p, s);
-    default: return launch_any<128, 128, 2, 2, 1, 1>(p, s);
-  }
+  return dwords ? launch_generic_tiles<true>(p, s) : launch_generic_tiles<false>(p, s);
 }
 
 // ---- built-in scratch of the entry point that allocates nothing
@@ -5486,10 +5510,10 @@ int mi355x_fp8_rowwise_grouped_form(int64_t G, int64_t M, int64_t N, int64_t K) 
   return grouped_form(G, M, N, K, K);
 }
 
-int mi355x_fp8_rowwise_generic_form(int64_t M, int64_t N, int64_t K) {
+int mi355x_fp8_rowwise_generic_form(int64_t M, int64_t N, int64_t K, int dwords) {
   const int st = check_shape(M, N, K);
   if (st != MI355X_FP8_OK) return st;
-  return generic_streams(M, N, K) ? MI355X_FP8_GENERIC_STREAM : generic_tiles(M, N, K).tiles + 1;
+  return generic_streams(M, N, K) ? MI355X_FP8_GENERIC_STREAM : generic_tiles(M, N, K, dwords != 0).tiles + 1;
 }
 
 int mi355x_fp8_blockwise_form(int64_t M, int64_t N, int64_t K) {
