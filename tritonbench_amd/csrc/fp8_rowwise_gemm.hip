@@ -4588,13 +4588,14 @@ inline float block_one_tile_cost_us(int64_t M, int64_t N, int64_t K, float off_l
   return fmaxf(off_lines * one_tile_cost_us(M, N, K), 3.0f + (wgs > kNumCu ? (float)(wgs - kNumCu) * per_wg : 0.0f));
 }
 // The form that keeps A on chip against its row-wise estimate, with one tile a workgroup as it is. One tile a CU: off the lines it is behind by more
-// the more rows of A and the longer K, and with up to 4 rows its start shows. Two: it is behind off the lines and where its second round of
-// steps begins. (2420 shapes, weights from HBM: 0.998 of the time without this form on average, 1 % of them more than 2 % behind; by the
-// row-wise estimate alone 1.000 and 5 %, 16x2528x3264 5.47 -> 6.08 us, 4x5376x3584 6.49 -> 7.08, 8x1088x4592 5.51 -> 6.07. What it
-// is for: 16x8192x8192 14.1 -> 13.1, 16x8192x3600 9.88 -> 8.80, 16x512x5936 7.53 -> 7.14.)
+// the more rows of A and the longer K, and with up to 4 rows its start shows. Two: it is behind off the lines, most on long rows (2x4368x7616
+// 11.3 us, on narrow tiles 10.3), and where its second round of steps begins. (2420 shapes, weights from HBM: 0.998 of the time without this form on
+// average, 1 % of them more than 2 % behind; by the row-wise estimate alone 1.000 and 5 %, 16x2528x3264 5.47 -> 6.08 us, 4x5376x3584 6.49 -> 7.08,
+// 8x1088x4592 5.51 -> 6.07. What it is for: 16x8192x8192 14.1 -> 13.1, 16x8192x3600 9.88 -> 8.80, 16x512x5936 7.53 -> 7.14.)
 inline float block_resident_factor(int64_t M, int64_t N, int64_t K, bool off_lines) {
   if (N <= 16 * kNumCu) return (off_lines ? 1.07f + 1.1e-6f * (float)M * (float)K : 1.01f) + (M <= 4 ? 0.08f : 0.0f);
   if (M > 8) return off_lines ? 1.2f : K > 4096 ? 1.0f : 1.09f;
+  if (off_lines && K > 4096) return 1.17f;
   return (off_lines ? 1.07f : 1.01f) * (K > 2048 && K <= 4096 ? 1.08f : 1.0f);
 }
 inline BlockForm block_form(int64_t M, int64_t N, int64_t K, bool off_lines, float* cost_us = nullptr) {
