@@ -5304,12 +5304,16 @@ constexpr RowForm row_form(RowSource source, int64_t R, int64_t chunks) {
     return {1024, (int)((chunks + 1023) / 1024)};
   }
   const bool many = R > 2048;
+  if (source == kRowBf16 && chunks <= 192 && R <= 1024) return {256, 1};  // (512 rows of 1536 3.07 us, in waves 3.67; 2048 4.91 and 4.96)
   if (chunks <= 192) return {64, chunks <= 128 ? 2 : 3};
   if (chunks <= 256) return many ? RowForm{64, 4} : RowForm{256, 1};
   if (chunks <= 512) return many && source == kRowF32 ? RowForm{64, chunks <= 384 ? 6 : 8} : RowForm{256, 2};
   if (chunks <= 768) return {256, 3};
-  if (chunks <= 1024) return many ? RowForm{256, 4} : RowForm{512, 2};
-  if (chunks <= 1280 && many) return {256, 5};
+  // (The quantiser: 2048 rows of 4096 f32 8.26 us as 256x4, 8.88 as 512x2, 1024 rows level; 8192 rows 28.8 and 27.5, of 3584 the other way
+  // round. 2048 rows of 5120 f32 9.8 as 256x5, 10.4 as 512x3, 8192 35.2 and 34.1; bf16 keeps 256x5, 8192 of 8960 40.7 and 42.6.)
+  if (source == kRowF32 && chunks > 960 && chunks <= 1024 && R > 4096) return {512, 2};
+  if (chunks <= 1024) return many || (source != kRowSiluMul && R > 1024) ? RowForm{256, 4} : RowForm{512, 2};
+  if (chunks <= 1280 && (many || (source == kRowF32 && R > 1024)) && !(source == kRowF32 && chunks > 1216 && R > 4096)) return {256, 5};
   if (chunks <= 3072) return {512, (int)((chunks + 511) / 512)};
   if (source == kRowSiluMul) return {1024, 4};
   return {512, chunks <= 3584 ? 7 : 8};
@@ -5323,7 +5327,7 @@ void launch_by_rows(int64_t R, int64_t lanes, Launch&& launch) {
 constexpr bool row_forms_are_sound() {  // (the rule's lines lie at multiples of 64 chunks)
   for (int source = kRowF32; source <= kRowSiluMul; ++source) {
     bool chosen[17][9] = {};  // by 64 lanes and rounds
-    for (int64_t R : {int64_t(1), int64_t(kNumCu), int64_t(kNumCu + 1), int64_t(2048), int64_t(2049)})
+    for (int64_t R : {int64_t(1), int64_t(kNumCu), int64_t(kNumCu + 1), int64_t(1024), int64_t(1025), int64_t(2048), int64_t(2049), int64_t(4096), int64_t(4097)})
       for (int64_t chunks = 64; chunks <= 8192; chunks += 64)
         for (int64_t c : {chunks, chunks + 1}) {
           const RowForm f = row_form((RowSource)source, R, c);
